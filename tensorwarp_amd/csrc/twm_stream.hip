@@ -17,6 +17,8 @@
 // tile and group).
 #include "twm_device.h"
 
+#include <type_traits>
+
 namespace twm {
 
 namespace {
@@ -248,18 +250,42 @@ __global__ __launch_bounds__(WAVES * 64) void k_stream(const uint4v *__restrict_
 // f32 row keeps about 21 bits per value relative to the row's largest, as the reference's f32 product would; in range
 // s = 0 and nothing changes), and row_scale[row] = 2^s, which the GEMM's store multiplies the row's sums by (exact).
 // TWO = false: the one rounded term only (the prefill GEMM's operand).
-template <bool TWO>
+// Bound: latency with few rows, HBM with many.  A thread holds its NV 16-byte pieces of the row in registers between the
+// maximum and the conversion (NV > 0: k <= 4096 NV), so the row is read once, all of it in flight at once, and written
+// 8 bytes at a time; NV = 0 reads the row twice, for any k.  (Against a scalar loop that read the row twice: a down
+// projection 18944 -> 3584 with its conversion at 8 rows 27.4 -> 21.8 us, at 32 rows 37.9 -> 31.6; 2048 x 11008 rows,
+// 90 MB in and 45 MB out, about 7 us of the layer less.)
+template <bool TWO, int NV>
 __global__ __launch_bounds__(1024) void k_f32_rows_to_f16(const float *__restrict__ a, _Float16 *__restrict__ hi,
                                                            _Float16 *__restrict__ lo, float *__restrict__ row_scale, uint32_t k)
 {
+    typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+    constexpr int kHeld = NV > 0 ? NV : 1;
     __shared__ float s_max[16];
-    const float *src = a + (size_t)blockIdx.x * k;
+    const size_t row0 = (size_t)blockIdx.x * k;
+    const float4v *src = (const float4v *)(a + row0);
+    const uint32_t quads = k >> 2;  // k is a multiple of 32, rows are 16-byte aligned
+    float4v v[kHeld];
     float m = 0.f;
     bool odd = false;  // an infinity or a NaN in the row
-    for (uint32_t i = threadIdx.x; i < k; i += 1024u) {
-        const float v = fabsf(src[i]);
-        odd = odd || !(v <= 3.4028234e38f);
-        m = fmaxf(m, v);
+    auto look = [&](const float4v &x) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float f = fabsf(x[j]);
+            odd = odd || !(f <= 3.4028234e38f);
+            m = fmaxf(m, f);
+        }
+    };
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const uint32_t q = threadIdx.x + 1024u * i;
+            v[i] = src[q < quads ? q : quads - 1u];
+        }
+#pragma unroll
+        for (int i = 0; i < NV; i++) look(v[i]);
+    } else {
+        for (uint32_t q = threadIdx.x; q < quads; q += 1024u) look(src[q]);
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
@@ -276,12 +302,26 @@ __global__ __launch_bounds__(1024) void k_f32_rows_to_f16(const float *__restric
         back = __uint_as_float((e - 13u) << 23);              // 2^((e - 127) - 13)
     }
     if (threadIdx.x == 0) row_scale[blockIdx.x] = back;
-    _Float16 *dh = hi + (size_t)blockIdx.x * k, *dl = TWO ? lo + (size_t)blockIdx.x * k : nullptr;
-    for (uint32_t i = threadIdx.x; i < k; i += 1024u) {
-        const float v = src[i] * down;
-        const _Float16 h = (_Float16)v;
-        dh[i] = h;
-        if (TWO) dl[i] = (_Float16)(v - (float)h);
+    half4v *dh = (half4v *)(hi + row0), *dl = TWO ? (half4v *)(lo + row0) : nullptr;
+    auto convert = [&](uint32_t q, const float4v &x) {
+        half4v h, l;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float f = x[j] * down;
+            h[j] = (_Float16)f;
+            l[j] = (_Float16)(f - (float)h[j]);
+        }
+        dh[q] = h;
+        if (TWO) dl[q] = l;
+    };
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const uint32_t q = threadIdx.x + 1024u * i;
+            if (q < quads) convert(q, v[i]);
+        }
+    } else {
+        for (uint32_t q = threadIdx.x; q < quads; q += 1024u) convert(q, src[q]);
     }
 }
 
@@ -289,8 +329,16 @@ hipError_t launch_f32_rows_to_f16(hipStream_t s, const float *a, _Float16 *hi, _
                                   uint32_t k)
 {
     if (rows == 0 || k == 0) return hipSuccess;
-    if (lo) hipLaunchKernelGGL(k_f32_rows_to_f16<true>, dim3(rows), dim3(1024), 0, s, a, hi, lo, row_scale, k);
-    else hipLaunchKernelGGL(k_f32_rows_to_f16<false>, dim3(rows), dim3(1024), 0, s, a, hi, lo, row_scale, k);
+    auto go = [&](auto nv) {
+        constexpr int NV = decltype(nv)::value;
+        if (lo) hipLaunchKernelGGL((k_f32_rows_to_f16<true, NV>), dim3(rows), dim3(1024), 0, s, a, hi, lo, row_scale, k);
+        else hipLaunchKernelGGL((k_f32_rows_to_f16<false, NV>), dim3(rows), dim3(1024), 0, s, a, hi, lo, row_scale, k);
+    };
+    if (k <= 4096u) go(std::integral_constant<int, 1>{});
+    else if (k <= 4096u * 3) go(std::integral_constant<int, 3>{});
+    else if (k <= 4096u * 5) go(std::integral_constant<int, 5>{});
+    else if (k <= 4096u * 8) go(std::integral_constant<int, 8>{});
+    else go(std::integral_constant<int, 0>{});
     return hipGetLastError();
 }
 

@@ -1,0 +1,49 @@
+"""GPU tests of single kernels at the sizes where their tilings change: against the CPU oracle's f64 dequant-then-matmul or
+its byte-exact format functions, through the C ABI."""
+import numpy as np
+import pytest
+
+import tensorwarp_amd as T
+from oracle import twm_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = T.WarpDevice(0)
+    yield d
+    d.close()
+
+
+def weight(dev, k, n, seed):
+    packed, scales = O.synth_packed(k, n, seed), O.synth_scales(k, n, seed + 1)
+    return packed, scales, T.MarlinWeight.upload(dev, packed, scales, k, n)
+
+
+def close_rows(got, truth, bar):
+    """Every row of `got` within `bar` of the truth, relative to max(|t|, 1e-3 of the row's largest)."""
+    assert np.isfinite(got).all()
+    for r in range(len(truth)):
+        floor = 1e-3 * np.abs(truth[r]).max() + 1e-300
+        err = (np.abs(got[r].astype(np.float64) - truth[r]) / np.maximum(np.abs(truth[r]), floor)).max()
+        assert err < bar, (r, err)
+
+
+# f32 sums of K products: K * 2^-24 relative to the sum of magnitudes at worst, 2e-4 of the floor above in practice
+F32_SUM = 2e-4
+
+
+@pytest.mark.parametrize("k", [32, 4096, 4128, 12288, 12320, 20512, 32800])
+def test_f32_row_conversion_at_the_edges_of_its_register_tiers(dev, k):
+    # rows of 4096, 12288, 20480 and 32768 values are the most that one, three, five and eight pieces per thread hold
+    m, n = 6, 24
+    packed, scales, w = weight(dev, k, n, 77 + k)
+    rows = O.synth_normal_f32(m * k, 7 + k).reshape(m, k).copy()
+    rows[1] *= np.float32(1e7)
+    rows[2, k - 1] = np.float32(3e6)      # the row's largest value is its last
+    rows[3] *= np.float32(1e-8)
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    T.gemm(dev, w, T.GpuTensor.from_host(dev, rows), m, c)
+    close_rows(c.to_host(), O.gemm_f64(rows, packed, scales, m, k, n), F32_SUM)
+    w.free()
