@@ -355,8 +355,8 @@ int twm_gemm_split(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_d
 /* twm_gemm with f16 result rows: c_dev_f16[M][N] = f16_rne(the f32 result of twm_gemm).  The reference's decode buffers
  * are f32 (generate.rs:1382-1404) and its FP16 pipeline keeps f16 rows (crates/kernels/src/fp16.rs:133-166 casts between
  * them); this entry point serves the second kind of caller without a buffer of its own: the kernels store f32 rows into
- * the back half of the context's scratch and the cast kernel rounds them into c_dev_f16, in row blocks when M x N x 4
- * bytes exceed that half (32 MB by default).  One more launch per block than twm_gemm, no allocation (capturable).
+ * the last 32 MB of the context's scratch and the cast kernel rounds them into c_dev_f16, in row blocks when M x N x 4
+ * bytes exceed that part.  One more launch per block than twm_gemm, no allocation (capturable).
  * TWM_MEMORY_ERROR when a single row of f32 results does not fit: call twm_gemm and twm_cast_f32_to_f16 instead. */
 int twm_gemm_f16out(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_dtype, uint32_t m, uint16_t *c_dev_f16,
                     uint32_t splits);

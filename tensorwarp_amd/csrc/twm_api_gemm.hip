@@ -719,7 +719,7 @@ int twm_gemm(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_dtype, 
 
 // twm_gemm with f16 result rows: the kernels store f32 (what the reference's buffers hold), so the rows are computed in
 // blocks into the back half of the context's scratch and rounded from there by the cast kernel -- no allocation, one
-// more launch per block; the front half stays the launch's own scratch (split-K sums, f32 activation terms).
+// more launch per block; the rest stays the launch's own scratch (split-K sums, f32 activation terms).
 int twm_gemm_f16out(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_dtype, uint32_t m, uint16_t *c_dev_f16,
                     uint32_t splits)
 {
@@ -729,16 +729,16 @@ int twm_gemm_f16out(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_
     if (m != 0 && w->n != 0 && !c_dev_f16) return api_fail(TWM_INVALID_HANDLE, "%s: null output", who);
     if (a_dtype != TWM_F16 && a_dtype != TWM_F32) return api_fail(TWM_UNSUPPORTED_OP, "%s: activations must be f16 or f32", who);
     if (m == 0 || w->n == 0) return TWM_OK;
-    const size_t row_bytes = (size_t)w->n * 4, half = (ctx->ws_bytes / 2) & ~(size_t)255;
-    if (!ctx->ws || row_bytes > half)
-        return api_fail(TWM_MEMORY_ERROR, "%s: one row of f32 results (%zu bytes) does not fit half of the context's scratch; "
+    const size_t row_bytes = (size_t)w->n * 4, staged = kF16OutBytes;
+    if (!ctx->ws || row_bytes > staged)
+        return api_fail(TWM_MEMORY_ERROR, "%s: one row of f32 results (%zu bytes) does not fit the staging part of the context's scratch; "
                         "use twm_gemm and twm_cast_f32_to_f16", who, row_bytes);
-    uint32_t block = half / row_bytes < m ? (uint32_t)(half / row_bytes) : m;
+    uint32_t block = staged / row_bytes < m ? (uint32_t)(staged / row_bytes) : m;
     if (block >= 128) block -= block % 128;   // (whole prefill row blocks)
-    float *stage = (float *)((char *)ctx->ws + ctx->ws_bytes - half);
+    float *stage = (float *)((char *)ctx->ws + ctx->ws_bytes - staged);
     const size_t a_row_bytes = (size_t)w->k * (a_dtype == TWM_F32 ? 4 : 2), saved = ctx->ws_bytes;
     int rc = TWM_OK;
-    ctx->ws_bytes = saved - half;
+    ctx->ws_bytes = saved - staged;
     for (uint32_t m0 = 0; m0 < m && rc == TWM_OK; m0 += block) {
         const uint32_t rows = m - m0 < block ? m - m0 : block;
         rc = twm_gemm(ctx, w, (const char *)a_dev + (size_t)m0 * a_row_bytes, a_dtype, rows, stage, splits);

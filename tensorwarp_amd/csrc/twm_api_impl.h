@@ -95,7 +95,11 @@ struct twm_graph {
     hipGraphExec_t exec;
 };
 
-constexpr size_t kWsBytes = 64ull << 20;    // split-K scratch of a context
+// Scratch of a context: split-K sums and the f16 terms of f32 rows.  256 MB of the card's 288 GB hold the terms of a
+// 2048 x 18944 prompt in one piece (with 64 MB a 2048 x 11008 one ran as 1408 + 640 rows, the
+// second part on split K: a LLaMA-7B layer at 2048 rows 816 us, now 793).
+constexpr size_t kWsBytes = 256ull << 20;
+constexpr size_t kF16OutBytes = 32ull << 20;  // its end, where twm_gemm_f16out stages f32 rows
 constexpr uint32_t kCounters = 1u << 16;     // arrival counters of a context
 
 // twm_api_weights.hip

@@ -413,16 +413,22 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_swiglu(const float *__res
     *(float4 *)(gate_out + (size_t)row * ffn + feat) = o;
 }
 
-// out[row][:] *= row_scale[row] over every segment, for the rows whose factor is not 1 (a workgroup per row; a row that
-// needs nothing costs its workgroup one load)
-__global__ __launch_bounds__(256) void k_scale_rows(OutSpec out, const float *__restrict__ row_scale)
+// out[row][:] *= row_scale[row] over every segment, for the rows whose factor is not 1.  Rows that need nothing are the
+// rule: a workgroup looks at the factors of kScaleRows rows with one load and usually ends there (2048 rows: 64 x 8
+// workgroups instead of one per row, whose launch alone was 5 us).
+constexpr uint32_t kScaleRows = 32, kScaleParts = 8;
+__global__ __launch_bounds__(256) void k_scale_rows(OutSpec out, const float *__restrict__ row_scale, uint32_t rows)
 {
-    const uint32_t row = blockIdx.x;
-    const float rs = row_scale[row];
-    if (rs == 1.f) return;
-    for (uint32_t sg = 0; sg < out.count && sg < (uint32_t)kMaxSegs; sg++) {
-        float *p = out.seg[sg].ptr + (size_t)row * out.seg[sg].width;
-        for (uint32_t c = threadIdx.x; c < out.seg[sg].width; c += 256u) p[c] *= rs;
+    const uint32_t row0 = blockIdx.x * kScaleRows, mine = row0 + (threadIdx.x & (kScaleRows - 1u));
+    const float own = mine < rows ? row_scale[mine] : 1.f;
+    uint32_t todo = (uint32_t)__builtin_amdgcn_ballot_w64(own != 1.f);  // (lanes 0 .. 31: the rows; 32 .. 63 repeat them)
+    for (; todo; todo &= todo - 1u) {
+        const uint32_t row = row0 + (uint32_t)__builtin_ctz(todo);
+        const float rs = row_scale[row];
+        for (uint32_t sg = 0; sg < out.count && sg < (uint32_t)kMaxSegs; sg++) {
+            float *p = out.seg[sg].ptr + (size_t)row * out.seg[sg].width;
+            for (uint32_t c = blockIdx.y * 256u + threadIdx.x; c < out.seg[sg].width; c += 256u * kScaleParts) p[c] *= rs;
+        }
     }
 }
 
@@ -611,7 +617,12 @@ hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, boo
     if (!scratch || scratch_bytes < row_bytes + 512) return hipErrorInvalidValue;
     uint32_t slab = (uint32_t)((scratch_bytes - 512) / 2 / row_bytes < m ? (scratch_bytes - 512) / 2 / row_bytes : m);
     if (slab == 0) slab = 1;
-    if (slab >= 128) slab -= slab % 128;
+    const uint32_t slabs = (m + slab - 1) / slab;
+    if (slab >= 128) {  // whole row blocks, the slabs of about equal height
+        slab -= slab % 128;
+        const uint32_t even = ((m + slabs - 1) / slabs + 127) / 128 * 128;
+        if (even < slab) slab = even;
+    }
     for (uint32_t r0 = 0; r0 < m; r0 += slab) {
         uint32_t rows = m - r0 < slab ? m - r0 : slab;
         float *row_scale = (float *)scratch;
@@ -630,7 +641,8 @@ hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, boo
                                                          scratch_bytes - used, false);
             const uint32_t cps = (w.k_chunks + plan.splits - 1) / plan.splits;
             if ((w.k_chunks + cps - 1) / cps == 1) {  // (with a K-split the sum kernel has applied the factors)
-                hipLaunchKernelGGL(k_scale_rows, dim3(rows), dim3(256), 0, s, o, (const float *)row_scale);
+                hipLaunchKernelGGL(k_scale_rows, dim3((rows + kScaleRows - 1) / kScaleRows, kScaleParts), dim3(256), 0, s, o,
+                                   (const float *)row_scale, rows);
                 e = hipGetLastError();
                 if (e != hipSuccess) return e;
             }

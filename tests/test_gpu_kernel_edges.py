@@ -47,3 +47,24 @@ def test_f32_row_conversion_at_the_edges_of_its_register_tiers(dev, k):
     T.gemm(dev, w, T.GpuTensor.from_host(dev, rows), m, c)
     close_rows(c.to_host(), O.gemm_f64(rows, packed, scales, m, k, n), F32_SUM)
     w.free()
+
+
+@pytest.mark.parametrize("m,k", [(33, 64), (65, 64), (160, 4128), (3600, 18944)])
+def test_scaled_f32_rows_of_a_prompt_in_one_and_two_slabs(dev, m, k):
+    # prompt rows outside the f16 range: the factors go back onto the sums 32 rows at a time (first, last and 32nd row of
+    # such a group among them); 3600 x 18944 rows do not fit the half of the scratch that holds their f16 terms
+    n, distinct = 72, 48
+    packed, scales, w = weight(dev, k, n, 500 + k)
+    base = O.synth_act_f16(distinct, k, 501).view(np.float16).astype(np.float32).reshape(distinct, k)
+    factor = np.ones(m, np.float32)
+    factor[[0, 31, 32, m // 2, m - 1]] = [2.0 ** 20, 2.0 ** -20, 2.0 ** 90, 2.0 ** 17, 2.0 ** -90]
+    rows = base[np.arange(m) % distinct] * factor[:, None]   # f16 values times powers of two: the f16 terms are exact
+    w16 = O.dequant_f16(packed, scales, k, n).view(np.float16).astype(np.float64).reshape(k, n)
+    truth = (base.astype(np.float64) @ w16)[np.arange(m) % distinct] * factor[:, None].astype(np.float64)
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    a = T.GpuTensor.from_host(dev, np.ascontiguousarray(rows))
+    T.gemm(dev, w, a, m, c)
+    close_rows(c.to_host(), truth, 1e-3)      # the prefill GEMM's bar: f32 sums over all of K inside the MFMAs
+    for t in (a, c):
+        t.free()
+    w.free()
