@@ -75,7 +75,7 @@ constexpr int kBtSlots = 4;
 // MT: 16-row blocks (1 or 2); TERMS: 1 = f16 activations, 2 = f32 activations as two f16 terms;
 // TPW: tiles per wave.  TPW = 1: the workgroup owns one quad of tiles (64 columns), wave w tile w.
 // TPW = 2: two quads (128 columns), wave w tiles (w & 1) and (w & 1) + 2 of quad w >> 1 -- in a paired gate/up
-// weight a gate tile and the up tile of the same features, which the gated store needs in one lane.
+// weight a gate tile and the up tile of the same features.
 // KS: k-slices per workgroup (1, 2, 4): the workgroup has 4 KS waves, slice s = wave / 4 takes the chunks s, s + KS, ...
 // of the workgroup's k-range with its own LDS buffers, and the slices' sums are added through LDS at the end -- more
 // waves per CU where the column quads alone are too few workgroups, without the partial-sum traffic of a K-split
@@ -316,6 +316,37 @@ __global__ __launch_bounds__(64 * WPS * KS) void k_batch(const uint4v *__restric
         }
         return;
     }
+    if constexpr (TPW == 1) {
+        if (out.swiglu) {
+            // paired gate/up weight, one tile per wave: tiles 0, 1 of a quad hold gate columns, tiles 2, 3 the up columns of
+            // the same features.  The waves of the up tiles hand their sums over through LDS (the staging buffers are idle)
+            // and the gate tiles' waves finish: the gated launch keeps the plain launch's form (3584 -> 2 x 18944 on three
+            // quads per workgroup instead of two tiles per wave, which put four quads on some CUs: 30.9 -> 26.2 us at 32
+            // rows, 22.0 -> 20.7 at 16; 4096 -> 2 x 11008 on two quads 22.5 -> 20.1 at 32).
+            if constexpr (KS > 1) __syncthreads();  // (slice 0 has read the other slices' sums)
+            float4v *handed = (float4v *)lds_all;   // [WPS / 2 waves][MT][64 lanes]
+            static_assert(WPS / 2 * MT * 1024 <= (int)sizeof(lds_all), "the up sums fit");
+            const uint32_t pair_of = (wave >> 2) * 2u + (wave & 1u);
+            if (wave & 2u) {
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) handed[(pair_of * MT + mt) * 64u + lane] = acc[mt][0];
+            }
+            __syncthreads();
+            if ((wave & 2u) || tile_of[0] >= n_tiles) return;
+            const uint32_t ffn = n >> 1, feat = paired_feature(tile_of[0] * 16u + c);
+            if (feat >= ffn) return;
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                const float4v up = handed[(pair_of * MT + mt) * 64u + lane];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const uint32_t row = 16u * mt + 4u * kb + r;
+                    if (row < m_rows) out.swiglu[(size_t)row * ffn + feat] = gated_mul(out.gate_act, acc[mt][0][r], up[r]);
+                }
+            }
+            return;
+        }
+    }
     if constexpr (TPW == 2) {
         if (out.swiglu) {
             // paired gate/up weight: tile 0 of this wave holds gate columns, tile 1 the up columns of the same features
@@ -400,7 +431,7 @@ static hipError_t launch_batch_slices(hipStream_t s, const WeightView &w, const 
 // M <= 32.  quads_per_group: 1, 2 or 3 column quads per workgroup sharing one activation tile (one tile per wave; with
 // two tiles per wave the workgroup owns two quads anyway).  rounded: weights rounded to f16 and accumulated over K by
 // the MFMAs (always on the 32-row variant, so that one call runs one arithmetic whatever its last block's height);
-// otherwise the exact per-group f32 scaling.  tiles_per_wave: 1 or 2 (a gated store without split-K needs 2).  `scratch` holds, for f32 activations,
+// otherwise the exact per-group f32 scaling.  tiles_per_wave: 1 or 2.  `scratch` holds, for f32 activations,
 // their two f16 terms (2 x M x K halves) and after them the split-K partials (splits x M x (n_tiles * 16) floats);
 // the split factor is cut to what fits.
 hipError_t launch_batch(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out_in,
@@ -436,7 +467,6 @@ hipError_t launch_batch(hipStream_t s, const WeightView &w, const void *a, bool 
     else if (splits > partial_bytes / per_split) splits = (uint32_t)(partial_bytes / per_split);
     if (splits < 1) splits = 1;
     if (w.k_chunks < splits) splits = w.k_chunks;
-    if (out.swiglu && splits == 1) tiles_per_wave = 2;
 #define TWM_BATCH_CASE(MT, R, T, P) return launch_batch_slices<MT, R, T, P>(s, w, a, m, out, splits, k_slices, quads_per_group, partials, lo_offset)
     if (rounded) {
         if (tiles_per_wave == 2) { if (a_f32) TWM_BATCH_CASE(2, true, 2, 2); TWM_BATCH_CASE(2, true, 1, 2); }

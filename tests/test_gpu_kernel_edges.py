@@ -68,3 +68,27 @@ def test_scaled_f32_rows_of_a_prompt_in_one_and_two_slabs(dev, m, k):
     for t in (a, c):
         t.free()
     w.free()
+
+
+@pytest.mark.parametrize("m", [9, 16, 17, 32])
+@pytest.mark.parametrize("ffn,nt,waves", [(32, 0, 0), (96, 3, 0), (160, 3, 0), (96, 4, 8), (64, 1, 16)])
+def test_batched_gate_through_lds(dev, m, ffn, nt, waves):
+    # one tile per wave: the up tiles' sums reach the gate tiles' waves through LDS; one to five quads on workgroups of one,
+    # two and three (the last one part empty), alone and with k-slices
+    k = 544                                          # 17 groups: four chunks and a quarter
+    gate, up = [(O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (811, 813)]
+    pair = [tuple(T.GpuTensor.from_host(dev, x, t) for x, t in zip(w, ("u8", "f16"))) for w in (gate, up)]
+    w = T.MarlinWeight.gate_up(dev, *pair, k, ffn)
+    a16 = O.synth_act_f16(m, k, 815)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k)
+    g, u = (O.gemm_f64(a, *x, m, k, ffn) for x in (gate, up))
+    out = T.GpuTensor.from_host(dev, np.full((m, ffn), np.nan, np.float32))
+    try:
+        for key, v in (("kernel", 4 if nt else 0), ("nt", nt), ("waves", waves)):
+            dev.set_option(key, v)
+        T.gemm_swiglu(dev, w, T.GpuTensor.from_host(dev, a16, "f16"), m, out)
+    finally:
+        for key in ("kernel", "nt", "waves"):
+            dev.set_option(key, 0)
+    close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
+    w.free()
