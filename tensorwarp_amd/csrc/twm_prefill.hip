@@ -363,29 +363,47 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *
     }
 }
 
-// out[row][col] = sum over splits, in split order (deterministic), of partials[split][row][col]
-__global__ __launch_bounds__(256) void k_splitk_reduce(const float *__restrict__ partials, OutSpec out, uint32_t m_rows, uint32_t n,
-                                                         uint32_t n_ld, uint32_t splits)
+// The partial sums of one place, added in split order (deterministic): four loads in flight at a time.
+__device__ __forceinline__ float4v splitk_sum(const float4v *src, size_t stride4, uint32_t splits)
 {
-    size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;  // one thread per four padded columns
-    uint32_t quads = n_ld / 4;
+    float4v s = src[0];
+    uint32_t z = 1;
+    for (; z + 4u <= splits; z += 4u) {
+        float4v v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = src[(z + j) * stride4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) s += v[j];
+    }
+    if (z + 2u <= splits) {
+        const float4v v = src[z * stride4], w = src[(z + 1u) * stride4];
+        s += v;
+        s += w;
+        z += 2u;
+    }
+    if (z < splits) s += src[z * stride4];
+    return s;
+}
+
+// out[row][col] = sum over splits of partials[split][row][col], one thread per four padded columns.  Bound: latency.  (A
+// loop of one load and one add per turn waited for memory once per split: nine splits of 96 x 3584 took 6.6 us in a kernel
+// trace, now 4.8, of which most is the launch; four splits of 32 x 3584 5.0 and 4.8.)
+__global__ __launch_bounds__(256) void k_splitk_reduce(const float *__restrict__ partials, OutSpec out, uint32_t m_rows, uint32_t n,
+                                                         uint32_t n_ld, uint32_t splits, uint32_t row_store)
+{
+    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t quads = n_ld / 4;
     if (idx >= (size_t)m_rows * quads) return;
-    uint32_t row = (uint32_t)(idx / quads), col = (uint32_t)(idx % quads) * 4u;
-    const float4 *src = (const float4 *)(partials + (size_t)row * n_ld + col);
-    size_t stride4 = (size_t)m_rows * n_ld / 4;
-    float4 s = src[0];
-    for (uint32_t z = 1; z < splits; z++) {
-        float4 v = src[z * stride4];
-        s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+    const uint32_t row = (uint32_t)(idx / quads), col = (uint32_t)(idx % quads) * 4u;
+    float4v s = splitk_sum((const float4v *)(partials + (size_t)row * n_ld + col), (size_t)m_rows * n_ld / 4, splits);
+    if (out.row_scale) s *= out.row_scale[row];  // (f32 rows scaled into the f16 range)
+    if (row_store) {
+        if (col < n) *(float4v *)(out.seg[0].ptr + (size_t)row * n + col) = s;
+        return;
     }
-    if (out.row_scale) {
-        const float rs = out.row_scale[row];  // (f32 rows scaled into the f16 range)
-        s.x *= rs; s.y *= rs; s.z *= rs; s.w *= rs;
-    }
-    if (col + 0 < n) pf_store_out(out, row, col + 0, s.x);
-    if (col + 1 < n) pf_store_out(out, row, col + 1, s.y);
-    if (col + 2 < n) pf_store_out(out, row, col + 2, s.z);
-    if (col + 3 < n) pf_store_out(out, row, col + 3, s.w);
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++)
+        if (col + j < n) pf_store_out(out, row, col + j, s[j]);
 }
 
 // The same sum for a paired gate/up weight: one thread per four features adds the gate and the up partials
@@ -394,23 +412,21 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_swiglu(const float *__res
                                                                 uint32_t m_rows, uint32_t ffn, uint32_t n_ld, uint32_t splits,
                                                                 uint32_t act, const float *__restrict__ row_scale)
 {
-    size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    uint32_t quads = ffn / 4;  // ffn is a multiple of 32
+    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t quads = ffn / 4;  // ffn is a multiple of 32
     if (idx >= (size_t)m_rows * quads) return;
-    uint32_t row = (uint32_t)(idx / quads), feat = (uint32_t)(idx % quads) * 4u;
-    uint32_t col = (feat >> 5) * 64u + (feat & 31u);
-    const float4 *src = (const float4 *)(partials + (size_t)row * n_ld + col);
-    size_t stride4 = (size_t)m_rows * n_ld / 4;
-    float4 g = src[0], u = src[8];
-    for (uint32_t z = 1; z < splits; z++) {
-        float4 v = src[z * stride4], w = src[z * stride4 + 8];
-        g.x += v.x; g.y += v.y; g.z += v.z; g.w += v.w;
-        u.x += w.x; u.y += w.y; u.z += w.z; u.w += w.w;
+    const uint32_t row = (uint32_t)(idx / quads), feat = (uint32_t)(idx % quads) * 4u;
+    const float4v *src = (const float4v *)(partials + (size_t)row * n_ld + paired_col(feat));
+    const size_t stride4 = (size_t)m_rows * n_ld / 4;
+    float4v g = splitk_sum(src, stride4, splits), u = splitk_sum(src + kPairWidth / 4, stride4, splits);
+    if (row_scale) {  // (f32 rows scaled into the f16 range)
+        g *= row_scale[row];
+        u *= row_scale[row];
     }
-    const float rs = row_scale ? row_scale[row] : 1.f;  // (f32 rows scaled into the f16 range)
-    float4 o = {gated_mul(act, g.x * rs, u.x * rs), gated_mul(act, g.y * rs, u.y * rs), gated_mul(act, g.z * rs, u.z * rs),
-                gated_mul(act, g.w * rs, u.w * rs)};
-    *(float4 *)(gate_out + (size_t)row * ffn + feat) = o;
+    float4v o;
+#pragma unroll
+    for (int j = 0; j < 4; j++) o[j] = gated_mul(act, g[j], u[j]);
+    *(float4v *)(gate_out + (size_t)row * ffn + feat) = o;
 }
 
 // out[row][:] *= row_scale[row] over every segment, for the rows whose factor is not 1.  Rows that need nothing are the
@@ -437,15 +453,21 @@ hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutS
 {
     size_t quads = (size_t)m * n_ld / 4;
     if (quads == 0) return hipSuccess;
+    // few places: one wave per workgroup, so that they spread over the CUs
+    auto block_of = [](size_t threads) { return threads < 256u * 256u ? 64u : 256u; };
     if (out.swiglu) {
         if (n % (2 * kPairWidth) != 0) return hipErrorInvalidValue;
-        size_t fq = (size_t)m * (n / 2) / 4;
-        hipLaunchKernelGGL(k_splitk_reduce_swiglu, dim3((unsigned)((fq + 255) / 256)), dim3(256), 0, s, partials, out.swiglu, m,
+        const size_t fq = (size_t)m * (n / 2) / 4;
+        const unsigned block = block_of(fq);
+        hipLaunchKernelGGL(k_splitk_reduce_swiglu, dim3((unsigned)((fq + block - 1) / block)), dim3(block), 0, s, partials, out.swiglu, m,
                            n / 2, n_ld, splits, out.gate_act, out.row_scale);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, partials, out, m, n, n_ld,
-                       splits);
+    const uint32_t row_store = out.count == 1 && out.seg[0].start == 0 && out.seg[0].width == n && !out.seg[0].bias && n % 4 == 0 &&
+                               ((uintptr_t)out.seg[0].ptr & 15) == 0;
+    const unsigned block = block_of(quads);
+    hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)((quads + block - 1) / block)), dim3(block), 0, s, partials, out, m, n, n_ld,
+                       splits, row_store);
     return hipGetLastError();
 }
 

@@ -92,3 +92,23 @@ def test_batched_gate_through_lds(dev, m, ffn, nt, waves):
             dev.set_option(key, 0)
     close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
     w.free()
+
+
+@pytest.mark.parametrize("splits", [2, 3, 4, 5, 6, 8, 9])
+@pytest.mark.parametrize("m,n", [(5, 68), (40, 68), (24, 65), (40, 130)])
+def test_split_sums_of_every_count(dev, m, n, splits):
+    # the sum kernel takes four, two and one partial sums at a time; 16-byte stores where N is a multiple of four
+    k = 9 * 128
+    packed, scales, w = weight(dev, k, n, 900 + n)
+    a16 = O.synth_act_f16(m, k, 903 + m)
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    dev.set_option("kernel", 4 if m <= 32 else 0)
+    try:
+        T.gemm(dev, w, T.GpuTensor.from_host(dev, a16, "f16"), m, c, splits)
+    finally:
+        dev.set_option("kernel", 0)
+    a = a16.view(np.float16).astype(np.float64).reshape(m, k)
+    w16 = O.dequant_f16(packed, scales, k, n).view(np.float16).astype(np.float64).reshape(k, n)
+    truth = O.gemm_f64(a.astype(np.float32), packed, scales, m, k, n) if m <= 32 else a @ w16
+    close_rows(c.to_host(), truth, F32_SUM if m <= 32 else 1e-3)
+    w.free()
