@@ -114,7 +114,9 @@ int twm_ctx_info(twm_ctx *ctx, char *buf, size_t buf_len);
  *   "kernel"        decode kernel: 2 = one-lane-per-column kernel on whole 64-column tiles
  *                   (M <= 4 only), 3 = batched-decode streaming kernel (32-row blocks), 4 = batched-decode kernel
  *                   with the activations shared through LDS (32-row blocks; "nt" 1 / 2 = tiles per wave, 4 / 3 =
- *                   two / three column quads per workgroup, "waves" 8 / 16 = two / four k-slices per workgroup)
+ *                   two / three column quads per workgroup, "waves" 8 / 16 = two / four k-slices per workgroup),
+ *                   5 = the kernel for narrow matrices whose waves take k-chunks of their own ("nt" 1, 2, 4 = 16-column
+ *                   tiles per workgroup; above 32 rows f16-rounded weights, as the prefill GEMM)
  *   "dequant_src"   which repacked copy twm_weight_dequant_f16 unpacks: 0 = 16-column tiles, 1 = column lanes
  *   "tune_on_upload" new weight handles (twm_weight_upload, twm_weight_from_device, twm_weight_fuse_n; not the paired
  *                   gate/up handles) get measured plans at once, as if twm_weight_tune had been called on them: 1 = for

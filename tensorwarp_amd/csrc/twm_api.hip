@@ -85,7 +85,7 @@ twm_ctx *twm_ctx_create(int ordinal)
         return nullptr;
     }
     ok = ok && hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking) == hipSuccess;
-    ok = ok && init_prefill() == hipSuccess;
+    ok = ok && init_prefill() == hipSuccess && init_waves() == hipSuccess;
     ok = ok && noalloc_scratch_for_current_device("twm_ctx_create") != nullptr;
     c->stream = c->own_stream;
     c->ws_bytes = kWsBytes;
@@ -201,7 +201,7 @@ int twm_ctx_info(twm_ctx *ctx, char *buf, size_t buf_len)
 
 /* Tuning knobs for sweeps (0 = heuristic): "nt" = tiles per workgroup (1, 2, 4); "waves" = waves per
  * workgroup; "kernel" = 2 the one-lane-per-column kernel (M <= 4), 3 the
- * streaming kernel, 4 the batched-decode kernel with LDS-shared activations;
+ * streaming kernel, 4 the batched-decode kernel with LDS-shared activations, 5 the one whose waves take k-chunks of their own;
  * "dequant_src" = which weight copy twm_weight_dequant_f16 unpacks; "prefill_min_m" = smallest M that
  * runs the prefill kernel. */
 int twm_ctx_set_option(twm_ctx *ctx, const char *key, int value)
@@ -276,7 +276,7 @@ int twm_ctx_set_option(twm_ctx *ctx, const char *key, int value)
         return TWM_OK;
     }
     if (strcmp(key, "kernel") == 0) {
-        if (value < 0 || value > 4 || value == 1) return api_fail(TWM_SHAPE_ERROR, "twm_ctx_set_option: kernel must be 0, 2, 3 or 4");
+        if (value < 0 || value > 5 || value == 1) return api_fail(TWM_SHAPE_ERROR, "twm_ctx_set_option: kernel must be 0, 2, 3, 4 or 5");
         ctx->force_kernel = value;
         return TWM_OK;
     }

@@ -218,7 +218,7 @@ static BatchPlan plan_batch(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, boo
 
 // ---- the launch form of a GEMM: chosen in one place, launched in another ---------------------------------
 // What twm_gemm will run for a weight's shape, a row count and the context's knobs.  Nothing here touches the device.
-enum FormKind { kFormPrefill = 0, kFormSubTile = 1, kFormWholeTile = 2, kFormBatch = 3, kFormStream = 4, kFormNone = 5 };
+enum FormKind { kFormPrefill = 0, kFormSubTile = 1, kFormWholeTile = 2, kFormBatch = 3, kFormStream = 4, kFormNone = 5, kFormWaves = 6 };
 struct LaunchForm {
     int kind;
     int copy;                 // the repacked order it reads (kCopyTile / kCopyCol)
@@ -230,14 +230,14 @@ struct LaunchForm {
     BatchPlan batch;
 };
 struct FormEnv {              // the knobs and limits of a context
-    int kernel, nt, waves, sub, sub_waves, prefill_min_m, batch_rounded;
+    int kernel, nt, waves, sub, sub_waves, prefill_min_m, batch_rounded, prefill_bm;
     size_t ws_bytes;          // split-K scratch
     uint32_t n_counters;      // arrival counters
 };
 static FormEnv form_env(const twm_ctx *c)
 {
     return FormEnv{c->force_kernel, c->force_nt, c->force_waves, c->force_sub, c->force_sub_waves, c->prefill_min_m,
-                   c->batch_rounded, c->ws_bytes, c->n_counters};
+                   c->batch_rounded, c->prefill_bm, c->ws_bytes, c->n_counters};
 }
 
 // n_tiles: 16-column tiles of the padded weight; gated: the gated store of a paired weight
@@ -246,6 +246,25 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
     LaunchForm f = {};
     const uint32_t n_ld = n_tiles * kTileN, tiles64 = n_ld / 64;
     f.splits = splits;
+    WavesPlan wp = {0, 0, 0};
+    if (e.kernel == 5) {  // forced: "nt" 16-column tiles per workgroup (1, 2 or 4), "waves" waves (4 or 8)
+        wp = WavesPlan{e.nt == 1 || e.nt == 2 ? (uint32_t)e.nt : m > 32 ? 2u : 4u, e.waves == 4 ? 4u : 8u, 1};
+        if (wp.waves == 4 && (m <= 32 || wp.nt != 2)) wp.waves = 8;                       // (forms that do not exist: the nearest)
+        if (wp.nt == 4 && (m > 32 || (a_f32 && m > 16))) wp.nt = 2;
+    } else if (e.kernel == 0 && !e.nt && !e.waves && !e.sub && !splits && !e.batch_rounded && !e.prefill_bm &&
+               e.prefill_min_m <= 33 && (m <= 32) == (m < (uint32_t)e.prefill_min_m)) {
+        // (its arithmetic is exact up to 32 rows and rounded above: only where the caller left or lowered that line, so that
+        // with the line raised a call of many rows and a call on each of its 32-row blocks are the same launches)
+        wp = plan_waves(n_tiles, k_chunks, m, a_f32, gated);
+    }
+    if (wp.nt) {
+        f.kind = kFormWaves;
+        f.copy = kCopyTile;
+        f.nt = wp.nt;
+        f.waves = wp.waves;
+        f.splits = splits ? splits : wp.splits;
+        return f;
+    }
     if (m >= (uint32_t)e.prefill_min_m) {
         f.kind = kFormPrefill;
         f.copy = kCopyTile;
@@ -358,7 +377,7 @@ static void tiles_of(uint32_t k, uint32_t n, uint32_t &n_tiles, uint32_t &k_chun
 }
 static FormEnv default_env()
 {
-    return FormEnv{0, 0, 0, 0, 0, 33, 0, kWsBytes, kCounters};
+    return FormEnv{0, 0, 0, 0, 0, 33, 0, 0, kWsBytes, kCounters};
 }
 
 uint32_t twm_pick_splits(uint32_t k, uint32_t n, uint32_t m)
@@ -370,7 +389,8 @@ uint32_t twm_pick_splits(uint32_t k, uint32_t n, uint32_t m)
     const LaunchForm f = choose_form(default_env(), n_tiles, k_chunks, m, false, 0, false);
     switch (f.kind) {
     case kFormSubTile:
-    case kFormWholeTile: return f.splits;
+    case kFormWholeTile:
+    case kFormWaves: return f.splits;
     case kFormBatch: return plan_batch(n_tiles, k_chunks, m < 32 ? m : 32, false).splits;
     case kFormStream: return plan_stream(n_tiles, k_chunks, m < 32 ? m : 32);
     default: return 1;  // prefill: see twm_plan_describe
@@ -415,6 +435,16 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
                  bp.slices == 1 ? "" : "s", bp.splits, bp.splits == 1 ? "" : "s", bp.splits > 1 ? " + k_splitk_reduce" : "");
         break;
     }
+    case kFormWaves:
+        // (named by the family whose decomposition it shares: sub-tiles with a pass per wave up to 16 rows, else batched decode)
+        if (m <= 16 && f.nt <= 2 && f.waves * (4 / f.nt) >= k_chunks)
+            snprintf(text, bytes, "k_gemv4s: %u-column sub-tiles, %u waves (k_waves: each on k-chunks of its own), %u K-split%s%s; 16-column tile copy",
+                     16 * f.nt, f.waves, f.splits, f.splits == 1 ? "" : "s", f.splits > 1 ? " + k_splitk_reduce" : "");
+        else
+            snprintf(text, bytes, "k_batch: %u waves (k_waves: each on k-chunks of its own), %u columns of 1 quad per workgroup, 1 tile per wave, "
+                     "%u K-split%s%s; 16-column tile copy", f.waves, 16 * f.nt, f.splits, f.splits == 1 ? "" : "s",
+                     f.splits > 1 ? " + k_splitk_reduce" : "");
+        break;
     case kFormStream: {
         const uint32_t sp = plan_stream(n_tiles, k_chunks, mb);
         snprintf(text, bytes, "k_stream: %u waves, %u K-split%s%s; 16-column tile copy", stream_waves(n_tiles, mb, e.waves), sp,
@@ -475,6 +505,10 @@ static int gemm_dispatch(twm_ctx *ctx, const twm_weight *w, const void *a_dev, i
                 TWM_DEVICE_ERROR, "prefill launch");
         return TWM_OK;
     }
+    case kFormWaves:
+        HIP_TRY(launch_waves(ctx->stream, v, a_dev, a_f32, m, gated, f.nt, f.waves, f.splits, ctx->ws, ctx->ws_bytes), TWM_DEVICE_ERROR,
+                "batched launch");
+        return TWM_OK;
     case kFormSubTile:
         HIP_TRY(launch_gemv4s(ctx->stream, v, a_dev, a_f32, m, gated, ctx->ws, ctx->counters, f.sub, f.waves, f.splits, ctx->trace), TWM_DEVICE_ERROR,
                 "sub-tile gemv launch");
@@ -551,6 +585,12 @@ static void tune_candidates(uint32_t m, uint32_t k_chunks, std::vector<TunedPlan
         for (int wv : {8, 16})
             for (int sp : {1, 2, 4, 8}) add(2, 1, wv, 0, 0, sp, 0);   // whole 64-column tiles, K split over workgroups
         add(2, 2, 8, 0, 0, 1, 0);
+    }
+    if (m > 4 && m <= 192)
+        for (int nt : {1, 2, 4})                                        // waves on k-ranges of their own
+            for (int sp : {1, 2, 4})
+                if (nt != 4 || m <= 32) add(5, nt, 0, 0, 0, sp, 0);
+    if (m <= 4) {
     } else if (m <= 32) {
         for (int sp : {1, 2, 3, 4, 6, 8}) add(3, 0, 0, 0, 0, sp, 0);  // streaming kernel
         for (int nt : {1, 2, 3, 4})                                     // LDS-shared kernel: tiles per wave / quads per workgroup

@@ -162,6 +162,15 @@ hipError_t launch_gemv4(hipStream_t s, const WeightView &w, const void *a, bool 
 hipError_t launch_gemv4_ref(hipStream_t s, const uint8_t *packed, const uint16_t *scales, uint32_t k, uint32_t n,
                             const float *a, float *c, float *ws, unsigned *counters, uint32_t waves, uint32_t splits);
 hipError_t init_prefill();
+hipError_t init_waves();
+// 5 .. 192 rows on narrow matrices, waves on k-ranges of their own (twm_waves.hip): 16-column tiles per workgroup (0: another
+// form runs), waves, K-splits
+struct WavesPlan {
+    uint32_t nt, waves, splits;
+};
+WavesPlan plan_waves(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated);
+hipError_t launch_waves(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out, uint32_t nt,
+                        uint32_t waves, uint32_t splits, void *scratch, size_t scratch_bytes);
 hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out,
                           uint32_t block_rows, uint32_t splits, void *scratch, size_t scratch_bytes);
 // out[row][col] = sum over splits (in order) of partials[split][row][col], partials rows n_ld floats wide

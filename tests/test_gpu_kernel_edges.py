@@ -112,3 +112,67 @@ def test_split_sums_of_every_count(dev, m, n, splits):
     truth = O.gemm_f64(a.astype(np.float32), packed, scales, m, k, n) if m <= 32 else a @ w16
     close_rows(c.to_host(), truth, F32_SUM if m <= 32 else 1e-3)
     w.free()
+
+
+def gemm_truth(a, packed, scales, m, k, n):
+    """Exact weights up to 32 rows, the FP16 Q4 unpack above (the library's default arithmetic), f64 sums."""
+    if m <= 32:
+        return O.gemm_f64(a, packed, scales, m, k, n)
+    w16 = O.dequant_f16(packed, scales, k, n).view(np.float16).astype(np.float64).reshape(k, n)
+    return a.astype(np.float64) @ w16
+
+
+@pytest.mark.parametrize("nt,waves,splits", [(1, 8, 1), (2, 8, 1), (4, 8, 1), (2, 4, 1), (1, 8, 4)])
+@pytest.mark.parametrize("m", [5, 8, 9, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97, 129, 192])
+def test_waves_on_their_own_k_ranges(dev, m, nt, waves, splits):
+    # row blocks of 16, 32, 48 and 64 rows and their remainders; K of one group, fewer chunks than waves, and more than one
+    # chunk per wave with a ragged end; N ragged; f16 rows, and f32 rows some of which leave the f16 range
+    for k, n in ((32, 9), (416, 65), (1312, 131)):
+        packed, scales, w = weight(dev, k, n, 1200 + k + m)
+        a16 = O.synth_act_f16(m, k, 1203 + m)
+        a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+        big = a.copy()
+        big[0] *= np.float32(2.0 ** 18)
+        big[m - 1] *= np.float32(2.0 ** -22)
+        bias = T.GpuTensor.from_host(dev, O.synth_normal_f32(n, 1207))
+        for rows, dt in ((a16, "f16"), (big, "f32")):
+            c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+            ad = T.GpuTensor.from_host(dev, rows, dt)
+            try:
+                for key, v in (("kernel", 5), ("nt", nt), ("waves", waves)):
+                    dev.set_option(key, v)
+                T.gemm_split(dev, w, ad, m, [c], [n], splits, biases=[bias] if dt == "f16" else None)
+            finally:
+                for key in ("kernel", "nt", "waves"):
+                    dev.set_option(key, 0)
+            truth = gemm_truth(a if dt == "f16" else big, packed, scales, m, k, n)
+            if dt == "f16":
+                truth = truth + bias.to_host().astype(np.float64)
+            close_rows(c.to_host(), truth, F32_SUM if m <= 32 else 1e-3)
+        w.free()
+
+
+@pytest.mark.parametrize("m,dtype", [(5, "f32"), (8, "f32"), (9, "f16"), (13, "f32"), (32, "f16"), (40, "f16"), (64, "f32"), (96, "f16")])
+def test_waves_gated_store(dev, m, dtype):
+    k, ffn = 1056, 96                                # 33 groups; three quads of gate and up tiles
+    gate, up = [(O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (1311, 1313)]
+    pair = [tuple(T.GpuTensor.from_host(dev, x, t) for x, t in zip(w, ("u8", "f16"))) for w in (gate, up)]
+    w = T.MarlinWeight.gate_up(dev, *pair, k, ffn)
+    a16 = O.synth_act_f16(m, k, 1315)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+    if dtype == "f32":
+        a[1] *= np.float32(2.0 ** -21)
+    g, u = (gemm_truth(a, *x, m, k, ffn) for x in (gate, up))
+    truth = g / (1.0 + np.exp(-g)) * u
+    ad = T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a)
+    for nt, splits in ((0, 0), (2, 1), (4, 1), (1, 3)):
+        out = T.GpuTensor.from_host(dev, np.full((m, ffn), np.nan, np.float32))
+        try:
+            dev.set_option("kernel", 5 if nt else 0)
+            dev.set_option("nt", nt)
+            T.gemm_swiglu(dev, w, ad, m, out, splits)
+        finally:
+            dev.set_option("kernel", 0)
+            dev.set_option("nt", 0)
+        close_rows(out.to_host(), truth, F32_SUM if m <= 32 else 2e-3)   # (a product of two sums at 1e-3 each)
+    w.free()
