@@ -93,17 +93,19 @@ struct QGroup {
     uint32_t w[4];
 };
 
-__device__ __forceinline__ QGroup quantize_group32(const float *vals)
+// Group grids: blockIdx.y and .z count the groups (.y holds at most 65535 of them), blockIdx.x the columns of one, so that
+// no thread divides a 64-bit index.
+__device__ __forceinline__ uint32_t block_group() { return blockIdx.z * gridDim.y + blockIdx.y; }
+
+static dim3 group_grid(uint32_t blocks, uint32_t groups)
 {
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; i++) {
-        float a = fabsf(vals[i]);
-        if (a > amax) amax = a;  // NaN never wins, as with Rust's f32::max fold
-    }
-    QGroup r;
-    r.scale = amax / 7.0f;                                 // correctly rounded division
-    float inv = (r.scale != 0.0f) ? 7.0f / amax : 0.0f;
+    const uint32_t y = groups < 65535u ? groups : 65535u;
+    return dim3(blocks, y, (groups + y - 1) / y);
+}
+
+// The general form: any values, NaN and infinity among them.
+__device__ __forceinline__ void quantize_words(const float *vals, float inv, uint32_t *w)
+{
 #pragma unroll
     for (int wi = 0; wi < 4; wi++) {
         uint32_t word = 0;
@@ -115,73 +117,130 @@ __device__ __forceinline__ QGroup quantize_group32(const float *vals)
             q = q < 0 ? 0 : (q > 15 ? 15 : q);
             word |= (uint32_t)q << (4 * j);
         }
-        r.w[wi] = word;
+        w[wi] = word;
     }
+}
+
+// Finite values and a finite factor: |x| <= 7 (1 + 2^-23), so the rounded value is -7 .. 7 and needs no clamp.  Half away
+// from zero is the integer part of x + 0.49999997 with x's sign (the largest f32 below a half: x = 0.5 still reaches 1 by
+// the sum's own rounding and 0.49999997 does not), which leaves five instructions per value instead of about fourteen.
+__device__ __forceinline__ void quantize_words_finite(const float *vals, float inv, uint32_t *w)
+{
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int wi = 0; wi < 4; wi++) {
+        uint32_t word = 0x88888888u;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float x = vals[wi * 8 + j] * inv;
+            const int r = (int)(x + copysignf(0.49999997f, x));
+            word += (uint32_t)r << (4 * j);
+        }
+        w[wi] = word;
+    }
+}
+
+__device__ __forceinline__ QGroup quantize_group32(const float *vals)
+{
+    float amax = 0.0f;
+    bool odd = false;  // an infinity or a NaN
+#pragma unroll
+    for (int i = 0; i < 32; i++) {
+        float a = fabsf(vals[i]);
+        odd = odd || !(a <= 3.40282347e38f);
+        if (a > amax) amax = a;  // NaN never wins, as with Rust's f32::max fold
+    }
+    QGroup r;
+    r.scale = amax / 7.0f;                                 // correctly rounded division
+    float inv = (r.scale != 0.0f) ? 7.0f / amax : 0.0f;
+    odd = odd || !(inv <= 3.40282347e38f);
+    if (__builtin_amdgcn_ballot_w64(odd) != 0) quantize_words(vals, inv, r.w);
+    else quantize_words_finite(vals, inv, r.w);
     return r;
 }
 
-// w row-major [K,N] (is_nk == 0) or [N,K] (is_nk != 0)
-__device__ __forceinline__ void gather_group(const float *w, int is_nk, uint32_t k, uint32_t n, uint32_t g,
-                                             uint32_t col, float *vals)
-{
-    if (is_nk) {
-        const float4 *p = (const float4 *)(w + (size_t)col * k + (size_t)g * 32);
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            float4 v = p[i];
-            vals[4 * i] = v.x; vals[4 * i + 1] = v.y; vals[4 * i + 2] = v.z; vals[4 * i + 3] = v.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 32; i++) vals[i] = w[((size_t)g * 32 + i) * n + col];
-    }
-}
-
+// One thread per (group, column) of a [K,N] matrix: lanes take neighbouring columns.
 __global__ __launch_bounds__(256) void k_quantize_q4_0(const float *__restrict__ w, uint32_t k, uint32_t n,
                                                         uint8_t *__restrict__ q4)
 {
-    uint32_t groups = k / 32;
-    size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;  // idx = g * n + col (coalesced reads of [K,N])
-    if (idx >= (size_t)groups * n) return;
-    uint32_t g = (uint32_t)(idx / n), col = (uint32_t)(idx % n);
+    const uint32_t groups = k / 32, g = block_group(), col = blockIdx.x * 256u + threadIdx.x;
+    if (g >= groups || col >= n) return;
     float vals[32];
-    gather_group(w, 0, k, n, g, col, vals);
+#pragma unroll
+    for (int i = 0; i < 32; i++) vals[i] = w[((size_t)g * 32 + i) * n + col];
     QGroup r = quantize_group32(vals);
     uint32_t *dst = (uint32_t *)(q4 + ((size_t)col * groups + g) * 20);  // 20-byte blocks are 4-byte aligned
     dst[0] = __float_as_uint(r.scale);
     dst[1] = r.w[0]; dst[2] = r.w[1]; dst[3] = r.w[2]; dst[4] = r.w[3];
 }
 
-__global__ __launch_bounds__(256) void k_quantize_twm(const float *__restrict__ w, int is_nk, uint32_t k, uint32_t n,
-                                                       uint4v *__restrict__ packed, uint16_t *__restrict__ scales)
+__global__ __launch_bounds__(256) void k_quantize_twm_kn(const float *__restrict__ w, uint32_t groups, uint32_t n, uint4v *__restrict__ packed,
+                                                          uint16_t *__restrict__ scales)
 {
-    uint32_t groups = k / 32;
-    size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;  // g * n + col
-    if (idx >= (size_t)groups * n) return;
-    uint32_t g = (uint32_t)(idx / n), col = (uint32_t)(idx % n);
+    const uint32_t g = block_group(), col = blockIdx.x * 256u + threadIdx.x;
+    if (g >= groups || col >= n) return;
     float vals[32];
-    gather_group(w, is_nk, k, n, g, col, vals);
+#pragma unroll
+    for (int i = 0; i < 32; i++) vals[i] = __builtin_nontemporal_load(w + ((size_t)g * 32 + i) * n + col);
     QGroup r = quantize_group32(vals);
-    uint4v o = {r.w[0], r.w[1], r.w[2], r.w[3]};
-    packed[idx] = o;
-    scales[idx] = f32_to_f16_bits(r.scale);
+    packed[(size_t)g * n + col] = uint4v{r.w[0], r.w[1], r.w[2], r.w[3]};
+    scales[(size_t)g * n + col] = f32_to_f16_bits(r.scale);
+}
+
+// [N,K]: a column's values lie along K and its neighbours K floats away, so a workgroup takes 64 columns x four groups
+// through LDS: 32 lanes read 512 contiguous bytes of a column (with a thread reading its own 128 bytes every load touched
+// 64 lines: 3584 x 18944, 314 MB, 80 us, now 52.2 at 6.0 TB/s), then a thread per (group, column) quantizes.  A column's 32
+// slots of 16 bytes stand 33 apart, so that the 64 columns of a read fall on different banks.  The f32 matrix is read once
+// and passes the caches (61 us through them).
+__global__ __launch_bounds__(256) void k_quantize_twm_nk(const float *__restrict__ w, uint32_t k, uint32_t n,
+                                                          uint4v *__restrict__ packed, uint16_t *__restrict__ scales)
+{
+    __shared__ float4v tile[64 * 33];
+    const uint32_t groups = k / 32, g0 = block_group() * 4u, col0 = blockIdx.x * 64u;
+    if (g0 >= groups) return;
+    const uint32_t slots = (groups - g0 < 4u ? groups - g0 : 4u) * 8u;  // 16-byte slots of a column in this tile
+    float4v v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const uint32_t at = i * 256u + threadIdx.x, c = at >> 5, slot = at & 31u;
+        const uint32_t col = col0 + c < n ? col0 + c : n - 1;
+        v[i] = __builtin_nontemporal_load((const float4v *)(w + (size_t)col * k + (size_t)g0 * 32) + (slot < slots ? slot : 0u));
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const uint32_t at = i * 256u + threadIdx.x;
+        tile[(at >> 5) * 33u + (at & 31u)] = v[i];
+    }
+    __syncthreads();
+    const uint32_t c = threadIdx.x & 63u, g = g0 + (threadIdx.x >> 6), col = col0 + c;
+    if (g >= groups) return;
+    float vals[32];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float4v x = tile[c * 33u + (threadIdx.x >> 6) * 8u + i];
+#pragma unroll
+        for (int j = 0; j < 4; j++) vals[4 * i + j] = x[j];
+    }
+    QGroup r = quantize_group32(vals);
+    if (col >= n) return;
+    packed[(size_t)g * n + col] = uint4v{r.w[0], r.w[1], r.w[2], r.w[3]};
+    scales[(size_t)g * n + col] = f32_to_f16_bits(r.scale);
 }
 
 hipError_t launch_quantize_q4_0(hipStream_t s, const float *w_kn, uint32_t k, uint32_t n, uint8_t *q4)
 {
-    size_t total = (size_t)(k / 32) * n;
-    if (total == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_quantize_q4_0, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, w_kn, k, n, q4);
+    if (k / 32 == 0 || n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_quantize_q4_0, group_grid((n + 255) / 256, k / 32), dim3(256), 0, s, w_kn, k, n, q4);
     return hipGetLastError();
 }
 
 hipError_t launch_quantize_twm(hipStream_t s, const float *w, int w_is_nk, uint32_t k, uint32_t n, uint8_t *packed,
                                uint16_t *scales)
 {
-    size_t total = (size_t)(k / 32) * n;
-    if (total == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_quantize_twm, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, w, w_is_nk, k, n,
-                       (uint4v *)packed, scales);
+    const uint32_t groups = k / 32;
+    if (groups == 0 || n == 0) return hipSuccess;
+    if (w_is_nk) hipLaunchKernelGGL(k_quantize_twm_nk, group_grid((n + 63) / 64, (groups + 3) / 4), dim3(256), 0, s, w, k, n, (uint4v *)packed, scales);
+    else hipLaunchKernelGGL(k_quantize_twm_kn, group_grid((n + 255) / 256, groups), dim3(256), 0, s, w, groups, n, (uint4v *)packed, scales);
     return hipGetLastError();
 }
 
@@ -211,13 +270,12 @@ hipError_t launch_reorder(hipStream_t s, const uint8_t *q4, uint32_t k, uint32_t
 }
 
 __global__ __launch_bounds__(256) void k_fuse_one(const uint4v *__restrict__ pin, const uint16_t *__restrict__ sin,
-                                                   uint32_t groups, uint32_t ni, uint32_t total_n, uint32_t col_off,
-                                                   uint4v *__restrict__ pout, uint16_t *__restrict__ sout)
+                                                   uint32_t groups, uint32_t ni, uint32_t total_n,
+                                                   uint32_t col_off, uint4v *__restrict__ pout, uint16_t *__restrict__ sout)
 {
-    size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;  // g * ni + c
-    if (idx >= (size_t)groups * ni) return;
-    uint32_t g = (uint32_t)(idx / ni), c = (uint32_t)(idx % ni);
-    size_t dst = (size_t)g * total_n + col_off + c;
+    const uint32_t g = block_group(), c = blockIdx.x * 256u + threadIdx.x;
+    if (g >= groups || c >= ni) return;
+    const size_t idx = (size_t)g * ni + c, dst = (size_t)g * total_n + col_off + c;
     pout[dst] = pin[idx];
     sout[dst] = sin[idx];
 }
@@ -225,27 +283,71 @@ __global__ __launch_bounds__(256) void k_fuse_one(const uint4v *__restrict__ pin
 hipError_t launch_fuse_one(hipStream_t s, const uint8_t *packed_in, const uint16_t *scales_in, uint32_t groups,
                            uint32_t ni, uint32_t total_n, uint32_t col_off, uint8_t *packed_out, uint16_t *scales_out)
 {
-    size_t total = (size_t)groups * ni;
-    if (total == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fuse_one, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, (const uint4v *)packed_in,
+    if (groups == 0 || ni == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_fuse_one, group_grid((ni + 255) / 256, groups), dim3(256), 0, s, (const uint4v *)packed_in,
                        scales_in, groups, ni, total_n, col_off, (uint4v *)packed_out, scales_out);
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------------
-// Q4 unpack from the reference layout: one thread per (k-pair... ) element column-coalesced
+// Q4 unpack from the reference layout
 // ---------------------------------------------------------------------------------
-template <bool F16OUT>
-__global__ __launch_bounds__(256) void k_dequant(const uint8_t *__restrict__ packed, const uint16_t *__restrict__ scales,
-                                                  uint32_t k, uint32_t n, void *__restrict__ out)
+// Memory bound.  A thread takes COLS neighbouring columns of one group: their 16-byte records once, then 32 rows of COLS
+// values.  3584 x 37888 to f16, 352 MB: 49.8 us, 7.1 TB/s (an element per thread, each reading its record's byte and
+// dividing its 64-bit index, took 235; four columns 52.3, eight 127).  The stores pass the caches, or the write-back falls
+// on whatever runs next; records loaded past the caches as well cost 25 us of the gain, since they are often just written.
+template <int COLS, bool F16OUT>
+__global__ __launch_bounds__(256) void k_dequant(const uint4v *__restrict__ packed, const uint16_t *__restrict__ scales,
+                                                  uint32_t groups, uint32_t n, void *__restrict__ out)
 {
-    size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;  // row * n + col
-    if (idx >= (size_t)k * n) return;
-    uint32_t row = (uint32_t)(idx / n), col = (uint32_t)(idx % n);
-    uint32_t g = row / 32, e = row % 32;
+    typedef uint16_t halves __attribute__((ext_vector_type(COLS)));
+    typedef float floats __attribute__((ext_vector_type(COLS)));
+    const uint32_t g = block_group(), col = (blockIdx.x * 256u + threadIdx.x) * COLS;
+    if (g >= groups || col >= n) return;
+    const size_t rec = (size_t)g * n + col;
+    uint4v w[COLS];
+    float sc[COLS];
+#pragma unroll
+    for (int c = 0; c < COLS; c++) {
+        w[c] = packed[rec + c];
+        sc[c] = f16_bits_to_f32(scales[rec + c]);
+        asm volatile("" : "+v"(sc[c]));
+    }
+    const size_t at = (size_t)g * 32 * n + col;
+#pragma unroll
+    for (int wi = 0; wi < 4; wi++) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            halves h;
+            floats f;
+#pragma unroll
+            for (int c = 0; c < COLS; c++) {
+                // (the product is exact in f32: 11-bit x 4-bit significands; see scale_times_q for the pins)
+                const uint32_t nibbles = ((e & 1) ? w[c][wi] >> 4 : w[c][wi]) & 0x0F0F0F0Fu;
+                float x = sc[c] * ((float)((nibbles >> (8 * (e >> 1))) & 0xFFu) - 8.0f);
+                asm volatile("" : "+v"(x));
+                f[c] = x;
+                h[c] = f32_to_f16_bits(x);
+            }
+            const size_t o = at + (size_t)(wi * 8 + e) * n;
+            if (F16OUT) __builtin_nontemporal_store(h, (halves *)((uint16_t *)out + o));
+            else __builtin_nontemporal_store(f, (floats *)((float *)out + o));
+        }
+    }
+}
+
+// records at any address: a byte and an element per thread
+template <bool F16OUT>
+__global__ __launch_bounds__(256) void k_dequant_bytes(const uint8_t *__restrict__ packed, const uint16_t *__restrict__ scales,
+                                                        uint32_t k, uint32_t n, void *__restrict__ out)
+{
+    const uint32_t row = block_group(), col = blockIdx.x * 256u + threadIdx.x;
+    if (row >= k || col >= n) return;
+    const uint32_t g = row / 32, e = row % 32;
+    const size_t idx = (size_t)row * n + col;
     uint8_t byte = packed[((size_t)g * n + col) * 16 + e / 2];
     int q = (e & 1) ? (byte >> 4) : (byte & 0xF);
-    float w = scale_times_q(scales[(size_t)g * n + col], q - 8);  // exact in f32: 11-bit x 4-bit significands
+    float w = scale_times_q(scales[(size_t)g * n + col], q - 8);
     if (F16OUT) ((uint16_t *)out)[idx] = f32_to_f16_bits(w);
     else ((float *)out)[idx] = w;
 }
@@ -253,11 +355,21 @@ __global__ __launch_bounds__(256) void k_dequant(const uint8_t *__restrict__ pac
 hipError_t launch_dequant(hipStream_t s, const uint8_t *packed, const uint16_t *scales, uint32_t k, uint32_t n,
                           void *out, bool f16_out)
 {
-    size_t total = (size_t)k * n;
-    if (total == 0) return hipSuccess;
-    dim3 grid((unsigned)((total + 255) / 256));
-    if (f16_out) hipLaunchKernelGGL(k_dequant<true>, grid, dim3(256), 0, s, packed, scales, k, n, out);
-    else hipLaunchKernelGGL(k_dequant<false>, grid, dim3(256), 0, s, packed, scales, k, n, out);
+    if (k == 0 || n == 0) return hipSuccess;
+    if (((uintptr_t)packed & 15) != 0) {
+        const dim3 grid = group_grid((n + 255) / 256, k);
+        if (f16_out) hipLaunchKernelGGL(k_dequant_bytes<true>, grid, dim3(256), 0, s, packed, scales, k, n, out);
+        else hipLaunchKernelGGL(k_dequant_bytes<false>, grid, dim3(256), 0, s, packed, scales, k, n, out);
+        return hipGetLastError();
+    }
+    // two columns per thread where a row's columns keep the alignment of the paired stores
+    const bool pairs = n % 2 == 0 && ((uintptr_t)out & (f16_out ? 3 : 7)) == 0;
+    const dim3 grid = group_grid((n + (pairs ? 511 : 255)) / (pairs ? 512 : 256), k / 32);
+    const uint4v *rec = (const uint4v *)packed;
+    if (pairs && f16_out) hipLaunchKernelGGL((k_dequant<2, true>), grid, dim3(256), 0, s, rec, scales, k / 32, n, out);
+    else if (pairs) hipLaunchKernelGGL((k_dequant<2, false>), grid, dim3(256), 0, s, rec, scales, k / 32, n, out);
+    else if (f16_out) hipLaunchKernelGGL((k_dequant<1, true>), grid, dim3(256), 0, s, rec, scales, k / 32, n, out);
+    else hipLaunchKernelGGL((k_dequant<1, false>), grid, dim3(256), 0, s, rec, scales, k / 32, n, out);
     return hipGetLastError();
 }
 

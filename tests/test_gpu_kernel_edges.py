@@ -176,3 +176,44 @@ def test_waves_gated_store(dev, m, dtype):
             dev.set_option("nt", 0)
         close_rows(out.to_host(), truth, F32_SUM if m <= 32 else 2e-3)   # (a product of two sums at 1e-3 each)
     w.free()
+
+
+# one group and one column; column and group tiles of the [N,K] form (64 x 4) with a remainder; more groups than a grid's
+# y dimension counts (65535), in both forms
+@pytest.mark.parametrize("k,n", [(32, 1), (96, 63), (128, 64), (160, 65), (288, 258), (2097184, 2), (8388704, 1)])
+def test_one_pass_quantizer_both_layouts(dev, k, n):
+    rng = np.random.default_rng(k + n)
+    w = rng.standard_normal((n, k), dtype=np.float32)
+    w[0, :9] = [0.5, -0.5, 1.5, -2.5, 7.0, -7.0, 0.49999997, 3.4999998, -6.5]  # ties and their neighbours: factor 1
+    w[0, 9:32] = 0.25
+    if k > 32:
+        w[0, 32:64] = 0.0
+        w[-1, 64:96] *= np.float32(1e-39)   # the factor overflows
+        w[-1, 40], w[-1, 41] = np.nan, np.inf
+    want_p, want_s = O.quantize_tw_marlin_nk(w, k, n)
+    for nk in (True, False):
+        x = w if nk else np.ascontiguousarray(w.T)
+        p, s = T.quantize_f32_to_tw_marlin(dev, T.GpuTensor.from_host(dev, x), k, n, weights_are_nk=nk)
+        assert np.array_equal(p.to_host(), want_p) and np.array_equal(s.to_host().view(np.uint16), want_s.view(np.uint16)), nk
+
+
+@pytest.mark.parametrize("k,n", [(32, 1), (64, 3), (64, 512), (96, 514), (32, 257), (2097184, 2)])
+@pytest.mark.parametrize("offset", [0, 4])
+def test_unpack_columns_and_alignments(dev, k, n, offset):
+    # pairs of columns, single ones, records that start off a 16-byte line, and more groups than a grid's y counts
+    packed, scales = O.synth_packed(k, n, 5), O.synth_scales(k, n, 6)
+    raw = T.GpuTensor.from_host(dev, np.concatenate([np.zeros(offset, np.uint8), packed.reshape(-1)]))
+    sc = T.GpuTensor.from_host(dev, scales)
+    for f16, want in ((True, O.dequant_f16(packed, scales, k, n)), (False, O.dequant_f32(packed, scales, k, n).view(np.uint32))):
+        out = T.GpuTensor(dev, (k, n), "f16" if f16 else "f32")
+        call = dev._l.twm_dequant_to_f16 if f16 else dev._l.twm_dequant_to_f32
+        assert call(dev.handle, raw.ptr + offset, sc.ptr, k, n, out.ptr) == 0
+        assert np.array_equal(out.to_host().view(want.dtype), want), f16
+
+
+@pytest.mark.parametrize("k,ns", [(32, [1]), (64, [255, 1, 257]), (2097184, [2, 1])])
+def test_fuse_of_ragged_parts(dev, k, ns):
+    parts = [(O.synth_packed(k, n, 7 + i), O.synth_scales(k, n, 8 + i)) for i, n in enumerate(ns)]
+    fp, fs = T.fuse_tw_marlin_n(dev, [tuple(T.GpuTensor.from_host(dev, x) for x in p) for p in parts], k, ns)
+    wp, ws = O.fuse_tw_marlin_n(parts, k, ns)
+    assert np.array_equal(fp.to_host(), wp) and np.array_equal(fs.to_host(), ws)
