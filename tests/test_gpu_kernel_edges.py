@@ -217,3 +217,22 @@ def test_fuse_of_ragged_parts(dev, k, ns):
     fp, fs = T.fuse_tw_marlin_n(dev, [tuple(T.GpuTensor.from_host(dev, x) for x in p) for p in parts], k, ns)
     wp, ws = O.fuse_tw_marlin_n(parts, k, ns)
     assert np.array_equal(fp.to_host(), wp) and np.array_equal(fs.to_host(), ws)
+
+
+def test_saved_plans_of_every_kernel_come_back(dev):
+    # a plan that the tuner keeps (valid, kernel, nt, waves, sub, sub_waves, splits, prefill_bm) is in an exported blob's last
+    # 96 bytes, eight per bucket of row counts; import drops only values that no option takes
+    k, n = 256, 128
+    packed, scales, w = weight(dev, k, n, 1701)
+    blob = w.export_blob()
+    kept = [1, 5, 2, 0, 0, 0, 1, 0]
+    blob[-96 + 8 * 5:-96 + 8 * 6] = np.array(kept, np.uint8)              # 17 .. 32 rows
+    blob[-96 + 8 * 6:-96 + 8 * 7] = np.array([1, 6, 0, 0, 0, 0, 0, 0], np.uint8)
+    back = T.MarlinWeight.import_blob(dev, blob)
+    assert back.tuned_plan(64) is None and list(back.tuned_plan(20).values())[-7:] == kept[1:]
+    a16 = O.synth_act_f16(20, k, 1703)
+    c = T.GpuTensor.from_host(dev, np.full((20, n), np.nan, np.float32))
+    T.gemm(dev, back, T.GpuTensor.from_host(dev, a16, "f16"), 20, c)
+    close_rows(c.to_host(), gemm_truth(a16.view(np.float16).astype(np.float32).reshape(20, k), packed, scales, 20, k, n), F32_SUM)
+    back.free()
+    w.free()
