@@ -161,6 +161,7 @@ hipError_t launch_gemv4(hipStream_t s, const WeightView &w, const void *a, bool 
                         float *swiglu_out = nullptr);
 hipError_t launch_gemv4_ref(hipStream_t s, const uint8_t *packed, const uint16_t *scales, uint32_t k, uint32_t n,
                             const float *a, float *c, float *ws, unsigned *counters, uint32_t waves, uint32_t splits);
+bool prefill_form_known(uint32_t form);  // a prefill block form (see launch_prefill)
 hipError_t init_prefill();
 hipError_t init_waves();
 // 5 .. 192 rows on narrow matrices, waves on k-ranges of their own (twm_waves.hip): 16-column tiles per workgroup (0: another

@@ -30,8 +30,10 @@ namespace twm {
 // HALF: the MFMAs of a 32-deep group run as two half steps of MT / 2 row blocks, and the A operands are read half a step
 // ahead instead of a whole one: MT / 2 x 2 operand registers less, which with NTW = 3 brings the kernel under 256
 // registers, so that two workgroups share a CU and one's MFMAs fill the issue gaps of the other.
-template <int MT, int NTW = 4, bool HALF = false>
-__global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc,
+// D: chunks in flight (LDS buffers of the A tile and register slots of B).  Two for the tall blocks, whose chunk of MFMAs is
+// as long as a trip to memory; a block of 48 .. 96 rows works through a chunk in a quarter of that and takes three or four.
+template <int MT, int NTW = 4, bool HALF = false, int D = 2>
+__global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc,
                                                   const _Float16 *__restrict__ a_any, OutSpec out, uint32_t m_rows,
                                                   uint32_t k, uint32_t n, uint32_t n_tiles, uint32_t k_chunks,
                                                   uint32_t chunks_per_split, float *__restrict__ partials,
@@ -40,7 +42,7 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *
     constexpr int kPfTileHalves = 16 * MT * kPfRowStride;
     constexpr int NV = MT;       // direct-to-LDS load instructions per wave and A tile (16 MT rows / 16)
     constexpr int HP = 2 * NTW;  // half fragments of B operands per 32-deep group
-    extern __shared__ _Float16 a_lds[];  // two tiles of kPfTileHalves (64 KB at MT = 8)
+    extern __shared__ _Float16 a_lds[];  // D tiles of kPfTileHalves (64 KB at MT = 8)
 
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
@@ -78,10 +80,15 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *
 
     const PfConsts dq = make_pf_consts();
 
-    // this wave's tiles; tiles past the end replay the last tile and are never stored
+    // this wave's tiles; tiles past the end replay the last tile and are never stored.  (Two tiles under a gated store: a
+    // gate tile and the up tile of the same features, which stand two tiles apart in a quad.)
+    const uint32_t pair0 = 4u * (nt0 >> 2) + ((nt0 >> 1) & 1u);
     uint32_t nt[NTW];
 #pragma unroll
-    for (int t = 0; t < NTW; t++) nt[t] = nt0 + t < n_tiles ? nt0 + t : n_tiles - 1;
+    for (int t = 0; t < NTW; t++) {
+        const uint32_t at = NTW == 2 && out.swiglu && !partials ? pair0 + 2u * t : nt0 + t;
+        nt[t] = at < n_tiles ? at : n_tiles - 1;
+    }
 
     // Accumulators live in AGPRs.  The empty asm pins them there across the loop back edge; without it the
     // compiler carries them in VGPRs and copies all of them to AGPRs and back every iteration.
@@ -124,10 +131,23 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *
     };
     // everything this wave has loaded (its parts of the A tile among it) has arrived: before a barrier
     auto wait_loads = [&]() { __builtin_amdgcn_s_waitcnt(0x0F70); };  // vmcnt(0), other counters untouched
+    // D > 2: this wave's LDS reads are back and all of its loads have arrived but the newest `chunks` chunks' (a chunk's loads
+    // are issued together, in chunk order), then the workgroup's barrier.  (__syncthreads would wait for every load.)
+    constexpr int kLoads = NV + 2 * NTW;  // loads per wave and chunk
+    static_assert(D == 2 || ((D - 1) * kLoads < 64 && !HALF), "the counter of loads in flight ends at 63");
+    auto wait_but = [&](auto chunks_c) {
+        constexpr int left = decltype(chunks_c)::value * kLoads;
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0070 | (left & 15) | ((left >> 4) << 14));  // vmcnt(left) lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
 
-    // ---- B: chunk kc lives in register slot kc % 2
-    uint4v bq[2][NTW];
-    uint2v bs[2][NTW];
+    // ---- B: chunk kc lives in register slot kc % D
+    uint4v bq[D][NTW];
+    uint2v bs[D][NTW];
     const uint32_t q_off = lane * 16u, s_off = c * 8u;
     auto load_bq = [&](int slot, uint32_t kc, int t) {
         bq[slot][t] = *(const TWM_GLOBAL uint4v *)(scalar_base(qw, (size_t)((kc0 + kc) * n_tiles + nt[t]) * 1024u) + q_off);
@@ -190,7 +210,7 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *
         }
     };
 
-    // One k-chunk (B slot S = kc & 1, LDS buffer kc & 1).  On entry af0 / bf0 hold group 0 of this chunk.
+    // One k-chunk (B slot and LDS buffer S = kc % D; D = 2 is described).  On entry af0 / bf0 hold group 0 of this chunk.
     //   step 0 .. 2: no loads; at the end of step 2 wait for this wave's loads, then the chunk's only barrier:
     //              A tile kc+1 and B of chunk kc+1 are complete (both requested a whole chunk ago, nothing newer
     //              is in flight), and every wave is done reading buffer kc & 1 (tile kc: its reads were issued
@@ -201,12 +221,14 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *
     // HALF: eight half steps; the last reads of tile kc are those of half step 6 (group 3, second half), so the wait
     // for the loads stands before half step 6 (which already unpacks chunk kc+1), the barrier behind it, and half step 7
     // issues the loads of chunk kc+2.  On entry af0 holds the first half of group 0.
-    auto chunk = [&](auto slot_c, uint32_t kc) {
-        constexpr int S = decltype(slot_c)::value, S1 = S ^ 1;
-        const uint32_t buf = kc & 1u;
-        const uint32_t kc2 = kc + 2 < last ? kc + 2 : last;
+    // D > 2: the chunks behind the last multiple of D (`tail`) load nothing more and wait for everything, since the compiler
+    // drops register loads that nothing will use, and then the count of loads in flight is no longer known.
+    auto chunk = [&](auto slot_c, uint32_t kc, auto tail) {
+        constexpr int S = decltype(slot_c)::value, S1 = (S + 1) % D;
+        constexpr uint32_t buf = S, buf1 = S1;
+        const uint32_t kc2 = kc + D < last ? kc + D : last;
         auto later_loads = [&](int u, int units) {
-            // (the A parts and the B tiles of chunk kc + 2, dealt over `units` units)
+            // (the A parts and the B tiles of chunk kc + D, dealt over `units` units)
 #pragma unroll
             for (int j = 0; j < NV; j++)
                 if (j * units / NV == u) load_a(buf, kc2, j);
@@ -226,35 +248,59 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *
             wait_loads();
             half_step(0, af0, bf1, af1, bf0, buf, 3, S1, 0, [&](int) {});
             __syncthreads();
-            half_step(1, af1, bf1, af0, bf0, buf ^ 1u, 0, S1, 0, [&](int u) { later_loads(u, AF); });
+            half_step(1, af1, bf1, af0, bf0, buf1, 0, S1, 0, [&](int u) { later_loads(u, AF); });
         } else {
             step(af0, bf0, af1, bf1, buf, 1, S, 1, [&](int) {});
             step(af1, bf1, af0, bf0, buf, 2, S, 2, [&](int) {});
             step(af0, bf0, af1, bf1, buf, 3, S, 3, [&](int) {});
-            wait_loads();
-            __syncthreads();
-            step(af1, bf1, af0, bf0, buf ^ 1u, 0, S1, 0, [&](int u) { later_loads(u, MT); });
+            if constexpr (D == 2) {
+                wait_loads();
+                __syncthreads();
+            } else {
+                wait_but(std::integral_constant<int, decltype(tail)::value ? 0 : D - 2>{});
+            }
+            step(af1, bf1, af0, bf0, buf1, 0, S1, 0, [&](int u) {
+                if constexpr (!decltype(tail)::value) later_loads(u, MT);
+            });
         }
         pin_acc();
     };
     using S0 = std::integral_constant<int, 0>;
     using S1 = std::integral_constant<int, 1>;
+    using S2 = std::integral_constant<int, 2 % D>;
+    using S3 = std::integral_constant<int, 3 % D>;
 
-    // prologue: tiles 0 and 1 -> LDS, B chunks 0 and 1 -> slots 0 and 1
+    // prologue: tiles 0 .. D - 1 -> LDS, B chunks 0 .. D - 1 -> slots 0 .. D - 1
     const uint32_t kc1p = 1 < last ? 1 : last;
+    if constexpr (D == 2) {
 #pragma unroll
-    for (int j = 0; j < NV; j++) load_a(0, 0, j);
+        for (int j = 0; j < NV; j++) load_a(0, 0, j);
 #pragma unroll
-    for (int t = 0; t < NTW; t++) {
-        load_bq(0, 0, t);
-        load_bs(0, 0, t);
-        load_bq(1, kc1p, t);
-        load_bs(1, kc1p, t);
+        for (int t = 0; t < NTW; t++) {
+            load_bq(0, 0, t);
+            load_bs(0, 0, t);
+            load_bq(1, kc1p, t);
+            load_bs(1, kc1p, t);
+        }
+#pragma unroll
+        for (int j = 0; j < NV; j++) load_a(1, kc1p, j);
+        wait_loads();
+        __syncthreads();
+    } else {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const uint32_t kcp = (uint32_t)d < last ? (uint32_t)d : last;
+#pragma unroll
+            for (int j = 0; j < NV; j++) load_a(d, kcp, j);
+#pragma unroll
+            for (int t = 0; t < NTW; t++) {
+                load_bq(d, kcp, t);
+                load_bs(d, kcp, t);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        wait_but(std::integral_constant<int, D - 1>{});
     }
-#pragma unroll
-    for (int j = 0; j < NV; j++) load_a(1, kc1p, j);
-    wait_loads();
-    __syncthreads();
 #pragma unroll
     for (int mt = 0; mt < AF; mt++) af0[mt] = read_a(0, 0, mt);
 #pragma unroll
@@ -262,11 +308,19 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *
     __builtin_amdgcn_sched_barrier(0);
 
     uint32_t kc = 0;
-    for (; kc + 2 <= nchunks; kc += 2) {
-        chunk(S0{}, kc);
-        chunk(S1{}, kc + 1);
+    for (; kc + D <= nchunks; kc += D) {
+        chunk(S0{}, kc, std::false_type{});
+        chunk(S1{}, kc + 1, std::false_type{});
+        if constexpr (D > 2) chunk(S2{}, kc + 2, std::false_type{});
+        if constexpr (D > 3) chunk(S3{}, kc + 3, std::false_type{});
     }
-    if (kc < nchunks) chunk(S0{}, kc);
+    using Tail = std::bool_constant<(D > 2)>;
+    if (kc < nchunks) chunk(S0{}, kc, Tail{});
+    if constexpr (D > 2)
+        if (kc + 1 < nchunks) chunk(S1{}, kc + 1, Tail{});
+    if constexpr (D > 3)
+        if (kc + 2 < nchunks) chunk(S2{}, kc + 2, Tail{});
+    if constexpr (D > 2) wait_loads();  // (what was loaded past the end lands before the buffers take the store's blocks, or end)
 
     // ---- store: lane (c, kb) holds rows 4*kb + r of row block mt, column 16*tile + c ----
     if (row_store) {
@@ -343,6 +397,30 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF) void k_prefill(const uint4v *
                     } else {
                         p[0] = v[0]; p[1] = v[1]; p[2] = v[2]; p[3] = v[3];
                     }
+                }
+            }
+        }
+        return;
+    }
+    if (NTW == 2 && out.swiglu) {
+        // the same with a gate tile and its up tile per wave: four lanes cover the 64 bytes of a row
+        const uint32_t ffn = n >> 1;
+        __syncthreads();
+        float *stage = (float *)a_lds + wave * (16 * 20);
+        const uint32_t row = lane >> 2, feat = paired_feature(pair0 * 16u) + (lane & 3u) * 4u;
+        const bool aligned = ((uintptr_t)out.swiglu & 15) == 0;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) stage[(kb * 4 + r) * 20 + c] = gated_mul(out.gate_act, acc[mt][0][r], acc[mt][NTW - 1][r]);
+            const float4v v = *(const float4v *)(stage + row * 20 + (lane & 3u) * 4u);
+            const uint32_t om = m0 + mt * 16u + row;
+            if (om < m_rows && feat < ffn && pair0 + 2u < n_tiles) {
+                float *p = out.swiglu + (size_t)om * ffn + feat;
+                if (aligned) {
+                    __builtin_nontemporal_store(v, (float4v *)p);
+                } else {
+                    p[0] = v[0]; p[1] = v[1]; p[2] = v[2]; p[3] = v[3];
                 }
             }
         }
@@ -485,7 +563,19 @@ hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutS
 // form, under 256 registers): 4096 -> 11008 at M = 1024 81.6 us against 102.5 on 256-column blocks, 3584 -> 4608 at
 // M = 2048 66.9 against 90.7, 3584 -> 37888 at M = 2048 462 against 476; level at 4096 -> 11008, M = 2048 (158.7 / 158.0).
 // Not with the gated store, whose waves hold gate and up tiles in pairs.
+//
+// Up to 256 rows also blocks of 128 columns (two tiles per wave) with 48, 64, 96 or 128 rows, named by their rows + 1: a few
+// rows on 256-column blocks leave half the CUs idle (3584 -> 2 x 18944 is 148 of them) or multiply rows that are not there.
+// kNarrow holds what a chunk takes with one, two and three workgroups on a CU (the 96-row form fits twice, the 128-row form
+// once, the rest of them follow).  Best form before and now (us): 3584 -> 2 x 18944 at 96 rows 50.5 / 45.1, 4096 -> 2 x 11008
+// at 96 35.2 / 29.1 and at 128 38.9 / 34.0, 896 -> 2 x 4864 at 64 13.4 / 8.1, 2048 -> 2 x 5632 at 192 22.7 / 17.6,
+// 18944 -> 3584 at 96 29.1 / 24.1, 11008 -> 4096 at 40 17.6 / 14.8, 3584 -> 4608 at 96 16.4 / 13.3, 4096 -> 12288 at 192
+// 33.5 / 27.9; 3584 -> 2 x 18944 at 128 rows is level or worse (50.8 / 55.4).  Under 2048 columns the wider blocks on more
+// K-splits stay ahead (4864 -> 896 at 96 rows 9.3 / 10.1).
 constexpr double kPf192 = 0.80;
+constexpr uint32_t kNarrowMaxRows = 256, kNarrowMinTiles = 128;
+static const struct { uint32_t form; double chunk[3]; } kNarrow[] = {
+    {49, {0.70, 1.05, 1.50}}, {65, {0.77, 1.30, 1.90}}, {97, {0.88, 1.45, 2.35}}, {129, {1.03, 2.10, 3.15}}};
 struct PrefillPlan {
     uint32_t block_rows, splits;   // block_rows: the form (64, 128, 192)
     double us;
@@ -496,18 +586,25 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
     PrefillPlan best = {force_rows ? force_rows : 64u, force_splits ? force_splits : 1u, 1e30};
     const size_t n_ld = (size_t)n_tiles * 16;
     const double partial_us = (double)rows * (double)n_ld * 4.0 / 4.0e6;  // the reduce kernel's read of one split
-    for (uint32_t bm = 64; bm <= 192; bm += 64) {
-        if (force_rows && bm != force_rows) continue;
+    static const uint32_t kForms[] = {64, 128, 192, 49, 65, 97, 129};
+    for (uint32_t bm : kForms) {
+        const bool narrow = (bm & 1u) != 0;
+        if (force_rows ? bm != force_rows : narrow && (rows > kNarrowMaxRows || n_tiles < kNarrowMinTiles)) continue;
         if (bm == 192 && gated) continue;
-        const uint32_t col_blocks = bm == 192 ? (n_tiles + 11) / 12 : (n_tiles + 15) / 16, height = bm == 64 ? 64u : 128u;
+        const uint32_t col_blocks = bm == 192 ? (n_tiles + 11) / 12 : narrow ? (n_tiles + 7) / 8 : (n_tiles + 15) / 16;
+        const uint32_t height = narrow ? bm - 1u : bm == 64 ? 64u : 128u;
         const double wgs = (double)((rows + height - 1) / height) * col_blocks;
         for (uint32_t sp = 1; sp <= 64; sp++) {
             if (force_splits ? sp != force_splits : sp * 2 > (k_chunks > 1 ? k_chunks : 2) && sp > 1) continue;
             const uint32_t cps = (k_chunks + sp - 1) / sp;
             if (!force_splits && (k_chunks + cps - 1) / cps != sp) continue;  // same work as a smaller factor
             const double total = wgs * sp;
-            double t;
-            if (bm == 192 && total > 256.0) {
+            double t = 0.0;
+            if (narrow) {
+                const uint32_t on_cu = ((uint32_t)total + 255u) / 256u;  // workgroups of the busiest CU
+                for (const auto &f : kNarrow)
+                    if (f.form == bm) t = cps * (on_cu / 3u * f.chunk[2] + (on_cu % 3u ? f.chunk[on_cu % 3u - 1u] : 0.0)) + 3.0;
+            } else if (bm == 192 && total > 256.0) {
                 // two workgroups share a CU: 2.45 per chunk each; a last round of up to one per CU runs at 1.45
                 const double full = (double)(uint64_t)(total / 512.0), rem = total - 512.0 * full;
                 t = full * (cps * 2.45 + 3.0) + (rem == 0.0 ? 0.0 : (rem <= 256.0 ? cps * 1.45 : cps * 2.45) + 3.0);
@@ -523,7 +620,7 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
             }
             if (sp > 1) t += 2.5 + sp * partial_us;
             // a larger factor, and the narrower block, have to pay for themselves
-            const double margin = (sp > best.splits && bm == best.block_rows) || bm == 192 ? 0.97 : 1.0;
+            const double margin = (sp > best.splits && bm == best.block_rows) || bm == 192 || narrow ? 0.97 : 1.0;
             if (t < best.us * margin) {
                 best.block_rows = bm;
                 best.splits = sp;
@@ -566,11 +663,11 @@ void prefill_plan_of(uint32_t rows, uint32_t block_rows, uint32_t splits, uint32
     *splits_out = plan.splits;
 }
 
-template <int MT, int NTW = 4, bool HALF = false>
+template <int MT, int NTW = 4, bool HALF = false, int D = 2>
 static hipError_t launch_prefill_t(hipStream_t s, const WeightView &w, const _Float16 *a, uint32_t m, const OutSpec &out,
                                    uint32_t splits, float *partials, bool via_partials = false)
 {
-    size_t lds = (size_t)2 * 16 * MT * kPfRowStride * sizeof(_Float16);
+    size_t lds = (size_t)D * 16 * MT * kPfRowStride * sizeof(_Float16);
     uint32_t cps = (w.k_chunks + splits - 1) / splits;
     splits = (w.k_chunks + cps - 1) / cps;  // no empty split
     const uint32_t col_blocks = (w.n_tiles + 4 * NTW - 1) / (4 * NTW), row_blocks = (m + 16 * MT - 1) / (16 * MT);
@@ -584,39 +681,52 @@ static hipError_t launch_prefill_t(hipStream_t s, const WeightView &w, const _Fl
     if (splits == 1 && !via_partials)
         row_store = !out.swiglu && out.count == 1 && out.seg[0].start == 0 && out.seg[0].width == w.n && !out.seg[0].bias &&
                     w.n % 4 == 0 && ((uintptr_t)out.seg[0].ptr & 15) == 0;
-    if (NTW != 4 && out.swiglu) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_prefill<MT, NTW, HALF>), grid, dim3(256), lds, s, (const uint4v *)w.qw, (const uint2v *)w.sc, a, out, m, w.k,
+    if (NTW == 3 && out.swiglu) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_prefill<MT, NTW, HALF, D>), grid, dim3(256), lds, s, (const uint4v *)w.qw, (const uint2v *)w.sc, a, out, m, w.k,
                        w.n, w.n_tiles, w.k_chunks, cps, splits > 1 || via_partials ? partials : nullptr, row_store, col_blocks, row_blocks);
     if (splits > 1 || via_partials) return launch_splitk_reduce(s, partials, out, m, w.n, w.n_tiles * 16, splits);
     return hipGetLastError();
 }
 
+bool prefill_form_known(uint32_t form)
+{
+    return form == 64 || form == 128 || form == 192 || form == 49 || form == 65 || form == 97 || form == 129;
+}
+
 // Once per device, outside any stream capture: the 128-row variant asks for all 64 KB of dynamic LDS.
 hipError_t init_prefill()
 {
-    hipError_t e = hipFuncSetAttribute((const void *)k_prefill<8>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       2 * 16 * 8 * kPfRowStride * (int)sizeof(_Float16));
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void *)k_prefill<8, 3>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            2 * 16 * 8 * kPfRowStride * (int)sizeof(_Float16));
-    if (e != hipSuccess) return e;
-    return hipFuncSetAttribute((const void *)k_prefill<8, 3, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               2 * 16 * 8 * kPfRowStride * (int)sizeof(_Float16));
+    auto ask = [](const void *fn, int mt, int d) {
+        return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, d * 16 * mt * kPfRowStride * (int)sizeof(_Float16));
+    };
+    hipError_t e = ask((const void *)k_prefill<8>, 8, 2);
+    if (e == hipSuccess) e = ask((const void *)k_prefill<8, 3>, 8, 2);
+    if (e == hipSuccess) e = ask((const void *)k_prefill<8, 3, true>, 8, 2);
+    if (e == hipSuccess) e = ask((const void *)k_prefill<4, 2, false, 4>, 4, 4);
+    if (e == hipSuccess) e = ask((const void *)k_prefill<6, 2, false, 3>, 6, 3);
+    if (e == hipSuccess) e = ask((const void *)k_prefill<8, 2, false, 3>, 8, 3);
+    return e;
 }
 
 // block_rows: the block form (64 = 64 rows x 256 columns, 128 = 128 x 256, 192 = 128 rows x 192 columns), splits: k-split
-// factor; 0 = choose (plan_prefill), within what `scratch` can hold as f32 partial sums.
+// factor, 49 / 65 / 97 / 129 = 48 / 64 / 96 / 128 rows x 128 columns; 0 = choose (plan_prefill), within what `scratch` can hold as f32 partial sums.
 // `scratch` (scratch_bytes) holds the f16 copy of f32 activations and / or the split-K partials; when it
 // cannot hold all M rows the rows are processed in slabs.
 hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out,
                           uint32_t block_rows, uint32_t splits, void *scratch, size_t scratch_bytes)
 {
     if (m == 0 || w.n == 0) return hipSuccess;
-    if (block_rows != 0 && block_rows != 64 && block_rows != 128 && block_rows != 192) return hipErrorInvalidValue;
+    if (block_rows != 0 && !prefill_form_known(block_rows)) return hipErrorInvalidValue;
     auto run = [&](const _Float16 *a16, uint32_t rows, const OutSpec &o, void *ws, size_t ws_bytes, bool via = false) {
         // (a forced 192-column form with the gated store: the 256-column one)
         const uint32_t form = block_rows == 192 && o.swiglu ? 128u : block_rows;
         const PrefillPlan plan = plan_prefill_within(rows, form, splits, w.n_tiles, w.k_chunks, ws ? ws_bytes : 0, o.swiglu != nullptr);
+        switch (plan.block_rows) {
+        case 49: return launch_prefill_t<3, 2, false, 4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
+        case 65: return launch_prefill_t<4, 2, false, 4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
+        case 97: return launch_prefill_t<6, 2, false, 3>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
+        case 129: return launch_prefill_t<8, 2, false, 3>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
+        }
         if (plan.block_rows == 64) return launch_prefill_t<4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
         if (plan.block_rows == 192) {
             // more workgroups than CUs: the variant of which two share a CU (4096 -> 11008 at M = 1024, 464 workgroups:

@@ -236,3 +236,51 @@ def test_saved_plans_of_every_kernel_come_back(dev):
     close_rows(c.to_host(), gemm_truth(a16.view(np.float16).astype(np.float32).reshape(20, k), packed, scales, 20, k, n), F32_SUM)
     back.free()
     w.free()
+
+
+# 48 .. 128-row blocks of 128 columns: a block's last row and the next one's first, K of one group, of two chunks and of an
+# odd number with a ragged end, N ragged below and above a block; K-split and plain stores, f16 rows and scaled f32 rows
+@pytest.mark.parametrize("form", [49, 65, 97, 129])
+@pytest.mark.parametrize("m", [33, 48, 49, 64, 65, 96, 97, 128, 129, 193])
+def test_prefill_blocks_of_128_columns(dev, m, form):
+    for k, n, splits in ((32, 9, 1), (256, 132, 1), (672, 257, 1), (1312, 260, 3)):
+        packed, scales, w = weight(dev, k, n, 1500 + k + m)
+        a16 = O.synth_act_f16(m, k, 1503 + m)
+        a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+        big = a.copy()
+        big[0] *= np.float32(2.0 ** 18)
+        for rows, dt, vals in ((a16, "f16", a), (big, "f32", big)):
+            c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+            ad = T.GpuTensor.from_host(dev, rows, dt)
+            try:
+                dev.set_option("prefill_bm", form)
+                T.gemm(dev, w, ad, m, c, splits=splits)
+            finally:
+                dev.set_option("prefill_bm", 0)
+            close_rows(c.to_host(), gemm_truth(vals, packed, scales, m, k, n), 1e-3)
+        w.free()
+
+
+@pytest.mark.parametrize("form", [0, 49, 65, 97, 129])
+@pytest.mark.parametrize("m,ffn,dtype", [(33, 32, "f16"), (48, 96, "f32"), (65, 160, "f16"), (96, 288, "f16"), (129, 96, "f32")])
+def test_prefill_gate_on_128_columns(dev, m, ffn, dtype, form):
+    k = 416
+    gate, up = [(O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (1611, 1613)]
+    pair = [tuple(T.GpuTensor.from_host(dev, x, t) for x, t in zip(w, ("u8", "f16"))) for w in (gate, up)]
+    w = T.MarlinWeight.gate_up(dev, *pair, k, ffn)
+    a16 = O.synth_act_f16(m, k, 1615)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+    if dtype == "f32":
+        a[1] *= np.float32(2.0 ** -21)
+    g, u = (gemm_truth(a, *x, m, k, ffn) for x in (gate, up))
+    truth = g / (1.0 + np.exp(-g)) * u
+    ad = T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a)
+    for splits in (1, 3):
+        out = T.GpuTensor.from_host(dev, np.full((m, ffn), np.nan, np.float32))
+        try:
+            dev.set_option("prefill_bm", form)
+            T.gemm_swiglu(dev, w, ad, m, out, splits)
+        finally:
+            dev.set_option("prefill_bm", 0)
+        close_rows(out.to_host(), truth, 2e-3)   # (a product of two sums at 1e-3 each)
+    w.free()
