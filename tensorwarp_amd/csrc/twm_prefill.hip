@@ -8,11 +8,11 @@
 // Block = 16*MT rows x 256 columns (MT = 8 or 4), 4 waves; wave w owns 64 columns (four 16-column tiles of
 // the tile-order copy) for all rows of the block, so no weight is unpacked twice inside a block.  Per
 // 128-deep k-chunk and wave:
-//   A tile (16*MT x 128 f16): global -> LDS directly (global_load_lds_dwordx4), double buffered, 256-byte rows
+//   A tile (16*MT x 128 f16): global -> LDS directly (global_load_lds_dwordx4), D buffers, 256-byte rows
 //                             whose 16-byte slots are XOR-swizzled so that the sixteen rows of an operand
 //                             read hit distinct banks;
-//   B : 16 bytes of nibbles + four scales per lane per tile, straight from HBM/L2 into registers, one
-//       chunk ahead (two register slots), unpacked to MFMA B operands one 32-deep group ahead;
+//   B : 16 bytes of nibbles + four scales per lane per tile, straight from HBM/L2 into registers,
+//       D - 1 chunks ahead (D register slots), unpacked to MFMA B operands one 32-deep group ahead;
 //   16*MT v_mfma_f32_16x16x32_f16 (MT row blocks x 4 column tiles x 4 groups), 16*MT accumulator registers.
 // One v_mfma issue slot hides about two other vector instructions, so the unpack (14 instructions per
 // tile and group, shared by MT row blocks) is only free from MT = 8 on.
@@ -30,9 +30,12 @@ namespace twm {
 // HALF: the MFMAs of a 32-deep group run as two half steps of MT / 2 row blocks, and the A operands are read half a step
 // ahead instead of a whole one: MT / 2 x 2 operand registers less, which with NTW = 3 brings the kernel under 256
 // registers, so that two workgroups share a CU and one's MFMAs fill the issue gaps of the other.
-// D: chunks in flight (LDS buffers of the A tile and register slots of B).  Two for the tall blocks, whose chunk of MFMAs is
-// as long as a trip to memory; a block of 48 .. 96 rows works through a chunk in a quarter of that and takes three or four.
-template <int MT, int NTW = 4, bool HALF = false, int D = 2>
+// D: chunks in flight (LDS buffers of the A tile and register slots of B): two with HALF, whose second workgroup covers the
+// wait, four for blocks of 48 and 64 rows x 128 columns, which work through a chunk in a quarter of a trip to memory, else
+// three (two before: 4096 -> 2 x 11008 at 96 rows 32.8 -> 29.1 us on 96 x 128, at 64 rows 27.0 -> 25.3 on 64 x 256; a LLaMA-7B
+// layer at 512 rows 254.1 -> 249.7, at 2048 787.9 -> 783.4 on 128 x 256; 3584 -> 2 x 18944 at 96 rows, two workgroups on some
+// CUs, 43.1 -> 45.2).
+template <int MT, int NTW = 4, bool HALF = false, int D = HALF ? 2 : 3>
 __global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc,
                                                   const _Float16 *__restrict__ a_any, OutSpec out, uint32_t m_rows,
                                                   uint32_t k, uint32_t n, uint32_t n_tiles, uint32_t k_chunks,
@@ -42,7 +45,7 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(co
     constexpr int kPfTileHalves = 16 * MT * kPfRowStride;
     constexpr int NV = MT;       // direct-to-LDS load instructions per wave and A tile (16 MT rows / 16)
     constexpr int HP = 2 * NTW;  // half fragments of B operands per 32-deep group
-    extern __shared__ _Float16 a_lds[];  // D tiles of kPfTileHalves (64 KB at MT = 8)
+    extern __shared__ _Float16 a_lds[];  // D tiles of kPfTileHalves (96 KB at MT = 8, D = 3)
 
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
@@ -134,7 +137,7 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(co
     // D > 2: this wave's LDS reads are back and all of its loads have arrived but the newest `chunks` chunks' (a chunk's loads
     // are issued together, in chunk order), then the workgroup's barrier.  (__syncthreads would wait for every load.)
     constexpr int kLoads = NV + 2 * NTW;  // loads per wave and chunk
-    static_assert(D == 2 || ((D - 1) * kLoads < 64 && !HALF), "the counter of loads in flight ends at 63");
+    static_assert(HALF ? D == 2 : D > 2 && (D - 1) * kLoads < 64, "the counter of loads in flight ends at 63");
     auto wait_but = [&](auto chunks_c) {
         constexpr int left = decltype(chunks_c)::value * kLoads;
         __builtin_amdgcn_sched_barrier(0);
@@ -210,15 +213,14 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(co
         }
     };
 
-    // One k-chunk (B slot and LDS buffer S = kc % D; D = 2 is described).  On entry af0 / bf0 hold group 0 of this chunk.
-    //   step 0 .. 2: no loads; at the end of step 2 wait for this wave's loads, then the chunk's only barrier:
-    //              A tile kc+1 and B of chunk kc+1 are complete (both requested a whole chunk ago, nothing newer
-    //              is in flight), and every wave is done reading buffer kc & 1 (tile kc: its reads were issued
-    //              up to step 2 and are waited for by the barrier)
-    //   step 3   : A tile kc+2 -> buffer kc & 1 and B of chunk kc+2 -> slot S (its last group was unpacked in
-    //              step 2); the step's own reads and unpack are already those of chunk kc+1, group 0
+    // One k-chunk (B slot and LDS buffer S = kc % D).  On entry af0 / bf0 hold group 0 of this chunk.
+    //   step 0 .. 2: no loads; at the end of step 2 wait for this wave's loads but the newest D - 2 chunks', then the chunk's
+    //              only barrier: A tile kc+1 and B of chunk kc+1 are complete, and every wave is done reading buffer S
+    //              (tile kc: its reads were issued up to step 2 and are back)
+    //   step 3   : A tile kc+D -> buffer S and B of chunk kc+D -> slot S (its last group was unpacked in step 2); the
+    //              step's own reads and unpack are already those of chunk kc+1, group 0
     // Past the end the last chunk is loaded again and never used.
-    // HALF: eight half steps; the last reads of tile kc are those of half step 6 (group 3, second half), so the wait
+    // HALF (D = 2): eight half steps; the last reads of tile kc are those of half step 6 (group 3, second half), so the wait
     // for the loads stands before half step 6 (which already unpacks chunk kc+1), the barrier behind it, and half step 7
     // issues the loads of chunk kc+2.  On entry af0 holds the first half of group 0.
     // D > 2: the chunks behind the last multiple of D (`tail`) load nothing more and wait for everything, since the compiler
@@ -253,12 +255,7 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(co
             step(af0, bf0, af1, bf1, buf, 1, S, 1, [&](int) {});
             step(af1, bf1, af0, bf0, buf, 2, S, 2, [&](int) {});
             step(af0, bf0, af1, bf1, buf, 3, S, 3, [&](int) {});
-            if constexpr (D == 2) {
-                wait_loads();
-                __syncthreads();
-            } else {
-                wait_but(std::integral_constant<int, decltype(tail)::value ? 0 : D - 2>{});
-            }
+            wait_but(std::integral_constant<int, decltype(tail)::value ? 0 : D - 2>{});
             step(af1, bf1, af0, bf0, buf1, 0, S1, 0, [&](int u) {
                 if constexpr (!decltype(tail)::value) later_loads(u, MT);
             });
@@ -272,7 +269,7 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(co
 
     // prologue: tiles 0 .. D - 1 -> LDS, B chunks 0 .. D - 1 -> slots 0 .. D - 1
     const uint32_t kc1p = 1 < last ? 1 : last;
-    if constexpr (D == 2) {
+    if constexpr (HALF) {
 #pragma unroll
         for (int j = 0; j < NV; j++) load_a(0, 0, j);
 #pragma unroll
@@ -663,7 +660,7 @@ void prefill_plan_of(uint32_t rows, uint32_t block_rows, uint32_t splits, uint32
     *splits_out = plan.splits;
 }
 
-template <int MT, int NTW = 4, bool HALF = false, int D = 2>
+template <int MT, int NTW = 4, bool HALF = false, int D = HALF ? 2 : 3>
 static hipError_t launch_prefill_t(hipStream_t s, const WeightView &w, const _Float16 *a, uint32_t m, const OutSpec &out,
                                    uint32_t splits, float *partials, bool via_partials = false)
 {
@@ -693,18 +690,18 @@ bool prefill_form_known(uint32_t form)
     return form == 64 || form == 128 || form == 192 || form == 49 || form == 65 || form == 97 || form == 129;
 }
 
-// Once per device, outside any stream capture: the 128-row variant asks for all 64 KB of dynamic LDS.
+// Once per device, outside any stream capture: the forms with 48 KB or more of dynamic LDS.
 hipError_t init_prefill()
 {
     auto ask = [](const void *fn, int mt, int d) {
         return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, d * 16 * mt * kPfRowStride * (int)sizeof(_Float16));
     };
-    hipError_t e = ask((const void *)k_prefill<8>, 8, 2);
-    if (e == hipSuccess) e = ask((const void *)k_prefill<8, 3>, 8, 2);
+    hipError_t e = ask((const void *)k_prefill<8>, 8, 3);
+    if (e == hipSuccess) e = ask((const void *)k_prefill<8, 3>, 8, 3);
     if (e == hipSuccess) e = ask((const void *)k_prefill<8, 3, true>, 8, 2);
     if (e == hipSuccess) e = ask((const void *)k_prefill<4, 2, false, 4>, 4, 4);
-    if (e == hipSuccess) e = ask((const void *)k_prefill<6, 2, false, 3>, 6, 3);
-    if (e == hipSuccess) e = ask((const void *)k_prefill<8, 2, false, 3>, 8, 3);
+    if (e == hipSuccess) e = ask((const void *)k_prefill<6, 2>, 6, 3);
+    if (e == hipSuccess) e = ask((const void *)k_prefill<8, 2>, 8, 3);
     return e;
 }
 
@@ -724,8 +721,8 @@ hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, boo
         switch (plan.block_rows) {
         case 49: return launch_prefill_t<3, 2, false, 4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
         case 65: return launch_prefill_t<4, 2, false, 4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
-        case 97: return launch_prefill_t<6, 2, false, 3>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
-        case 129: return launch_prefill_t<8, 2, false, 3>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
+        case 97: return launch_prefill_t<6, 2>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
+        case 129: return launch_prefill_t<8, 2>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
         }
         if (plan.block_rows == 64) return launch_prefill_t<4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
         if (plan.block_rows == 192) {

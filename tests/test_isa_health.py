@@ -65,3 +65,22 @@ def test_no_prefetch_was_moved_down_to_its_use(kernels):
             checked += 1
             assert not pattern.search(body), name
     assert checked >= 40
+
+
+def test_counted_waits_match_the_loads_of_a_chunk(kernels):
+    # k_prefill's forms with three or four chunks in flight wait for "all but the newest D - 2 chunks' loads" by number: every
+    # chunk of the main loop has to issue that number of loads between two barriers, the start D chunks' worth
+    checked = 0
+    for name, (body, _) in kernels.items():
+        form = re.search(r"9k_prefillILi(\d+)ELi(\d+)ELb0ELi(\d)E", name)
+        if not form:
+            continue
+        mt, ntw, depth = (int(x) for x in form.groups())
+        per_chunk = mt + 2 * ntw
+        parts = re.split(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)\n\s*s_barrier", body)
+        loads = [len(re.findall(r"\bglobal_load_(?:lds_)?dword", p)) for p in parts[0::2]]
+        waits = [int(x) for x in parts[1::2]]
+        assert waits[:depth + 1] == [(depth - 1) * per_chunk] + [(depth - 2) * per_chunk] * depth, (name, waits)
+        assert loads[:depth + 1] == [depth * per_chunk, 0] + [per_chunk] * (depth - 1), (name, loads)
+        checked += 1
+    assert checked == 7
