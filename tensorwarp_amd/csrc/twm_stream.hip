@@ -255,6 +255,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_stream(const uint4v *__restrict_
 // 8 bytes at a time; NV = 0 reads the row twice, for any k.  (Against a scalar loop that read the row twice: a down
 // projection 18944 -> 3584 with its conversion at 8 rows 27.4 -> 21.8 us, at 32 rows 37.9 -> 31.6; 2048 x 11008 rows,
 // 90 MB in and 45 MB out, about 7 us of the layer less.)
+// gridDim.y = NV > 1: workgroup y reads the whole row for its maximum and converts and writes only stretch y of it, so that
+// a few rows' stores leave from more CUs (four 18944-wide conversions a pass: 201.8 -> 200.2 us at 8 rows, 285.0 -> 283.8 at
+// 32; three stretches of 11008 level; with 96 rows, 480 workgroups, the repeated reads cost more than that: two conversions
+// 198.7 -> 200.3).
 template <bool TWO, int NV>
 __global__ __launch_bounds__(1024) void k_f32_rows_to_f16(const float *__restrict__ a, _Float16 *__restrict__ hi,
                                                            _Float16 *__restrict__ lo, float *__restrict__ row_scale, uint32_t k)
@@ -301,7 +305,7 @@ __global__ __launch_bounds__(1024) void k_f32_rows_to_f16(const float *__restric
         down = __uint_as_float((254u + 13u - e) << 23);       // 2^(13 - (e - 127))
         back = __uint_as_float((e - 13u) << 23);              // 2^((e - 127) - 13)
     }
-    if (threadIdx.x == 0) row_scale[blockIdx.x] = back;
+    if (threadIdx.x == 0 && blockIdx.y == 0) row_scale[blockIdx.x] = back;
     half4v *dh = (half4v *)(hi + row0), *dl = TWO ? (half4v *)(lo + row0) : nullptr;
     auto convert = [&](uint32_t q, const float4v &x) {
         half4v h, l;
@@ -318,7 +322,7 @@ __global__ __launch_bounds__(1024) void k_f32_rows_to_f16(const float *__restric
 #pragma unroll
         for (int i = 0; i < NV; i++) {
             const uint32_t q = threadIdx.x + 1024u * i;
-            if (q < quads) convert(q, v[i]);
+            if ((gridDim.y == 1u || blockIdx.y == (uint32_t)i) && q < quads) convert(q, v[i]);
         }
     } else {
         for (uint32_t q = threadIdx.x; q < quads; q += 1024u) convert(q, src[q]);
@@ -331,8 +335,10 @@ hipError_t launch_f32_rows_to_f16(hipStream_t s, const float *a, _Float16 *hi, _
     if (rows == 0 || k == 0) return hipSuccess;
     auto go = [&](auto nv) {
         constexpr int NV = decltype(nv)::value;
-        if (lo) hipLaunchKernelGGL((k_f32_rows_to_f16<true, NV>), dim3(rows), dim3(1024), 0, s, a, hi, lo, row_scale, k);
-        else hipLaunchKernelGGL((k_f32_rows_to_f16<false, NV>), dim3(rows), dim3(1024), 0, s, a, hi, lo, row_scale, k);
+        // a row's NV stretches on workgroups of their own while all of them fit the CUs at once
+        const dim3 grid(rows, NV > 1 && rows <= 256u / (NV > 0 ? NV : 1) ? NV : 1);
+        if (lo) hipLaunchKernelGGL((k_f32_rows_to_f16<true, NV>), grid, dim3(1024), 0, s, a, hi, lo, row_scale, k);
+        else hipLaunchKernelGGL((k_f32_rows_to_f16<false, NV>), grid, dim3(1024), 0, s, a, hi, lo, row_scale, k);
     };
     if (k <= 4096u) go(std::integral_constant<int, 1>{});
     else if (k <= 4096u * 3) go(std::integral_constant<int, 3>{});

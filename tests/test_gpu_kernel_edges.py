@@ -49,6 +49,30 @@ def test_f32_row_conversion_at_the_edges_of_its_register_tiers(dev, k):
     w.free()
 
 
+@pytest.mark.parametrize("m,k", [(85, 12288), (86, 12288), (51, 20480), (52, 20480), (31, 32768), (32, 32768), (33, 32768), (1, 32768)])
+def test_f32_rows_converted_by_one_or_several_workgroups(dev, m, k):
+    # the stretches of a row run as workgroups of their own up to 85, 51 and 32 rows of these lengths: rows of f16 values
+    # times powers of two, the row's largest value in its first and in its last stretch
+    n = 24
+    packed, scales, w = weight(dev, k, n, 300 + m)
+    base = O.synth_act_f16(m, k, 301).view(np.float16).astype(np.float32).reshape(m, k).copy()
+    base[0, k - 1], base[m - 1, 0] = 64.0, 64.0
+    factor = np.ones(m, np.float32)
+    factor[::3] = 2.0 ** 40
+    rows = base * factor[:, None]
+    if m <= 32:
+        truth = O.gemm_f64(rows, packed, scales, m, k, n)
+    else:
+        truth = (base.astype(np.float64) @ O.dequant_f16(packed, scales, k, n).view(np.float16).astype(np.float64).reshape(k, n)) * factor[:, None]
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    a = T.GpuTensor.from_host(dev, rows)
+    T.gemm(dev, w, a, m, c)
+    close_rows(c.to_host(), truth, F32_SUM if m <= 32 else 1e-3)   # above 32 rows the prefill GEMM's bar
+    for t in (a, c):
+        t.free()
+    w.free()
+
+
 @pytest.mark.parametrize("m,k", [(33, 64), (65, 64), (160, 4128), (3600, 18944)])
 def test_scaled_f32_rows_of_a_prompt_in_one_and_two_slabs(dev, m, k):
     # prompt rows outside the f16 range: the factors go back onto the sums 32 rows at a time (first, last and 32nd row of
