@@ -240,6 +240,15 @@ static FormEnv form_env(const twm_ctx *c)
                    c->batch_rounded, c->prefill_bm, c->ws_bytes, c->n_counters};
 }
 
+// k_waves' arithmetic follows the row count alone: exact weights up to 32 rows, f16-rounded ones above.  It may stand in for
+// the other forms only where the options ask for the same: the prefill GEMM's line left at 33 or lowered (with it raised a
+// call of many rows and a call on each of its 32-row blocks are the same launches), this row count on its usual side of it,
+// no rounded batches.
+static bool waves_arithmetic_asked_for(const FormEnv &e, uint32_t m)
+{
+    return !e.batch_rounded && e.prefill_min_m <= 33 && (m <= 32) == (m < (uint32_t)e.prefill_min_m);
+}
+
 // n_tiles: 16-column tiles of the padded weight; gated: the gated store of a paired weight
 static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, uint32_t splits, bool gated)
 {
@@ -251,10 +260,7 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
         wp = WavesPlan{e.nt == 1 || e.nt == 2 ? (uint32_t)e.nt : m > 32 ? 2u : 4u, e.waves == 4 ? 4u : 8u, 1};
         if (wp.waves == 4 && (m <= 32 || wp.nt != 2)) wp.waves = 8;                       // (forms that do not exist: the nearest)
         if (wp.nt == 4 && (m > 32 || (a_f32 && m > 16))) wp.nt = 2;
-    } else if (e.kernel == 0 && !e.nt && !e.waves && !e.sub && !splits && !e.batch_rounded && !e.prefill_bm &&
-               e.prefill_min_m <= 33 && (m <= 32) == (m < (uint32_t)e.prefill_min_m)) {
-        // (its arithmetic is exact up to 32 rows and rounded above: only where the caller left or lowered that line, so that
-        // with the line raised a call of many rows and a call on each of its 32-row blocks are the same launches)
+    } else if (e.kernel == 0 && !e.nt && !e.waves && !e.sub && !splits && !e.prefill_bm && waves_arithmetic_asked_for(e, m)) {
         wp = plan_waves(n_tiles, k_chunks, m, a_f32, gated);
     }
     if (wp.nt) {
@@ -550,22 +556,24 @@ static void set_knobs(twm_ctx *c, const Knobs &k)
     c->prefill_bm = k.prefill_bm;
 }
 
-// With nothing forced by the caller, a plan that twm_weight_tune measured for this weight and row count is what runs.
+// With nothing forced by the caller, a plan that twm_weight_tune measured for this weight and row count is what runs --
+// unless it is one of k_waves and the options have come to ask for another arithmetic at this row count.
 static int gemm_common(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_dtype, uint32_t m, const OutSpec &out,
                        uint32_t splits, const char *who, float *swiglu_out = nullptr, uint32_t gate_act = 2)
 {
     const Knobs user = knobs_of(ctx);
     const bool free_choice = !splits && !user.kernel && !user.nt && !user.waves && !user.sub && !user.sub_waves && !user.prefill_bm;
     const TunedPlan *tp = (m >= 1 && free_choice && !swiglu_out && a_dtype == TWM_F16) ? &w->tuned[tune_bucket(m)] : nullptr;
-    if (!tp || !tp->valid) return gemm_dispatch(ctx, w, a_dev, a_dtype, m, out, splits, who, swiglu_out, gate_act);
+    if (!tp || !tp->valid || (tp->kernel == 5 && !waves_arithmetic_asked_for(form_env(ctx), m)))
+        return gemm_dispatch(ctx, w, a_dev, a_dtype, m, out, splits, who, swiglu_out, gate_act);
     set_knobs(ctx, Knobs{tp->kernel, tp->nt, tp->waves, tp->sub, tp->sub_waves, tp->prefill_bm});
     const int rc = gemm_dispatch(ctx, w, a_dev, a_dtype, m, out, tp->splits, who, swiglu_out, gate_act);
     set_knobs(ctx, user);
     return rc;
 }
 
-// Candidate launch forms for `m` rows: what the option knobs can ask for.  The first entry is the planners' own choice.
-static void tune_candidates(uint32_t m, uint32_t k_chunks, std::vector<TunedPlan> &out)
+// Candidate launch forms for `m` rows: what the option knobs can ask for (waves: k_waves among them).  The first entry is the planners' own choice.
+static void tune_candidates(uint32_t m, uint32_t k_chunks, bool waves, std::vector<TunedPlan> &out)
 {
     auto add = [&](int kernel, int nt, int waves, int sub, int sub_waves, int splits, int bm) {
         out.push_back(TunedPlan{1, (uint8_t)kernel, (uint8_t)nt, (uint8_t)waves, (uint8_t)sub, (uint8_t)sub_waves, (uint8_t)splits, (uint8_t)bm});
@@ -586,7 +594,7 @@ static void tune_candidates(uint32_t m, uint32_t k_chunks, std::vector<TunedPlan
             for (int sp : {1, 2, 4, 8}) add(2, 1, wv, 0, 0, sp, 0);   // whole 64-column tiles, K split over workgroups
         add(2, 2, 8, 0, 0, 1, 0);
     }
-    if (m > 4 && m <= 192)
+    if (waves && m > 4 && m <= 192)
         for (int nt : {1, 2, 4})                                        // waves on k-ranges of their own
             for (int sp : {1, 2, 4})
                 if (nt != 4 || m <= 32) add(5, nt, 0, 0, 0, sp, 0);
@@ -673,7 +681,7 @@ int twm_weight_tune(twm_ctx *ctx, twm_weight *w, const uint32_t *ms, uint32_t co
     for (uint32_t i = 0; i < count && rc == TWM_OK; i++) {
         const uint32_t m = ms[i];
         std::vector<TunedPlan> cands;
-        tune_candidates(m, w->k_chunks, cands);
+        tune_candidates(m, w->k_chunks, waves_arithmetic_asked_for(form_env(ctx), m), cands);
         const int reps = m <= 32 ? 24 : 6;
         float best_ms = 0.f, own_ms = 0.f;
         TunedPlan best = cands[0];

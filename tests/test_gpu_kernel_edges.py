@@ -308,3 +308,34 @@ def test_prefill_gate_on_128_columns(dev, m, ffn, dtype, form):
             dev.set_option("prefill_bm", 0)
         close_rows(out.to_host(), truth, 2e-3)   # (a product of two sums at 1e-3 each)
     w.free()
+
+
+@pytest.mark.parametrize("m,option,value,exact", [(40, "prefill_min_m", 1 << 30, True), (24, "prefill_min_m", 8, False), (24, "batch_rounded", 1, False),
+                                                  (40, None, 0, False), (24, None, 0, True)])
+def test_measured_plans_keep_the_arithmetic_that_the_options_ask_for(dev, m, option, value, exact):
+    # a measured plan of kernel 5 (exact weights up to 32 rows, f16-rounded ones above) on a context whose options ask for the
+    # other arithmetic at that row count: the planners' choice runs.  At 2e-4 and 1e-3 of the floor in close_rows the two
+    # arithmetics, 2^-12 of each weight apart, are told apart by the outputs that nearly cancel.
+    k, n = 256, 128
+    packed, scales, w = weight(dev, k, n, 1801)
+    blob = w.export_blob()
+    for bucket in (5, 6):                                                  # 17 .. 32 and 33 .. 64 rows
+        blob[-96 + 8 * bucket:-96 + 8 * (bucket + 1)] = np.array([1, 5, 2, 0, 0, 0, 1, 0], np.uint8)
+    back = T.MarlinWeight.import_blob(dev, blob)
+    a16 = O.synth_act_f16(m, k, 1803)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k)
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    try:
+        if option:
+            dev.set_option(option, value)
+        T.gemm(dev, back, T.GpuTensor.from_host(dev, a16, "f16"), m, c)
+    finally:
+        dev.set_option("prefill_min_m", 33)
+        dev.set_option("batch_rounded", 0)
+    w16 = O.dequant_f16(packed, scales, k, n).view(np.float16).astype(np.float64).reshape(k, n)
+    truths = {True: O.gemm_f64(a, packed, scales, m, k, n), False: a.astype(np.float64) @ w16}
+    close_rows(c.to_host(), truths[exact], F32_SUM if exact else 1e-3)
+    with pytest.raises(AssertionError):
+        close_rows(c.to_host(), truths[not exact], 1e-3)
+    back.free()
+    w.free()
