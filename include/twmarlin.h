@@ -296,9 +296,11 @@ void twm_weight_destroy(twm_weight *w);
 int twm_weight_dims(const twm_weight *w, uint32_t *k, uint32_t *n);
 /* device bytes held by the repacked weight */
 size_t twm_weight_bytes(const twm_weight *w);
-/* The handle holds the weight in up to two orders: the 16-column tile order (copy 1: the kernels for M >= 5 and the
- * prefill GEMM) and the column-lane order (copy 2: M <= 4, and M = 5 .. 16 on narrow matrices), 4.5 bits per weight
- * each.  Option "weight_copies" says which ones a new handle gets (0 or 3 = both, the default; 1; 2); a call that needs
+/* The handle holds the weight in up to two orders, 4.5 bits per weight each: the 16-column tile order (copy 1: the kernels
+ * for M >= 5 and the prefill GEMM) and the column-lane order (copy 2: M <= 4; with f16 rows also M = 5 .. 8 on wide
+ * matrices and M = 5 .. 16 on narrow ones, N up to 4096 with K 2048 .. 8192 and N up to 8192 with K 2048 .. 4096 -- of
+ * which M = 7 .. 16 run faster from copy 1 and do so where the handle holds it: the same sums in another order).
+ * Option "weight_copies" says which ones a new handle gets (0 or 3 = both, the default; 1; 2); a call that needs
  * a copy the handle does not hold builds it from the other one on the spot -- which allocates, so inside a graph
  * capture such a call fails with TWM_UNSUPPORTED_OP: ask for the copy beforehand with twm_weight_ensure.
  * twm_weight_drop frees one of two copies (synchronises the stream); twm_weight_copies returns the mask held.

@@ -249,8 +249,10 @@ static bool waves_arithmetic_asked_for(const FormEnv &e, uint32_t m)
     return !e.batch_rounded && e.prefill_min_m <= 33 && (m <= 32) == (m < (uint32_t)e.prefill_min_m);
 }
 
-// n_tiles: 16-column tiles of the padded weight; gated: the gated store of a paired weight
-static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, uint32_t splits, bool gated)
+// n_tiles: 16-column tiles of the padded weight; gated: the gated store of a paired weight; copies: the repacked orders that
+// the handle holds
+static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, uint32_t splits, bool gated,
+                              int copies = kCopyTile | kCopyCol)
 {
     LaunchForm f = {};
     const uint32_t n_ld = n_tiles * kTileN, tiles64 = n_ld / 64;
@@ -262,6 +264,10 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
         if (wp.nt == 4 && (m > 32 || (a_f32 && m > 16))) wp.nt = 2;
     } else if (e.kernel == 0 && !e.nt && !e.waves && !e.sub && !splits && !e.prefill_bm && waves_arithmetic_asked_for(e, m)) {
         wp = plan_waves(n_tiles, k_chunks, m, a_f32, gated);
+        // A handle with the column-lane copy alone keeps the sub-tile kernel, which reads that copy, where there is one for
+        // this shape: a little slower (3584 -> 3584 at 16 rows 7.4 us, k_waves 5.6), but the tile copy would be a second
+        // allocation of the weight's size, and inside a graph capture a refusal.
+        if (!(copies & kCopyTile) && !a_f32 && m <= 16 && plan_gemv4_sub_rows(tiles64, k_chunks).sub) wp.nt = 0;
     }
     if (wp.nt) {
         f.kind = kFormWaves;
@@ -489,7 +495,7 @@ static int gemm_dispatch(twm_ctx *ctx, const twm_weight *w, const void *a_dev, i
     OutSpec gated = out;
     gated.swiglu = swiglu_out;
     gated.gate_act = gate_act;
-    const LaunchForm f = choose_form(form_env(ctx), w->n_tiles, w->k_chunks, m, a_f32, splits, swiglu_out != nullptr);
+    const LaunchForm f = choose_form(form_env(ctx), w->n_tiles, w->k_chunks, m, a_f32, splits, swiglu_out != nullptr, copies_of(w));
     if (f.kind == kFormNone) return api_fail(TWM_UNSUPPORTED_OP, "%s: the one-lane-per-column kernel takes M <= 4", who);
     // the copy the launch reads is built here if the handle does not hold it yet
     if (int rc = weight_ensure(ctx, w, f.copy, who)) return rc;

@@ -339,3 +339,26 @@ def test_measured_plans_keep_the_arithmetic_that_the_options_ask_for(dev, m, opt
         close_rows(c.to_host(), truths[not exact], 1e-3)
     back.free()
     w.free()
+
+
+@pytest.mark.parametrize("m", [7, 9, 16])
+def test_a_column_lane_handle_keeps_its_one_copy_on_narrow_matrices(dev, m):
+    # the documented range of the column-lane copy: captured without a second copy, and run eagerly without building one
+    k, n = 2048, 2048
+    dev.set_option("weight_copies", T.MarlinWeight.COPY_COLUMN_LANE)
+    packed, scales, w = weight(dev, k, n, 1901)
+    dev.set_option("weight_copies", 0)
+    a16 = O.synth_act_f16(m, k, 1903 + m)
+    a = T.GpuTensor.from_host(dev, a16, "f16")
+    truth = O.gemm_f64(a16.view(np.float16).astype(np.float32).reshape(m, k), packed, scales, m, k, n)
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    graph = T.GraphCapture.record_with_device(dev, lambda: T.gemm(dev, w, a, m, c))
+    graph.replay()
+    dev.synchronize()
+    close_rows(c.to_host(), truth, F32_SUM)
+    c.copy_from_host(np.full((m, n), np.nan, np.float32))
+    T.gemm(dev, w, a, m, c)
+    close_rows(c.to_host(), truth, F32_SUM)
+    assert w.copies == T.MarlinWeight.COPY_COLUMN_LANE
+    graph.destroy()
+    w.free()
