@@ -448,14 +448,9 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
         break;
     }
     case kFormWaves:
-        // (named by the family whose decomposition it shares: sub-tiles with a pass per wave up to 16 rows, else batched decode)
-        if (m <= 16 && f.nt <= 2 && f.waves * (4 / f.nt) >= k_chunks)
-            snprintf(text, bytes, "k_gemv4s: %u-column sub-tiles, %u waves (k_waves: each on k-chunks of its own), %u K-split%s%s; 16-column tile copy",
-                     16 * f.nt, f.waves, f.splits, f.splits == 1 ? "" : "s", f.splits > 1 ? " + k_splitk_reduce" : "");
-        else
-            snprintf(text, bytes, "k_batch: %u waves (k_waves: each on k-chunks of its own), %u columns of 1 quad per workgroup, 1 tile per wave, "
-                     "%u K-split%s%s; 16-column tile copy", f.waves, 16 * f.nt, f.splits, f.splits == 1 ? "" : "s",
-                     f.splits > 1 ? " + k_splitk_reduce" : "");
+        snprintf(text, bytes, "k_waves: %u-row x %u-column blocks, %u waves on k-chunks of their own, %s weights, %u K-split%s%s; "
+                 "16-column tile copy", waves_block_rows(m), 16 * f.nt, f.waves, m <= 32 ? "exact" : "f16-rounded", f.splits,
+                 f.splits == 1 ? "" : "s", f.splits > 1 ? " + k_splitk_reduce" : "");
         break;
     case kFormStream: {
         const uint32_t sp = plan_stream(n_tiles, k_chunks, mb);

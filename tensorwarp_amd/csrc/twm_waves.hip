@@ -358,6 +358,8 @@ uint32_t waves_mt(uint32_t m)
 
 }  // namespace
 
+uint32_t waves_block_rows(uint32_t m) { return 16u * waves_mt(m); }
+
 // Once per device, outside any stream capture: the forms that ask for more than 64 KB of LDS.
 hipError_t init_waves()
 {
@@ -376,13 +378,14 @@ hipError_t init_waves()
 //   32 rows 15.0 / 14.5), 4608 with 17 .. 32 f32 rows on two tiles (5120 -> 5120 18.9 / 18.2), any depth with up to eight f32 rows (18944 -> 3584 20.2 / 20.7, 11008 -> 4096 14.4 / 15.5);
 // * up to six f16 rows, or eight on more than one tile, the lane-per-column sub-tiles are ahead from K = 2048 on (3584 ->
 //   3584 at 5 rows 5.3 / 4.8, at 8 rows 5.3 / 5.4);
-// * K is cut four ways only where at most 64 workgroups would run, each range keeping eight chunks (4864 -> 896 at 32
-//   rows 6.9 on four, 8.3 the other form);
+// * K is cut only where few workgroups would run, each range keeping eight chunks and more: four ways up to 64 of them
+//   (4864 -> 896 at 32 rows 6.9 on four, 8.3 the other form), two ways up to 128 with up to eight f32 rows on K above 12288
+//   and up to 112 above 32 rows;
 // * above 32 rows: while one or two tiles make one round (3584 -> 3584 at 128 rows 12.0 / 17.4, at 192 18.8 / 17.6), K up to
 //   6144, above 4096 only with most CUs busy (5632 -> 2048 at 64 rows 11.7 / 11.1, at 128 13.4 / 17.0); 33 .. 64 rows on a
-//   shallow K also two rounds of four-wave workgroups (2048 -> 11264 gated at 64 rows 15.8 / 17.9).  K = 896 and less would
-//   gain as well (896 -> 1152 at 64 rows 5.4 / 9.7) but stays with the prefill GEMM's blocks: the planner's tests hold that
-//   shape to them.
+//   shallow K also two rounds of four-wave workgroups (2048 -> 11264 gated at 64 rows 15.8 / 17.9).  The lower
+//   line, K of about 1024, is where the sweep above 32 rows began and not where the other forms get ahead: 896 -> 1152 at
+//   64 rows takes 5.4 here and 9.7 on the prefill GEMM's blocks, where it still runs.
 WavesPlan plan_waves(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated)
 {
     const WavesPlan none = {0, 0, 0};

@@ -51,7 +51,7 @@ def workgroups(f, k, n, m):
         return -(-(n_pad // 64) // (f["quads"] * f["tiles_per_wave"])) * f["splits"]
     if f["kernel"] == "k_stream":
         return n_pad // 64 * f["splits"]
-    if f["kernel"] == "k_prefill":
+    if f["kernel"] in ("k_prefill", "k_waves"):
         return -(-m // f["block_rows"]) * -(-n_pad // f["block_cols"]) * f["splits"]
     raise AssertionError(f["text"])
 
@@ -73,16 +73,16 @@ def test_plans_of_the_qwen7b_projections(lib, name, m, dtype):
         assert f["kernel"] in ("k_gemv4s", "k_gemv4") and f["copy"] == "column-lane copy", f["text"]
         assert f["splits"] == 1, f["text"]                   # (a hand-over between workgroups costs over a microsecond)
     elif m <= 16:
-        assert f["kernel"] in ("k_gemv4s", "k_gemv4", "k_stream", "k_batch"), f["text"]
+        assert f["kernel"] in ("k_gemv4s", "k_gemv4", "k_stream", "k_batch", "k_waves"), f["text"]
     else:
-        assert f["kernel"] == "k_batch" and f["copy"] == "16-column tile copy", f["text"]
+        assert f["kernel"] in ("k_batch", "k_waves") and f["copy"] == "16-column tile copy", f["text"]
     if m == 1:
         assert f["kernel"] == "k_gemv4s" and wgs >= CUS // 2, f["text"]
         if k_chunks <= 32:                                    # K up to 4096: a wave makes one pass or two, no loop
             assert f["waves"] * (64 // f["sub"]) * 2 >= k_chunks, f["text"]
         else:                                                 # deep K: sixteen columns, few waves, the pass loop
             assert f["sub"] == 16 and f["waves"] in (4, 8, 16), f["text"]
-    if f["kernel"] in ("k_stream", "k_batch"):
+    if f["kernel"] in ("k_stream", "k_batch", "k_waves"):
         assert f["copy"] == "16-column tile copy" and 1 <= f["splits"] <= 16, f["text"]
         unsplit = wgs // f["splits"]
         if f["splits"] > 1:
@@ -136,12 +136,37 @@ def test_pick_splits_agrees_with_the_described_plan(lib):
             assert kernel in ("k_gemv4", "k_gemv4s"), (k, n, m, text)
             assert "column-lane copy" in text
         if m > 16:
-            assert kernel == "k_batch", (k, n, m, text)
+            assert kernel in ("k_batch", "k_waves"), (k, n, m, text)
         if kernel == "k_gemv4s":
             sub, waves = map(int, re.search(r"(\d+)-column sub-tiles, (\d+) waves", text).groups())
             assert sub in (16, 32) and 1 <= waves <= 16
             if m > 4:   # rows beyond four repeat the MFMA chain: only in the one-pass form
                 assert waves * (64 // sub) >= k_chunks, (k, n, m, text)
+
+
+def test_plans_of_the_kernel_on_narrow_matrices(lib):
+    # k_waves: blocks of whole tiles that divide the padded columns and whose rows pad less than a block, its arithmetic by
+    # the row count, one round of workgroups on the CUs (two of the four-wave form), K cut only where that leaves CUs idle
+    rng = np.random.default_rng(11)
+    taken = set()
+    for _ in range(3000):
+        k, n = 32 * int(rng.integers(1, 200)), int(rng.integers(1, 20000))
+        m, gated = int(rng.integers(1, 260)), int(rng.integers(0, 2))
+        n = n // 64 * 64 + 64 if gated else n
+        dtype = _lib.F32 if rng.integers(0, 2) else _lib.F16
+        f = parse(describe(lib, k, n, m, dtype, gated))
+        if f["kernel"] != "k_waves":
+            continue
+        wgs, k_chunks = workgroups(f, k, n, m), (k // 32 + 3) // 4
+        assert 5 <= m <= 192 and f["copy"] == "16-column tile copy", f["text"]
+        assert f["block_cols"] in ((32, 64) if gated else (16, 32, 64)) and f["block_rows"] in (16, 32, 48, 64), f["text"]
+        assert (m <= 32) == (f["block_rows"] <= 32) == ("exact weights" in f["text"]) != ("f16-rounded weights" in f["text"]), f["text"]
+        assert -(-m // f["block_rows"]) * f["block_rows"] - m < f["block_rows"], f["text"]
+        assert wgs <= (CUS if f["waves"] == 8 else 2 * CUS) and (f["waves"] == 8 or 33 <= m <= 64), f["text"]
+        if f["splits"] > 1:
+            assert wgs // f["splits"] <= CUS // 2 and k_chunks // f["splits"] >= 8 and "k_splitk_reduce" in f["text"], f["text"]
+        taken.add((f["block_rows"], f["block_cols"]))
+    assert len(taken) >= 10, taken
 
 
 def test_describe_rejects_what_twm_gemm_rejects(lib):
