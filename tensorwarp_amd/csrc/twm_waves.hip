@@ -110,7 +110,8 @@ __global__ __launch_bounds__(64 * W) void k_waves(const uint4v *__restrict__ qw,
 
     // Load j of the tile takes rows 4 j .. 4 j + 3: lane L row 4 j + L / 16, vector (L % 16) ^ (row % 16) of its sixteen,
     // and writes it to slot L % 16 of that row.  Rows past m_rows replay the last row and are never stored; vectors past K
-    // replay the row's first vector of the chunk, where the padded weights are zero.
+    // replay the row's first vector of the chunk and are staged as zeros: an infinity there times the padded weights' zero
+    // would make the row's sums NaN.
     const char *a_blk = (const char *)a_any + (size_t)m0 * k * 2u;
     uint32_t a_off[NV], a_vec[4];
 #pragma unroll
@@ -151,7 +152,14 @@ __global__ __launch_bounds__(64 * W) void k_waves(const uint4v *__restrict__ qw,
             ws[slot][t] = __builtin_nontemporal_load((const TWM_GLOBAL uint2v *)(wv_scalar_base(sc, tile * 128u) + (s_off & on)));
         }
     };
-    auto stage_a = [&]() {
+    auto stage_a = [&](uint32_t i) {
+        const uint32_t left = k - chunk_at(i) * 128u;  // the row's values from this chunk on
+        if (left < 128u) {
+#pragma unroll
+            for (int t = 0; t < TERMS; t++)
+#pragma unroll
+                for (int j = 0; j < NV; j++) ar[t][j] = a_vec[j & 3] * 8u < left ? ar[t][j] : uint4v{0u, 0u, 0u, 0u};
+        }
 #pragma unroll
         for (int t = 0; t < TERMS; t++)
 #pragma unroll
@@ -229,7 +237,7 @@ __global__ __launch_bounds__(64 * W) void k_waves(const uint4v *__restrict__ qw,
         load_b(1, 1);
         __builtin_amdgcn_sched_barrier(0);
         auto step = [&](int slot, uint32_t i) {
-            stage_a();
+            stage_a(i);
             __builtin_amdgcn_sched_barrier(0);
             load_a(i + 1u);
             __builtin_amdgcn_sched_barrier(0);

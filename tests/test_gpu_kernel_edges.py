@@ -362,3 +362,27 @@ def test_a_column_lane_handle_keeps_its_one_copy_on_narrow_matrices(dev, m):
     assert w.copies == T.MarlinWeight.COPY_COLUMN_LANE
     graph.destroy()
     w.free()
+
+
+@pytest.mark.parametrize("k,m", [(416, 9), (416, 24), (2080, 7), (2080, 16), (1056, 40), (1056, 96)])
+def test_an_infinite_activation_reaches_every_column_as_itself(dev, k, m):
+    # K one group past a 128-deep chunk: the padded part of the last chunk must not multiply an infinity by its zero weights.
+    # The infinity stands in the first and last piece of that chunk, and in the first of the row.
+    n = 96
+    packed, scales, w = weight(dev, k, n, 2001)
+    dense = O.dequant_f32(packed, scales, k, n).reshape(k, n)
+    a16 = O.synth_act_f16(m, k, 2003)
+    rows = a16.view(np.float16).reshape(m, k).copy()
+    places = {1: k // 128 * 128, 3: k - 1, m - 1: 0}
+    for r, p in places.items():
+        rows[r, p] = np.inf
+    c = T.GpuTensor.from_host(dev, np.full((m, n), -1.0, np.float32))
+    T.gemm(dev, w, T.GpuTensor.from_host(dev, rows.view(np.uint16), "f16"), m, c)
+    got = c.to_host()
+    for r, p in places.items():
+        want = np.where(dense[p] == 0, np.nan, np.copysign(np.inf, dense[p])).astype(np.float32)
+        assert np.array_equal(got[r], want, equal_nan=True), (r, p)
+    others = [r for r in range(m) if r not in places]
+    truth = gemm_truth(rows[others].astype(np.float32), packed, scales, len(others), k, n)
+    close_rows(got[others], truth, F32_SUM if m <= 32 else 1e-3)
+    w.free()
