@@ -583,6 +583,16 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
     PrefillPlan best = {force_rows ? force_rows : 64u, force_splits ? force_splits : 1u, 1e30};
     const size_t n_ld = (size_t)n_tiles * 16;
     const double partial_us = (double)rows * (double)n_ld * 4.0 / 4.0e6;  // the reduce kernel's read of one split
+    // the split factors that differ in their work, once for all forms (a prompt's call plans on the host each time)
+    struct { uint32_t splits, chunks; } cuts[64];
+    uint32_t n_cuts = 0;
+    for (uint32_t sp = 1; sp <= 64; sp++) {
+        if (force_splits ? sp != force_splits : sp * 2 > (k_chunks > 1 ? k_chunks : 2) && sp > 1) continue;
+        const uint32_t cps = (k_chunks + sp - 1) / sp;
+        if (!force_splits && (k_chunks + cps - 1) / cps != sp) continue;  // same work as a smaller factor
+        cuts[n_cuts].splits = sp;
+        cuts[n_cuts++].chunks = cps;
+    }
     static const uint32_t kForms[] = {64, 128, 192, 49, 65, 97, 129};
     for (uint32_t bm : kForms) {
         const bool narrow = (bm & 1u) != 0;
@@ -591,16 +601,17 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
         const uint32_t col_blocks = bm == 192 ? (n_tiles + 11) / 12 : narrow ? (n_tiles + 7) / 8 : (n_tiles + 15) / 16;
         const uint32_t height = narrow ? bm - 1u : bm == 64 ? 64u : 128u;
         const double wgs = (double)((rows + height - 1) / height) * col_blocks;
-        for (uint32_t sp = 1; sp <= 64; sp++) {
-            if (force_splits ? sp != force_splits : sp * 2 > (k_chunks > 1 ? k_chunks : 2) && sp > 1) continue;
-            const uint32_t cps = (k_chunks + sp - 1) / sp;
-            if (!force_splits && (k_chunks + cps - 1) / cps != sp) continue;  // same work as a smaller factor
+        const double *chunk = nullptr;
+        for (const auto &f : kNarrow)
+            if (f.form == bm) chunk = f.chunk;
+        for (uint32_t i = 0; i < n_cuts; i++) {
+            const uint32_t sp = cuts[i].splits, cps = cuts[i].chunks;
+            if (!force_splits && sp > 1 && 5.5 + sp * partial_us >= best.us) break;  // (the sum kernel alone takes longer)
             const double total = wgs * sp;
             double t = 0.0;
             if (narrow) {
                 const uint32_t on_cu = ((uint32_t)total + 255u) / 256u;  // workgroups of the busiest CU
-                for (const auto &f : kNarrow)
-                    if (f.form == bm) t = cps * (on_cu / 3u * f.chunk[2] + (on_cu % 3u ? f.chunk[on_cu % 3u - 1u] : 0.0)) + 3.0;
+                t = cps * (on_cu / 3u * chunk[2] + (on_cu % 3u ? chunk[on_cu % 3u - 1u] : 0.0)) + 3.0;
             } else if (bm == 192 && total > 256.0) {
                 // two workgroups share a CU: 2.45 per chunk each; a last round of up to one per CU runs at 1.45
                 const double full = (double)(uint64_t)(total / 512.0), rem = total - 512.0 * full;
@@ -714,10 +725,13 @@ hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, boo
 {
     if (m == 0 || w.n == 0) return hipSuccess;
     if (block_rows != 0 && !prefill_form_known(block_rows)) return hipErrorInvalidValue;
+    uint32_t ran_splits = 1;  // of the last run
     auto run = [&](const _Float16 *a16, uint32_t rows, const OutSpec &o, void *ws, size_t ws_bytes, bool via = false) {
         // (a forced 192-column form with the gated store: the 256-column one)
         const uint32_t form = block_rows == 192 && o.swiglu ? 128u : block_rows;
         const PrefillPlan plan = plan_prefill_within(rows, form, splits, w.n_tiles, w.k_chunks, ws ? ws_bytes : 0, o.swiglu != nullptr);
+        const uint32_t cps = (w.k_chunks + plan.splits - 1) / plan.splits;
+        ran_splits = (w.k_chunks + cps - 1) / cps;
         switch (plan.block_rows) {
         case 49: return launch_prefill_t<3, 2, false, 4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
         case 65: return launch_prefill_t<4, 2, false, 4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
@@ -765,16 +779,11 @@ hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, boo
         size_t used = (size_t)((char *)a16 - (char *)scratch) + (((size_t)rows * w.k * 2 + 255) & ~(size_t)255);
         hipError_t e = run(a16, rows, o, (char *)scratch + used, scratch_bytes - used, after_sum);
         if (e != hipSuccess) return e;
-        if (!after_sum) {
-            const PrefillPlan plan = plan_prefill_within(rows, block_rows == 192 && o.swiglu ? 128u : block_rows, splits, w.n_tiles, w.k_chunks,
-                                                         scratch_bytes - used, false);
-            const uint32_t cps = (w.k_chunks + plan.splits - 1) / plan.splits;
-            if ((w.k_chunks + cps - 1) / cps == 1) {  // (with a K-split the sum kernel has applied the factors)
-                hipLaunchKernelGGL(k_scale_rows, dim3((rows + kScaleRows - 1) / kScaleRows, kScaleParts), dim3(256), 0, s, o,
-                                   (const float *)row_scale, rows);
-                e = hipGetLastError();
-                if (e != hipSuccess) return e;
-            }
+        if (!after_sum && ran_splits == 1) {  // (with a K-split the sum kernel has applied the factors)
+            hipLaunchKernelGGL(k_scale_rows, dim3((rows + kScaleRows - 1) / kScaleRows, kScaleParts), dim3(256), 0, s, o,
+                               (const float *)row_scale, rows);
+            e = hipGetLastError();
+            if (e != hipSuccess) return e;
         }
     }
     return hipGetLastError();
