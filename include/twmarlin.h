@@ -121,7 +121,7 @@ int twm_ctx_info(twm_ctx *ctx, char *buf, size_t buf_len);
  *   "tune_on_upload" new weight handles (twm_weight_upload, twm_weight_from_device, twm_weight_fuse_n; not the paired
  *                   gate/up handles) get measured plans at once, as if twm_weight_tune had been called on them: 1 = for
  *                   the decode row counts 1, 4, 8, 16, 32; 2 = also for the prefill row counts 128, 512, 2048; 0 (default)
- *                   = no.  Costs about half a second per row count and handle; a handle whose tuning fails is not returned.
+ *                   = no.  Costs up to 0.2 s per row count and handle; a handle whose tuning fails is not returned.
  *                   The tuner measures kernels of both repacked orders, so a tuned handle holds both copies whatever
  *                   "weight_copies" says (twm_weight_drop frees one afterwards).
  *   "weight_copies" the repacked orders a new weight handle is given: 0 or 3 = both, 1 = 16-column tiles only,
@@ -307,8 +307,8 @@ size_t twm_weight_bytes(const twm_weight *w);
  * No counterpart in the reference, whose kernels read the one TW-Marlin order. */
 /* Measured plans, the role of AutoTuner::tune_gemm and its per-shape table (crates/kernels/src/autotune.rs:254-396):
  * for each of the `count` row counts in ms[], times this weight's GEMM in the launch forms that the option knobs can
- * ask for (sub-tile widths and waves, whole tiles with K-splits, streaming and LDS-shared batched-decode forms, prefill
- * block heights and K-splits) on synthetic f16 activations -- as captured graphs replayed over copies of the weight that
+ * ask for (sub-tile widths and waves, whole tiles with K-splits, streaming and LDS-shared batched-decode forms, waves on
+ * k-chunks of their own, prefill block forms and K-splits) on synthetic f16 activations -- as captured graphs replayed over copies of the weight that
  * together exceed the 256 MB cache -- and keeps the fastest for that bucket of row counts (1, 2, 3-4, 5-8, ...
  * 513-1024, above) when it beats the planners' own choice by more than 2 %.  Later calls with f16
  * activations, splits = 0 and no knob set run the kept form (one of kernel 5 only while "prefill_min_m" and

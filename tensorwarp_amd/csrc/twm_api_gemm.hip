@@ -599,6 +599,7 @@ static void tune_candidates(uint32_t m, uint32_t k_chunks, bool waves, std::vect
         for (int nt : {1, 2, 4})                                        // waves on k-ranges of their own
             for (int sp : {1, 2, 4})
                 if (nt != 4 || m <= 32) add(5, nt, 0, 0, 0, sp, 0);
+    if (waves && m > 32 && m <= 64) add(5, 2, 4, 0, 0, 1, 0);           // (the four-wave form)
     if (m <= 4) {
     } else if (m <= 32) {
         for (int sp : {1, 2, 3, 4, 6, 8}) add(3, 0, 0, 0, 0, sp, 0);  // streaming kernel
@@ -607,8 +608,9 @@ static void tune_candidates(uint32_t m, uint32_t k_chunks, bool waves, std::vect
                 for (int sp : {1, 2, 3, 4, 6})
                     if (!(wv == 16 && nt != 1) && !(wv == 8 && nt == 3)) add(4, nt, wv, 0, 0, sp, 0);
     } else {
-        for (int bm : {64, 128, 192})
-            for (int sp : {1, 2, 3, 4, 6, 8}) add(0, 0, 0, 0, 0, sp, bm);
+        for (int bm : {64, 128, 192, 49, 65, 97, 129})                   // (128-column blocks: up to 256 rows, as the planner)
+            if (!(bm & 1) || m <= 256)
+                for (int sp : {1, 2, 3, 4, 6, 8}) add(0, 0, 0, 0, 0, sp, bm);
     }
 }
 
