@@ -93,14 +93,29 @@ struct QGroup {
     uint32_t w[4];
 };
 
-// Group grids: blockIdx.y and .z count the groups (.y holds at most 65535 of them), blockIdx.x the columns of one, so that
-// no thread divides a 64-bit index.
-__device__ __forceinline__ uint32_t block_group() { return blockIdx.z * gridDim.y + blockIdx.y; }
-
-static dim3 group_grid(uint32_t blocks, uint32_t groups)
+// One thread per (group, column) of a matrix, columns next to each other, groups one after the other without a gap whatever
+// the width: blockIdx.x counts the places of `slab` groups, as many as 31 bits index, and blockIdx.y the slabs, so that a
+// thread divides 32 bits and not 64.  (A workgroup on 256 columns of one group leaves most of its threads idle on narrow
+// matrices and behind the last 256 columns: 1048576 x 1 quantized 20.4 us, now 7.0, 18944 x 260 7.0, now 5.0.)
+struct Place {
+    uint32_t group, column;
+};
+__device__ __forceinline__ bool place_of(uint32_t groups, uint32_t columns, uint32_t slab, Place &p)
 {
-    const uint32_t y = groups < 65535u ? groups : 65535u;
-    return dim3(blocks, y, (groups + y - 1) / y);
+    const uint32_t at = blockIdx.x * 256u + threadIdx.x, q = at / columns;
+    p.group = blockIdx.y * slab + q;
+    p.column = at - q * columns;
+    return q < slab && p.group < groups;
+}
+static uint32_t place_slab(uint32_t groups, uint32_t columns)
+{
+    const uint32_t most = columns < 0x80000000u ? 0x7FFFFFFFu / columns : 1u;
+    return groups < most ? groups : most;
+}
+static dim3 place_grid(uint32_t groups, uint32_t columns)
+{
+    const uint32_t slab = place_slab(groups, columns);
+    return dim3((unsigned)(((uint64_t)slab * columns + 255) / 256), (groups + slab - 1) / slab);
 }
 
 // The general form: any values, NaN and infinity among them.
@@ -161,10 +176,12 @@ __device__ __forceinline__ QGroup quantize_group32(const float *vals)
 
 // One thread per (group, column) of a [K,N] matrix: lanes take neighbouring columns.
 __global__ __launch_bounds__(256) void k_quantize_q4_0(const float *__restrict__ w, uint32_t k, uint32_t n,
-                                                        uint8_t *__restrict__ q4)
+                                                        uint8_t *__restrict__ q4, uint32_t slab)
 {
-    const uint32_t groups = k / 32, g = block_group(), col = blockIdx.x * 256u + threadIdx.x;
-    if (g >= groups || col >= n) return;
+    const uint32_t groups = k / 32;
+    Place at;
+    if (!place_of(groups, n, slab, at)) return;
+    const uint32_t g = at.group, col = at.column;
     float vals[32];
 #pragma unroll
     for (int i = 0; i < 32; i++) vals[i] = w[((size_t)g * 32 + i) * n + col];
@@ -175,10 +192,11 @@ __global__ __launch_bounds__(256) void k_quantize_q4_0(const float *__restrict__
 }
 
 __global__ __launch_bounds__(256) void k_quantize_twm_kn(const float *__restrict__ w, uint32_t groups, uint32_t n, uint4v *__restrict__ packed,
-                                                          uint16_t *__restrict__ scales)
+                                                          uint16_t *__restrict__ scales, uint32_t slab)
 {
-    const uint32_t g = block_group(), col = blockIdx.x * 256u + threadIdx.x;
-    if (g >= groups || col >= n) return;
+    Place at;
+    if (!place_of(groups, n, slab, at)) return;
+    const uint32_t g = at.group, col = at.column;
     float vals[32];
 #pragma unroll
     for (int i = 0; i < 32; i++) vals[i] = __builtin_nontemporal_load(w + ((size_t)g * 32 + i) * n + col);
@@ -188,36 +206,40 @@ __global__ __launch_bounds__(256) void k_quantize_twm_kn(const float *__restrict
 }
 
 // [N,K]: a column's values lie along K and its neighbours K floats away, so a workgroup takes 64 columns x four groups
-// through LDS: 32 lanes read 512 contiguous bytes of a column (with a thread reading its own 128 bytes every load touched
-// 64 lines: 3584 x 18944, 314 MB, 80 us, now 52.2 at 6.0 TB/s), then a thread per (group, column) quantizes.  A column's 32
-// slots of 16 bytes stand 33 apart, so that the 64 columns of a read fall on different banks.  The f32 matrix is read once
-// and passes the caches (61 us through them).
+// (bits = 6; NARROW: of matrices with fewer columns 2^bits of them x more groups: 1048576 x 1 22.4 us on 64, now 3.4) through LDS:
+// 32 lanes read 512 contiguous bytes of a column (with a thread reading its own 128 bytes every load touched 64 lines:
+// 3584 x 18944, 314 MB, 80 us, now 52.2 at 6.0 TB/s), then a thread per (group, column) quantizes.  A column's 32 slots of
+// 16 bytes stand 33 apart, so that the 64 columns of a read fall on different banks.  The f32 matrix is read once and passes
+// the caches (61 us through them).  blockIdx.y and .z count the groups (.y holds at most 65535).
+template <bool NARROW>
 __global__ __launch_bounds__(256) void k_quantize_twm_nk(const float *__restrict__ w, uint32_t k, uint32_t n,
-                                                          uint4v *__restrict__ packed, uint16_t *__restrict__ scales)
+                                                          uint4v *__restrict__ packed, uint16_t *__restrict__ scales, uint32_t narrow_bits)
 {
-    __shared__ float4v tile[64 * 33];
-    const uint32_t groups = k / 32, g0 = block_group() * 4u, col0 = blockIdx.x * 64u;
+    const uint32_t bits = NARROW ? narrow_bits : 6u;
+    __shared__ float4v tile[64 * 33];  // (2^bits columns of 2^(11 - bits) slots and one more: 2048 + 2^bits of them)
+    const uint32_t groups = k / 32, tall = 256u >> bits, g0 = (blockIdx.z * gridDim.y + blockIdx.y) * tall, col0 = blockIdx.x << bits;
     if (g0 >= groups) return;
-    const uint32_t slots = (groups - g0 < 4u ? groups - g0 : 4u) * 8u;  // 16-byte slots of a column in this tile
+    const uint32_t slots = (groups - g0 < tall ? groups - g0 : tall) * 8u;  // 16-byte slots of a column in this tile
+    const uint32_t slot_bits = 11u - bits, slot_mask = (1u << slot_bits) - 1u, stride = slot_mask + 2u;
     float4v v[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const uint32_t at = i * 256u + threadIdx.x, c = at >> 5, slot = at & 31u;
+        const uint32_t at = i * 256u + threadIdx.x, c = at >> slot_bits, slot = at & slot_mask;
         const uint32_t col = col0 + c < n ? col0 + c : n - 1;
         v[i] = __builtin_nontemporal_load((const float4v *)(w + (size_t)col * k + (size_t)g0 * 32) + (slot < slots ? slot : 0u));
     }
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         const uint32_t at = i * 256u + threadIdx.x;
-        tile[(at >> 5) * 33u + (at & 31u)] = v[i];
+        tile[(at >> slot_bits) * stride + (at & slot_mask)] = v[i];
     }
     __syncthreads();
-    const uint32_t c = threadIdx.x & 63u, g = g0 + (threadIdx.x >> 6), col = col0 + c;
+    const uint32_t c = threadIdx.x & ((1u << bits) - 1u), row = threadIdx.x >> bits, g = g0 + row, col = col0 + c;
     if (g >= groups) return;
     float vals[32];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const float4v x = tile[c * 33u + (threadIdx.x >> 6) * 8u + i];
+        const float4v x = tile[c * stride + row * 8u + i];
 #pragma unroll
         for (int j = 0; j < 4; j++) vals[4 * i + j] = x[j];
     }
@@ -230,7 +252,7 @@ __global__ __launch_bounds__(256) void k_quantize_twm_nk(const float *__restrict
 hipError_t launch_quantize_q4_0(hipStream_t s, const float *w_kn, uint32_t k, uint32_t n, uint8_t *q4)
 {
     if (k / 32 == 0 || n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_quantize_q4_0, group_grid((n + 255) / 256, k / 32), dim3(256), 0, s, w_kn, k, n, q4);
+    hipLaunchKernelGGL(k_quantize_q4_0, place_grid(k / 32, n), dim3(256), 0, s, w_kn, k, n, q4, place_slab(k / 32, n));
     return hipGetLastError();
 }
 
@@ -239,8 +261,16 @@ hipError_t launch_quantize_twm(hipStream_t s, const float *w, int w_is_nk, uint3
 {
     const uint32_t groups = k / 32;
     if (groups == 0 || n == 0) return hipSuccess;
-    if (w_is_nk) hipLaunchKernelGGL(k_quantize_twm_nk, group_grid((n + 63) / 64, (groups + 3) / 4), dim3(256), 0, s, w, k, n, (uint4v *)packed, scales);
-    else hipLaunchKernelGGL(k_quantize_twm_kn, group_grid((n + 255) / 256, groups), dim3(256), 0, s, w, groups, n, (uint4v *)packed, scales);
+    if (w_is_nk) {
+        uint32_t bits = 0;
+        while (bits < 6 && (1u << bits) < n) bits++;
+        const uint32_t tall = 256u >> bits, blocks = (groups + tall - 1) / tall, y = blocks < 65535u ? blocks : 65535u;
+        const dim3 grid((n >> bits) + ((n & ((1u << bits) - 1u)) != 0), y, (blocks + y - 1) / y);
+        if (bits < 6) hipLaunchKernelGGL(k_quantize_twm_nk<true>, grid, dim3(256), 0, s, w, k, n, (uint4v *)packed, scales, bits);
+        else hipLaunchKernelGGL(k_quantize_twm_nk<false>, grid, dim3(256), 0, s, w, k, n, (uint4v *)packed, scales, bits);
+    } else {
+        hipLaunchKernelGGL(k_quantize_twm_kn, place_grid(groups, n), dim3(256), 0, s, w, groups, n, (uint4v *)packed, scales, place_slab(groups, n));
+    }
     return hipGetLastError();
 }
 
@@ -271,10 +301,12 @@ hipError_t launch_reorder(hipStream_t s, const uint8_t *q4, uint32_t k, uint32_t
 
 __global__ __launch_bounds__(256) void k_fuse_one(const uint4v *__restrict__ pin, const uint16_t *__restrict__ sin,
                                                    uint32_t groups, uint32_t ni, uint32_t total_n,
-                                                   uint32_t col_off, uint4v *__restrict__ pout, uint16_t *__restrict__ sout)
+                                                   uint32_t col_off, uint4v *__restrict__ pout, uint16_t *__restrict__ sout,
+                                                   uint32_t slab)
 {
-    const uint32_t g = block_group(), c = blockIdx.x * 256u + threadIdx.x;
-    if (g >= groups || c >= ni) return;
+    Place at;
+    if (!place_of(groups, ni, slab, at)) return;
+    const uint32_t g = at.group, c = at.column;
     const size_t idx = (size_t)g * ni + c, dst = (size_t)g * total_n + col_off + c;
     pout[dst] = pin[idx];
     sout[dst] = sin[idx];
@@ -284,8 +316,8 @@ hipError_t launch_fuse_one(hipStream_t s, const uint8_t *packed_in, const uint16
                            uint32_t ni, uint32_t total_n, uint32_t col_off, uint8_t *packed_out, uint16_t *scales_out)
 {
     if (groups == 0 || ni == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fuse_one, group_grid((ni + 255) / 256, groups), dim3(256), 0, s, (const uint4v *)packed_in,
-                       scales_in, groups, ni, total_n, col_off, (uint4v *)packed_out, scales_out);
+    hipLaunchKernelGGL(k_fuse_one, place_grid(groups, ni), dim3(256), 0, s, (const uint4v *)packed_in,
+                       scales_in, groups, ni, total_n, col_off, (uint4v *)packed_out, scales_out, place_slab(groups, ni));
     return hipGetLastError();
 }
 
@@ -298,12 +330,13 @@ hipError_t launch_fuse_one(hipStream_t s, const uint8_t *packed_in, const uint16
 // on whatever runs next; records loaded past the caches as well cost 25 us of the gain, since they are often just written.
 template <int COLS, bool F16OUT>
 __global__ __launch_bounds__(256) void k_dequant(const uint4v *__restrict__ packed, const uint16_t *__restrict__ scales,
-                                                  uint32_t groups, uint32_t n, void *__restrict__ out)
+                                                  uint32_t groups, uint32_t n, void *__restrict__ out, uint32_t slab)
 {
     typedef uint16_t halves __attribute__((ext_vector_type(COLS)));
     typedef float floats __attribute__((ext_vector_type(COLS)));
-    const uint32_t g = block_group(), col = (blockIdx.x * 256u + threadIdx.x) * COLS;
-    if (g >= groups || col >= n) return;
+    Place place;
+    if (!place_of(groups, n / COLS, slab, place)) return;
+    const uint32_t g = place.group, col = place.column * COLS;
     const size_t rec = (size_t)g * n + col;
     uint4v w[COLS];
     float sc[COLS];
@@ -339,10 +372,11 @@ __global__ __launch_bounds__(256) void k_dequant(const uint4v *__restrict__ pack
 // records at any address: a byte and an element per thread
 template <bool F16OUT>
 __global__ __launch_bounds__(256) void k_dequant_bytes(const uint8_t *__restrict__ packed, const uint16_t *__restrict__ scales,
-                                                        uint32_t k, uint32_t n, void *__restrict__ out)
+                                                        uint32_t k, uint32_t n, void *__restrict__ out, uint32_t slab)
 {
-    const uint32_t row = block_group(), col = blockIdx.x * 256u + threadIdx.x;
-    if (row >= k || col >= n) return;
+    Place at;
+    if (!place_of(k, n, slab, at)) return;
+    const uint32_t row = at.group, col = at.column;
     const uint32_t g = row / 32, e = row % 32;
     const size_t idx = (size_t)row * n + col;
     uint8_t byte = packed[((size_t)g * n + col) * 16 + e / 2];
@@ -356,20 +390,24 @@ hipError_t launch_dequant(hipStream_t s, const uint8_t *packed, const uint16_t *
                           void *out, bool f16_out)
 {
     if (k == 0 || n == 0) return hipSuccess;
-    if (((uintptr_t)packed & 15) != 0) {
-        const dim3 grid = group_grid((n + 255) / 256, k);
-        if (f16_out) hipLaunchKernelGGL(k_dequant_bytes<true>, grid, dim3(256), 0, s, packed, scales, k, n, out);
-        else hipLaunchKernelGGL(k_dequant_bytes<false>, grid, dim3(256), 0, s, packed, scales, k, n, out);
+    // An element per thread where the records are not aligned -- and where a record per thread would be few workgroups (4096 x
+    // 64: 2.5 us, here 2.2) or put a wave's stores on as many lines as it has lanes (1048576 x 1: 9.4, here 3.2).
+    if (((uintptr_t)packed & 15) != 0 || n < 8 || (uint64_t)(k / 32) * n < 32768u) {
+        const dim3 grid = place_grid(k, n);
+        const uint32_t slab = place_slab(k, n);
+        if (f16_out) hipLaunchKernelGGL(k_dequant_bytes<true>, grid, dim3(256), 0, s, packed, scales, k, n, out, slab);
+        else hipLaunchKernelGGL(k_dequant_bytes<false>, grid, dim3(256), 0, s, packed, scales, k, n, out, slab);
         return hipGetLastError();
     }
     // two columns per thread where a row's columns keep the alignment of the paired stores
     const bool pairs = n % 2 == 0 && ((uintptr_t)out & (f16_out ? 3 : 7)) == 0;
-    const dim3 grid = group_grid((n + (pairs ? 511 : 255)) / (pairs ? 512 : 256), k / 32);
+    const uint32_t groups = k / 32, columns = pairs ? n / 2 : n, slab = place_slab(groups, columns);
+    const dim3 grid = place_grid(groups, columns);
     const uint4v *rec = (const uint4v *)packed;
-    if (pairs && f16_out) hipLaunchKernelGGL((k_dequant<2, true>), grid, dim3(256), 0, s, rec, scales, k / 32, n, out);
-    else if (pairs) hipLaunchKernelGGL((k_dequant<2, false>), grid, dim3(256), 0, s, rec, scales, k / 32, n, out);
-    else if (f16_out) hipLaunchKernelGGL((k_dequant<1, true>), grid, dim3(256), 0, s, rec, scales, k / 32, n, out);
-    else hipLaunchKernelGGL((k_dequant<1, false>), grid, dim3(256), 0, s, rec, scales, k / 32, n, out);
+    if (pairs && f16_out) hipLaunchKernelGGL((k_dequant<2, true>), grid, dim3(256), 0, s, rec, scales, groups, n, out, slab);
+    else if (pairs) hipLaunchKernelGGL((k_dequant<2, false>), grid, dim3(256), 0, s, rec, scales, groups, n, out, slab);
+    else if (f16_out) hipLaunchKernelGGL((k_dequant<1, true>), grid, dim3(256), 0, s, rec, scales, groups, n, out, slab);
+    else hipLaunchKernelGGL((k_dequant<1, false>), grid, dim3(256), 0, s, rec, scales, groups, n, out, slab);
     return hipGetLastError();
 }
 

@@ -235,6 +235,40 @@ def test_unpack_columns_and_alignments(dev, k, n, offset):
         assert np.array_equal(out.to_host().view(want.dtype), want), f16
 
 
+# [N,K] tiles of 2 .. 64 columns, of which 67 groups leave a remainder; rows of a workgroup's 256 places that end anywhere
+@pytest.mark.parametrize("n", [2, 5, 16, 31, 64, 100, 130, 250, 260, 512])
+def test_format_kernels_on_narrow_matrices(dev, n):
+    k = 67 * 32
+    w = np.random.default_rng(n).standard_normal((n, k), dtype=np.float32)
+    kn = np.ascontiguousarray(w.T)
+    want_p, want_s = O.quantize_tw_marlin_nk(w, k, n)
+    for x, nk in ((w, True), (kn, False)):
+        p, s = T.quantize_f32_to_tw_marlin(dev, T.GpuTensor.from_host(dev, x), k, n, weights_are_nk=nk)
+        assert np.array_equal(p.to_host(), want_p) and np.array_equal(s.to_host().view(np.uint16), want_s.view(np.uint16)), nk
+    q4 = T.quantize_weights_q4_0(dev, T.GpuTensor.from_host(dev, kn), k, n)
+    assert np.array_equal(q4.to_host().reshape(-1), O.quantize_weights_q4_0_kn(kn, k, n).reshape(-1))
+    fp, fs = T.fuse_tw_marlin_n(dev, [(p, s), (p, s)], k, [n, n])
+    wp, ws = O.fuse_tw_marlin_n([(want_p, want_s)] * 2, k, [n, n])
+    assert np.array_equal(fp.to_host(), wp) and np.array_equal(fs.to_host(), ws)
+    assert np.array_equal(T.dequant_to_f16(dev, p, s, k, n).to_host().view(np.uint16), O.dequant_f16(want_p, want_s, k, n))
+    assert np.array_equal(T.dequant_to_f32(dev, p, s, k, n).to_host().view(np.uint32), O.dequant_f32(want_p, want_s, k, n).view(np.uint32))
+
+
+# from 32768 records and eight columns on a thread unpacks whole records, two of them where columns and output allow it
+@pytest.mark.parametrize("k,n", [(4096, 256), (4096, 257), (4096, 258), (131072, 8), (116544, 9), (4096, 255)])
+@pytest.mark.parametrize("out_offset", [0, 1])
+def test_unpack_of_whole_records(dev, k, n, out_offset):
+    packed, scales = O.synth_packed(k, n, 5), O.synth_scales(k, n, 6)
+    raw, sc = T.GpuTensor.from_host(dev, packed), T.GpuTensor.from_host(dev, scales)
+    for f16, want in ((True, O.dequant_f16(packed, scales, k, n)), (False, O.dequant_f32(packed, scales, k, n).view(np.uint32))):
+        out = T.GpuTensor.from_host(dev, np.full(k * n + 2, 7, want.dtype if f16 else np.int32))
+        call = dev._l.twm_dequant_to_f16 if f16 else dev._l.twm_dequant_to_f32
+        assert call(dev.handle, raw.ptr, sc.ptr, k, n, out.ptr + out_offset * (2 if f16 else 4)) == 0
+        got = out.to_host().view(want.dtype)
+        assert np.array_equal(got[out_offset:out_offset + k * n], want.reshape(-1)), f16
+        assert (got[:out_offset] == 7).all() and (got[out_offset + k * n:] == 7).all()
+
+
 @pytest.mark.parametrize("k,ns", [(32, [1]), (64, [255, 1, 257]), (2097184, [2, 1])])
 def test_fuse_of_ragged_parts(dev, k, ns):
     parts = [(O.synth_packed(k, n, 7 + i), O.synth_scales(k, n, 8 + i)) for i, n in enumerate(ns)]
