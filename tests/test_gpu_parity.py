@@ -1689,6 +1689,8 @@ def test_plan_description_follows_the_context_options(dev):
     # the split factor is: it changes the summation order)
     k, n = 3584, 3584
     assert dev.plan(k, n, 1).startswith("k_gemv4s: 16-column sub-tiles, 8 waves")
+    plain16 = dev.plan(k, n, 16)
+    assert plain16.startswith(("k_gemv4s:", "k_waves:"))
     dev.set_option("sub", 1)
     try:
         assert dev.plan(k, n, 1).startswith("k_gemv4: 1 x 64-column tiles per workgroup")
@@ -1704,7 +1706,7 @@ def test_plan_description_follows_the_context_options(dev):
         assert dev.plan(k, n, 16).startswith("k_prefill:")
     finally:
         dev.set_option("prefill_min_m", 33)
-    assert dev.plan(k, n, 16).startswith("k_gemv4s:")
+    assert dev.plan(k, n, 16) == plain16
     assert dev.plan(3584, 37888, 1, gated=True).startswith("k_gemv4s: 32-column sub-tiles")
     assert dev.plan(18944, 3584, 1, dtype="f32") == "k_gemv4s: 16-column sub-tiles, 4 waves, 1 K-split; column-lane copy"
     # the drop-in on the reference's arrays: its own planner and options
