@@ -110,8 +110,9 @@ __global__ __launch_bounds__(64 * W) void k_waves(const uint4v *__restrict__ qw,
 
     // Load j of the tile takes rows 4 j .. 4 j + 3: lane L row 4 j + L / 16, vector (L % 16) ^ (row % 16) of its sixteen,
     // and writes it to slot L % 16 of that row.  Rows past m_rows replay the last row and are never stored; vectors past K
-    // replay the row's first vector of the chunk and are staged as zeros: an infinity there times the padded weights' zero
-    // would make the row's sums NaN.
+    // replay the row's first vector of the chunk, where the padded weights are zero -- and, up to sixteen f16 rows, are staged
+    // as zeros: an infinity in that vector times a zero weight would make the row's sums NaN.  (Above that k_batch and
+    // k_prefill, which take these rows on other shapes, replay it as well; there the masks cost 1 % of the launch.)
     const char *a_blk = (const char *)a_any + (size_t)m0 * k * 2u;
     uint32_t a_off[NV], a_vec[4];
 #pragma unroll
@@ -153,12 +154,12 @@ __global__ __launch_bounds__(64 * W) void k_waves(const uint4v *__restrict__ qw,
         }
     };
     auto stage_a = [&](uint32_t i) {
-        const uint32_t left = k - chunk_at(i) * 128u;  // the row's values from this chunk on
-        if (left < 128u) {
+        if constexpr (MT == 1 && TERMS == 1) {
+            const uint32_t left = k - chunk_at(i) * 128u;  // the row's values from this chunk on
+            if (left < 128u) {
 #pragma unroll
-            for (int t = 0; t < TERMS; t++)
-#pragma unroll
-                for (int j = 0; j < NV; j++) ar[t][j] = a_vec[j & 3] * 8u < left ? ar[t][j] : uint4v{0u, 0u, 0u, 0u};
+                for (int j = 0; j < NV; j++) ar[0][j] = a_vec[j & 3] * 8u < left ? ar[0][j] : uint4v{0u, 0u, 0u, 0u};
+            }
         }
 #pragma unroll
         for (int t = 0; t < TERMS; t++)

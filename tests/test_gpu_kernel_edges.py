@@ -398,10 +398,11 @@ def test_a_column_lane_handle_keeps_its_one_copy_on_narrow_matrices(dev, m):
     w.free()
 
 
-@pytest.mark.parametrize("k,m", [(416, 9), (416, 24), (2080, 7), (2080, 16), (1056, 40), (1056, 96)])
+@pytest.mark.parametrize("k,m", [(416, 9), (416, 16), (992, 5), (2080, 8), (2080, 16)])
 def test_an_infinite_activation_reaches_every_column_as_itself(dev, k, m):
     # K one group past a 128-deep chunk: the padded part of the last chunk must not multiply an infinity by its zero weights.
-    # The infinity stands in the first and last piece of that chunk, and in the first of the row.
+    # The infinity stands in the first and last piece of that chunk, and in the first of the row.  (Row counts and depths
+    # that k_waves takes.)
     n = 96
     packed, scales, w = weight(dev, k, n, 2001)
     dense = O.dequant_f32(packed, scales, k, n).reshape(k, n)
@@ -417,6 +418,6 @@ def test_an_infinite_activation_reaches_every_column_as_itself(dev, k, m):
         want = np.where(dense[p] == 0, np.nan, np.copysign(np.inf, dense[p])).astype(np.float32)
         assert np.array_equal(got[r], want, equal_nan=True), (r, p)
     others = [r for r in range(m) if r not in places]
-    truth = gemm_truth(rows[others].astype(np.float32), packed, scales, len(others), k, n)
-    close_rows(got[others], truth, F32_SUM if m <= 32 else 1e-3)
+    truth = O.gemm_f64(rows[others].astype(np.float32), packed, scales, len(others), k, n)
+    close_rows(got[others], truth, F32_SUM)
     w.free()
