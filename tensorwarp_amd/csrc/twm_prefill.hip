@@ -760,11 +760,10 @@ hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, boo
     if (!scratch || scratch_bytes < row_bytes + 512) return hipErrorInvalidValue;
     uint32_t slab = (uint32_t)((scratch_bytes - 512) / 2 / row_bytes < m ? (scratch_bytes - 512) / 2 / row_bytes : m);
     if (slab == 0) slab = 1;
-    const uint32_t slabs = (m + slab - 1) / slab;
-    if (slab >= 128) {  // whole row blocks, the slabs of about equal height
+    if (slab < m && slab >= 128) {  // several slabs: of whole row blocks, about equally high
         slab -= slab % 128;
-        const uint32_t even = ((m + slabs - 1) / slabs + 127) / 128 * 128;
-        if (even < slab) slab = even;
+        const uint32_t slabs = (m + slab - 1) / slab;
+        slab = ((m + slabs - 1) / slabs + 127) / 128 * 128;
     }
     for (uint32_t r0 = 0; r0 < m; r0 += slab) {
         uint32_t rows = m - r0 < slab ? m - r0 : slab;

@@ -94,6 +94,35 @@ def test_scaled_f32_rows_of_a_prompt_in_one_and_two_slabs(dev, m, k):
     w.free()
 
 
+@pytest.mark.parametrize("m", [130, 160, 255, 400])
+@pytest.mark.parametrize("gated", [False, True])
+def test_f32_prompt_rows_that_fit_run_as_the_f16_rows_do(dev, m, gated):
+    # f16 values as f32 rows, all of them in the scratch at once: one launch under the f16 rows' plan, so the same sums in the
+    # same order (a gated launch goes through the K-split's buffer: the same products of the same sums)
+    k, n = 2720, 1088
+    packed, scales = O.synth_packed(k, n, 611), O.synth_scales(k, n, 612)
+    if gated:
+        half = n // 2
+        p, s = packed.reshape(k // 32, n, 16), scales.reshape(k // 32, n)
+        pair = [(T.GpuTensor.from_host(dev, np.ascontiguousarray(p[:, c])), T.GpuTensor.from_host(dev, np.ascontiguousarray(s[:, c]), "f16"))
+                for c in (slice(0, half), slice(half, n))]
+        w = T.MarlinWeight.gate_up(dev, *pair, k, half)
+    else:
+        half, w = n, T.MarlinWeight.upload(dev, packed, scales, k, n)
+    a16 = O.synth_act_f16(m, k, 613)
+    got = []
+    dev.set_option("prefill_bm", 64)     # (the prefill GEMM at every one of these row counts)
+    try:
+        for rows in (T.GpuTensor.from_host(dev, a16, "f16"), T.GpuTensor.from_host(dev, a16.view(np.float16).astype(np.float32))):
+            out = T.GpuTensor.from_host(dev, np.full((m, half), np.nan, np.float32))
+            (T.gemm_swiglu if gated else T.gemm)(dev, w, rows, m, out)
+            got.append(out.to_host())
+    finally:
+        dev.set_option("prefill_bm", 0)
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
+    w.free()
+
+
 @pytest.mark.parametrize("m", [9, 16, 17, 32])
 @pytest.mark.parametrize("ffn,nt,waves", [(32, 0, 0), (96, 3, 0), (160, 3, 0), (96, 4, 8), (64, 1, 16)])
 def test_batched_gate_through_lds(dev, m, ffn, nt, waves):
