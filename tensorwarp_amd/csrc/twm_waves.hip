@@ -385,16 +385,21 @@ hipError_t init_waves()
 //   up to eight f32 rows (2048 -> 11264 gated 10.2 / 11.1), and not for 17 .. 32 f32 rows (25.2 / 23.6);
 // * deep K: up to 8192 with f16 rows and 16 of them (11008 -> 4096 level), 6144 with more or with f32 rows (11008 -> 4096 at
 //   32 rows 15.0 / 14.5), 4608 with 17 .. 32 f32 rows on two tiles (5120 -> 5120 18.9 / 18.2), any depth with up to eight f32 rows (18944 -> 3584 20.2 / 20.7, 11008 -> 4096 14.4 / 15.5);
-// * up to six f16 rows, or eight on more than one tile, the lane-per-column sub-tiles are ahead from K = 2048 on (3584 ->
-//   3584 at 5 rows 5.3 / 4.8, at 8 rows 5.3 / 5.4);
+// * up to six f16 rows, seven up to K = 4096, or eight on more than one tile, the lane-per-column sub-tiles are ahead from
+//   K = 2048 on (3584 -> 3584 at 5 rows 5.3 / 4.8, 4096 -> 4096 at 7 rows 6.2 / 5.9, at 8 rows 6.2 / 6.1, 4224 -> 896 at 7
+//   rows 5.7 / 6.2); up to eight f16 rows on more than one tile the streaming kernel is on K of 800 .. 1024 (896 -> 8192 at 5
+//   rows 4.8 / 4.6, 1024 -> 6144 gated at 7 rows 5.1 / 4.7; 640 -> 5120 4.2 / 4.4, 1536 -> 8192 5.6 / 5.7) and on more than
+//   6144 gated columns of a shallower K (512 -> 8192 gated at 8 rows 4.4 / 4.2);
 // * K is cut only where few workgroups would run, each range keeping eight chunks and more: four ways up to 64 of them
 //   (4864 -> 896 at 32 rows 6.9 on four, 8.3 the other form), two ways up to 128 with up to eight f32 rows on K above 12288
 //   and up to 112 above 32 rows;
-// * above 32 rows: while one or two tiles make one round (3584 -> 3584 at 128 rows 12.0 / 17.4, at 192 18.8 / 17.6), K up to
-//   6144, above 4096 only with most CUs busy (5632 -> 2048 at 64 rows 11.7 / 11.1, at 128 13.4 / 17.0); 33 .. 64 rows on a
-//   shallow K also two rounds of four-wave workgroups (2048 -> 11264 gated at 64 rows 15.8 / 17.9).  The lower
-//   line, K of about 1024, is where the sweep above 32 rows began and not where the other forms get ahead: 896 -> 1152 at
-//   64 rows takes 5.4 here and 9.7 on the prefill GEMM's blocks, where it still runs.
+// * above 32 rows: while one or two tiles make one round (3584 -> 3584 at 128 rows 12.0 / 17.4, at 192 18.8 / 17.6), which
+//   with several row blocks is 32 workgroups on each XCD, column groups being dealt eight at a time: 2656 -> 2656 at 192 rows
+//   is 252 workgroups, but 33 of them on four of the XCDs (20.2 / 13.1), and 5120 -> 320 at 160 rows on four K-ranges 36 on
+//   each (13.3, on two 10.5).  K up to 6144, above 4096 only with most CUs busy (5632 -> 2048 at 64 rows 11.7 / 11.1, at 128
+//   13.4 / 17.0); 33 .. 64 rows on a shallow K also two rounds of four-wave workgroups (2048 -> 11264 gated at 64 rows 15.8 /
+//   17.9).  The lower line, K of about 1024, is where the sweep above 32 rows began and not where the other forms get ahead:
+//   896 -> 1152 at 64 rows takes 5.4 here and 9.7 on the prefill GEMM's blocks, where it still runs.
 WavesPlan plan_waves(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated)
 {
     const WavesPlan none = {0, 0, 0};
@@ -404,7 +409,10 @@ WavesPlan plan_waves(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32
         uint32_t nt = n_tiles <= 256 ? 1u : n_tiles <= 512 ? 2u : n_tiles <= 1024 ? 4u : 0u;
         if (gated && nt == 1) nt = 2;
         if (nt == 0 || (nt == 4 && !few_f32 && (k_chunks < 24 || (a_f32 && m > 16)))) return none;
-        if (!a_f32 && m <= 8 && k_chunks >= 16 && (m <= 6 || nt > 1)) return none;
+        if (!a_f32 && m <= 8) {
+            if (k_chunks >= 16 && (m <= 6 || nt > 1 || (m == 7 && k_chunks <= 32))) return none;
+            if (k_chunks <= 8 && nt > 1 && (k_chunks >= 7 || (gated && n_tiles > 384))) return none;
+        }
         if (!few_f32 && k_chunks > (!a_f32 && m <= 16 ? 64u : a_f32 && m > 16 && nt == 2 ? 36u : 48u)) return none;
         const uint32_t groups = n_tiles / nt;
         uint32_t splits = 1;
@@ -415,9 +423,9 @@ WavesPlan plan_waves(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32
     if (k_chunks < 8 || k_chunks > 48) return none;
     const uint32_t blocks = (m + 16 * waves_mt(m) - 1) / (16 * waves_mt(m));
     for (uint32_t nt = gated ? 2 : 1; nt <= 2; nt++) {
-        const uint32_t groups = n_tiles / nt * blocks;
-        if (groups > 256) continue;
-        const uint32_t splits = k_chunks < 32 ? 1u : groups <= 64 ? 4u : groups <= 112 ? 2u : 1u;
+        const uint32_t groups = n_tiles / nt * blocks, on_xcd = (n_tiles / nt + 7) / 8 * blocks;
+        if (on_xcd > 32) continue;
+        const uint32_t splits = k_chunks < 32 ? 1u : on_xcd <= 8 ? 4u : groups <= 112 ? 2u : 1u;
         if (k_chunks > 32 && splits == 1 && groups < 160) return none;
         return WavesPlan{nt, 8, splits};
     }

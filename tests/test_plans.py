@@ -149,8 +149,8 @@ def test_plans_of_the_kernel_on_narrow_matrices(lib):
     # the row count, one round of workgroups on the CUs (two of the four-wave form), K cut only where that leaves CUs idle
     rng = np.random.default_rng(11)
     taken = set()
-    for _ in range(3000):
-        k, n = 32 * int(rng.integers(1, 200)), int(rng.integers(1, 20000))
+    for _ in range(6000):
+        k, n = 32 * int(rng.integers(1, 200)), int(rng.choice([400, 3000, 20000]) * rng.random()) + 1
         m, gated = int(rng.integers(1, 260)), int(rng.integers(0, 2))
         n = n // 64 * 64 + 64 if gated else n
         dtype = _lib.F32 if rng.integers(0, 2) else _lib.F16
@@ -163,6 +163,9 @@ def test_plans_of_the_kernel_on_narrow_matrices(lib):
         assert (m <= 32) == (f["block_rows"] <= 32) == ("exact weights" in f["text"]) != ("f16-rounded weights" in f["text"]), f["text"]
         assert -(-m // f["block_rows"]) * f["block_rows"] - m < f["block_rows"], f["text"]
         assert wgs <= (CUS if f["waves"] == 8 else 2 * CUS) and (f["waves"] == 8 or 33 <= m <= 64), f["text"]
+        blocks, groups = -(-m // f["block_rows"]), (n + 63) // 64 * 64 // f["block_cols"]
+        if blocks > 1:  # the row blocks of a column group stay on one of the eight XCDs: one round on its 32 CUs
+            assert -(-groups // 8) * blocks * f["splits"] <= CUS // 8, f["text"]
         if f["splits"] > 1:
             assert wgs // f["splits"] <= CUS // 2 and k_chunks // f["splits"] >= 8 and "k_splitk_reduce" in f["text"], f["text"]
         taken.add((f["block_rows"], f["block_cols"]))
