@@ -564,7 +564,9 @@ hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutS
 // Up to 256 rows also blocks of 128 columns (two tiles per wave) with 48, 64, 96 or 128 rows, named by their rows + 1: a few
 // rows on 256-column blocks leave half the CUs idle (3584 -> 2 x 18944 is 148 of them) or multiply rows that are not there.
 // kNarrow holds what a chunk takes with one, two and three workgroups on a CU (the 96-row form fits twice, the 128-row form
-// once, the rest of them follow).  Best form before and now (us): 3584 -> 2 x 18944 at 96 rows 50.5 / 45.1, 4096 -> 2 x 11008
+// once, the rest of them follow); each further three start and store once more, 2 us that a shallow K feels (160 rows of
+// 1024 -> 49476 on three to five 64 x 128 blocks a CU 37.1, on 64 x 256 32.8; 896 -> 152064 on 96 x 128 76.7, 64 x 256 69.9).
+// Best form before and now (us): 3584 -> 2 x 18944 at 96 rows 50.5 / 45.1, 4096 -> 2 x 11008
 // at 96 35.2 / 29.1 and at 128 38.9 / 34.0, 896 -> 2 x 4864 at 64 13.4 / 8.1, 2048 -> 2 x 5632 at 192 22.7 / 17.6,
 // 18944 -> 3584 at 96 29.1 / 24.1, 11008 -> 4096 at 40 17.6 / 14.8, 3584 -> 4608 at 96 16.4 / 13.3, 4096 -> 12288 at 192
 // 33.5 / 27.9; 3584 -> 2 x 18944 at 128 rows is level or worse (50.8 / 55.4).  Under 2048 columns the wider blocks on more
@@ -611,7 +613,7 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
             double t = 0.0;
             if (narrow) {
                 const uint32_t on_cu = ((uint32_t)total + 255u) / 256u;  // workgroups of the busiest CU
-                t = cps * (on_cu / 3u * chunk[2] + (on_cu % 3u ? chunk[on_cu % 3u - 1u] : 0.0)) + 3.0;
+                t = cps * (on_cu / 3u * chunk[2] + (on_cu % 3u ? chunk[on_cu % 3u - 1u] : 0.0)) + 3.0 + 2.0 * ((on_cu - 1u) / 3u);
             } else if (bm == 192 && total > 256.0) {
                 // two workgroups share a CU: 2.45 per chunk each; a last round of up to one per CU runs at 1.45
                 const double full = (double)(uint64_t)(total / 512.0), rem = total - 512.0 * full;
