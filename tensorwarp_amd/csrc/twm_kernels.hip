@@ -330,13 +330,12 @@ hipError_t launch_fuse_one(hipStream_t s, const uint8_t *packed_in, const uint16
 // on whatever runs next; records loaded past the caches as well cost 25 us of the gain, since they are often just written.
 template <int COLS, bool F16OUT>
 __global__ __launch_bounds__(256) void k_dequant(const uint4v *__restrict__ packed, const uint16_t *__restrict__ scales,
-                                                  uint32_t groups, uint32_t n, void *__restrict__ out, uint32_t slab)
+                                                  uint32_t groups, uint32_t n, void *__restrict__ out)
 {
     typedef uint16_t halves __attribute__((ext_vector_type(COLS)));
     typedef float floats __attribute__((ext_vector_type(COLS)));
-    Place place;
-    if (!place_of(groups, n / COLS, slab, place)) return;
-    const uint32_t g = place.group, col = place.column * COLS;
+    const uint32_t g = blockIdx.z * gridDim.y + blockIdx.y, col = (blockIdx.x * 256u + threadIdx.x) * COLS;
+    if (g >= groups || col >= n) return;
     const size_t rec = (size_t)g * n + col;
     uint4v w[COLS];
     float sc[COLS];
@@ -391,8 +390,9 @@ hipError_t launch_dequant(hipStream_t s, const uint8_t *packed, const uint16_t *
 {
     if (k == 0 || n == 0) return hipSuccess;
     // An element per thread where the records are not aligned -- and where a record per thread would be few workgroups (4096 x
-    // 64: 2.5 us, here 2.2) or put a wave's stores on as many lines as it has lanes (1048576 x 1: 9.4, here 3.2).
-    if (((uintptr_t)packed & 15) != 0 || n < 8 || (uint64_t)(k / 32) * n < 32768u) {
+    // 64: 2.6 us and here 2.2) or leave most of one idle (1048576 x 1: 16.5, here 3.2; 262144 x 16: 7.7, here 7.5, to f32 11.4
+    // and 7.9).
+    if (((uintptr_t)packed & 15) != 0 || n <= 16 || (uint64_t)(k / 32) * n < 32768u) {
         const dim3 grid = place_grid(k, n);
         const uint32_t slab = place_slab(k, n);
         if (f16_out) hipLaunchKernelGGL(k_dequant_bytes<true>, grid, dim3(256), 0, s, packed, scales, k, n, out, slab);
@@ -401,13 +401,13 @@ hipError_t launch_dequant(hipStream_t s, const uint8_t *packed, const uint16_t *
     }
     // two columns per thread where a row's columns keep the alignment of the paired stores
     const bool pairs = n % 2 == 0 && ((uintptr_t)out & (f16_out ? 3 : 7)) == 0;
-    const uint32_t groups = k / 32, columns = pairs ? n / 2 : n, slab = place_slab(groups, columns);
-    const dim3 grid = place_grid(groups, columns);
+    const uint32_t groups = k / 32, y = groups < 65535u ? groups : 65535u;
+    const dim3 grid((n + (pairs ? 511 : 255)) / (pairs ? 512 : 256), y, (groups + y - 1) / y);
     const uint4v *rec = (const uint4v *)packed;
-    if (pairs && f16_out) hipLaunchKernelGGL((k_dequant<2, true>), grid, dim3(256), 0, s, rec, scales, groups, n, out, slab);
-    else if (pairs) hipLaunchKernelGGL((k_dequant<2, false>), grid, dim3(256), 0, s, rec, scales, groups, n, out, slab);
-    else if (f16_out) hipLaunchKernelGGL((k_dequant<1, true>), grid, dim3(256), 0, s, rec, scales, groups, n, out, slab);
-    else hipLaunchKernelGGL((k_dequant<1, false>), grid, dim3(256), 0, s, rec, scales, groups, n, out, slab);
+    if (pairs && f16_out) hipLaunchKernelGGL((k_dequant<2, true>), grid, dim3(256), 0, s, rec, scales, groups, n, out);
+    else if (pairs) hipLaunchKernelGGL((k_dequant<2, false>), grid, dim3(256), 0, s, rec, scales, groups, n, out);
+    else if (f16_out) hipLaunchKernelGGL((k_dequant<1, true>), grid, dim3(256), 0, s, rec, scales, groups, n, out);
+    else hipLaunchKernelGGL((k_dequant<1, false>), grid, dim3(256), 0, s, rec, scales, groups, n, out);
     return hipGetLastError();
 }
 

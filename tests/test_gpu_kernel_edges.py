@@ -283,8 +283,9 @@ def test_format_kernels_on_narrow_matrices(dev, n):
     assert np.array_equal(T.dequant_to_f32(dev, p, s, k, n).to_host().view(np.uint32), O.dequant_f32(want_p, want_s, k, n).view(np.uint32))
 
 
-# from 32768 records and eight columns on a thread unpacks whole records, two of them where columns and output allow it
-@pytest.mark.parametrize("k,n", [(4096, 256), (4096, 257), (4096, 258), (131072, 8), (116544, 9), (4096, 255)])
+# from 32768 records and 17 columns on a thread unpacks whole records, two of them where columns and output allow it; more
+# groups than a grid's y dimension counts
+@pytest.mark.parametrize("k,n", [(4096, 256), (4096, 257), (4096, 514), (61728, 17), (63552, 18), (4096, 255), (65568, 16), (2097184, 18)])
 @pytest.mark.parametrize("out_offset", [0, 1])
 def test_unpack_of_whole_records(dev, k, n, out_offset):
     packed, scales = O.synth_packed(k, n, 5), O.synth_scales(k, n, 6)
