@@ -785,7 +785,7 @@ int twm_gemm_f16out(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_
         return api_fail(TWM_MEMORY_ERROR, "%s: one row of f32 results (%zu bytes) does not fit the staging part of the context's scratch; "
                         "use twm_gemm and twm_cast_f32_to_f16", who, row_bytes);
     uint32_t block = staged / row_bytes < m ? (uint32_t)(staged / row_bytes) : m;
-    if (block >= 128) block -= block % 128;   // (whole prefill row blocks)
+    if (block < m && block >= 128) block -= block % 128;   // (several blocks: whole prefill row blocks)
     float *stage = (float *)((char *)ctx->ws + ctx->ws_bytes - staged);
     const size_t a_row_bytes = (size_t)w->k * (a_dtype == TWM_F32 ? 4 : 2), saved = ctx->ws_bytes;
     int rc = TWM_OK;
