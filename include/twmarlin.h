@@ -83,7 +83,8 @@ int twm_last_error_kind(void);
 
 /* c_api.rs:52-59 warp_device_create / WarpDevice::new (device.rs) + KernelCache::new.
  * All kernels are precompiled gfx950 code inside the library, so there is no
- * JIT step.  Creates the context's own stream and its split-K scratch.
+ * JIT step.  Creates the context's own stream and its scratch (256 MB of device memory until twm_ctx_destroy:
+ * split-K sums and the f16 terms of f32 rows).
  * Returns NULL on failure. */
 twm_ctx *twm_ctx_create(int ordinal);
 /* c_api.rs:61-67 warp_device_destroy */
@@ -474,7 +475,8 @@ int twm_gemm_tw_marlin_m1_indirect(twm_ctx *ctx, const float *a_dev, const uint8
 uint32_t twm_pick_splits(uint32_t k, uint32_t n, uint32_t m);
 
 /* What twm_gemm would launch for a K x N weight, m rows of f16 / f32 activations and (gated != 0) the gated store of a
- * paired weight, as one line of text: the kernel, its workgroup shape, the K-split and the repacked copy it reads.
+ * paired weight, as one line of text: the kernel, its workgroup shape, the K-split and the repacked copy it reads (for a
+ * handle that holds both copies, without a measured plan).
  * ctx = NULL: a fresh context's defaults; otherwise the context's options count.  Touches no device: usable to
  * see what the planners decide -- the counterpart of AutoTuner::heuristic_variant and ::report
  * (crates/kernels/src/autotune.rs:505-515, 648-668) -- and to test them without a GPU. */

@@ -769,7 +769,7 @@ int twm_gemm(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_dtype, 
 }
 
 // twm_gemm with f16 result rows: the kernels store f32 (what the reference's buffers hold), so the rows are computed in
-// blocks into the back half of the context's scratch and rounded from there by the cast kernel -- no allocation, one
+// blocks into the end of the context's scratch (kF16OutBytes) and rounded from there by the cast kernel -- no allocation, one
 // more launch per block; the rest stays the launch's own scratch (split-K sums, f32 activation terms).
 int twm_gemm_f16out(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_dtype, uint32_t m, uint16_t *c_dev_f16,
                     uint32_t splits)

@@ -37,7 +37,8 @@ struct twm_ctx {
     int force_sub_waves;  // sub-tile kernels with a forced width: waves per workgroup (1 .. 16), 0 = "waves" or eight
     int force_sub;        // M <= 4: 0 = heuristic, 1 = whole 64-column tiles per workgroup, 32 or 16 = the sub-tile kernel
     int force_kernel;     // 0 = heuristic, 2 = one-lane-per-column kernel on whole tiles (M <= 4), 3 = streaming kernel (M <= 32),
-                          // 4 = batched-decode kernel with LDS-shared activations (M <= 32; "nt" = tiles per wave, "waves" 8 / 16 = 2 / 4 k-slices)
+                          // 4 = batched-decode kernel with LDS-shared activations (M <= 32; "nt" = tiles per wave, "waves" 8 / 16 = 2 / 4 k-slices),
+                          // 5 = waves on k-chunks of their own ("nt" = 16-column tiles per workgroup, "waves" 4 / 8)
     int prefill_bm;       // prefill block form: 0 = choose, 64 = 64 rows x 256 columns, 128 = 128 x 256, 192 = 128 rows x 192 columns, 49 / 65 / 97 / 129 = 48 / 64 / 96 / 128 rows x 128 columns
     int prefill_min_m;    // M from which the LDS/MFMA prefill kernel runs instead of 16-row decode blocks
     int dequant_src;      // which copy twm_weight_dequant_f16 unpacks: 0 = 16-column tiles, 1 = column-lane
@@ -95,9 +96,9 @@ struct twm_graph {
     hipGraphExec_t exec;
 };
 
-// Scratch of a context: split-K sums and the f16 terms of f32 rows.  256 MB of the card's 288 GB hold the terms of a
-// 2048 x 18944 prompt in one piece (with 64 MB a 2048 x 11008 one ran as 1408 + 640 rows, the
-// second part on split K: a LLaMA-7B layer at 2048 rows 816 us, now 793).
+// Scratch of a context, held from its creation on: split-K sums and the f16 terms of f32 rows.  256 MB of the card's 288 GB
+// hold the terms of a 2048 x 18944 prompt in one piece (with 64 MB a 2048 x 11008 one ran as 1408 + 640 rows, the second part
+// on split K: a LLaMA-7B layer at 2048 rows 816 us, now 793; 4096 -> 2 x 18944 at 1280 f32 rows 595, now 420).
 constexpr size_t kWsBytes = 256ull << 20;
 constexpr size_t kF16OutBytes = 32ull << 20;  // its end, where twm_gemm_f16out stages f32 rows
 constexpr uint32_t kCounters = 1u << 16;     // arrival counters of a context

@@ -5,8 +5,8 @@
 // f16_rne(f32(scale) * (q - 8)) (quantize.rs:534-571), produced in registers: (q - 8) is exact in f16 and
 // one packed f16 multiply by the scale rounds exactly like the reference's __float2half(scale * q).
 //
-// Block = 16*MT rows x 256 columns (MT = 8 or 4), 4 waves; wave w owns 64 columns (four 16-column tiles of
-// the tile-order copy) for all rows of the block, so no weight is unpacked twice inside a block.  Per
+// Block = 16*MT rows x 64*NTW columns (MT = 3, 4, 6, 8; NTW = 4, 3, 2), 4 waves; wave w owns 16*NTW columns (NTW tiles
+// of the tile-order copy) for all rows of the block, so no weight is unpacked twice inside a block.  Per
 // 128-deep k-chunk and wave:
 //   A tile (16*MT x 128 f16): global -> LDS directly (global_load_lds_dwordx4), D buffers, 256-byte rows
 //                             whose 16-byte slots are XOR-swizzled so that the sixteen rows of an operand
@@ -25,8 +25,9 @@
 
 namespace twm {
 
-// MT = 16-row blocks per workgroup tile (BM = 16 * MT rows); NTW = 16-column tiles per wave: 4 (256-column blocks) or
-// 3 (192-column blocks, for shapes whose 256-column blocks leave a round of workgroups mostly empty)
+// MT = 16-row blocks per workgroup tile (BM = 16 * MT rows); NTW = 16-column tiles per wave: 4 (256-column blocks), 3
+// (192-column blocks, for shapes whose 256-column blocks leave a round of workgroups mostly empty) or 2 (128-column blocks,
+// for up to 256 rows)
 // HALF: the MFMAs of a 32-deep group run as two half steps of MT / 2 row blocks, and the A operands are read half a step
 // ahead instead of a whole one: MT / 2 x 2 operand registers less, which with NTW = 3 brings the kernel under 256
 // registers, so that two workgroups share a CU and one's MFMAs fill the issue gaps of the other.
@@ -505,8 +506,8 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_swiglu(const float *__res
 }
 
 // out[row][:] *= row_scale[row] over every segment, for the rows whose factor is not 1.  Rows that need nothing are the
-// rule: a workgroup looks at the factors of kScaleRows rows with one load and usually ends there (2048 rows: 64 x 8
-// workgroups instead of one per row, whose launch alone was 5 us).
+// rule: a workgroup looks at the factors of kScaleRows rows with one load and usually ends there (2048 x 4096 without a factor,
+// in a kernel trace: 5.0 us in the median and 1.2 at least on 64 x 8 workgroups, 4.9 and 3.9 on one per row).
 constexpr uint32_t kScaleRows = 32, kScaleParts = 8;
 __global__ __launch_bounds__(256) void k_scale_rows(OutSpec out, const float *__restrict__ row_scale, uint32_t rows)
 {
@@ -576,7 +577,7 @@ constexpr uint32_t kNarrowMaxRows = 256, kNarrowMinTiles = 128;
 static const struct { uint32_t form; double chunk[3]; } kNarrow[] = {
     {49, {0.70, 1.05, 1.50}}, {65, {0.77, 1.30, 1.90}}, {97, {0.88, 1.45, 2.35}}, {129, {1.03, 2.10, 3.15}}};
 struct PrefillPlan {
-    uint32_t block_rows, splits;   // block_rows: the form (64, 128, 192)
+    uint32_t block_rows, splits;   // block_rows: the form, see launch_prefill
     double us;
 };
 static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t force_splits, uint32_t n_tiles, uint32_t k_chunks,
@@ -718,8 +719,9 @@ hipError_t init_prefill()
     return e;
 }
 
-// block_rows: the block form (64 = 64 rows x 256 columns, 128 = 128 x 256, 192 = 128 rows x 192 columns), splits: k-split
-// factor, 49 / 65 / 97 / 129 = 48 / 64 / 96 / 128 rows x 128 columns; 0 = choose (plan_prefill), within what `scratch` can hold as f32 partial sums.
+// block_rows: the block form (64 = 64 rows x 256 columns, 128 = 128 x 256, 192 = 128 rows x 192 columns, 49 / 65 / 97 / 129 =
+// 48 / 64 / 96 / 128 rows x 128 columns), splits: k-split factor; 0 = choose (plan_prefill), within what `scratch` can hold as
+// f32 partial sums.
 // `scratch` (scratch_bytes) holds the f16 copy of f32 activations and / or the split-K partials; when it
 // cannot hold all M rows the rows are processed in slabs.
 hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out,

@@ -378,7 +378,8 @@ hipError_t init_waves()
 }
 
 // Where this kernel takes a GEMM, and in which form; nt = 0: it does not.  Lines fitted to forced sweeps on twenty projection
-// shapes (and checked on twenty others: 1.25 times as fast over 520 cells, none more than 3 % slower), 5 .. 192 rows, f16 and f32 rows (us, this kernel against the best other form):
+// shapes and redrawn after a comparison with the forms of before on 3000 random ones, 5 .. 192 rows, f16 and f32 rows (us, this
+// kernel against the best other form):
 // * one round of workgroups on 256 CUs: one tile each up to 4096 columns, two up to 8192, four up to 16384 (beyond, the
 //   forms that share the activation tile among more columns are level or ahead: 4096 -> 22016 gated at 32 rows 22.8 / 21.0);
 //   four tiles only from K = 3072 on (4096 -> 12288 at 32 rows 14.0 / 15.6, but 2048 -> 11264 gated at 16 7.9 / 7.4) -- except
