@@ -313,7 +313,8 @@ size_t twm_weight_bytes(const twm_weight *w);
  * together exceed the 256 MB cache -- and keeps the fastest for that bucket of row counts (1, 2, 3-4, 5-8, ...
  * 513-1024, above) when it beats the planners' own choice by more than 2 %.  Later calls with f16
  * activations, splits = 0 and no knob set run the kept form (one of kernel 5 only while "prefill_min_m" and
- * "batch_rounded" ask for that kernel's arithmetic at the call's row count); the table travels with twm_weight_export /
+ * "batch_rounded" ask for that kernel's arithmetic at the call's row count, any only while the handle holds the copy that
+ * it reads); the table travels with twm_weight_export /
  * _import.
  * Allocates trial buffers and synchronises: a load-time call, not for a graph capture.
  * twm_weight_tuned_plan returns the bucket's entry as eight ints: valid, kernel, nt, waves, sub, sub_waves, splits,

@@ -558,7 +558,8 @@ static void set_knobs(twm_ctx *c, const Knobs &k)
 }
 
 // With nothing forced by the caller, a plan that twm_weight_tune measured for this weight and row count is what runs --
-// unless it is one of k_waves and the options have come to ask for another arithmetic at this row count.
+// unless it is one of k_waves and the options have come to ask for another arithmetic at this row count, or it reads a copy
+// that the handle has dropped since: building that again allocates, so the planners choose from what is held.
 static int gemm_common(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int a_dtype, uint32_t m, const OutSpec &out,
                        uint32_t splits, const char *who, float *swiglu_out = nullptr, uint32_t gate_act = 2)
 {
@@ -568,7 +569,10 @@ static int gemm_common(twm_ctx *ctx, const twm_weight *w, const void *a_dev, int
     if (!tp || !tp->valid || (tp->kernel == 5 && !waves_arithmetic_asked_for(form_env(ctx), m)))
         return gemm_dispatch(ctx, w, a_dev, a_dtype, m, out, splits, who, swiglu_out, gate_act);
     set_knobs(ctx, Knobs{tp->kernel, tp->nt, tp->waves, tp->sub, tp->sub_waves, tp->prefill_bm});
-    const int rc = gemm_dispatch(ctx, w, a_dev, a_dtype, m, out, tp->splits, who, swiglu_out, gate_act);
+    const bool held = w->copy_bytes == 0 ||
+                      (copies_of(w) & choose_form(form_env(ctx), w->n_tiles, w->k_chunks, m, false, tp->splits, false).copy);
+    if (!held) set_knobs(ctx, user);
+    const int rc = gemm_dispatch(ctx, w, a_dev, a_dtype, m, out, held ? tp->splits : splits, who, swiglu_out, gate_act);
     set_knobs(ctx, user);
     return rc;
 }

@@ -442,6 +442,34 @@ def test_a_column_lane_handle_keeps_its_one_copy_on_narrow_matrices(dev, m):
     w.free()
 
 
+def test_a_measured_plan_does_not_ask_for_a_dropped_copy(dev):
+    # a plan of kernel 5 (16-column tiles) on a handle that holds the column lanes: the planners' choice from what is held,
+    # inside a capture too; with the copy back, the plan
+    m, k, n = 16, 2048, 1024
+    dev.set_option("weight_copies", T.MarlinWeight.COPY_COLUMN_LANE)
+    packed, scales, w = weight(dev, k, n, 1951)
+    dev.set_option("weight_copies", 0)
+    blob = w.export_blob()
+    blob[-96 + 8 * 4:-96 + 8 * 5] = np.array([1, 5, 1, 0, 0, 0, 1, 0], np.uint8)       # 9 .. 16 rows
+    back = T.MarlinWeight.import_blob(dev, blob)
+    a16 = O.synth_act_f16(m, k, 1953)
+    a = T.GpuTensor.from_host(dev, a16, "f16")
+    truth = O.gemm_f64(a16.view(np.float16).astype(np.float32).reshape(m, k), packed, scales, m, k, n)
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    graph = T.GraphCapture.record_with_device(dev, lambda: T.gemm(dev, back, a, m, c))
+    graph.replay()
+    dev.synchronize()
+    close_rows(c.to_host(), truth, F32_SUM)
+    assert back.copies == T.MarlinWeight.COPY_COLUMN_LANE
+    back.ensure(3)
+    c.copy_from_host(np.full((m, n), np.nan, np.float32))
+    T.gemm(dev, back, a, m, c)
+    close_rows(c.to_host(), truth, F32_SUM)
+    graph.destroy()
+    back.free()
+    w.free()
+
+
 @pytest.mark.parametrize("k,m", [(416, 9), (416, 16), (992, 5), (2080, 8), (2080, 16)])
 def test_an_infinite_activation_reaches_every_column_as_itself(dev, k, m):
     # K one group past a 128-deep chunk: the padded part of the last chunk must not multiply an infinity by its zero weights.
