@@ -240,7 +240,7 @@ static FormEnv form_env(const twm_ctx *c)
                    c->batch_rounded, c->prefill_bm, c->ws_bytes, c->n_counters};
 }
 
-// k_waves' arithmetic follows the row count alone: exact weights up to 32 rows, f16-rounded ones above.  It may stand in for
+// k_waves_exact takes up to 32 rows, k_waves (f16-rounded weights) more: the arithmetic follows the row count alone.  They may stand in for
 // the other forms only where the options ask for the same: the prefill GEMM's line left at 33 or lowered (with it raised a
 // call of many rows and a call on each of its 32-row blocks are the same launches), this row count on its usual side of it,
 // no rounded batches.
@@ -263,11 +263,11 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
         if (wp.waves == 4 && (m <= 32 || wp.nt != 2)) wp.waves = 8;                       // (forms that do not exist: the nearest)
         if (wp.nt == 4 && (m > 32 || (a_f32 && m > 16))) wp.nt = 2;
     } else if (e.kernel == 0 && !e.nt && !e.waves && !e.sub && !splits && !e.prefill_bm && waves_arithmetic_asked_for(e, m)) {
-        wp = plan_waves(n_tiles, k_chunks, m, a_f32, gated);
-        // A handle with the column-lane copy alone keeps the sub-tile kernel, which reads that copy, where there is one for
-        // this shape: a little slower (3584 -> 3584 at 16 rows 7.4 us, k_waves 5.6), but the tile copy would be a second
-        // allocation of the weight's size, and inside a graph capture a refusal.
-        if (!(copies & kCopyTile) && !a_f32 && m <= 16 && plan_gemv4_sub_rows(tiles64, k_chunks).sub) wp.nt = 0;
+        wp = m <= 32 ? plan_waves_exact(n_tiles, k_chunks, m, a_f32, gated) : plan_waves(n_tiles, k_chunks, m, gated);
+        // A handle with the column-lane copy alone keeps the kernels that read that copy where there is one for this shape: a
+        // little slower (3584 -> 3584 at 16 rows 7.4 us, k_waves_exact 5.4), but the tile copy would be a second allocation of
+        // the weight's size, and inside a graph capture a refusal.
+        if (!(copies & kCopyTile) && !a_f32 && m <= 16 && (plan_gemv4_sub_rows(tiles64, k_chunks).sub || (m <= 8 && tiles64 > 128))) wp.nt = 0;
     }
     if (wp.nt) {
         f.kind = kFormWaves;
@@ -448,6 +448,15 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
         break;
     }
     case kFormWaves:
+        if (f.nt != 1 && f.nt != 2 && f.nt != 4) {
+            const uint32_t quads = (f.nt + 3) / 4, less = quads * 4 - f.nt;
+            char part[32] = "";
+            if (less) snprintf(part, sizeof part, " less %u tile%s", less, less == 1 ? "" : "s");
+            snprintf(text, bytes, "k_batch: %u quad%s per workgroup%s, 1 tile per wave in turn, %u waves on k-chunks of their own, %u K-split%s%s; "
+                     "16-column tile copy", quads, quads == 1 ? "" : "s", part, f.waves, f.splits, f.splits == 1 ? "" : "s",
+                     f.splits > 1 ? " + k_splitk_reduce" : "");
+            break;
+        }
         snprintf(text, bytes, "k_waves: %u-row x %u-column blocks, %u waves on k-chunks of their own, %s weights, %u K-split%s%s; "
                  "16-column tile copy", waves_block_rows(m), 16 * f.nt, f.waves, m <= 32 ? "exact" : "f16-rounded", f.splits,
                  f.splits == 1 ? "" : "s", f.splits > 1 ? " + k_splitk_reduce" : "");
@@ -513,8 +522,9 @@ static int gemm_dispatch(twm_ctx *ctx, const twm_weight *w, const void *a_dev, i
         return TWM_OK;
     }
     case kFormWaves:
-        HIP_TRY(launch_waves(ctx->stream, v, a_dev, a_f32, m, gated, f.nt, f.waves, f.splits, ctx->ws, ctx->ws_bytes), TWM_DEVICE_ERROR,
-                "batched launch");
+        HIP_TRY(m <= 32 ? launch_waves_exact(ctx->stream, v, a_dev, a_f32, m, gated, f.nt, f.splits, ctx->ws, ctx->ws_bytes)
+                        : launch_waves(ctx->stream, v, a_dev, a_f32, m, gated, f.nt, f.waves, f.splits, ctx->ws, ctx->ws_bytes),
+                TWM_DEVICE_ERROR, "batched launch");
         return TWM_OK;
     case kFormSubTile:
         HIP_TRY(launch_gemv4s(ctx->stream, v, a_dev, a_f32, m, gated, ctx->ws, ctx->counters, f.sub, f.waves, f.splits, ctx->trace), TWM_DEVICE_ERROR,

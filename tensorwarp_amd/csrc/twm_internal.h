@@ -164,13 +164,17 @@ hipError_t launch_gemv4_ref(hipStream_t s, const uint8_t *packed, const uint16_t
 bool prefill_form_known(uint32_t form);  // a prefill block form (see launch_prefill)
 hipError_t init_prefill();
 hipError_t init_waves();
-// 5 .. 192 rows on narrow matrices, waves on k-ranges of their own (twm_waves.hip): 16-column tiles per workgroup (0: another
-// form runs), waves, K-splits
+hipError_t init_waves_exact();
+// waves on k-chunks of their own: 5 .. 32 rows with exact weights (twm_waves_exact.hip), 33 .. 192 rows on narrow matrices with
+// f16-rounded ones (twm_waves.hip): 16-column tiles per workgroup (0: another form runs), waves, K-splits
 struct WavesPlan {
     uint32_t nt, waves, splits;
 };
-WavesPlan plan_waves(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated);
+WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated);
+WavesPlan plan_waves(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool gated);
 uint32_t waves_block_rows(uint32_t m);  // rows per workgroup
+hipError_t launch_waves_exact(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out, uint32_t nt,
+                              uint32_t splits, void *scratch, size_t scratch_bytes);
 hipError_t launch_waves(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out, uint32_t nt,
                         uint32_t waves, uint32_t splits, void *scratch, size_t scratch_bytes);
 hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out,

@@ -219,6 +219,47 @@ def test_waves_on_their_own_k_ranges(dev, m, nt, waves, splits):
         w.free()
 
 
+# column groups of 3, 5, 6, 8 and 10 tiles whose last one is ragged, K one group past whole chunks and fewer chunks than two per
+# wave; one and two row blocks, f16 rows, f32 rows in one block and in two tiles with rows outside the f16 range
+@pytest.mark.parametrize("n", [12001, 17001, 22016, 30016, 40001])
+@pytest.mark.parametrize("m,dtype", [(9, "f16"), (16, "f32"), (20, "f16"), (7, "f32"), (32, "f32")])
+def test_waves_on_many_column_tiles(dev, m, dtype, n):
+    k = 1312 if n < 40000 else 1056
+    packed, scales, w = weight(dev, k, n, 1401 + m)
+    a16 = O.synth_act_f16(m, k, 1403 + m)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+    if dtype == "f32":
+        a[0] *= np.float32(2.0 ** 60)
+        a[1, 128:256] *= np.float32(2.0 ** -30)      # a stretch of a row far below the rest of it
+        a[m - 1] *= np.float32(2.0 ** -40)
+    third = n // 3
+    parts = [third, third + 1, n - 2 * third - 1]
+    outs = [T.GpuTensor.from_host(dev, np.full((m, x), np.nan, np.float32)) for x in parts]
+    bias = [T.GpuTensor.from_host(dev, np.zeros(x, np.float32)) for x in parts]
+    T.gemm_split(dev, w, T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a), m, outs, parts, biases=bias)
+    close_rows(np.concatenate([o.to_host() for o in outs], axis=1), O.gemm_f64(a, packed, scales, m, k, n), F32_SUM)
+    w.free()
+
+
+# the gated store of groups of four, six, eight and ten tiles, the last group ragged
+@pytest.mark.parametrize("ffn", [6176, 10016, 14112, 18464])
+@pytest.mark.parametrize("m,dtype", [(9, "f16"), (13, "f32"), (8, "f32"), (32, "f16")])
+def test_waves_gated_store_on_many_column_tiles(dev, m, dtype, ffn):
+    k = 1056
+    gate, up = [(O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (1511, 1513)]
+    pair = [tuple(T.GpuTensor.from_host(dev, x, t) for x, t in zip(w, ("u8", "f16"))) for w in (gate, up)]
+    w = T.MarlinWeight.gate_up(dev, *pair, k, ffn)
+    a16 = O.synth_act_f16(m, k, 1515)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+    if dtype == "f32":
+        a[1] *= np.float32(2.0 ** -21)
+    g, u = (O.gemm_f64(a, *x, m, k, ffn) for x in (gate, up))
+    out = T.GpuTensor.from_host(dev, np.full((m, ffn), np.nan, np.float32))
+    T.gemm_swiglu(dev, w, T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a), m, out)
+    close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
+    w.free()
+
+
 @pytest.mark.parametrize("m,dtype", [(5, "f32"), (8, "f32"), (9, "f16"), (13, "f32"), (32, "f16"), (40, "f16"), (64, "f32"), (96, "f16")])
 def test_waves_gated_store(dev, m, dtype):
     k, ffn = 1056, 96                                # 33 groups; three quads of gate and up tiles
