@@ -579,8 +579,8 @@ __device__ __forceinline__ void gemv4s_compute(const ChunkS<SUB, (RL + 3) / 4> &
 // NP passes per wave - first, first + stride, ... - with every load of the wave issued before the first unpack: NP
 // register sets, no loop.  The loads are unconditional (a pass past the last one replays the k-range's last chunk and
 // nobody unpacks it), so the wait in front of each unpack is an exact count of the loads issued after its own.
-template <int SUB, int NP, int RG = 1, class Load, class Compute>
-__device__ __forceinline__ void gemv4s_run_upfront(uint32_t first, uint32_t stride, uint32_t passes, Load load, Compute compute)
+template <int SUB, int NP, int RG = 1, class Load, class Compute, class Between>
+__device__ __forceinline__ void gemv4s_run_upfront(uint32_t first, uint32_t stride, uint32_t passes, Load load, Compute compute, Between between)
 {
     ChunkS<SUB, RG> r[NP];
 #pragma unroll
@@ -588,6 +588,7 @@ __device__ __forceinline__ void gemv4s_run_upfront(uint32_t first, uint32_t stri
         load(r[i], first + i * stride);
         __builtin_amdgcn_sched_barrier(0);
     }
+    between();
 #pragma unroll
     for (int i = 0; i < NP; i++) {
         if (first + i * stride < passes) compute(r[i]);
@@ -622,13 +623,19 @@ __device__ __forceinline__ float sum_lane_groups(float v)
 // and waits for the newest loads before the unpack may read the older ones - which is what the plain form below
 // does: its second register set only saves the address arithmetic.  The pipelined form needs both sets live through
 // the unpack; the variants with more rows or f32 activations would spill, and stay with the plain form.
-template <int SUB, bool ONE, int RG = 1, bool PIPE = false, class Load, class Compute>
-__device__ __forceinline__ void gemv4s_run_passes(uint32_t first, uint32_t stride, uint32_t passes, Load load, Compute compute)
+// between: what the wave does once its first loads are on their way.
+struct Gemv4sNothing {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <int SUB, bool ONE, int RG = 1, bool PIPE = false, class Load, class Compute, class Between = Gemv4sNothing>
+__device__ __forceinline__ void gemv4s_run_passes(uint32_t first, uint32_t stride, uint32_t passes, Load load, Compute compute,
+                                                  Between between = Between())
 {
     if (ONE) {
         ChunkS<SUB, RG> r0;
         if (first < passes) {
             load(r0, first);
+            between();
             compute(r0);
         }
         return;
@@ -637,6 +644,7 @@ __device__ __forceinline__ void gemv4s_run_passes(uint32_t first, uint32_t strid
     ChunkS<SUB, RG> r0, r1;
     uint32_t p = first;
     load(r0, p);
+    between();
     if (PIPE) {
         const uint32_t mine = (passes - first + stride - 1u) / stride;  // this wave's passes
         for (uint32_t i = 1; i < mine; i += 2) {

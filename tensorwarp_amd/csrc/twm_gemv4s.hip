@@ -58,14 +58,14 @@ __device__ __forceinline__ void gemv4s_store_out(const OutSpec &out, uint32_t m,
 // NP >= 2 (16 columns, one row): every wave makes up to NP passes and issues all their loads before its first unpack
 // (gemv4s_run_upfront): a workgroup that is alone on its CU has its whole share of the matrix in flight at once, like
 // the one-pass form, where the pass loop keeps two passes per wave in flight and walks K one memory round trip at a time.
-template <int SUB, int RL, bool AF32, bool ONE, bool REFL, int NP = 0>
+template <int SUB, int RL, bool AF32, bool ONE, bool REFL, int NP, bool SPLIT>
 __device__ __forceinline__ void gemv4s_body(const char *__restrict__ cw, const void *__restrict__ a_any, const OutSpec &out,
                                             float *__restrict__ ws, unsigned *__restrict__ counters, uint32_t cfg,
                                             uint32_t k, uint32_t n, uint32_t n_pad, uint32_t k_chunks,
                                             uint32_t sub_tiles, uint32_t cps,
                                             const uint16_t *__restrict__ ref_scales, uint32_t *trace_loaded)
 {
-    const uint32_t splits = cfg_splits(cfg), waves = cfg_waves(cfg), m_rows = cfg_rows(cfg);
+    const uint32_t splits = SPLIT ? cfg_splits(cfg) : 1u, waves = cfg_waves(cfg), m_rows = cfg_rows(cfg);
     const bool gated_store = cfg_gated(cfg);
     static_assert(!REFL || (AF32 && RL == 1), "the reference-layout variant is the M = 1, f32-activation entry point");
     constexpr int CPP = 64 / SUB;     // chunks per pass
@@ -86,7 +86,7 @@ __device__ __forceinline__ void gemv4s_body(const char *__restrict__ cw, const v
     const uint32_t b = blockIdx.x;
     const uint32_t xcd = b & 7u, jj = b >> 3;
     // (unsplit, as the planner's sub-tile forms are: no division in front of the first loads)
-    const uint32_t sp = splits == 1 ? 0u : jj % splits, jt = splits == 1 ? jj : jj / splits;
+    const uint32_t sp = SPLIT ? jj % splits : 0u, jt = SPLIT ? jj / splits : jj;
     // Workgroups reach the eight XCDs in turn by linear id.  Repacked copy: sub-tile = id (every block of the copy belongs
     // to one workgroup).  The reference's arrays: neighbouring sub-tiles share the 128-byte lines of the scale rows (32 or
     // 64 bytes per sub-tile and group), so each XCD takes a contiguous run of sub-tiles and the shared lines meet in its L2.
@@ -129,14 +129,11 @@ __device__ __forceinline__ void gemv4s_body(const char *__restrict__ cw, const v
             gemv4s_load_pass_ref<SUB, TERMS, RG>(r, cw, ref_scales, a_any, arow, kc, live, ref_col, st * SUB + cl < n, n, ref_groups,
                                                  cl, k, lane_is_lo);
         } else {
-            if (PIPE || UPFRONT) {
-                // activations first: loads complete in the order of their issue, and these come from the cache
+            if (PIPE || UPFRONT || F32_PIECE || (AF32 && RL == 2 && ONE)) {
+                // activations first: loads complete in the order of their issue, and these come from the cache (two f32 rows
+                // 3584 -> 4608 5.35 -> 4.86 us; in the pass loop, 9984 -> 2048, 7.6 -> 7.9)
                 gemv4s_load_a<SUB, AF32, TERMS, REFL, RG>(r, a_any, arow, kc, cl, k, lane_is_lo, m_rows);
                 gemv4s_load_w<SUB, RG, true>(r, tbase + (size_t)kc * kColBlockBytes, col_in_tile(cl), live);
-            } else if (F32_PIECE) {
-                // (the same order: the split of the f32 piece can then run while the weights are on their way)
-                gemv4s_load_a<SUB, AF32, TERMS, REFL, RG>(r, a_any, arow, kc, cl, k, lane_is_lo, m_rows);
-                gemv4s_load_w<SUB, RG, false>(r, tbase + (size_t)kc * kColBlockBytes, col_in_tile(cl), live);
             } else {
                 gemv4s_load_w<SUB, RG, false>(r, tbase + (size_t)kc * kColBlockBytes, col_in_tile(cl), live);
                 gemv4s_load_a<SUB, AF32, TERMS, REFL, RG>(r, a_any, arow, kc, cl, k, lane_is_lo, m_rows);
@@ -144,9 +141,50 @@ __device__ __forceinline__ void gemv4s_body(const char *__restrict__ cw, const v
         }
     };
     auto compute_pass = [&](const ChunkS<SUB, RG> &r) { gemv4s_compute<SUB, RL, TERMS, REFL>(r, dq, acc); };
+    // Where the lanes of wave 0 will store (E <= 64, unsplit: lane e = r * SUB + column), and the bias there: behind the barrier
+    // each is a round trip of its own.  f32 rows fetch them while the weights are on their way (4864 -> 896 4.09 -> 3.70 us,
+    // 3584 -> 4608 4.85 -> 4.56), f16 rows ahead of the barrier (on their way they cost 3584 -> 2 x 18944 0.5 us).
+    const uint32_t early_col = (REFL ? st * SUB + cl : tile * 64u + col_in_tile(cl));
+    float *early_dst = nullptr;
+    uint32_t early_ld = 0;
+    float early_bias = 0.f;
+    bool early_has_bias = false;
+    auto fetch_early = [&]() {
+        if (gated) {
+            const uint32_t feat = tile * 32u + part * (SUB / 2) + cl;
+            early_ld = n >> 1;
+            if (cl < SUB / 2 && feat < early_ld) early_dst = out.swiglu + feat;
+            return;
+        }
+        if (early_col >= n) return;
+#pragma unroll
+        for (uint32_t sg = 0; sg < kMaxSegs; sg++) {
+            if (sg < out.count) {
+                const uint32_t rel = early_col - out.seg[sg].start;
+                if (rel < out.seg[sg].width) {
+                    early_dst = out.seg[sg].ptr + rel;
+                    early_ld = out.seg[sg].width;
+                    if (out.seg[sg].bias) {
+                        early_bias = out.seg[sg].bias[rel];
+                        early_has_bias = true;
+                    }
+                }
+            }
+        }
+    };
     // (ONE: the launcher saw that no wave has a second pass: one register set, no loop)
-    if constexpr (UPFRONT) gemv4s_run_upfront<SUB, NP, RG>(wave, waves, passes, load_pass, compute_pass);
-    else gemv4s_run_passes<SUB, ONE, RG, PIPE>(wave, waves, passes, load_pass, compute_pass);
+    constexpr bool EARLY = !SPLIT && RL * SUB <= 64 && (ONE || UPFRONT);   // (the pass loops have no registers left for it)
+    auto between = [&]() {
+        if constexpr (EARLY && AF32) {
+            if (wave == 0) fetch_early();
+        } else {
+            // (so that the output description is in the scalar cache when the store asks for it)
+            asm volatile("" ::"s"(out.seg[0].ptr), "s"(out.seg[2].ptr), "s"(out.count));
+        }
+    };
+    if constexpr (UPFRONT) gemv4s_run_upfront<SUB, NP, RG>(wave, waves, passes, load_pass, compute_pass, between);
+    else gemv4s_run_passes<SUB, ONE, RG, PIPE>(wave, waves, passes, load_pass, compute_pass, between);
+    if (EARLY && !AF32 && wave == 0) fetch_early();
     if (trace_loaded && threadIdx.x == 0) *trace_loaded = (uint32_t)__builtin_amdgcn_s_memrealtime();  // data arrived and unpacked
 
     // ---- sum over the chunks of a pass (lane groups) inside the wave, over the waves through LDS ----
@@ -210,8 +248,11 @@ __device__ __forceinline__ void gemv4s_body(const char *__restrict__ cw, const v
         const uint32_t e = lane % E, r = e / SUB, c = e % SUB;
         float total = sum_lane_groups<E>(sum_waves(e, lane / E, PARTS));   // (every lane of an entry holds it)
         const bool owner = lane < E;
-        if (splits == 1) {
-            finish(r, c, total, gated ? __shfl_down(total, SUB / 2, 64) : 0.f, owner);
+        if constexpr (!SPLIT) {
+            const float up = gated ? __shfl_down(total, SUB / 2, 64) : 0.f;
+            if constexpr (!EARLY) finish(r, c, total, up, owner);
+            else if (owner && early_dst && r < m_rows)
+                early_dst[(size_t)r * early_ld] = gated ? gated_mul(out.gate_act, total, up) : early_has_bias ? total + early_bias : total;
             return;
         }
         // cross-workgroup split-K as in k_gemv4: park the partial, count arrivals, the last one adds in split order
@@ -240,7 +281,7 @@ __device__ __forceinline__ void gemv4s_body(const char *__restrict__ cw, const v
                 for (int q = 0; q < CPP; q++) v += red[(w * RL + r) * 64 + q * SUB + c];
             return v;
         };
-        if (splits == 1) {
+        if (!SPLIT) {
             for (uint32_t e = threadIdx.x; e < (uint32_t)E; e += threads) {
                 const uint32_t r = e / SUB, c = e % SUB;
                 if (gated) {
@@ -290,26 +331,26 @@ __device__ __forceinline__ void gemv4s_body(const char *__restrict__ cw, const v
 // one round trip to the scalar cache later, and with one workgroup per CU nothing hides that -- hence also the packed
 // word `cfg` (gemv4s_cfg: split factor, gated store, waves per workgroup, rows), which keeps the workgroup size out of
 // the dispatch packet's hidden arguments, where a read of blockDim would fetch it from.
-template <int SUB, int RL, bool AF32, bool ONE, bool REFL = false>
+template <int SUB, int RL, bool AF32, bool ONE, bool REFL, bool SPLIT>
 __global__ __launch_bounds__(1024) void k_gemv4s(const char *__restrict__ cw, const void *__restrict__ a_any,
                                                   const uint16_t *__restrict__ ref_scales, uint32_t cfg, uint32_t k,
                                                   uint32_t k_chunks, uint32_t sub_tiles, uint32_t cps, uint32_t n,
                                                   uint32_t n_pad, float *__restrict__ ws, unsigned *__restrict__ counters,
                                                   OutSpec out)
 {
-    gemv4s_body<SUB, RL, AF32, ONE, REFL>(cw, a_any, out, ws, counters, cfg, k, n, n_pad, k_chunks, sub_tiles, cps, ref_scales,
+    gemv4s_body<SUB, RL, AF32, ONE, REFL, 0, SPLIT>(cw, a_any, out, ws, counters, cfg, k, n, n_pad, k_chunks, sub_tiles, cps, ref_scales,
                                           nullptr);
 }
 
 // 16 columns, one row, up to NP passes per wave with all their loads issued up front.
-template <bool AF32, bool REFL, int NP>
+template <bool AF32, bool REFL, int NP, bool SPLIT>
 __global__ __launch_bounds__(1024) void k_gemv4s_upfront(const char *__restrict__ cw, const void *__restrict__ a_any,
                                                           const uint16_t *__restrict__ ref_scales, uint32_t cfg, uint32_t k,
                                                           uint32_t k_chunks, uint32_t sub_tiles, uint32_t cps, uint32_t n,
                                                           uint32_t n_pad, float *__restrict__ ws, unsigned *__restrict__ counters,
                                                           OutSpec out)
 {
-    gemv4s_body<16, 1, AF32, false, REFL, NP>(cw, a_any, out, ws, counters, cfg, k, n, n_pad, k_chunks, sub_tiles, cps, ref_scales,
+    gemv4s_body<16, 1, AF32, false, REFL, NP, SPLIT>(cw, a_any, out, ws, counters, cfg, k, n, n_pad, k_chunks, sub_tiles, cps, ref_scales,
                                               nullptr);
 }
 
@@ -331,7 +372,7 @@ __global__ __launch_bounds__(1024) void k_gemv4s_traced(const char *__restrict__
         // HW_ID (register 4): wave, SIMD, CU, SH, SE ids; XCC_ID (register 20): the XCD
         tr[3] = (__builtin_amdgcn_s_getreg((31 << 11) | 4) & 0xFFFFu) | (__builtin_amdgcn_s_getreg((3 << 11) | 20) << 16);
     }
-    gemv4s_body<SUB, 1, false, ONE, false>(cw, a_any, out, ws, counters, gemv4s_cfg(splits, out.swiglu != nullptr, blockDim.x >> 6, m_rows),
+    gemv4s_body<SUB, 1, false, ONE, false, 0, true>(cw, a_any, out, ws, counters, gemv4s_cfg(splits, out.swiglu != nullptr, blockDim.x >> 6, m_rows),
                                            k, n, n_pad, k_chunks, sub_tiles, cps, nullptr, tr + 1);
     if (threadIdx.x == 0) tr[2] = (uint32_t)__builtin_amdgcn_s_memrealtime();
 }
@@ -349,10 +390,15 @@ static hipError_t launch_gemv4s_t(hipStream_t s, const WeightView &w, const void
     size_t lds = (size_t)waves * RL * (RL * SUB > 64 ? 64 : SUB) * sizeof(float);   // (five rows and more: every lane writes, see gemv4s_body)
     const bool one = (cps + 64 / SUB - 1) / (64 / SUB) <= waves;
     const bool runs = blocks <= 512;  // few workgroups per CU: a contiguous run of sub-tiles per XCD
-#define TWM_S_LAUNCH(AF, ONEV)                                                                                          \
-    hipLaunchKernelGGL((k_gemv4s<SUB, RL, AF, ONEV>), dim3(blocks), dim3(waves * 64), lds, s, (const char *)w.cq, a,         \
+#define TWM_S_LAUNCH_S(AF, ONEV, SPLITV)                                                                                 \
+    hipLaunchKernelGGL((k_gemv4s<SUB, RL, AF, ONEV, false, SPLITV>), dim3(blocks), dim3(waves * 64), lds, s, (const char *)w.cq, a, \
                        (const uint16_t *)nullptr, gemv4s_cfg(splits, out.swiglu != nullptr, waves, m, runs), w.k, w.k_chunks, \
                        sub_tiles, cps, w.n, n_pad, ws, counters, out)
+#define TWM_S_LAUNCH(AF, ONEV)                   \
+    do {                                         \
+        if (splits > 1) TWM_S_LAUNCH_S(AF, ONEV, true); \
+        else TWM_S_LAUNCH_S(AF, ONEV, false);    \
+    } while (0)
     if constexpr (RL == 1) {
         if (!a_f32 && trace.ptr && blocks <= trace.capacity) {
             if (one)
@@ -367,13 +413,19 @@ static hipError_t launch_gemv4s_t(hipStream_t s, const WeightView &w, const void
     if constexpr (SUB == 16 && RL == 1) {
         const uint32_t np = ((cps + 3) / 4 + waves - 1) / waves;  // passes per wave
         if ((np == 2 || np == 3) && !out.swiglu) {
-#define TWM_S_UP(AF, NPV)                                                                                               \
-    hipLaunchKernelGGL((k_gemv4s_upfront<AF, false, NPV>), dim3(blocks), dim3(waves * 64), lds, s, (const char *)w.cq, a,    \
+#define TWM_S_UP_S(AF, NPV, SPLITV)                                                                                      \
+    hipLaunchKernelGGL((k_gemv4s_upfront<AF, false, NPV, SPLITV>), dim3(blocks), dim3(waves * 64), lds, s, (const char *)w.cq, a,    \
                        (const uint16_t *)nullptr, gemv4s_cfg(splits, false, waves, m, runs), w.k, w.k_chunks, sub_tiles, cps, \
                        w.n, n_pad, ws, counters, out)
+#define TWM_S_UP(AF, NPV)                      \
+    do {                                       \
+        if (splits > 1) TWM_S_UP_S(AF, NPV, true); \
+        else TWM_S_UP_S(AF, NPV, false);       \
+    } while (0)
             if (a_f32) { if (np == 2) TWM_S_UP(true, 2); else TWM_S_UP(true, 3); }
             else { if (np == 2) TWM_S_UP(false, 2); else TWM_S_UP(false, 3); }
 #undef TWM_S_UP
+#undef TWM_S_UP_S
             return hipGetLastError();
         }
     }
@@ -389,6 +441,7 @@ static hipError_t launch_gemv4s_t(hipStream_t s, const WeightView &w, const void
         else TWM_S_LAUNCH(false, false);
     }
 #undef TWM_S_LAUNCH
+#undef TWM_S_LAUNCH_S
     return hipGetLastError();
 }
 
@@ -438,28 +491,29 @@ hipError_t launch_gemv4s_ref(hipStream_t s, const uint8_t *packed, const uint16_
     out.seg[0].ptr = c;
     out.seg[0].start = 0;
     out.seg[0].width = n;
-#define TWM_S_REF(SUBV, ONEV)                                                                                          \
-    hipLaunchKernelGGL((k_gemv4s<SUBV, 1, true, ONEV, true>), dim3(blocks), dim3(waves * 64), lds, s, (const char *)packed, \
-                       (const void *)a, scales, gemv4s_cfg(splits, false, waves, 1u), k, k_chunks, sub_tiles, cps, n, n_pad, ws,  \
-                       counters, out)
+#define TWM_S_REF_ARGS                                                                                                   \
+    dim3(blocks), dim3(waves * 64), lds, s, (const char *)packed, (const void *)a, scales, gemv4s_cfg(splits, false, waves, 1u), k, k_chunks, \
+        sub_tiles, cps, n, n_pad, ws, counters, out
+#define TWM_S_REF(SUBV, ONEV)                                                                                            \
+    do {                                                                                                                 \
+        if (splits > 1) hipLaunchKernelGGL((k_gemv4s<SUBV, 1, true, ONEV, true, true>), TWM_S_REF_ARGS);                    \
+        else hipLaunchKernelGGL((k_gemv4s<SUBV, 1, true, ONEV, true, false>), TWM_S_REF_ARGS);                              \
+    } while (0)
+#define TWM_S_REF_UP(NPV)                                                                                                \
+    do {                                                                                                                 \
+        if (splits > 1) hipLaunchKernelGGL((k_gemv4s_upfront<true, true, NPV, true>), TWM_S_REF_ARGS);                       \
+        else hipLaunchKernelGGL((k_gemv4s_upfront<true, true, NPV, false>), TWM_S_REF_ARGS);                                 \
+    } while (0)
     const uint32_t np = ((cps + 3) / 4 + waves - 1) / waves;  // passes per wave on 16 columns
-    if (sub == 16 && (np == 2 || np == 3)) {
-        if (np == 2)
-            hipLaunchKernelGGL((k_gemv4s_upfront<true, true, 2>), dim3(blocks), dim3(waves * 64), lds, s, (const char *)packed, (const void *)a,
-                               scales, gemv4s_cfg(splits, false, waves, 1u), k, k_chunks, sub_tiles, cps, n, n_pad, ws, counters, out);
-        else
-            hipLaunchKernelGGL((k_gemv4s_upfront<true, true, 3>), dim3(blocks), dim3(waves * 64), lds, s, (const char *)packed, (const void *)a,
-                               scales, gemv4s_cfg(splits, false, waves, 1u), k, k_chunks, sub_tiles, cps, n, n_pad, ws, counters, out);
-        return hipGetLastError();
-    }
-    if (sub == 32) {
-        if (one) TWM_S_REF(32, true);
-        else TWM_S_REF(32, false);
-    } else {
-        if (one) TWM_S_REF(16, true);
-        else TWM_S_REF(16, false);
-    }
+    if (sub == 16 && np == 2) TWM_S_REF_UP(2);
+    else if (sub == 16 && np == 3) TWM_S_REF_UP(3);
+    else if (sub == 32 && one) TWM_S_REF(32, true);
+    else if (sub == 32) TWM_S_REF(32, false);
+    else if (one) TWM_S_REF(16, true);
+    else TWM_S_REF(16, false);
+#undef TWM_S_REF_UP
 #undef TWM_S_REF
+#undef TWM_S_REF_ARGS
     return hipGetLastError();
 }
 
