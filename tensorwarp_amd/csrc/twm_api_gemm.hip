@@ -218,7 +218,7 @@ static BatchPlan plan_batch(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, boo
 
 // ---- the launch form of a GEMM: chosen in one place, launched in another ---------------------------------
 // What twm_gemm will run for a weight's shape, a row count and the context's knobs.  Nothing here touches the device.
-enum FormKind { kFormPrefill = 0, kFormSubTile = 1, kFormWholeTile = 2, kFormBatch = 3, kFormStream = 4, kFormNone = 5, kFormWaves = 6 };
+enum FormKind { kFormPrefill = 0, kFormSubTile = 1, kFormWholeTile = 2, kFormBatch = 3, kFormStream = 4, kFormNone = 5, kFormWaves = 6, kFormGroupLane = 7 };
 struct LaunchForm {
     int kind;
     int copy;                 // the repacked order it reads (kCopyTile / kCopyCol)
@@ -359,6 +359,12 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
         sub.waves = e.sub_waves ? (uint32_t)e.sub_waves : e.waves ? (uint32_t)e.waves : 8;
     } else if (e.sub == 0 && !e.nt && !e.waves && !splits) {
         // (an explicit nt, waves or split factor asks for the 64-column kernel's plan)
+        if (e.kernel == 0 && (f.waves = plan_gemv4g(tiles64, k_chunks, m, a_f32, gated)) != 0) {
+            f.kind = kFormGroupLane;
+            f.sub = 16;
+            f.splits = 1;
+            return f;
+        }
         sub = plan_gemv4_sub(tiles64, k_chunks, m, a_f32, gated);
         // the gated store splits a sub-tile into a gate and an up half: 16 columns would read 128-byte runs
         // (3584 -> 2 x 18944 at M = 1: 17.0 us on 16 columns, 16.3 on 32, 17.1 on whole tiles)
@@ -401,6 +407,7 @@ uint32_t twm_pick_splits(uint32_t k, uint32_t n, uint32_t m)
     const LaunchForm f = choose_form(default_env(), n_tiles, k_chunks, m, false, 0, false);
     switch (f.kind) {
     case kFormSubTile:
+    case kFormGroupLane:
     case kFormWholeTile:
     case kFormWaves: return f.splits;
     case kFormBatch: return plan_batch(n_tiles, k_chunks, m < 32 ? m : 32, false).splits;
@@ -433,6 +440,7 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
         break;
     }
     case kFormSubTile:
+    case kFormGroupLane:   // (k_gemv4g: the same columns, waves and copy)
         snprintf(text, bytes, "k_gemv4s: %u-column sub-tiles, %u waves, %u K-split%s; column-lane copy", f.sub, f.waves, f.splits,
                  f.splits == 1 ? "" : "s");
         break;
@@ -529,6 +537,9 @@ static int gemm_dispatch(twm_ctx *ctx, const twm_weight *w, const void *a_dev, i
     case kFormSubTile:
         HIP_TRY(launch_gemv4s(ctx->stream, v, a_dev, a_f32, m, gated, ctx->ws, ctx->counters, f.sub, f.waves, f.splits, ctx->trace), TWM_DEVICE_ERROR,
                 "sub-tile gemv launch");
+        return TWM_OK;
+    case kFormGroupLane:
+        HIP_TRY(launch_gemv4g(ctx->stream, v, a_dev, a_f32, m, gated, f.waves, ctx->trace), TWM_DEVICE_ERROR, "group-lane gemv launch");
         return TWM_OK;
     case kFormWholeTile:
         HIP_TRY(launch_gemv4(ctx->stream, v, a_dev, a_f32, m, gated, ctx->ws, ctx->counters, f.nt, f.waves, f.splits, swiglu_out),

@@ -153,6 +153,10 @@ hipError_t launch_weight_dequant_f16_col(hipStream_t s, const WeightView &w, uin
 // of the N columns, write silu(gate) * up of every feature to swiglu_out[m][ffn]; `out` is ignored.
 hipError_t launch_gemv4s(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out,
                          float *ws, unsigned *counters, uint32_t sub, uint32_t waves, uint32_t splits, TraceBuf trace = TraceBuf{nullptr, 0});
+// a lane per column and group on small and narrow matrices (twm_gemv4g.hip): waves per workgroup (0: another form runs)
+uint32_t plan_gemv4g(uint32_t tiles64, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated);
+hipError_t launch_gemv4g(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out, uint32_t waves,
+                         TraceBuf trace = TraceBuf{nullptr, 0});
 hipError_t launch_gemv4s_ref(hipStream_t s, const uint8_t *packed, const uint16_t *scales, uint32_t k, uint32_t n,
                              const float *a, float *c, float *ws, unsigned *counters, uint32_t sub, uint32_t waves,
                              uint32_t splits);

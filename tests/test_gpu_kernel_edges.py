@@ -534,3 +534,40 @@ def test_an_infinite_activation_reaches_every_column_as_itself(dev, k, m):
     truth = O.gemm_f64(rows[others].astype(np.float32), packed, scales, len(others), k, n)
     close_rows(got[others], truth, F32_SUM)
     w.free()
+
+
+# one chunk in part, the most chunks with one each per wave and one more, K one group past whole chunks, four chunks per wave of
+# sixteen waves; a column and a sub-tile more than whole tiles
+@pytest.mark.parametrize("k,n", [(32, 1), (96, 17), (1408, 81), (1440, 64), (2592, 130), (3616, 33), (8192, 65)])
+@pytest.mark.parametrize("m,dtype", [(1, "f16"), (2, "f16"), (3, "f16"), (4, "f16"), (1, "f32")])
+def test_up_to_four_rows_on_small_matrices(dev, k, n, m, dtype):
+    packed, scales, w = weight(dev, k, n, 2101)
+    a16 = O.synth_act_f16(m, k, 2103)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+    if dtype == "f32":
+        a[0, : k // 2] *= np.float32(2.0 ** 20)      # half of the row outside the f16 range
+    parts = [n] if n < 3 else [n // 2, n - n // 2]
+    outs = [T.GpuTensor.from_host(dev, np.full((m, x), np.nan, np.float32)) for x in parts]
+    b = O.synth_normal_f32(n, 2105)
+    bias = [T.GpuTensor.from_host(dev, x) for x in np.split(b, np.cumsum(parts)[:-1])]
+    T.gemm_split(dev, w, T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a), m, outs, parts, biases=bias)
+    truth = O.gemm_f64(a, packed, scales, m, k, n)
+    got = np.concatenate([o.to_host() for o in outs], axis=1)
+    floor = np.maximum(np.abs(truth), 1e-3 * np.abs(truth).max(axis=1, keepdims=True))
+    assert (np.abs(got - (truth + b)) <= F32_SUM * floor + 2.0 ** -23 * np.abs(truth + b)).all()
+    w.free()
+
+
+@pytest.mark.parametrize("k,ffn", [(32, 32), (1440, 96), (2720, 32), (8192, 64)])
+@pytest.mark.parametrize("m,dtype", [(1, "f16"), (2, "f16"), (4, "f16"), (1, "f32")])
+def test_up_to_four_rows_gated_on_small_matrices(dev, k, ffn, m, dtype):
+    gate, up = [(O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (2111, 2113)]
+    pair = [tuple(T.GpuTensor.from_host(dev, x, t) for x, t in zip(w, ("u8", "f16"))) for w in (gate, up)]
+    w = T.MarlinWeight.gate_up(dev, *pair, k, ffn)
+    a16 = O.synth_act_f16(m, k, 2115)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k)
+    g, u = (O.gemm_f64(a, *x, m, k, ffn) for x in (gate, up))
+    out = T.GpuTensor.from_host(dev, np.full((m, ffn), np.nan, np.float32))
+    T.gemm_swiglu(dev, w, T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a), m, out)
+    close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
+    w.free()
