@@ -28,127 +28,150 @@ __device__ __forceinline__ uint32_t expert_of(float id, uint32_t experts)
     return (id >= 0.f && id < (float)experts) ? (uint32_t)id : experts;
 }
 
-// Both kernels work on sub-tiles of SUB = 16 or 32 columns (see twm_gemv4_core.h): a wave covers 64 / SUB
-// consecutive chunks of them in one pass, so that the short K of an expert matrix (a few chunks) still gives
-// every wave of a workgroup one pass and the launch many workgroups.
+// Both kernels work on sub-tiles of 16 columns (see twm_gemv4_core.h): a wave covers four consecutive chunks of them in one
+// pass, so that the short K of an expert matrix (a few chunks) still gives every wave of a workgroup one pass and the launch
+// many workgroups.
+// What bounds these launches is a chain of round trips, not the 9 or 18 MB of weights: the slot's expert id, then its weights,
+// then the store.  So nothing else waits: the arguments that the loads need arrive preloaded (thirteen words), the activations
+// are loaded ahead of the id, the accumulator and the slots' weights ahead of the weights, the wave's four chunks are summed by
+// lane swaps, and the waves' sums by reads that do not wait for each other -- the sums are in chunk order within a pass ((0 + 2)
+// + (1 + 3)) and in pass order behind it, the same in both kernels.
+// (us in a graph, against one thread per column walking 22 and 64 dependent LDS reads, the activations behind the id and the
+// accumulator and weights behind the barrier: 2816 -> 2 x 704 gated, eight of 128 experts 6.07 -> 5.27, 704 -> 2816 level at 6.1;
+// 4096 -> 2 x 1408, six of 16, 10.6 -> 9.15, 1408 -> 4096 8.36 -> 7.76.)
 
-// Workgroup = `waves` waves on one sub-tile of one slot's expert; wave w takes passes w, w + waves, ...
-// grid = (sub-tiles, slots).  ACT 0: out[slot][n]; 1 / 2: paired bank (each 64-column tile is 32 gate columns,
-// then the up columns of the same features; the workgroup takes SUB / 2 of each),
-// out[slot][n/2] = gelu_tanh / silu (gate) * up.
-template <int SUB, bool AF32, int ACT, bool ONE>
-__global__ __launch_bounds__(1024) void k_bank_gemv(const char *__restrict__ bank, size_t expert_bytes, uint32_t experts,
-                                                     const void *__restrict__ a_any, uint32_t a_slot_stride,
-                                                     const float *__restrict__ ids, float *__restrict__ out,
-                                                     uint32_t k, uint32_t n, uint32_t k_chunks, uint32_t sub_tiles)
+// What a wave sums over its passes first, first + stride, ... of a sub-tile; ONE: it has one.  between: what it does once its
+// loads are on their way.  An id that is no expert reads expert 0 and counts as zero (a branch would take the activations'
+// loads behind the id).
+template <bool AF32, bool ONE, class Between>
+__device__ __forceinline__ float bank_dot(const char *__restrict__ bank, size_t expert_bytes, uint32_t experts, const void *__restrict__ a_row,
+                                          const float *__restrict__ id, uint32_t first, uint32_t stride, uint32_t tile, uint32_t col,
+                                          uint32_t k, uint32_t k_chunks, Between between)
 {
-    constexpr int CPP = 64 / SUB;
-    constexpr int TERMS = AF32 ? kTermsOneRowF32 : kTermsOne;   // one row: f32 activations as two f16 terms of one shared piece per lane
-    extern __shared__ float red[];  // [waves][64]
-    // (gridDim.x is a multiple of 8, workgroups reach the eight XCDs in turn: a contiguous run of sub-tiles per XCD, so
-    // that the sub-tiles of a 64-column tile, whose pieces interleave inside the copy's blocks, stream through one L2)
-    const uint32_t st = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3), slot = blockIdx.y;
-    if (st >= sub_tiles) return;
-    const uint32_t waves = blockDim.x >> 6;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int SUB = 16, CPP = 4;
+    constexpr int TERMS = AF32 ? kTermsOneRowF32 : kTermsOneRow;   // one row: a lane loads one piece of its chunk
     const uint32_t lane = threadIdx.x & 63u, cl = lane % SUB, cg = lane / SUB;
-    const uint32_t tile = st / CPP, part = st % CPP;
-    const uint32_t eid = __builtin_amdgcn_readfirstlane(expert_of(ids[slot], experts));
-    const uint32_t col = ACT ? (cl / (SUB / 2)) * 32u + part * (SUB / 2) + cl % (SUB / 2) : part * SUB + cl;
     const uint32_t passes = (k_chunks + CPP - 1) / CPP;
-
     float acc[1] = {0.f};
-    if (eid < experts) {
-        const char *tbase = bank + (size_t)eid * expert_bytes + (size_t)tile * k_chunks * kColBlockBytes;
-        const void *a_row = (const char *)a_any + (size_t)slot * a_slot_stride * (AF32 ? 4 : 2);
+    bool ok;
+    if (ONE) {
+        ChunkS<SUB> r;
+        uint32_t kc = first * CPP + cg;
+        const bool live = kc < k_chunks;
+        kc = live ? kc : k_chunks - 1u;
+        gemv4s_load_a<SUB, AF32, TERMS>(r, a_row, 0, kc, cl, k, false);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t eid = __builtin_amdgcn_readfirstlane(expert_of(*id, experts));
+        ok = eid < experts;
+        gemv4s_load_w<SUB, 1, true>(r, bank + (size_t)(ok ? eid : 0u) * expert_bytes + ((size_t)tile * k_chunks + kc) * kColBlockBytes, col, live);
+        __builtin_amdgcn_sched_barrier(0);
+        between();
+        gemv4s_compute<SUB, 1, TERMS>(r, make_gemv4_consts(), acc);
+    } else {
+        const uint32_t eid = __builtin_amdgcn_readfirstlane(expert_of(*id, experts));
+        ok = eid < experts;
+        const char *tbase = bank + (size_t)(ok ? eid : 0u) * expert_bytes + (size_t)tile * k_chunks * kColBlockBytes;
         const Gemv4Consts dq = make_gemv4_consts();
-        const bool is_lo = (cl & 1u) != 0;
-        gemv4s_run_passes<SUB, ONE>(
-            wave, waves, passes,
+        gemv4s_run_passes<SUB, false, 1, true>(
+            first, stride, passes,
             [&](ChunkS<SUB> &r, uint32_t pass) {
                 uint32_t kc = pass * CPP + cg;
                 const bool live = kc < k_chunks;
                 kc = live ? kc : k_chunks - 1u;
-                gemv4s_load_w<SUB>(r, tbase + (size_t)kc * kColBlockBytes, col, live);
-                gemv4s_load_a<SUB, AF32, TERMS>(r, a_row, 0, kc, cl, k, is_lo);
+                gemv4s_load_a<SUB, AF32, TERMS>(r, a_row, 0, kc, cl, k, false);
+                gemv4s_load_w<SUB, 1, true>(r, tbase + (size_t)kc * kColBlockBytes, col, live);
             },
-            [&](const ChunkS<SUB> &r) { gemv4s_compute<SUB, 1, TERMS>(r, dq, acc); });
+            [&](const ChunkS<SUB> &r) { gemv4s_compute<SUB, 1, TERMS>(r, dq, acc); }, between);
     }
-    red[wave * 64 + lane] = acc[0];
-    __syncthreads();
-    auto summed = [&](uint32_t c) {
-        float v = 0.f;
-        for (uint32_t w = 0; w < waves; w++)
+    const float dot = sum_lane_groups<SUB>(acc[0]);
+    return ok ? dot : 0.f;
+}
+
+// The sum of count (<= 16) values at, at + 16, ... in their order: the reads are independent
+__device__ __forceinline__ float bank_sum(const float *at, uint32_t count)
+{
+    float x[16];
 #pragma unroll
-            for (int q = 0; q < CPP; q++) v += red[w * 64 + q * SUB + c];
-        return v;
-    };
+    for (uint32_t w = 0; w < 16; w++) x[w] = at[(w < count ? w : 0u) * 16u];
+    float v = x[0];
+#pragma unroll
+    for (uint32_t w = 1; w < 16; w++) v += w < count ? x[w] : 0.f;
+    return v;
+}
+
+// Workgroup = `waves` waves on one sub-tile of one slot's expert; wave w takes passes w, w + waves, ...
+// grid = (sub-tiles, slots).  ACT 0: out[slot][n]; 1 / 2: paired bank (each 64-column tile is 32 gate columns,
+// then the up columns of the same features; the workgroup takes eight of each),
+// out[slot][n/2] = gelu_tanh / silu (gate) * up.
+template <bool AF32, int ACT, bool ONE>
+__global__ __launch_bounds__(1024) void k_bank_gemv(const float *__restrict__ ids, const void *__restrict__ a_any,
+                                                     const char *__restrict__ bank, size_t expert_bytes, uint32_t experts,
+                                                     uint32_t a_slot_stride, uint32_t k, uint32_t sub_tiles, uint32_t waves,
+                                                     uint32_t n, float *__restrict__ out)
+{
+    constexpr int SUB = 16, CPP = 4;
+    __shared__ float red[16 * SUB];  // [waves][16]
+    // (workgroups reach the eight XCDs in turn: a contiguous run of sub-tiles per XCD, so that the sub-tiles of a 64-column
+    // tile, whose pieces interleave inside the copy's blocks, stream through one L2)
+    const uint32_t st = (blockIdx.x & 7u) * ((sub_tiles + 7u) >> 3) + (blockIdx.x >> 3), slot = blockIdx.y;
+    if (st >= sub_tiles) return;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u, cl = lane % SUB;
+    const uint32_t tile = st / CPP, part = st % CPP;
+    const uint32_t col = ACT ? (cl / (SUB / 2)) * 32u + part * (SUB / 2) + cl % (SUB / 2) : part * SUB + cl;
+    const void *a_row = (const char *)a_any + (size_t)slot * a_slot_stride * (AF32 ? 4 : 2);
+    const float dot = bank_dot<AF32, ONE>(bank, expert_bytes, experts, a_row, ids + slot, wave, waves, tile, col, k, (k + 127u) >> 7, [&]() {
+        asm volatile("" ::"s"(out), "s"(n));   // (the store's arguments, fetched meanwhile)
+    });
+    if (lane < SUB) red[wave * SUB + cl] = dot;
+    __syncthreads();
+    if (wave != 0) return;
+    const float total = bank_sum(red + cl, waves);
     if (ACT == 0) {
-        if (threadIdx.x < SUB) {
-            uint32_t on = st * SUB + threadIdx.x;
-            if (on < n) out[(size_t)slot * n + on] = summed(threadIdx.x);
-        }
-    } else if (threadIdx.x < SUB / 2) {
-        uint32_t dim = n >> 1, feat = tile * 32u + part * (SUB / 2) + threadIdx.x;
-        if (feat < dim) out[(size_t)slot * dim + feat] = gate_mul<ACT>(summed(threadIdx.x), summed(SUB / 2 + threadIdx.x));
+        const uint32_t on = st * SUB + cl;
+        if (lane < SUB && on < n) out[(size_t)slot * n + on] = total;
+    } else {
+        const float up = __shfl_down(total, SUB / 2, 64);
+        const uint32_t dim = n >> 1, feat = tile * 32u + part * (SUB / 2) + cl;
+        if (lane < SUB / 2 && feat < dim) out[(size_t)slot * dim + feat] = gate_mul<ACT>(total, up);
     }
 }
 
 // Workgroup = slots * wps waves on one sub-tile: wave (slot, j) takes passes j, j + wps, ... of its slot's
 // expert with its slot's activation row; one thread per column then adds weight[slot] * dot to the accumulator
-// slot by slot.
-template <int SUB, bool AF32, bool ONE>
-__global__ __launch_bounds__(1024) void k_bank_down_axpy(const char *__restrict__ bank, size_t expert_bytes, uint32_t experts,
-                                                          const void *__restrict__ a_all, const float *__restrict__ ids,
-                                                          const float *__restrict__ weights, float *__restrict__ accum,
-                                                          uint32_t k, uint32_t n, uint32_t k_chunks, uint32_t sub_tiles,
-                                                          uint32_t slots, uint32_t wps)
+// slot by slot.  slots_wps: slots | wps << 8 | ceil(256 / wps) << 16 (which makes wave / wps, up to 16, a product and a shift).
+template <bool AF32, bool ONE>
+__global__ __launch_bounds__(1024) void k_bank_down_axpy(const float *__restrict__ ids, const void *__restrict__ a_all,
+                                                          const char *__restrict__ bank, size_t expert_bytes, uint32_t experts,
+                                                          uint32_t k, uint32_t sub_tiles, uint32_t slots_wps, uint32_t n,
+                                                          const float *__restrict__ weights, float *__restrict__ accum)
 {
-    constexpr int CPP = 64 / SUB;
-    constexpr int TERMS = AF32 ? kTermsOneRowF32 : kTermsOne;
-    extern __shared__ float red[];  // [slots * wps][64]
-    const uint32_t st = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);  // (a contiguous run per XCD, as in k_bank_gemv)
+    constexpr int SUB = 16, CPP = 4;
+    __shared__ float red[16 * SUB];  // [slots * wps][16]
+    const uint32_t slots = slots_wps & 255u, wps = (slots_wps >> 8) & 255u;
+    const uint32_t st = (blockIdx.x & 7u) * ((sub_tiles + 7u) >> 3) + (blockIdx.x >> 3);  // (a contiguous run per XCD, as in k_bank_gemv)
     if (st >= sub_tiles) return;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t lane = threadIdx.x & 63u, cl = lane % SUB, cg = lane / SUB;
-    const uint32_t tile = st / CPP, part = st % CPP;
-    const uint32_t slot = wave / wps, j = wave % wps;
-    const uint32_t eid = __builtin_amdgcn_readfirstlane(expert_of(ids[slot], experts));
-    const uint32_t passes = (k_chunks + CPP - 1) / CPP;
-
-    float acc[1] = {0.f};
-    if (eid < experts) {
-        const char *tbase = bank + (size_t)eid * expert_bytes + (size_t)tile * k_chunks * kColBlockBytes;
-        const void *a_row = (const char *)a_all + (size_t)slot * k * (AF32 ? 4 : 2);
-        const Gemv4Consts dq = make_gemv4_consts();
-        const bool is_lo = (cl & 1u) != 0;
-        gemv4s_run_passes<SUB, ONE>(
-            j, wps, passes,
-            [&](ChunkS<SUB> &r, uint32_t pass) {
-                uint32_t kc = pass * CPP + cg;
-                const bool live = kc < k_chunks;
-                kc = live ? kc : k_chunks - 1u;
-                gemv4s_load_w<SUB>(r, tbase + (size_t)kc * kColBlockBytes, part * SUB + cl, live);
-                gemv4s_load_a<SUB, AF32, TERMS>(r, a_row, 0, kc, cl, k, is_lo);
-            },
-            [&](const ChunkS<SUB> &r) { gemv4s_compute<SUB, 1, TERMS>(r, dq, acc); });
-    }
-    red[wave * 64 + lane] = acc[0];
-    __syncthreads();
-    if (threadIdx.x < SUB) {
-        uint32_t on = st * SUB + threadIdx.x;
-        if (on < n) {
-            float total = accum[on];
-            for (uint32_t s = 0; s < slots; s++) {
-                float dot = 0.f;
-                for (uint32_t q = 0; q < wps; q++)
+    const uint32_t lane = threadIdx.x & 63u, cl = lane % SUB;
+    const uint32_t slot = (wave * (slots_wps >> 16)) >> 8, j = wave - slot * wps;
+    const uint32_t on = st * SUB + cl;
+    float total = 0.f, w[kMaxBankSlots];
+    auto fetch = [&]() {
+        if (wave != 0) return;
+        if (on < n) total = accum[on];
 #pragma unroll
-                    for (int c = 0; c < CPP; c++) dot += red[(s * wps + q) * 64 + c * SUB + threadIdx.x];
-                total += weights[s] * dot;
-            }
-            accum[on] = total;
-        }
+        for (uint32_t s = 0; s < (uint32_t)kMaxBankSlots; s++) w[s] = weights[s < slots ? s : 0u];
+    };
+    const void *a_row = (const char *)a_all + (size_t)slot * k * (AF32 ? 4 : 2);
+    const float dot = bank_dot<AF32, ONE>(bank, expert_bytes, experts, a_row, ids + slot, j, wps, st / CPP, (st % CPP) * SUB + cl, k, (k + 127u) >> 7, fetch);
+    if (lane < SUB) red[wave * SUB + cl] = dot;
+    __syncthreads();
+    if (wave != 0 || lane >= SUB || on >= n) return;
+#pragma unroll
+    for (uint32_t s = 0; s < (uint32_t)kMaxBankSlots; s++) {
+        if (s < slots) total += w[s] * bank_sum(red + s * wps * SUB + cl, wps);
     }
+    accum[on] = total;
 }
 
 // ---- the same two launches on the reference's own slabs (no bank, nothing repacked) --------------------------
@@ -310,76 +333,66 @@ hipError_t launch_geglu_rows(hipStream_t s, const float *gu, float *out, uint32_
     return hipGetLastError();
 }
 
-// Sub-tile width of the bank kernels (force_sub = 16 or 32 overrides: a tuning knob of the context).  The
+// Sub-tile width of the kernels on the reference's slabs (force_sub = 16 or 32 overrides: a tuning knob of the context).  The
 // per-slot GEMV runs best on 32 columns once that gives a workgroup per CU (Gemma, Qwen and Mixtral expert
 // shapes: 7.0 against 7.6, 5.5 against 5.9, 26.9 against 29.7 us); the down projection, whose workgroups hold
 // every slot, on 16 (6.6 against 7.9, 5.6 against 7.6, 15.4 against 18.6 us).
-static uint32_t bank_sub(uint32_t n_pad, uint32_t slots, bool per_slot, int force_sub)
+static uint32_t raw_sub(uint32_t n_pad, uint32_t slots, bool per_slot, int force_sub)
 {
     if (force_sub == 16 || force_sub == 32) return (uint32_t)force_sub;
     return per_slot && (uint64_t)(n_pad / 32) * slots >= 256 ? 32 : 16;
 }
 
 hipError_t launch_bank_gemv(hipStream_t s, const BankView &b, const void *a, bool a_f32, uint32_t a_slot_stride,
-                            const float *ids, uint32_t slots, int act, float *out, int force_sub, int force_waves)
+                            const float *ids, uint32_t slots, int act, float *out, int force_waves)
 {
     if (slots == 0 || b.n == 0) return hipSuccess;
     if (!b.cq || act < 0 || act > 2 || slots > 65535u) return hipErrorInvalidValue;
     if (act != 0 && b.n % (2 * kPairWidth) != 0) return hipErrorInvalidValue;
-    const uint32_t sub = bank_sub(b.n_pad, slots, true, force_sub), sub_tiles = b.n_pad / sub;
-    const uint32_t passes = (b.k_chunks + 64 / sub - 1) / (64 / sub);
+    const uint32_t sub_tiles = b.n_pad / 16, passes = (b.k_chunks + 3) / 4;
     uint32_t waves = passes < 16 ? passes : 16;
     if (force_waves >= 1 && force_waves <= 16) waves = (uint32_t)force_waves;
     const bool one = passes <= waves;
     dim3 grid(((sub_tiles + 7) / 8) * 8, slots), block(waves * 64);  // (whole rounds of the eight XCDs: see k_bank_gemv)
-    size_t lds = (size_t)waves * 64 * sizeof(float);
-#define TWM_BANK_LAUNCH(SUBV, F32, A, ONEV)                                                                            \
-    hipLaunchKernelGGL((k_bank_gemv<SUBV, F32, A, ONEV>), grid, block, lds, s, (const char *)b.cq, b.expert_bytes,      \
-                       b.experts, a, a_slot_stride, ids, out, b.k, b.n, b.k_chunks, sub_tiles)
-#define TWM_BANK_ONE(SUBV, F32, A)                  \
-    if (one) TWM_BANK_LAUNCH(SUBV, F32, A, true);   \
-    else TWM_BANK_LAUNCH(SUBV, F32, A, false)
-#define TWM_BANK_ACT(SUBV, F32)                     \
-    if (act == 0) { TWM_BANK_ONE(SUBV, F32, 0); }   \
-    else if (act == 1) { TWM_BANK_ONE(SUBV, F32, 1); } \
-    else { TWM_BANK_ONE(SUBV, F32, 2); }
-    if (sub == 16) {
-        if (a_f32) { TWM_BANK_ACT(16, true) } else { TWM_BANK_ACT(16, false) }
-    } else {
-        if (a_f32) { TWM_BANK_ACT(32, true) } else { TWM_BANK_ACT(32, false) }
-    }
+#define TWM_BANK_LAUNCH(F32, A, ONEV)                                                                                  \
+    hipLaunchKernelGGL((k_bank_gemv<F32, A, ONEV>), grid, block, 0, s, ids, a, (const char *)b.cq, b.expert_bytes,     \
+                       b.experts, a_slot_stride, b.k, sub_tiles, waves, b.n, out)
+#define TWM_BANK_ACT(F32, ONEV)                            \
+    do {                                                   \
+        if (act == 0) TWM_BANK_LAUNCH(F32, 0, ONEV);       \
+        else if (act == 1) TWM_BANK_LAUNCH(F32, 1, ONEV);  \
+        else TWM_BANK_LAUNCH(F32, 2, ONEV);                \
+    } while (0)
+    if (a_f32 && one) TWM_BANK_ACT(true, true);
+    else if (a_f32) TWM_BANK_ACT(true, false);
+    else if (one) TWM_BANK_ACT(false, true);
+    else TWM_BANK_ACT(false, false);
 #undef TWM_BANK_ACT
-#undef TWM_BANK_ONE
 #undef TWM_BANK_LAUNCH
     return hipGetLastError();
 }
 
 hipError_t launch_bank_down_axpy(hipStream_t s, const BankView &b, const void *a_all, bool a_f32, const float *ids,
-                                 const float *weights, uint32_t slots, float *accum, int force_sub, int force_waves)
+                                 const float *weights, uint32_t slots, float *accum, int force_waves)
 {
     if (slots == 0 || b.n == 0) return hipSuccess;
     if (!b.cq || slots > (uint32_t)kMaxBankSlots) return hipErrorInvalidValue;
-    const uint32_t sub = bank_sub(b.n_pad, slots, false, force_sub), sub_tiles = b.n_pad / sub;
-    const uint32_t passes = (b.k_chunks + 64 / sub - 1) / (64 / sub);
+    const uint32_t sub_tiles = b.n_pad / 16, passes = (b.k_chunks + 3) / 4;
     uint32_t wps = 16 / slots;                // waves per slot: up to one per pass, sixteen waves in all
     if (wps > passes) wps = passes;
     if (force_waves >= 1 && (uint32_t)force_waves * slots <= 16) wps = (uint32_t)force_waves;
     if (wps == 0) wps = 1;
-    const bool one = passes <= wps;
-    const uint32_t waves = slots * wps;
-    size_t lds = (size_t)waves * 64 * sizeof(float);
-#define TWM_DOWN_LAUNCH(SUBV, F32, ONEV)                                                                               \
-    hipLaunchKernelGGL((k_bank_down_axpy<SUBV, F32, ONEV>), dim3(((sub_tiles + 7) / 8) * 8), dim3(waves * 64), lds, s, (const char *)b.cq, \
-                       b.expert_bytes, b.experts, a_all, ids, weights, accum, b.k, b.n, b.k_chunks, sub_tiles, slots, wps)
-#define TWM_DOWN_ONE(SUBV, F32)                  \
-    if (one) TWM_DOWN_LAUNCH(SUBV, F32, true);   \
-    else TWM_DOWN_LAUNCH(SUBV, F32, false)
-    if (sub == 16) {
-        if (a_f32) { TWM_DOWN_ONE(16, true); } else { TWM_DOWN_ONE(16, false); }
+    const uint32_t slots_wps = slots | (wps << 8) | (((256u + wps - 1u) / wps) << 16);
+#define TWM_DOWN_LAUNCH(F32, ONEV)                                                                                     \
+    hipLaunchKernelGGL((k_bank_down_axpy<F32, ONEV>), dim3(((sub_tiles + 7) / 8) * 8), dim3(slots * wps * 64), 0, s, ids, a_all, \
+                       (const char *)b.cq, b.expert_bytes, b.experts, b.k, sub_tiles, slots_wps, b.n, weights, accum)
+    if (passes <= wps) {
+        if (a_f32) TWM_DOWN_LAUNCH(true, true);
+        else TWM_DOWN_LAUNCH(false, true);
     } else {
-        if (a_f32) { TWM_DOWN_ONE(32, true); } else { TWM_DOWN_ONE(32, false); }
+        if (a_f32) TWM_DOWN_LAUNCH(true, false);
+        else TWM_DOWN_LAUNCH(false, false);
     }
-#undef TWM_DOWN_ONE
 #undef TWM_DOWN_LAUNCH
     return hipGetLastError();
 }
@@ -403,7 +416,7 @@ hipError_t launch_raw_gemv(hipStream_t s, const RawView &v, const float *a, uint
     if (slots == 0 || v.n == 0) return hipSuccess;
     if (v.k == 0 || v.k % 32 != 0 || slots > 65535u) return hipErrorInvalidValue;
     const uint32_t n_pad = ((v.n + 63) / 64) * 64, k_chunks = (v.k / 32 + 3) / 4;
-    const uint32_t sub = bank_sub(n_pad, slots, true, force_sub), sub_tiles = (v.n + sub - 1) / sub;
+    const uint32_t sub = raw_sub(n_pad, slots, true, force_sub), sub_tiles = (v.n + sub - 1) / sub;
     const uint32_t passes = (k_chunks + 64 / sub - 1) / (64 / sub);
     uint32_t waves = passes < 16 ? passes : 16;
     if (force_waves >= 1 && force_waves <= 16) waves = (uint32_t)force_waves;
@@ -434,7 +447,7 @@ hipError_t launch_raw_down_axpy(hipStream_t s, const RawView &v, const float *a_
     const RawSlab e = raw_slab(v);
     for (uint32_t s0 = 0; s0 < slots; s0 += kMaxBankSlots) {
         const uint32_t now = slots - s0 < (uint32_t)kMaxBankSlots ? slots - s0 : (uint32_t)kMaxBankSlots;
-        const uint32_t sub = bank_sub(n_pad, now, false, force_sub), sub_tiles = (v.n + sub - 1) / sub;
+        const uint32_t sub = raw_sub(n_pad, now, false, force_sub), sub_tiles = (v.n + sub - 1) / sub;
         const uint32_t passes = (k_chunks + 64 / sub - 1) / (64 / sub);
         uint32_t wps = 16 / now;
         if (wps > passes) wps = passes;
