@@ -22,6 +22,15 @@
         }                                                                              \
     } while (0)
 
+constexpr size_t kPlainNodes = 20;   // most nodes of a graph that is replayed launch by launch (plain_chain, twm_api.hip)
+// a device copy recorded into an open capture, and its node
+struct PlainCopy {
+    hipGraphNode_t node;
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+
 struct twm_ctx {
     int ordinal;
     twm::TraceBuf trace;  // twm_debug_trace: where this context's M = 1 sub-tile launches record their clocks (null: off)
@@ -32,6 +41,7 @@ struct twm_ctx {
     unsigned *counters;   // one arrival counter per tile group, zero between launches
     uint32_t n_counters;
     bool capturing;
+    std::vector<PlainCopy> captured_copies;  // twm_memcpy_d2d's of the open capture
     int force_nt;         // 0 = heuristic
     int force_waves;      // 0 = heuristic
     int force_sub_waves;  // sub-tile kernels with a forced width: waves per workgroup (1 .. 16), 0 = "waves" or eight
@@ -91,9 +101,16 @@ struct twm_bank {
     bool paired;
 };
 
+// A captured graph.  `plain`: it is a chain of at most kPlainNodes kernels and twm_memcpy_d2d copies, which a replay launches
+// one by one (see twm_graph_end); exec is null then.  Otherwise exec is launched.
+struct PlainNode {
+    hipKernelNodeParams kernel;   // (its arguments belong to the graph)
+    PlainCopy copy;               // bytes != 0: a copy
+};
 struct twm_graph {
     hipGraph_t graph;
     hipGraphExec_t exec;
+    std::vector<PlainNode> plain;
 };
 
 // Scratch of a context, held from its creation on: split-K sums and the f16 terms of f32 rows.  256 MB of the card's 288 GB

@@ -571,3 +571,40 @@ def test_up_to_four_rows_gated_on_small_matrices(dev, k, ffn, m, dtype):
     T.gemm_swiglu(dev, w, T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a), m, out)
     close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
     w.free()
+
+
+@pytest.mark.parametrize("copies,gemms", [(1, 0), (1, 1), (3, 17), (4, 16), (5, 16), (2, 30)])
+def test_graphs_about_the_longest_that_replays_launch_by_launch(dev, copies, gemms):
+    # twenty nodes and twenty-one, copies between the launches, replays with new inputs and eager work between them
+    k, n = 256, 64
+    packed, scales, w = weight(dev, k, n, 2201)
+    a = T.GpuTensor.zeros(dev, (1, k), "f16")
+    src = [T.GpuTensor.zeros(dev, (n,), "f32") for _ in range(copies)]
+    dst = [T.GpuTensor.zeros(dev, (n,), "f32") for _ in range(copies)]
+    outs = [T.GpuTensor.zeros(dev, (1, n), "f32") for _ in range(gemms)]
+
+    def work():
+        for i in range(max(copies, gemms)):
+            if i < copies:
+                T.quantize._check(T._lib.load().twm_memcpy_d2d(dev.handle, dst[i].ptr, src[i].ptr, 4 * n))
+            if i < gemms:
+                T.gemm(dev, w, a, 1, outs[i])
+
+    graph = T.GraphCapture.record_with_device(dev, work)
+    for rep in range(3):
+        rows = O.synth_act_f16(1, k, 2203 + rep)
+        a.copy_from_host(rows.reshape(1, k))
+        for i, s in enumerate(src):
+            s.copy_from_host(np.full(n, 10 * rep + i, np.float32))
+        graph.replay()
+        dev.synchronize()
+        truth = O.gemm_f64(rows.view(np.float16).astype(np.float32).reshape(1, k), packed, scales, 1, k, n)
+        for o in outs:
+            close_rows(o.to_host(), truth, F32_SUM)
+        for i, d in enumerate(dst):
+            assert (d.to_host() == 10 * rep + i).all()
+        eager = T.GpuTensor.zeros(dev, (1, n), "f32")
+        T.gemm(dev, w, a, 1, eager)
+        assert all(np.array_equal(eager.to_host(), o.to_host()) for o in outs)
+    graph.destroy()
+    w.free()
