@@ -130,7 +130,7 @@ int twm_ctx_info(twm_ctx *ctx, char *buf, size_t buf_len);
  *   "sub_waves"     waves per workgroup of the sub-tile kernels when "sub" forces their width (1 .. 16)
  *   "prefill_min_m" smallest M that runs the prefill GEMM (default 33; below it the decode kernels run)
  *   "prefill_bm"    prefill block form: 64 = 64 rows x 256 columns, 128 = 128 x 256, 192 = 128 rows x 192 columns;
- *                   49, 65, 97, 129 = 48, 64, 96, 128 rows x 128 columns
+ *                   49, 65, 97, 129 = 48, 64, 96, 128 rows x 128 columns; 66, 98 = 64, 96 rows x 192 columns
  *   "m1_exact"      twm_gemm_tw_marlin_m1: 1 = f32 activations and f32 FMAs in the reference kernel's order with
  *                   the reference's split-K rule and float atomics (bit-equal to the reference order when that
  *                   rule yields one split); 0 (default) = the MFMA kernel

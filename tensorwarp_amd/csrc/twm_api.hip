@@ -231,7 +231,7 @@ int twm_ctx_set_option(twm_ctx *ctx, const char *key, int value)
     }
     if (strcmp(key, "prefill_bm") == 0) {
         if (value != 0 && (value < 0 || !prefill_form_known((uint32_t)value)))
-            return api_fail(TWM_SHAPE_ERROR, "twm_ctx_set_option: prefill_bm must be 0, 49, 64, 65, 97, 128, 129 or 192");
+            return api_fail(TWM_SHAPE_ERROR, "twm_ctx_set_option: prefill_bm must be 0, 49, 64, 65, 66, 97, 98, 128, 129 or 192");
         ctx->prefill_bm = value;
         return TWM_OK;
     }

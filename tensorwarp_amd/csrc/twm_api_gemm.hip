@@ -435,8 +435,8 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
     case kFormPrefill: {
         uint32_t bm = 0, sp = 0;
         prefill_plan_of(m, 0, 0, n_tiles, k_chunks, e.ws_bytes, gated != 0, &bm, &sp);
-        snprintf(text, bytes, "k_prefill: %u-row x %u-column blocks, %u K-split%s%s; 16-column tile copy", (bm & 1u) ? bm - 1u : bm == 64 ? 64u : 128u,
-                 (bm & 1u) ? 128u : bm == 192 ? 192u : 256u, sp, sp == 1 ? "" : "s", sp > 1 ? " + k_splitk_reduce" : "");
+        snprintf(text, bytes, "k_prefill: %u-row x %u-column blocks, %u K-split%s%s; 16-column tile copy", (bm & 1u) ? bm - 1u : bm == 66 || bm == 98 ? bm - 2u : bm == 64 ? 64u : 128u,
+                 (bm & 1u) ? 128u : bm == 192 || bm == 66 || bm == 98 ? 192u : 256u, sp, sp == 1 ? "" : "s", sp > 1 ? " + k_splitk_reduce" : "");
         break;
     }
     case kFormSubTile:
@@ -633,8 +633,8 @@ static void tune_candidates(uint32_t m, uint32_t k_chunks, bool waves, std::vect
                 for (int sp : {1, 2, 3, 4, 6})
                     if (!(wv == 16 && nt != 1) && !(wv == 8 && nt == 3)) add(4, nt, wv, 0, 0, sp, 0);
     } else {
-        for (int bm : {64, 128, 192, 49, 65, 97, 129})                   // (128-column blocks: up to 256 rows, as the planner)
-            if (!(bm & 1) || m <= 256)
+        for (int bm : {64, 128, 192, 49, 65, 97, 129, 66, 98})           // (the lower blocks: up to as many rows as the planner)
+            if ((!(bm & 1) || m <= 256) && ((bm != 66 && bm != 98) || m <= 1024))
                 for (int sp : {1, 2, 3, 4, 6, 8}) add(0, 0, 0, 0, 0, sp, bm);
     }
 }

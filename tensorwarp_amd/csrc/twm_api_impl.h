@@ -49,7 +49,7 @@ struct twm_ctx {
     int force_kernel;     // 0 = heuristic, 2 = one-lane-per-column kernel on whole tiles (M <= 4), 3 = streaming kernel (M <= 32),
                           // 4 = batched-decode kernel with LDS-shared activations (M <= 32; "nt" = tiles per wave, "waves" 8 / 16 = 2 / 4 k-slices),
                           // 5 = waves on k-chunks of their own ("nt" = 16-column tiles per workgroup, "waves" 4 / 8)
-    int prefill_bm;       // prefill block form: 0 = choose, 64 = 64 rows x 256 columns, 128 = 128 x 256, 192 = 128 rows x 192 columns, 49 / 65 / 97 / 129 = 48 / 64 / 96 / 128 rows x 128 columns
+    int prefill_bm;       // prefill block form: 0 = choose, 64 = 64 rows x 256 columns, 128 = 128 x 256, 192 = 128 rows x 192 columns, 49 / 65 / 97 / 129 = 48 / 64 / 96 / 128 rows x 128 columns, 66 / 98 = 64 / 96 rows x 192
     int prefill_min_m;    // M from which the LDS/MFMA prefill kernel runs instead of 16-row decode blocks
     int dequant_src;      // which copy twm_weight_dequant_f16 unpacks: 0 = 16-column tiles, 1 = column-lane
     int tune_on_upload;   // new plain weight handles are tuned at once: 0 = no, 1 = decode row counts, 2 = prefill row counts too

@@ -36,12 +36,11 @@ namespace twm {
 // three (two before: 4096 -> 2 x 11008 at 96 rows 32.8 -> 29.1 us on 96 x 128, at 64 rows 27.0 -> 25.3 on 64 x 256; a LLaMA-7B
 // layer at 512 rows 254.1 -> 249.7, at 2048 787.9 -> 783.4 on 128 x 256; 3584 -> 2 x 18944 at 96 rows, two workgroups on some
 // CUs, 43.1 -> 45.2).
-template <int MT, int NTW = 4, bool HALF = false, int D = HALF ? 2 : 3>
-__global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc,
-                                                  const _Float16 *__restrict__ a_any, OutSpec out, uint32_t m_rows,
-                                                  uint32_t k, uint32_t n, uint32_t n_tiles, uint32_t k_chunks,
-                                                  uint32_t chunks_per_split, float *__restrict__ partials,
-                                                  uint32_t row_store, uint32_t col_blocks, uint32_t row_blocks)
+template <int MT, int NTW, bool HALF, int D>
+__device__ __forceinline__ void prefill_block(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc, const _Float16 *__restrict__ a_any,
+                                              const OutSpec out, uint32_t m_rows, uint32_t k, uint32_t n, uint32_t n_tiles, uint32_t k_chunks,
+                                              uint32_t chunks_per_split, float *__restrict__ partials, uint32_t row_store, uint32_t col_blocks,
+                                              uint32_t row_blocks)
 {
     constexpr int kPfTileHalves = 16 * MT * kPfRowStride;
     constexpr int NV = MT;       // direct-to-LDS load instructions per wave and A tile (16 MT rows / 16)
@@ -400,6 +399,42 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(co
         }
         return;
     }
+    if (NTW == 3 && out.swiglu) {
+        // three quads of tiles on four waves of three: the gate and up tiles of a feature lie with different waves, so half of the
+        // block's rows at a time go through LDS (rows of 196 floats: the four row groups kb fall on different banks) and every
+        // thread gates and stores four features of a row, 24 lanes a row's 384 bytes
+        constexpr int HB = MT / 2, kLd = 64 * NTW + 4;
+        const uint32_t ffn = n >> 1, col0 = wave * (16u * NTW) + c;
+        const bool aligned = ((uintptr_t)out.swiglu & 15) == 0;
+        float *stage = (float *)a_lds;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            __syncthreads();
+#pragma unroll
+            for (int mt = 0; mt < HB; mt++)
+#pragma unroll
+                for (int t = 0; t < NTW; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) stage[(mt * 16 + kb * 4 + r) * kLd + col0 + t * 16] = acc[h * HB + mt][t][r];
+            __syncthreads();
+            for (uint32_t idx = threadIdx.x; idx < 16u * HB * 24u; idx += 256u) {
+                const uint32_t row = idx / 24u, f4 = idx % 24u, om = m0 + 16u * HB * h + row, feat = bx * 96u + f4 * 4u;
+                if (om >= m_rows || feat >= ffn) continue;
+                const float *src = stage + row * kLd + (f4 >> 3) * 64u + (f4 & 7u) * 4u;
+                const float4v g = *(const float4v *)src, u = *(const float4v *)(src + kPairWidth);
+                float4v v;
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = gated_mul(out.gate_act, g[j], u[j]);
+                float *p = out.swiglu + (size_t)om * ffn + feat;
+                if (aligned) {
+                    __builtin_nontemporal_store(v, (float4v *)p);
+                } else {
+                    p[0] = v[0]; p[1] = v[1]; p[2] = v[2]; p[3] = v[3];
+                }
+            }
+        }
+        return;
+    }
     if (NTW == 2 && out.swiglu) {
         // the same with a gate tile and its up tile per wave: four lanes cover the 64 bytes of a row
         const uint32_t ffn = n >> 1;
@@ -437,6 +472,29 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(co
                 if (om < m_rows) pf_store_out(out, om, on, acc[mt][t][r]);
             }
     }
+}
+
+template <int MT, int NTW = 4, bool HALF = false, int D = HALF ? 2 : 3>
+__global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc,
+                                                  const _Float16 *__restrict__ a_any, OutSpec out, uint32_t m_rows,
+                                                  uint32_t k, uint32_t n, uint32_t n_tiles, uint32_t k_chunks,
+                                                  uint32_t chunks_per_split, float *__restrict__ partials,
+                                                  uint32_t row_store, uint32_t col_blocks, uint32_t row_blocks)
+{
+    prefill_block<MT, NTW, HALF, D>(qw, sc, a_any, out, m_rows, k, n, n_tiles, k_chunks, chunks_per_split, partials, row_store, col_blocks, row_blocks);
+}
+
+// Blocks of 64 or 96 rows x 192 columns, for the shapes whose 128-column blocks put two on some CUs and whose 256-column blocks
+// leave many without (3584 -> 37888 at 64 rows 39.3 -> 28.3 us, at 96 39.6 -> 33.3; 4096 -> 22016 at 128 36.1 -> 31.2, at 192
+// 44.5 -> 38.7).
+template <int MT>
+__global__ __launch_bounds__(256) TWM_PF_OCC(MT == 4) void k_prefill192(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc,
+                                                  const _Float16 *__restrict__ a_any, OutSpec out, uint32_t m_rows,
+                                                  uint32_t k, uint32_t n, uint32_t n_tiles, uint32_t k_chunks,
+                                                  uint32_t chunks_per_split, float *__restrict__ partials,
+                                                  uint32_t row_store, uint32_t col_blocks, uint32_t row_blocks)
+{
+    prefill_block<MT, 3, false, 3>(qw, sc, a_any, out, m_rows, k, n, n_tiles, k_chunks, chunks_per_split, partials, row_store, col_blocks, row_blocks);
 }
 
 // The partial sums of one place, added in split order (deterministic): four loads in flight at a time.
@@ -560,7 +618,6 @@ hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutS
 // up to 256 workgroups, not that ratio).  With more workgroups than CUs its two-per-CU variant runs (the kernel's HALF
 // form, under 256 registers): 4096 -> 11008 at M = 1024 81.6 us against 102.5 on 256-column blocks, 3584 -> 4608 at
 // M = 2048 66.9 against 90.7, 3584 -> 37888 at M = 2048 462 against 476; level at 4096 -> 11008, M = 2048 (158.7 / 158.0).
-// Not with the gated store, whose waves hold gate and up tiles in pairs.
 //
 // Up to 256 rows also blocks of 128 columns (two tiles per wave) with 48, 64, 96 or 128 rows, named by their rows + 1: a few
 // rows on 256-column blocks leave half the CUs idle (3584 -> 2 x 18944 is 148 of them) or multiply rows that are not there.
@@ -572,8 +629,15 @@ hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutS
 // 18944 -> 3584 at 96 29.1 / 24.1, 11008 -> 4096 at 40 17.6 / 14.8, 3584 -> 4608 at 96 16.4 / 13.3, 4096 -> 12288 at 192
 // 33.5 / 27.9; 3584 -> 2 x 18944 at 128 rows is level or worse (50.8 / 55.4).  Under 2048 columns the wider blocks on more
 // K-splits stay ahead (4864 -> 896 at 96 rows 9.3 / 10.1).
-constexpr double kPf192 = 0.80;
-constexpr uint32_t kNarrowMaxRows = 256, kNarrowMinTiles = 128;
+// Up to 1024 rows also blocks of 64 or 96 rows x 192 columns (k_prefill192), named by their rows + 2: kMiddle holds what a chunk
+// takes with one and two of them on a CU, further ones follow (best form before and now, us: 3584 -> 37888 at 64 rows 39.3 /
+// 28.3, gated at 96 44.4 / 36.0; 4096 -> 2 x 11008 at 384 92 / 72, at 192 47.1 / 41.6; 4096 -> 6144 at 512 36.8 / 32.2; 2560 -> 2 x
+// 8192, 86 blocks of 192 columns where 64 of 256 fill the CUs, stays with those).  Gated, the 192-column forms take 1.07 times
+// the plain ones (4096 -> 2 x 11008 at 512 rows 98.3 / 89.4, at 768 154 / 133, at 2048 356 / 346; 3584 -> 2 x 18944 at 2048 537 /
+// 507).
+constexpr double kPf192 = 0.80, kPf192Gated = 1.07;
+constexpr uint32_t kNarrowMaxRows = 256, kNarrowMinTiles = 128, kMiddleMaxRows = 1024;
+static const struct { uint32_t form; double chunk[2]; } kMiddle[] = {{66, {0.94, 1.62}}, {98, {1.17, 2.10}}};
 static const struct { uint32_t form; double chunk[3]; } kNarrow[] = {
     {49, {0.70, 1.05, 1.50}}, {65, {0.77, 1.30, 1.90}}, {97, {0.88, 1.45, 2.35}}, {129, {1.03, 2.10, 3.15}}};
 struct PrefillPlan {
@@ -596,16 +660,17 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
         cuts[n_cuts].splits = sp;
         cuts[n_cuts++].chunks = cps;
     }
-    static const uint32_t kForms[] = {64, 128, 192, 49, 65, 97, 129};
+    static const uint32_t kForms[] = {64, 128, 192, 49, 65, 97, 129, 66, 98};
     for (uint32_t bm : kForms) {
-        const bool narrow = (bm & 1u) != 0;
-        if (force_rows ? bm != force_rows : narrow && (rows > kNarrowMaxRows || n_tiles < kNarrowMinTiles)) continue;
-        if (bm == 192 && gated) continue;
-        const uint32_t col_blocks = bm == 192 ? (n_tiles + 11) / 12 : narrow ? (n_tiles + 7) / 8 : (n_tiles + 15) / 16;
-        const uint32_t height = narrow ? bm - 1u : bm == 64 ? 64u : 128u;
+        const bool narrow = (bm & 1u) != 0, middle = bm == 66 || bm == 98;
+        if (force_rows ? bm != force_rows : (narrow && rows > kNarrowMaxRows) || (middle && rows > kMiddleMaxRows) || ((narrow || middle) && n_tiles < kNarrowMinTiles)) continue;
+        const uint32_t col_blocks = bm == 192 || middle ? (n_tiles + 11) / 12 : narrow ? (n_tiles + 7) / 8 : (n_tiles + 15) / 16;
+        const uint32_t height = narrow ? bm - 1u : middle ? bm - 2u : bm == 64 ? 64u : 128u;
         const double wgs = (double)((rows + height - 1) / height) * col_blocks;
         const double *chunk = nullptr;
         for (const auto &f : kNarrow)
+            if (f.form == bm) chunk = f.chunk;
+        for (const auto &f : kMiddle)
             if (f.form == bm) chunk = f.chunk;
         for (uint32_t i = 0; i < n_cuts; i++) {
             const uint32_t sp = cuts[i].splits, cps = cuts[i].chunks;
@@ -615,6 +680,9 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
             if (narrow) {
                 const uint32_t on_cu = ((uint32_t)total + 255u) / 256u;  // workgroups of the busiest CU
                 t = cps * (on_cu / 3u * chunk[2] + (on_cu % 3u ? chunk[on_cu % 3u - 1u] : 0.0)) + 3.0 + 2.0 * ((on_cu - 1u) / 3u);
+            } else if (middle) {
+                const uint32_t on_cu = ((uint32_t)total + 255u) / 256u;
+                t = cps * (on_cu / 2u * chunk[1] + (on_cu % 2u ? chunk[0] : 0.0)) * (gated && sp == 1 ? kPf192Gated : 1.0) + 3.0 + 2.0 * ((on_cu - 1u) / 2u);
             } else if (bm == 192 && total > 256.0) {
                 // two workgroups share a CU: 2.45 per chunk each; a last round of up to one per CU runs at 1.45
                 const double full = (double)(uint64_t)(total / 512.0), rem = total - 512.0 * full;
@@ -629,9 +697,10 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
                 const double full = (double)(uint64_t)(total / 512.0), rem = total - 512.0 * full;
                 t = full * (cps * 2.0 + 3.0) + (rem == 0.0 ? 0.0 : (rem <= 256.0 ? cps * 1.1 : cps * 2.0) + 3.0);
             }
+            if (bm == 192 && gated && sp == 1) t *= kPf192Gated;
             if (sp > 1) t += 2.5 + sp * partial_us;
             // a larger factor, and the narrower block, have to pay for themselves
-            const double margin = (sp > best.splits && bm == best.block_rows) || bm == 192 || narrow ? 0.97 : 1.0;
+            const double margin = (sp > best.splits && bm == best.block_rows) || bm == 192 || narrow || middle ? 0.97 : 1.0;
             if (t < best.us * margin) {
                 best.block_rows = bm;
                 best.splits = sp;
@@ -692,8 +761,11 @@ static hipError_t launch_prefill_t(hipStream_t s, const WeightView &w, const _Fl
     if (splits == 1 && !via_partials)
         row_store = !out.swiglu && out.count == 1 && out.seg[0].start == 0 && out.seg[0].width == w.n && !out.seg[0].bias &&
                     w.n % 4 == 0 && ((uintptr_t)out.seg[0].ptr & 15) == 0;
-    if (NTW == 3 && out.swiglu) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_prefill<MT, NTW, HALF, D>), grid, dim3(256), lds, s, (const uint4v *)w.qw, (const uint2v *)w.sc, a, out, m, w.k,
+    auto kernel = [] {
+        if constexpr (NTW == 3 && MT < 8) return k_prefill192<MT>;
+        else return k_prefill<MT, NTW, HALF, D>;
+    }();
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, (const uint4v *)w.qw, (const uint2v *)w.sc, a, out, m, w.k,
                        w.n, w.n_tiles, w.k_chunks, cps, splits > 1 || via_partials ? partials : nullptr, row_store, col_blocks, row_blocks);
     if (splits > 1 || via_partials) return launch_splitk_reduce(s, partials, out, m, w.n, w.n_tiles * 16, splits);
     return hipGetLastError();
@@ -701,7 +773,7 @@ static hipError_t launch_prefill_t(hipStream_t s, const WeightView &w, const _Fl
 
 bool prefill_form_known(uint32_t form)
 {
-    return form == 64 || form == 128 || form == 192 || form == 49 || form == 65 || form == 97 || form == 129;
+    return form == 64 || form == 128 || form == 192 || form == 49 || form == 65 || form == 97 || form == 129 || form == 66 || form == 98;
 }
 
 // Once per device, outside any stream capture: the forms with 48 KB or more of dynamic LDS.
@@ -716,11 +788,13 @@ hipError_t init_prefill()
     if (e == hipSuccess) e = ask((const void *)k_prefill<4, 2, false, 4>, 4, 4);
     if (e == hipSuccess) e = ask((const void *)k_prefill<6, 2>, 6, 3);
     if (e == hipSuccess) e = ask((const void *)k_prefill<8, 2>, 8, 3);
+    if (e == hipSuccess) e = ask((const void *)k_prefill192<4>, 4, 3);
+    if (e == hipSuccess) e = ask((const void *)k_prefill192<6>, 6, 3);
     return e;
 }
 
 // block_rows: the block form (64 = 64 rows x 256 columns, 128 = 128 x 256, 192 = 128 rows x 192 columns, 49 / 65 / 97 / 129 =
-// 48 / 64 / 96 / 128 rows x 128 columns), splits: k-split factor; 0 = choose (plan_prefill), within what `scratch` can hold as
+// 48 / 64 / 96 / 128 rows x 128 columns, 66 / 98 = 64 / 96 rows x 192 columns), splits: k-split factor; 0 = choose (plan_prefill), within what `scratch` can hold as
 // f32 partial sums.
 // `scratch` (scratch_bytes) holds the f16 copy of f32 activations and / or the split-K partials; when it
 // cannot hold all M rows the rows are processed in slabs.
@@ -731,9 +805,7 @@ hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, boo
     if (block_rows != 0 && !prefill_form_known(block_rows)) return hipErrorInvalidValue;
     uint32_t ran_splits = 1;  // of the last run
     auto run = [&](const _Float16 *a16, uint32_t rows, const OutSpec &o, void *ws, size_t ws_bytes, bool via = false) {
-        // (a forced 192-column form with the gated store: the 256-column one)
-        const uint32_t form = block_rows == 192 && o.swiglu ? 128u : block_rows;
-        const PrefillPlan plan = plan_prefill_within(rows, form, splits, w.n_tiles, w.k_chunks, ws ? ws_bytes : 0, o.swiglu != nullptr);
+        const PrefillPlan plan = plan_prefill_within(rows, block_rows, splits, w.n_tiles, w.k_chunks, ws ? ws_bytes : 0, o.swiglu != nullptr);
         const uint32_t cps = (w.k_chunks + plan.splits - 1) / plan.splits;
         ran_splits = (w.k_chunks + cps - 1) / cps;
         switch (plan.block_rows) {
@@ -741,6 +813,8 @@ hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, boo
         case 65: return launch_prefill_t<4, 2, false, 4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
         case 97: return launch_prefill_t<6, 2>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
         case 129: return launch_prefill_t<8, 2>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
+        case 66: return launch_prefill_t<4, 3>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
+        case 98: return launch_prefill_t<6, 3>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
         }
         if (plan.block_rows == 64) return launch_prefill_t<4>(s, w, a16, rows, o, plan.splits, (float *)ws, via);
         if (plan.block_rows == 192) {

@@ -608,3 +608,46 @@ def test_graphs_about_the_longest_that_replays_launch_by_launch(dev, copies, gem
         assert all(np.array_equal(eager.to_host(), o.to_host()) for o in outs)
     graph.destroy()
     w.free()
+
+
+# 64- and 96-row blocks of 192 columns, and the 128-row ones with the gated store: a block's last row and the next one's first,
+# K of one group and with a ragged end, columns a quad below and above a block's three
+@pytest.mark.parametrize("form", [66, 98])
+@pytest.mark.parametrize("m", [33, 64, 65, 96, 97, 193])
+def test_prefill_blocks_of_192_columns(dev, m, form):
+    for k, n, splits in ((32, 9, 1), (672, 193, 1), (1312, 388, 3)):
+        packed, scales, w = weight(dev, k, n, 2300 + k + m)
+        a16 = O.synth_act_f16(m, k, 2303 + m)
+        a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+        big = a.copy()
+        big[m - 1] *= np.float32(2.0 ** 18)
+        for rows, dt, vals in ((a16, "f16", a), (big, "f32", big)):
+            c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+            try:
+                dev.set_option("prefill_bm", form)
+                T.gemm(dev, w, T.GpuTensor.from_host(dev, rows, dt), m, c, splits=splits)
+            finally:
+                dev.set_option("prefill_bm", 0)
+            close_rows(c.to_host(), gemm_truth(vals, packed, scales, m, k, n), 1e-3)
+        w.free()
+
+
+@pytest.mark.parametrize("form", [66, 98, 192])
+@pytest.mark.parametrize("m,ffn", [(33, 32), (65, 96), (97, 128), (129, 288), (260, 6304)])
+def test_prefill_gate_on_192_columns(dev, m, ffn, form):
+    # (260 rows x 6304 features: more workgroups of 128 x 192 than CUs, the form of which two share one)
+    k = 416
+    gate, up = [(O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (2311, 2313)]
+    pair = [tuple(T.GpuTensor.from_host(dev, x, t) for x, t in zip(w, ("u8", "f16"))) for w in (gate, up)]
+    w = T.MarlinWeight.gate_up(dev, *pair, k, ffn)
+    a16 = O.synth_act_f16(m, k, 2315)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k)
+    g, u = (gemm_truth(a, *x, m, k, ffn) for x in (gate, up))
+    out = T.GpuTensor.from_host(dev, np.full((m, ffn), np.nan, np.float32))
+    try:
+        dev.set_option("prefill_bm", form)
+        T.gemm_swiglu(dev, w, T.GpuTensor.from_host(dev, a16, "f16"), m, out, 1)
+    finally:
+        dev.set_option("prefill_bm", 0)
+    close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, 2e-3)   # (a product of two sums at 1e-3 each)
+    w.free()
