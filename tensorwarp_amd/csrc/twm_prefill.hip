@@ -321,16 +321,24 @@ __device__ __forceinline__ void prefill_block(const uint4v *__restrict__ qw, con
 
     // ---- store: lane (c, kb) holds rows 4*kb + r of row block mt, column 16*tile + c ----
     if (row_store) {
-        // One destination (the output itself or this split's partial sums), rows 16-byte aligned: each wave turns
-        // its 16 x 64 block of a row block through LDS (272-byte rows: the four row groups kb fall on different
-        // banks) so that a lane stores 16 bytes and sixteen lanes cover 256 consecutive bytes of a row, instead
-        // of 64-byte pieces of four rows from 4-byte stores.
+        // Every four columns have one destination (this split's partial sums, or a segment of the output with all its rows
+        // 16-byte aligned): each wave turns its 16 x 64 block of a row block through LDS (272-byte rows: the four row
+        // groups kb fall on different banks) so that a lane stores 16 bytes and sixteen lanes cover 256 consecutive bytes
+        // of a row, instead of 64-byte pieces of four rows from 4-byte stores.
+        const uint32_t col = nt0 * 16u + (lane & 15u) * 4u;
+        constexpr bool SEGS = NTW == 3;                        // (see launch_prefill_t)
         float *dst = partials ? partials + ((size_t)blockIdx.z * m_rows) * (n_tiles * 16u) : out.seg[0].ptr;
-        const uint32_t ld = partials ? n_tiles * 16u : n;
-        const uint32_t n_lim = partials ? n_tiles * 16u : n;  // a multiple of 4
+        uint32_t ld = partials ? n_tiles * 16u : n, at = col;
+        bool mine = (lane & 15u) * 4u < 16u * NTW && col < ld;   // (ld is a multiple of 4)
+        float4v bias = {0.f, 0.f, 0.f, 0.f};
+        const bool has_bias = SEGS && row_store == kRowsSegments && out.seg[0].bias != nullptr;   // (all segments have one or none does)
+        if (SEGS && row_store == kRowsSegments) {
+            at = 0;
+            dst = mine ? pf_quad_of(out, col, ld, bias) : nullptr;
+            mine = dst != nullptr;
+        }
         __syncthreads();                                       // every wave is done with the A tiles
         float *stage = (float *)a_lds + wave * (16 * 68);
-        const uint32_t col = nt0 * 16u + (lane & 15u) * 4u;
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
 #pragma unroll
@@ -340,10 +348,10 @@ __device__ __forceinline__ void prefill_block(const uint4v *__restrict__ qw, con
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const uint32_t row = (lane >> 4) + 4u * i;
-                const float4v v = *(const float4v *)(stage + row * 68 + (lane & 15u) * 4u);
+                float4v v = *(const float4v *)(stage + row * 68 + (lane & 15u) * 4u);
                 const uint32_t om = m0 + mt * 16u + row;
-                if (om < m_rows && col < n_lim && (lane & 15u) * 4u < 16u * NTW)
-                    __builtin_nontemporal_store(v, (float4v *)(dst + (size_t)om * ld + col));
+                if (has_bias) v += bias;
+                if (om < m_rows && mine) __builtin_nontemporal_store(v, (float4v *)(dst + (size_t)om * ld + at));
             }
         }
         return;
@@ -522,17 +530,27 @@ __device__ __forceinline__ float4v splitk_sum(const float4v *src, size_t stride4
 // out[row][col] = sum over splits of partials[split][row][col], one thread per four padded columns.  Bound: latency.  (A
 // loop of one load and one add per turn waited for memory once per split: nine splits of 96 x 3584 took 6.6 us in a kernel
 // trace, now 4.8, of which most is the launch; four splits of 32 x 3584 5.0 and 4.8.)
+template <RowStore ROWS>
 __global__ __launch_bounds__(256) void k_splitk_reduce(const float *__restrict__ partials, OutSpec out, uint32_t m_rows, uint32_t n,
-                                                         uint32_t n_ld, uint32_t splits, uint32_t row_store)
+                                                         uint32_t n_ld, uint32_t splits)
 {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t quads = n_ld / 4;
     if (idx >= (size_t)m_rows * quads) return;
     const uint32_t row = (uint32_t)(idx / quads), col = (uint32_t)(idx % quads) * 4u;
+    uint32_t ld = 0;
+    float4v bias = {0.f, 0.f, 0.f, 0.f};
+    float *dst = nullptr;
+    if (ROWS == kRowsSegments && col < n) dst = pf_quad_of(out, col, ld, bias);   // (the bias is on its way during the sum)
     float4v s = splitk_sum((const float4v *)(partials + (size_t)row * n_ld + col), (size_t)m_rows * n_ld / 4, splits);
     if (out.row_scale) s *= out.row_scale[row];  // (f32 rows scaled into the f16 range)
-    if (row_store) {
+    if constexpr (ROWS == kRowsPlain) {
         if (col < n) *(float4v *)(out.seg[0].ptr + (size_t)row * n + col) = s;
+        return;
+    }
+    if constexpr (ROWS == kRowsSegments) {
+        if (out.seg[0].bias) s += bias;
+        if (dst) *(float4v *)(dst + (size_t)row * ld) = s;
         return;
     }
 #pragma unroll
@@ -582,6 +600,19 @@ __global__ __launch_bounds__(256) void k_scale_rows(OutSpec out, const float *__
     }
 }
 
+// How rows are stored: kRowsPlain where the output is one [M, N] matrix without a bias, kRowsSegments where every four columns
+// are 16 aligned bytes of one segment and all segments have a bias or none (4096 -> 12288 split into three at 512 rows 57.5 ->
+// 50.9 us, at 2048 190.5 -> 179.5 against 4-byte stores; with K-splits 3584 -> 3584 + 2 * 512 with biases at 512 rows 34.4 ->
+// 31.4 us).
+static uint32_t row_store_of(const OutSpec &out, uint32_t n)
+{
+    for (uint32_t i = 0; i < out.count; i++)
+        if (out.seg[i].start % 4 != 0 || out.seg[i].width % 4 != 0 || ((uintptr_t)out.seg[i].ptr & 15) != 0 || !out.seg[i].bias != !out.seg[0].bias)
+            return kRowsNone;
+    if (out.count == 0) return kRowsNone;
+    return out.count == 1 && out.seg[0].start == 0 && out.seg[0].width == n && !out.seg[0].bias ? kRowsPlain : kRowsSegments;
+}
+
 hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutSpec &out, uint32_t m, uint32_t n,
                                 uint32_t n_ld, uint32_t splits)
 {
@@ -597,11 +628,12 @@ hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutS
                            n / 2, n_ld, splits, out.gate_act, out.row_scale);
         return hipGetLastError();
     }
-    const uint32_t row_store = out.count == 1 && out.seg[0].start == 0 && out.seg[0].width == n && !out.seg[0].bias && n % 4 == 0 &&
-                               ((uintptr_t)out.seg[0].ptr & 15) == 0;
+    const uint32_t rows = row_store_of(out, n);
+    auto kernel = rows == kRowsPlain      ? k_splitk_reduce<kRowsPlain>
+                  : rows == kRowsSegments ? k_splitk_reduce<kRowsSegments>
+                                          : k_splitk_reduce<kRowsNone>;
     const unsigned block = block_of(quads);
-    hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)((quads + block - 1) / block)), dim3(block), 0, s, partials, out, m, n, n_ld,
-                       splits, row_store);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((quads + block - 1) / block)), dim3(block), 0, s, partials, out, m, n, n_ld, splits);
     return hipGetLastError();
 }
 
@@ -752,15 +784,18 @@ static hipError_t launch_prefill_t(hipStream_t s, const WeightView &w, const _Fl
     splits = (w.k_chunks + cps - 1) / cps;  // no empty split
     const uint32_t col_blocks = (w.n_tiles + 4 * NTW - 1) / (4 * NTW), row_blocks = (m + 16 * MT - 1) / (16 * MT);
     dim3 grid(col_blocks * row_blocks, 1, splits);  // the kernel turns the linear id into an XCD-aware tile
-    // 16-byte row stores: into the partial sums always (padded width, a multiple of 64); into the output when it
-    // is one plain [M, N] matrix with N a multiple of 4 at a 16-byte aligned address
+    // 16-byte row stores: into the partial sums always (padded width, a multiple of 64); into the output when every four
+    // columns are whole 16-byte places of one segment.  Segments only from 192-column blocks: the others are no faster with
+    // the segment's search in them, not even where it is skipped (128 x 256 blocks, 3584 -> 4608 plain at 200 rows 22.4 us
+    // without it, 24.2 with it).
     // (via_partials: the sums of a single split go through the partial-sum buffer too and k_splitk_reduce stores them:
     // it is the store that applies the rows' power-of-two factors of f32 activations ahead of a bias or a gate)
     via_partials = via_partials && partials != nullptr;
-    uint32_t row_store = 1;
-    if (splits == 1 && !via_partials)
-        row_store = !out.swiglu && out.count == 1 && out.seg[0].start == 0 && out.seg[0].width == w.n && !out.seg[0].bias &&
-                    w.n % 4 == 0 && ((uintptr_t)out.seg[0].ptr & 15) == 0;
+    uint32_t row_store = kRowsPlain;
+    if (splits == 1 && !via_partials) {
+        row_store = out.swiglu ? kRowsNone : row_store_of(out, w.n);
+        if (NTW != 3 && row_store == kRowsSegments) row_store = kRowsNone;
+    }
     auto kernel = [] {
         if constexpr (NTW == 3 && MT < 8) return k_prefill192<MT>;
         else return k_prefill<MT, NTW, HALF, D>;

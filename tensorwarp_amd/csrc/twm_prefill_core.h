@@ -64,4 +64,27 @@ __device__ __forceinline__ void pf_store_out(const OutSpec &out, uint32_t m, uin
     }
 }
 
+enum RowStore : uint32_t { kRowsNone, kRowsPlain, kRowsSegments };   // (see row_store_of)
+
+// Where columns col .. col + 3 of row 0 go (row r: r * ld further), and their bias; a segment's columns are multiples of four
+__device__ __forceinline__ float *pf_quad_of(const OutSpec &out, uint32_t col, uint32_t &ld, float4v &bias)
+{
+    float *dst = nullptr;
+#pragma unroll
+    for (uint32_t s = 0; s < kMaxSegs; s++) {
+        if (s < out.count) {
+            const uint32_t rel = col - out.seg[s].start;
+            if (rel < out.seg[s].width) {
+                dst = out.seg[s].ptr + rel;
+                ld = out.seg[s].width;
+                if (out.seg[s].bias) {
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; j++) bias[j] = out.seg[s].bias[rel + j];
+                }
+            }
+        }
+    }
+    return dst;
+}
+
 }  // namespace twm

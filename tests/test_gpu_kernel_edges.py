@@ -1,5 +1,7 @@
 """GPU tests of single kernels at the sizes where their tilings change: against the CPU oracle's f64 dequant-then-matmul or
 its byte-exact format functions, through the C ABI."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -630,6 +632,33 @@ def test_prefill_blocks_of_192_columns(dev, m, form):
                 dev.set_option("prefill_bm", 0)
             close_rows(c.to_host(), gemm_truth(vals, packed, scales, m, k, n), 1e-3)
         w.free()
+
+
+# Row stores of split outputs: segments that start on every fourth column and one that does not, across blocks' columns, with
+# and without biases and K-splits, at an output address that is not 16-byte aligned
+@pytest.mark.parametrize("widths", [(8, 200, 4), (184, 8, 200), (192, 192, 192), (201, 7, 60)])
+@pytest.mark.parametrize("form,splits", [(98, 1), (192, 1), (66, 3), (128, 1), (65, 2)])
+def test_prefill_rows_into_segments(dev, widths, form, splits):
+    m, k, n = 99, 672, sum(widths)
+    packed, scales, w = weight(dev, k, n, 2330)
+    a16 = O.synth_act_f16(m, k, 2333)
+    truth = gemm_truth(a16.view(np.float16).astype(np.float32).reshape(m, k), packed, scales, m, k, n)
+    a = T.GpuTensor.from_host(dev, a16, "f16")
+    biases = [np.linspace(-1, 1, x, dtype=np.float32) for x in widths]
+    for shift in (0, 1):
+        full = [T.GpuTensor.from_host(dev, b) for b in biases]
+        for bias in (None, full, [full[0], None, full[2]]):
+            outs = [T.GpuTensor.from_host(dev, np.full(m * x + shift, np.nan, np.float32)) for x in widths]
+            places = [SimpleNamespace(ptr=o.ptr + 4 * shift) for o in outs]
+            try:
+                dev.set_option("prefill_bm", form)
+                T.gemm_split(dev, w, a, m, places, list(widths), biases=bias, splits=splits)
+            finally:
+                dev.set_option("prefill_bm", 0)
+            got = np.concatenate([o.to_host()[shift:].reshape(m, -1) for o in outs], 1)
+            added = [b if t is not None else 0 * b for b, t in zip(biases, bias or [None] * 3)]
+            close_rows(got, truth + np.concatenate(added), 1e-3)
+    w.free()
 
 
 @pytest.mark.parametrize("form", [66, 98, 192])
