@@ -110,14 +110,14 @@ int twm_ctx_info(twm_ctx *ctx, char *buf, size_t buf_len);
  * crates/kernels/src/autotune.rs:254-396); 0 = library's choice unless noted:
  *   "nt"            column tiles per workgroup of the decode kernels (1, 2, 4)
  *   "waves"         waves per workgroup of the decode kernels (1, 2, 4, 8, 16; streaming kernel 4 or 8)
- *   "sub"           M <= 4 and expert-bank kernels: 1 = whole 64-column tiles per workgroup, 16 or 32 = sub-tiles
+ *   "sub"           M <= 4, and the expert kernels on the reference's slabs: 1 = whole 64-column tiles per workgroup, 16 or 32 = sub-tiles
  *                   of that many columns (with "waves" waves, default 8), 0 = the planner's choice per shape
  *   "kernel"        decode kernel: 2 = one-lane-per-column kernel on whole 64-column tiles
  *                   (M <= 4 only), 3 = batched-decode streaming kernel (32-row blocks), 4 = batched-decode kernel
  *                   with the activations shared through LDS (32-row blocks; "nt" 1 / 2 = tiles per wave, 4 / 3 =
  *                   two / three column quads per workgroup, "waves" 8 / 16 = two / four k-slices per workgroup),
- *                   5 = the kernel for narrow matrices whose waves take k-chunks of their own ("nt" 1, 2, 4 = 16-column
- *                   tiles per workgroup; above 32 rows f16-rounded weights, as the prefill GEMM)
+ *                   5 = the kernels whose waves take k-chunks of their own ("nt" 1, 2, 4 = 16-column tiles per
+ *                   workgroup; above 32 rows f16-rounded weights, as the prefill GEMM)
  *   "dequant_src"   which repacked copy twm_weight_dequant_f16 unpacks: 0 = 16-column tiles, 1 = column lanes
  *   "tune_on_upload" new weight handles (twm_weight_upload, twm_weight_from_device, twm_weight_fuse_n; not the paired
  *                   gate/up handles) get measured plans at once, as if twm_weight_tune had been called on them: 1 = for
@@ -494,7 +494,7 @@ int twm_plan_describe_m1(const twm_ctx *ctx, uint32_t k, uint32_t n, char *text,
 int twm_graph_begin(twm_ctx *ctx);
 /* Ends capture and instantiates; NULL on failure. */
 twm_graph *twm_graph_end(twm_ctx *ctx);
-/* GraphCapture::replay */
+/* GraphCapture::replay.  A chain of at most twenty nodes is issued as its launches, a longer or branching one as a graph. */
 int twm_graph_launch(twm_ctx *ctx, twm_graph *g);
 void twm_graph_destroy(twm_graph *g);
 

@@ -325,6 +325,7 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
     const bool batch_auto = e.kernel == 0 && !e.nt && !e.waves &&
                             (m > 16 || (!splits && ((m > 8 && (tiles64 > 128 || a_f32)) || (a_f32 && m > 4 && k_chunks <= 64))));
     if (e.kernel == 4 || batch_auto) {
+        // (what plan_waves_exact left; the figures compare these two kernels)
         // batched decode with the activations shared through LDS, in 32-row blocks: from 17 rows on (the same exact
         // arithmetic as below 17 rows; option "batch_rounded" runs the f16-rounded weights of the prefill kernel
         // there), and from 9 rows on wide

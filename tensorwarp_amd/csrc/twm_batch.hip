@@ -1,5 +1,6 @@
-// Batched-decode kernel with the activations shared through LDS (M = 17 .. 32; M = 9 .. 16 on wide matrices and with
-// f32 rows; M = 5 .. 8 with f32 rows on shallow K).
+// Batched-decode kernel with the activations shared through LDS, where k_waves_exact (twm_waves_exact.hip) is not planned:
+// M = 17 .. 32 on vocabularies, of f32 rows on wide or very deep matrices, and with "batch_rounded"; M = 9 .. 16 on
+// vocabularies and with an explicit number of splits.
 //
 // Semantics, up to 16 rows: as the streaming kernel (reference order, crates/kernels/src/quantize.rs:1219-1238; M > 1
 // has the meaning of gemm_q4_0, quantize.rs:1825-1858): per 32-deep group the products a * (q - 8) are summed in f32

@@ -1,4 +1,5 @@
-// Batched-decode kernel (M = 5 .. 32): streams the 16-column tile copy once for up to 32 rows.
+// Batched-decode kernel (M = 5 .. 32, where neither the lane-per-column kernels nor k_waves_exact nor k_batch is planned:
+// few f16 rows on narrow matrices of deep K, explicit splits): streams the 16-column tile copy once for up to 32 rows.
 //
 // Semantics: as the M = 1 kernels (reference order, crates/kernels/src/quantize.rs:1219-1238): per 32-deep
 // group the products a * (q - 8) are summed in f32 (here by one v_mfma_f32_16x16x32_f16 with a zero
