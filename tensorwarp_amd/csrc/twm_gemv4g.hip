@@ -52,7 +52,7 @@ __global__ __launch_bounds__(1024) void k_gemv4g(const char *__restrict__ cw, co
     uint16_t sc[NP];
 #pragma unroll
     for (int i = 0; i < NP; i++) {
-        const uint32_t kc0 = wave + i * waves, kc = kc0 < k_chunks ? kc0 : k_chunks - 1u;   // (past the end: replayed, scale 0)
+        const uint32_t kc0 = wave + i * waves, kc = kc0 < k_chunks ? kc0 : k_chunks - 1u;   // (past the end: replayed and left out)
         uint32_t k0 = kc * 128u + gl * 32u + (cl >> 2) * 8u;
         if (k0 > k - 8u) k0 = k - 8u;   // only the zero-padded groups of a last partial chunk get here
         if (AF32) {
@@ -103,7 +103,9 @@ __global__ __launch_bounds__(1024) void k_gemv4g(const char *__restrict__ cw, co
     for (int r = 0; r < RL; r++) acc[r] = 0.f;
 #pragma unroll
     for (int i = 0; i < NP; i++) {
-        const bool live = wave + i * waves < k_chunks;
+        // A chunk past the end and a padded group replay other values of the row: their sums are left out, not scaled by zero
+        // (an infinity among those values would come out as NaN in every column).
+        const bool live = ((wave + i * waves) * 4u + gl) * 32u < k;
         float inv[4] = {1.f, 1.f, 1.f, 1.f};
         union { uint4v u; half4v h[2]; } av;
         av.u = a[i];
@@ -124,11 +126,11 @@ __global__ __launch_bounds__(1024) void k_gemv4g(const char *__restrict__ cw, co
 #undef TWM_4G_PIECE
         union { uint16_t u; _Float16 h; } sv;
         sv.u = sc[i];
-        const float s = live ? (float)sv.h : 0.f;
-        if (AF32) acc[0] = fmaf(d[0] + d[1], s * inv[0], acc[0]);
+        const float s = (float)sv.h;
+        if (AF32) acc[0] = live ? fmaf(d[0] + d[1], s * inv[0], acc[0]) : acc[0];
         else {
 #pragma unroll
-            for (int r = 0; r < RL; r++) acc[r] = fmaf(d[r], s, acc[r]);
+            for (int r = 0; r < RL; r++) acc[r] = live ? fmaf(d[r], s, acc[r]) : acc[r];
         }
     }
     if constexpr (TRACE) {

@@ -538,6 +538,27 @@ def test_an_infinite_activation_reaches_every_column_as_itself(dev, k, m):
     w.free()
 
 
+# One to four rows on a lane per column and group: whole chunks that leave slots of a wave without one (28 chunks on eight waves
+# of four), chunks that each wave has one of, a padded last chunk, and both
+@pytest.mark.parametrize("k,m", [(3584, 1), (3584, 2), (3584, 4), (256, 1), (1920, 1), (1440, 1), (1440, 3), (2592, 2), (3616, 4), (96, 1)])
+def test_an_infinite_activation_of_a_few_rows_reaches_every_column_as_itself(dev, k, m):
+    n = 96
+    packed, scales, w = weight(dev, k, n, 2011)
+    dense = O.dequant_f32(packed, scales, k, n).reshape(k, n)
+    a16 = O.synth_act_f16(m, k, 2013)
+    for p in (0, k // 128 * 128 if k % 128 else k - 128, k - 1):
+        rows = a16.view(np.float16).reshape(m, k).copy()
+        rows[m - 1, p] = np.inf
+        c = T.GpuTensor.from_host(dev, np.full((m, n), -1.0, np.float32))
+        T.gemm(dev, w, T.GpuTensor.from_host(dev, rows.view(np.uint16), "f16"), m, c)
+        got = c.to_host()
+        want = np.where(dense[p] == 0, np.nan, np.copysign(np.inf, dense[p])).astype(np.float32)
+        assert np.array_equal(got[m - 1], want, equal_nan=True), p
+        if m > 1:
+            close_rows(got[:m - 1], O.gemm_f64(rows[:m - 1].astype(np.float32), packed, scales, m - 1, k, n), F32_SUM)
+    w.free()
+
+
 # one chunk in part, the most chunks with one each per wave and one more, K one group past whole chunks, four chunks per wave of
 # sixteen waves; a column and a sub-tile more than whole tiles
 @pytest.mark.parametrize("k,n", [(32, 1), (96, 17), (1408, 81), (1440, 64), (2592, 130), (3616, 33), (8192, 65)])
