@@ -53,6 +53,13 @@ __device__ __forceinline__ float bank_dot(const char *__restrict__ bank, size_t 
     const uint32_t lane = threadIdx.x & 63u, cl = lane % SUB, cg = lane / SUB;
     const uint32_t passes = (k_chunks + CPP - 1) / CPP;
     float acc[1] = {0.f};
+    // (the sums of a replayed chunk are left out: they have been scaled by zero, and an infinity in the row would have made
+    // that NaN)
+    auto add = [&](const ChunkS<SUB> &r, const Gemv4Consts &dq) {
+        const float before = acc[0];
+        gemv4s_compute<SUB, 1, TERMS>(r, dq, acc);
+        acc[0] = r.live ? acc[0] : before;
+    };
     bool ok;
     if (ONE) {
         ChunkS<SUB> r;
@@ -66,7 +73,7 @@ __device__ __forceinline__ float bank_dot(const char *__restrict__ bank, size_t 
         gemv4s_load_w<SUB, 1, true>(r, bank + (size_t)(ok ? eid : 0u) * expert_bytes + ((size_t)tile * k_chunks + kc) * kColBlockBytes, col, live);
         __builtin_amdgcn_sched_barrier(0);
         between();
-        gemv4s_compute<SUB, 1, TERMS>(r, make_gemv4_consts(), acc);
+        add(r, make_gemv4_consts());
     } else {
         const uint32_t eid = __builtin_amdgcn_readfirstlane(expert_of(*id, experts));
         ok = eid < experts;
@@ -81,7 +88,7 @@ __device__ __forceinline__ float bank_dot(const char *__restrict__ bank, size_t 
                 gemv4s_load_a<SUB, AF32, TERMS>(r, a_row, 0, kc, cl, k, false);
                 gemv4s_load_w<SUB, 1, true>(r, tbase + (size_t)kc * kColBlockBytes, col, live);
             },
-            [&](const ChunkS<SUB> &r) { gemv4s_compute<SUB, 1, TERMS>(r, dq, acc); }, between);
+            [&](const ChunkS<SUB> &r) { add(r, dq); }, between);
     }
     const float dot = sum_lane_groups<SUB>(acc[0]);
     return ok ? dot : 0.f;

@@ -559,6 +559,37 @@ def test_an_infinite_activation_of_a_few_rows_reaches_every_column_as_itself(dev
     w.free()
 
 
+# 256 and 768 values are two and six chunks: the last pass of a wave has lane groups without one; four waves, of which all but
+# one or two have no pass; a shape whose every lane group has a chunk of its own
+@pytest.mark.parametrize("k,waves", [(256, 0), (768, 0), (768, 4), (512, 0), (512, 4), (2816, 0)])
+def test_an_infinite_activation_of_a_bank_row_reaches_every_column_as_itself(dev, k, waves):
+    n, experts, ids_h = 192, 3, np.array([2, 0], np.float32)
+    raw = [(O.synth_packed(k, n, 2021 + e), O.synth_scales(k, n, 2031 + e)) for e in range(experts)]
+    p, s = (T.GpuTensor.from_host(dev, np.concatenate([x[i].reshape(-1) for x in raw])) for i in (0, 1))
+    bank = T.ExpertBank.from_device(dev, p, s, raw[0][0].size, raw[0][1].size, k, n, experts)
+    dense = [O.dequant_f32(*raw[int(e)], k, n).reshape(k, n) for e in ids_h]
+    ids, wts = T.GpuTensor.from_host(dev, ids_h), T.GpuTensor.from_host(dev, np.array([0.5, 0.25], np.float32))
+    a16 = O.synth_act_f16(2, k, 2041)
+    for at in (0, k - 128, k - 1):
+        rows = a16.view(np.float16).reshape(2, k).copy()
+        rows[:, at] = np.inf
+        each = np.stack([np.where(d[at] == 0, np.nan, np.copysign(np.inf, d[at])) for d in dense]).astype(np.float32)
+        a = T.GpuTensor.from_host(dev, rows.view(np.uint16), "f16")
+        out = T.GpuTensor.from_host(dev, np.full((2, n), -1.0, np.float32))
+        acc = T.GpuTensor.zeros(dev, (n,), "f32")
+        dev.set_option("waves", waves)
+        try:
+            T.batched_marlin_gate_up(dev, a, bank, ids, out, 2, per_slot_rows=True)
+            T.batched_marlin_down_axpy(dev, a, bank, ids, wts, acc, 2)
+        finally:
+            dev.set_option("waves", 0)
+        assert np.array_equal(out.to_host(), each, equal_nan=True), at
+        with np.errstate(invalid="ignore"):
+            both = each[0] + each[1]
+        assert np.array_equal(acc.to_host(), both, equal_nan=True), at
+    bank.free()
+
+
 # one chunk in part, the most chunks with one each per wave and one more, K one group past whole chunks, four chunks per wave of
 # sixteen waves; a column and a sub-tile more than whole tiles
 @pytest.mark.parametrize("k,n", [(32, 1), (96, 17), (1408, 81), (1440, 64), (2592, 130), (3616, 33), (8192, 65)])
