@@ -7,6 +7,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <dlfcn.h>
 #include <new>
 #include <string>
 #include <vector>
@@ -771,16 +772,30 @@ int twm_graph_begin(twm_ctx *ctx)
     return TWM_OK;
 }
 
-// The nodes of a graph that is a chain of at most kPlainNodes kernels of this process and copies that twm_memcpy_d2d recorded;
-// empty when it is anything else.  A replay launches these one by one: hipGraphLaunch takes 8 us of the device's time beyond its
-// nodes and 11 - 12 us of the host's, a launch 2.5 us of the host's and nothing beyond the kernel (a chain of six 12 us kernels
-// 78.0 as a graph, 72.3 launched; two mixture-of-experts layers, six nodes, 34.8 -> 26.9; the LM head and its argmax 55.5 -> 51.5).
-// With the line at twenty, launching is behind only if the nodes took less than 2.05 us each, which is less than a kernel that
-// loads and stores takes from node to node of a graph once a matrix is behind it (128 -> 512 at one row: 2.1).
+// Whether a kernel is one of this library's.  Its launches are function, grid, block, arguments and LDS size and nothing else; a
+// kernel that the caller captured on the stream may have been launched with attributes (cooperatively, say), so its graph is not
+// taken apart.
+static bool own_kernel(const void *func)
+{
+    static const char here = 0;
+    Dl_info kernel, self;
+    return dladdr(func, &kernel) && dladdr(&here, &self) && kernel.dli_fbase == self.dli_fbase;
+}
+
+// The nodes of a graph that is a short chain of this library's kernels and of copies that twm_memcpy_d2d recorded; empty when it
+// is anything else.  A replay launches these one by one.  hipGraphLaunch takes 8 us of the device's time beyond its nodes, and of
+// the calling thread's 23 us alone and 18 in a row, where a launch takes 2.1 and 2.5 .. 3.8 (from process to process) -- until
+// the eighth: with eight launches and more the last one is seen done later than with a graph.  us until a replay is seen done,
+// graph / launched, at 5, 7 and 8 nodes: 128 -> 512 at one row 35 / 22, 37 / 26, 35 / 50 .. 62, 3584 -> 3584 35 / 27, 42 / 33,
+// 41 / 40 .. 53.  Replays in a row, in a process whose launches take 3.8 us: 128 -> 512 18.9 / 18.8 at 5 nodes and 21.6 / 25.4
+// at 7 (the calling thread is the limit), 3584 -> 3584 29.2 / 27.4 at 7; in one whose launches take 2.5, 21.5 / 18.0 and 29.2 /
+// 22.3.  So up to five nodes, and up to seven whose launches are long enough for the thread to keep ahead in either process:
+// those that give every SIMD of the 256 CUs a wave, in the mean.  (Two mixture-of-experts layers, six nodes, 34.8 -> 26.9; the
+// LM head and its argmax 55.5 -> 51.5.)
 static std::vector<PlainNode> plain_chain(hipGraph_t graph, const std::vector<PlainCopy> &copies)
 {
     const std::vector<PlainNode> none;
-    size_t count = 0;
+    size_t count = 0, threads = 0;
     hipGraphNode_t nodes[kPlainNodes];
     if (hipGraphGetNodes(graph, nullptr, &count) != hipSuccess || count == 0 || count > kPlainNodes) return none;
     if (hipGraphGetNodes(graph, nodes, &count) != hipSuccess) return none;
@@ -794,16 +809,16 @@ static std::vector<PlainNode> plain_chain(hipGraph_t graph, const std::vector<Pl
         if (hipGraphNodeGetType(nodes[i], &type) != hipSuccess) return none;
         chain[i].copy = PlainCopy{nullptr, nullptr, nullptr, 0};
         if (type == hipGraphNodeTypeKernel) {
-            hipFuncAttributes attr;
-            if (hipGraphKernelNodeGetParams(nodes[i], &chain[i].kernel) != hipSuccess || !chain[i].kernel.kernelParams || chain[i].kernel.extra ||
-                hipFuncGetAttributes(&attr, chain[i].kernel.func) != hipSuccess)   // (a kernel of a loaded module: not by this call)
-                return none;
+            hipKernelNodeParams &p = chain[i].kernel;
+            if (hipGraphKernelNodeGetParams(nodes[i], &p) != hipSuccess || !p.kernelParams || p.extra || !own_kernel(p.func)) return none;
+            threads += (size_t)p.gridDim.x * p.gridDim.y * p.gridDim.z * p.blockDim.x * p.blockDim.y * p.blockDim.z;
         } else {
             for (const PlainCopy &c : copies)
                 if (c.node == nodes[i]) chain[i].copy = c;
             if (!chain[i].copy.node) return none;
         }
     }
+    if (count > kPlainNodesOfAnySize && threads < count * (256 * 4 * 64)) return none;
     return chain;
 }
 

@@ -22,7 +22,7 @@
         }                                                                              \
     } while (0)
 
-constexpr size_t kPlainNodes = 20;   // most nodes of a graph that is replayed launch by launch (plain_chain, twm_api.hip)
+constexpr size_t kPlainNodes = 7, kPlainNodesOfAnySize = 5;   // most nodes of a graph that is replayed launch by launch (plain_chain, twm_api.hip)
 // a device copy recorded into an open capture, and its node
 struct PlainCopy {
     hipGraphNode_t node;
@@ -101,8 +101,8 @@ struct twm_bank {
     bool paired;
 };
 
-// A captured graph.  `plain`: it is a chain of at most kPlainNodes kernels and twm_memcpy_d2d copies, which a replay launches
-// one by one (see twm_graph_end); exec is null then.  Otherwise exec is launched.
+// A captured graph.  `plain`: it is a short chain of this library's kernels and twm_memcpy_d2d copies, which a replay launches
+// one by one (see plain_chain); exec is null then.  Otherwise exec is launched.
 struct PlainNode {
     hipKernelNodeParams kernel;   // (its arguments belong to the graph)
     PlainCopy copy;               // bytes != 0: a copy

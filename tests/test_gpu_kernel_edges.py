@@ -1,5 +1,7 @@
 """GPU tests of single kernels at the sizes where their tilings change: against the CPU oracle's f64 dequant-then-matmul or
 its byte-exact format functions, through the C ABI."""
+import ctypes as C
+import shutil
 from types import SimpleNamespace
 
 import numpy as np
@@ -629,7 +631,7 @@ def test_up_to_four_rows_gated_on_small_matrices(dev, k, ffn, m, dtype):
 
 @pytest.mark.parametrize("copies,gemms", [(1, 0), (1, 1), (3, 17), (4, 16), (5, 16), (2, 30)])
 def test_graphs_about_the_longest_that_replays_launch_by_launch(dev, copies, gemms):
-    # twenty nodes and twenty-one, copies between the launches, replays with new inputs and eager work between them
+    # one node to 46, copies between the launches, replays with new inputs and eager work between them
     k, n = 256, 64
     packed, scales, w = weight(dev, k, n, 2201)
     a = T.GpuTensor.zeros(dev, (1, k), "f16")
@@ -662,6 +664,68 @@ def test_graphs_about_the_longest_that_replays_launch_by_launch(dev, copies, gem
         assert all(np.array_equal(eager.to_host(), o.to_host()) for o in outs)
     graph.destroy()
     w.free()
+
+
+def replays_as_launches(graph):
+    # (the second pointer of the handle is the instantiated graph; null: the nodes are launched)
+    return C.c_void_p.from_address(graph.handle + 8).value is None
+
+
+# small launches up to five nodes, those that give every SIMD a wave up to seven, copies counted as nodes without a wave
+@pytest.mark.parametrize("k,n,gemms,copies,launched", [(128, 512, 5, 0, True), (128, 512, 6, 0, False), (128, 512, 1, 4, True), (128, 512, 1, 5, False),
+                                                       (3584, 3584, 7, 0, True), (3584, 3584, 8, 0, False), (3584, 3584, 5, 1, True),
+                                                       (3584, 3584, 3, 3, False)])
+def test_which_graphs_replay_launch_by_launch(dev, k, n, gemms, copies, launched):
+    w = T.MarlinWeight.upload(dev, O.synth_packed(k, n, 2401), O.synth_scales(k, n, 2402), k, n)
+    a = T.GpuTensor.from_host(dev, O.synth_act_f16(1, k, 2403), "f16")
+    outs = [T.GpuTensor.zeros(dev, (1, n), "f32") for _ in range(gemms + copies)]
+
+    def work():
+        for o in outs[:gemms]:
+            T.gemm(dev, w, a, 1, o)
+        for o in outs[gemms:]:
+            T.quantize._check(T._lib.load().twm_memcpy_d2d(dev.handle, o.ptr, outs[0].ptr, 4 * n))
+
+    graph = T.GraphCapture.record_with_device(dev, work)
+    assert replays_as_launches(graph) == launched
+    eager = T.GpuTensor.zeros(dev, (1, n), "f32")
+    T.gemm(dev, w, a, 1, eager)
+    for _ in range(3):
+        for o in outs:
+            o.copy_from_host(np.full(n, np.nan, np.float32))
+        graph.replay()
+        dev.synchronize()
+        assert all(np.array_equal(o.to_host(), eager.to_host()) for o in outs)
+    graph.destroy()
+    w.free()
+
+
+def test_a_graph_with_a_kernel_of_the_callers_own_stays_one(dev, tmp_path):
+    # a second copy of the library stands for the caller's own code: its fill kernel, launched on the context's stream
+    class Dim3(C.Structure):
+        _fields_ = [(c, C.c_uint32) for c in "xyz"]
+
+    other = C.CDLL(shutil.copy(T._lib.LIB_PATH, tmp_path / "other.so"))
+    hip = C.CDLL("libamdhip64.so.7")
+    hip.hipLaunchKernel.argtypes = [C.c_void_p, Dim3, Dim3, C.POINTER(C.c_void_p), C.c_size_t, C.c_void_p]
+    words = 64
+    buf = T.GpuTensor.from_host(dev, np.full(words, 7, np.int32))
+    ptr, count = C.c_void_p(buf.ptr), C.c_size_t(words)
+    args = (C.c_void_p * 2)(C.addressof(ptr), C.addressof(count))
+
+    def work(lib):
+        kernel = C.addressof(C.c_char.in_dll(lib, "_ZN3twm11k_fill_zeroEPjm"))
+        assert hip.hipLaunchKernel(kernel, Dim3(1, 1, 1), Dim3(64, 1, 1), args, 0, T._lib.load().twm_ctx_stream(dev.handle)) == 0
+
+    for lib, launched in ((T._lib.load(), True), (other, False)):
+        graph = T.GraphCapture.record_with_device(dev, lambda: work(lib))
+        assert replays_as_launches(graph) == launched
+        for _ in range(2):
+            buf.copy_from_host(np.full(words, 7, np.int32))
+            graph.replay()
+            dev.synchronize()
+            assert not buf.to_host().any()
+        graph.destroy()
 
 
 # 64- and 96-row blocks of 192 columns, and the 128-row ones with the gated store: a block's last row and the next one's first,
