@@ -275,6 +275,7 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
         f.nt = wp.nt;
         f.waves = wp.waves;
         f.splits = splits ? splits : wp.splits;
+        if (gated && f.splits <= 1 && f.nt % 2) f.nt++;   // (a gate tile and its up tile lie in one workgroup)
         return f;
     }
     if (m >= (uint32_t)e.prefill_min_m) {
@@ -440,8 +441,13 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
                  (bm & 1u) ? 128u : bm == 192 || bm == 66 || bm == 98 ? 192u : 256u, sp, sp == 1 ? "" : "s", sp > 1 ? " + k_splitk_reduce" : "");
         break;
     }
+    case kFormGroupLane: {
+        const uint32_t each = (k_chunks + f.waves - 1) / f.waves;
+        snprintf(text, bytes, "k_gemv4g: %u-column sub-tiles, %u wave%s of up to %u chunk%s, 1 K-split; column-lane copy", f.sub, f.waves,
+                 f.waves == 1 ? "" : "s", each, each == 1 ? "" : "s");
+        break;
+    }
     case kFormSubTile:
-    case kFormGroupLane:   // (k_gemv4g: the same columns, waves and copy)
         snprintf(text, bytes, "k_gemv4s: %u-column sub-tiles, %u waves, %u K-split%s; column-lane copy", f.sub, f.waves, f.splits,
                  f.splits == 1 ? "" : "s");
         break;
@@ -457,17 +463,8 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
         break;
     }
     case kFormWaves:
-        if (f.nt != 1 && f.nt != 2 && f.nt != 4) {
-            const uint32_t quads = (f.nt + 3) / 4, less = quads * 4 - f.nt;
-            char part[32] = "";
-            if (less) snprintf(part, sizeof part, " less %u tile%s", less, less == 1 ? "" : "s");
-            snprintf(text, bytes, "k_batch: %u quad%s per workgroup%s, 1 tile per wave in turn, %u waves on k-chunks of their own, %u K-split%s%s; "
-                     "16-column tile copy", quads, quads == 1 ? "" : "s", part, f.waves, f.splits, f.splits == 1 ? "" : "s",
-                     f.splits > 1 ? " + k_splitk_reduce" : "");
-            break;
-        }
-        snprintf(text, bytes, "k_waves: %u-row x %u-column blocks, %u waves on k-chunks of their own, %s weights, %u K-split%s%s; "
-                 "16-column tile copy", waves_block_rows(m), 16 * f.nt, f.waves, m <= 32 ? "exact" : "f16-rounded", f.splits,
+        snprintf(text, bytes, "%s: %u-row x %u-column blocks, %u waves on k-chunks of their own, %s weights, %u K-split%s%s; 16-column tile copy",
+                 m <= 32 ? "k_waves_exact" : "k_waves", waves_block_rows(m), 16 * f.nt, f.waves, m <= 32 ? "exact" : "f16-rounded", f.splits,
                  f.splits == 1 ? "" : "s", f.splits > 1 ? " + k_splitk_reduce" : "");
         break;
     case kFormStream: {

@@ -1688,9 +1688,9 @@ def test_plan_description_follows_the_context_options(dev):
     # described form is the one that runs (same result bits as forcing it by hand is not observable from outside;
     # the split factor is: it changes the summation order)
     k, n = 3584, 3584
-    assert dev.plan(k, n, 1).startswith("k_gemv4s: 16-column sub-tiles, 8 waves")
+    assert dev.plan(k, n, 1).startswith("k_gemv4g: 16-column sub-tiles, 8 waves")
     plain16 = dev.plan(k, n, 16)
-    assert plain16.startswith(("k_gemv4s:", "k_waves:"))
+    assert plain16.startswith(("k_gemv4s:", "k_waves_exact:"))
     dev.set_option("sub", 1)
     try:
         assert dev.plan(k, n, 1).startswith("k_gemv4: 1 x 64-column tiles per workgroup")

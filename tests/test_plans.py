@@ -31,7 +31,7 @@ QWEN7B = {"qkv": (3584, 4608), "o": (3584, 3584), "gate_up": (3584, 37888), "dow
 def parse(text):
     """The fields of a plan line."""
     f = {"kernel": text.split(":")[0], "copy": text.rsplit(";", 1)[1].strip(), "text": text}
-    for key, pat in (("sub", r"(\d+)-column sub-tiles"), ("waves", r"(\d+) waves"), ("splits", r"(\d+) K-split"),
+    for key, pat in (("sub", r"(\d+)-column sub-tiles"), ("waves", r"(\d+) waves?"), ("chunks", r"of up to (\d+) chunk"), ("splits", r"(\d+) K-split"),
                      ("quads", r"(\d+) quads? per workgroup"), ("tiles_per_wave", r"(\d+) tiles? per wave"),
                      ("slices", r"(\d+) k-slice"), ("tiles64", r"(\d+) x 64-column tiles"),
                      ("block_rows", r"(\d+)-row x"), ("block_cols", r"x (\d+)-column blocks")):
@@ -43,7 +43,7 @@ def parse(text):
 
 def workgroups(f, k, n, m):
     n_pad = (n + 63) // 64 * 64
-    if f["kernel"] == "k_gemv4s":
+    if f["kernel"] in ("k_gemv4s", "k_gemv4g"):
         return n_pad // f["sub"] * f["splits"]
     if f["kernel"] == "k_gemv4":
         return -(-(n_pad // 64) // f["tiles64"]) * f["splits"]
@@ -51,7 +51,7 @@ def workgroups(f, k, n, m):
         return -(-(n_pad // 64) // (f["quads"] * f["tiles_per_wave"])) * f["splits"]
     if f["kernel"] == "k_stream":
         return n_pad // 64 * f["splits"]
-    if f["kernel"] in ("k_prefill", "k_waves"):
+    if f["kernel"] in ("k_prefill", "k_waves", "k_waves_exact"):
         return -(-m // f["block_rows"]) * -(-n_pad // f["block_cols"]) * f["splits"]
     raise AssertionError(f["text"])
 
@@ -70,19 +70,21 @@ def test_plans_of_the_qwen7b_projections(lib, name, m, dtype):
     f = parse(describe(lib, k, n, m, _lib.F32 if dtype == "f32" else _lib.F16))
     k_chunks, wgs = (k // 32 + 3) // 4, workgroups(f, k, n, m)
     if m <= 4:
-        assert f["kernel"] in ("k_gemv4s", "k_gemv4") and f["copy"] == "column-lane copy", f["text"]
+        assert f["kernel"] in ("k_gemv4s", "k_gemv4g", "k_gemv4") and f["copy"] == "column-lane copy", f["text"]
         assert f["splits"] == 1, f["text"]                   # (a hand-over between workgroups costs over a microsecond)
     elif m <= 16:
-        assert f["kernel"] in ("k_gemv4s", "k_gemv4", "k_stream", "k_batch", "k_waves"), f["text"]
+        assert f["kernel"] in ("k_gemv4s", "k_gemv4", "k_stream", "k_batch", "k_waves_exact"), f["text"]
     else:
-        assert f["kernel"] in ("k_batch", "k_waves") and f["copy"] == "16-column tile copy", f["text"]
+        assert f["kernel"] in ("k_batch", "k_waves_exact") and f["copy"] == "16-column tile copy", f["text"]
     if m == 1:
-        assert f["kernel"] == "k_gemv4s" and wgs >= CUS // 2, f["text"]
-        if k_chunks <= 32:                                    # K up to 4096: a wave makes one pass or two, no loop
+        assert f["kernel"] in ("k_gemv4s", "k_gemv4g") and wgs >= CUS // 2, f["text"]
+        if f["kernel"] == "k_gemv4g":                         # a wave has up to four chunks, all of them in flight
+            assert f["waves"] * f["chunks"] >= k_chunks and f["chunks"] <= 4, f["text"]
+        elif k_chunks <= 32:                                  # K up to 4096: a wave makes one pass or two, no loop
             assert f["waves"] * (64 // f["sub"]) * 2 >= k_chunks, f["text"]
         else:                                                 # deep K: sixteen columns, few waves, the pass loop
             assert f["sub"] == 16 and f["waves"] in (4, 8, 16), f["text"]
-    if f["kernel"] in ("k_stream", "k_batch", "k_waves"):
+    if f["kernel"] in ("k_stream", "k_batch", "k_waves_exact"):
         assert f["copy"] == "16-column tile copy" and 1 <= f["splits"] <= 16, f["text"]
         unsplit = wgs // f["splits"]
         if f["splits"] > 1:
@@ -110,7 +112,7 @@ def test_plans_of_lm_head_and_small_shapes(lib):
     lm = parse(describe(lib, 3584, 152064, 1))
     assert lm["kernel"] in ("k_gemv4", "k_gemv4s") and lm["splits"] == 1 and workgroups(lm, 3584, 152064, 1) >= 8 * CUS, lm["text"]
     small = parse(describe(lib, 896, 1152, 1))
-    assert small["kernel"] == "k_gemv4s" and small["splits"] == 1, small["text"]            # shallow K, one row: sub-tiles
+    assert small["kernel"] == "k_gemv4g" and small["splits"] == 1, small["text"]            # small matrix, one row: a lane per column and group
 
 
 def test_the_gated_store_takes_32_column_sub_tiles(lib):
@@ -133,10 +135,10 @@ def test_pick_splits_agrees_with_the_described_plan(lib):
         # which rows go to which kernel family
         kernel = text.split(":")[0]
         if m <= 4:
-            assert kernel in ("k_gemv4", "k_gemv4s"), (k, n, m, text)
+            assert kernel in ("k_gemv4", "k_gemv4s", "k_gemv4g"), (k, n, m, text)
             assert "column-lane copy" in text
         if m > 16:
-            assert kernel in ("k_batch", "k_waves"), (k, n, m, text)
+            assert kernel in ("k_batch", "k_waves_exact"), (k, n, m, text)
         if kernel == "k_gemv4s":
             sub, waves = map(int, re.search(r"(\d+)-column sub-tiles, (\d+) waves", text).groups())
             assert sub in (16, 32) and 1 <= waves <= 16
@@ -158,9 +160,8 @@ def test_plans_of_the_kernel_on_narrow_matrices(lib):
         if f["kernel"] != "k_waves":
             continue
         wgs, k_chunks = workgroups(f, k, n, m), (k // 32 + 3) // 4
-        assert 5 <= m <= 192 and f["copy"] == "16-column tile copy", f["text"]
-        assert f["block_cols"] in ((32, 64) if gated else (16, 32, 64)) and f["block_rows"] in (16, 32, 48, 64), f["text"]
-        assert (m <= 32) == (f["block_rows"] <= 32) == ("exact weights" in f["text"]) != ("f16-rounded weights" in f["text"]), f["text"]
+        assert 33 <= m <= 192 and f["copy"] == "16-column tile copy" and "f16-rounded weights" in f["text"], f["text"]
+        assert f["block_cols"] in ((32,) if gated else (16, 32)) and f["block_rows"] in (48, 64), f["text"]
         assert -(-m // f["block_rows"]) * f["block_rows"] - m < f["block_rows"], f["text"]
         assert wgs <= (CUS if f["waves"] == 8 else 2 * CUS) and (f["waves"] == 8 or 33 <= m <= 64), f["text"]
         blocks, groups = -(-m // f["block_rows"]), (n + 63) // 64 * 64 // f["block_cols"]
@@ -169,7 +170,37 @@ def test_plans_of_the_kernel_on_narrow_matrices(lib):
         if f["splits"] > 1:
             assert wgs // f["splits"] <= CUS // 2 and k_chunks // f["splits"] >= 8 and "k_splitk_reduce" in f["text"], f["text"]
         taken.add((f["block_rows"], f["block_cols"]))
-    assert len(taken) >= 10, taken
+    assert taken == {(48, 16), (48, 32), (64, 16), (64, 32)}, taken
+
+
+def test_plans_of_the_few_row_kernels(lib):
+    # k_gemv4g: up to four f16 rows or one f32 row, every wave's chunks in flight at once.  k_waves_exact: 5 .. 32 rows, blocks of
+    # 16 or 32 rows x 1 .. 10 column tiles, a gate tile beside its up tile unless K is split, K split only into ranges of some
+    # depth where the columns leave CUs idle
+    rng = np.random.default_rng(13)
+    seen = {"k_gemv4g": 0, "k_waves_exact": 0}
+    for _ in range(6000):
+        k, n = 32 * int(rng.integers(1, 600)), int(rng.choice([400, 3000, 40000]) * rng.random()) + 1
+        m, gated = int(rng.integers(1, 5) if rng.integers(0, 2) else rng.integers(5, 34)), int(rng.integers(0, 2))
+        n = n // 64 * 64 + 64 if gated else n
+        f32 = bool(rng.integers(0, 2))
+        f = parse(describe(lib, k, n, m, _lib.F32 if f32 else _lib.F16, gated))
+        k_chunks, wgs = (k // 32 + 3) // 4, workgroups(f, k, n, m)
+        if f["kernel"] == "k_gemv4g":
+            assert m <= (1 if f32 else 4) and f["copy"] == "column-lane copy" and f["sub"] == 16, f["text"]
+            assert 1 <= f["waves"] <= 16 and f["chunks"] <= 4 and f["waves"] * f["chunks"] >= k_chunks, f["text"]
+        elif f["kernel"] == "k_waves_exact":
+            assert 5 <= m <= 32 and f["copy"] == "16-column tile copy" and "exact weights" in f["text"] and f["waves"] == 8, f["text"]
+            assert f["block_rows"] == (16 if m <= 16 else 32) and f["block_cols"] % 16 == 0, f["text"]
+            nt = f["block_cols"] // 16
+            assert nt in (1, 2, 3, 4, 5, 6, 8, 10) and not (gated and f["splits"] == 1 and nt % 2), f["text"]
+            assert not f32 or nt <= (10 if m <= 8 else 8 if m <= 16 else 4), f["text"]      # (where their registers end)
+            if f["splits"] > 1:
+                assert wgs <= CUS and k_chunks // f["splits"] >= 8 and "k_splitk_reduce" in f["text"], f["text"]
+        else:
+            continue
+        seen[f["kernel"]] += 1
+    assert min(seen.values()) >= 400, seen
 
 
 def test_describe_rejects_what_twm_gemm_rejects(lib):
