@@ -358,7 +358,7 @@ __global__ __launch_bounds__(1024) void k_gemv4s_upfront(const char *__restrict_
 // trace[4 b]: the 100 MHz clock at its start, after wave 0 has unpacked its passes, and at its end, and the hardware
 // id of the CU it ran on.  A kernel of its own: reading the trace pointer first would put a second, dependent kernel
 // argument fetch in front of every wave of the product kernel.
-template <int SUB, bool ONE>
+template <int SUB, bool ONE, bool SPLIT>
 __global__ __launch_bounds__(1024) void k_gemv4s_traced(const char *__restrict__ cw, const void *__restrict__ a_any, OutSpec out,
                                                          float *__restrict__ ws, unsigned *__restrict__ counters,
                                                          uint32_t m_rows, uint32_t k, uint32_t n, uint32_t n_pad,
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(1024) void k_gemv4s_traced(const char *__restrict__
         // HW_ID (register 4): wave, SIMD, CU, SH, SE ids; XCC_ID (register 20): the XCD
         tr[3] = (__builtin_amdgcn_s_getreg((31 << 11) | 4) & 0xFFFFu) | (__builtin_amdgcn_s_getreg((3 << 11) | 20) << 16);
     }
-    gemv4s_body<SUB, 1, false, ONE, false, 0, true>(cw, a_any, out, ws, counters, gemv4s_cfg(splits, out.swiglu != nullptr, blockDim.x >> 6, m_rows),
+    gemv4s_body<SUB, 1, false, ONE, false, 0, SPLIT>(cw, a_any, out, ws, counters, gemv4s_cfg(splits, out.swiglu != nullptr, blockDim.x >> 6, m_rows),
                                            k, n, n_pad, k_chunks, sub_tiles, cps, nullptr, tr + 1);
     if (threadIdx.x == 0) tr[2] = (uint32_t)__builtin_amdgcn_s_memrealtime();
 }
@@ -401,12 +401,10 @@ static hipError_t launch_gemv4s_t(hipStream_t s, const WeightView &w, const void
     } while (0)
     if constexpr (RL == 1) {
         if (!a_f32 && trace.ptr && blocks <= trace.capacity) {
-            if (one)
-                hipLaunchKernelGGL((k_gemv4s_traced<SUB, true>), dim3(blocks), dim3(waves * 64), lds, s, (const char *)w.cq, a, out,
-                                   ws, counters, m, w.k, w.n, n_pad, w.k_chunks, sub_tiles, splits, cps, trace.ptr);
-            else
-                hipLaunchKernelGGL((k_gemv4s_traced<SUB, false>), dim3(blocks), dim3(waves * 64), lds, s, (const char *)w.cq, a, out,
-                                   ws, counters, m, w.k, w.n, n_pad, w.k_chunks, sub_tiles, splits, cps, trace.ptr);
+            auto kernel = splits > 1 ? (one ? k_gemv4s_traced<SUB, true, true> : k_gemv4s_traced<SUB, false, true>)
+                                     : (one ? k_gemv4s_traced<SUB, true, false> : k_gemv4s_traced<SUB, false, false>);
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(waves * 64), lds, s, (const char *)w.cq, a, out, ws, counters, m, w.k, w.n, n_pad,
+                               w.k_chunks, sub_tiles, splits, cps, trace.ptr);
             return hipGetLastError();
         }
     }

@@ -666,6 +666,31 @@ def test_graphs_about_the_longest_that_replays_launch_by_launch(dev, copies, gem
     w.free()
 
 
+# one pass per wave and the loop over passes, with and without a K-split, on both widths
+@pytest.mark.parametrize("k,n,sub,splits", [(3584, 200, 16, 0), (3584, 200, 32, 0), (9344, 128, 16, 0), (9344, 128, 32, 3), (3584, 200, 16, 2)])
+def test_traced_sub_tiles_compute_what_the_untraced_do(dev, k, n, sub, splits):
+    packed, scales, w = weight(dev, k, n, 2501)
+    a16 = O.synth_act_f16(1, k, 2503)
+    a = T.GpuTensor.from_host(dev, a16, "f16")
+    trace = T.GpuTensor.zeros(dev, (4 * 64,), "i32")
+    got = []
+    dev.set_option("sub", sub)
+    try:
+        for on in (False, True):
+            if on:
+                T.quantize._check(T._lib.load().twm_debug_trace(dev.handle, trace.ptr, 64))
+            c = T.GpuTensor.from_host(dev, np.full((1, n), np.nan, np.float32))
+            T.gemm(dev, w, a, 1, c, splits=splits)
+            got.append(c.to_host())
+            assert trace.to_host().any() == on
+    finally:
+        dev.set_option("sub", 0)
+        T.quantize._check(T._lib.load().twm_debug_trace(dev.handle, None, 0))
+    close_rows(got[0], O.gemm_f64(a16.view(np.float16).astype(np.float32).reshape(1, k), packed, scales, 1, k, n), F32_SUM)
+    assert np.array_equal(got[0], got[1])
+    w.free()
+
+
 def replays_as_launches(graph):
     # (the second pointer of the handle is the instantiated graph; null: the nodes are launched)
     return C.c_void_p.from_address(graph.handle + 8).value is None

@@ -84,3 +84,14 @@ def test_counted_waits_match_the_loads_of_a_chunk(kernels):
         assert loads[:depth + 1] == [depth * per_chunk, 0] + [per_chunk] * (depth - 1), (name, loads)
         checked += 1
     assert checked == 7
+
+
+def test_unsplit_sub_tile_launches_hand_nothing_over(kernels):
+    # k_gemv4s, its upfront form and the traced twin that stands for both: without a K-split no arrival counter is touched (there
+    # may be fewer of them than sub-tiles) and no partial sum parked
+    forms = [(name, body) for name, (body, _) in kernels.items() if re.search(r"\d+k_gemv4s(_upfront|_traced)?I", name)]
+    unsplit = [(name, body) for name, body in forms if re.search(r"Lb0EEEvPKc", name)]
+    assert len(unsplit) >= 20 and sum("k_gemv4s_traced" in name for name, _ in unsplit) == 4
+    for name, body in unsplit:
+        assert "global_atomic" not in body, name
+    assert all("global_atomic" in body for name, body in forms if re.search(r"Lb1EEEvPKc", name))
