@@ -40,9 +40,10 @@ __device__ __forceinline__ uint32_t expert_of(float id, uint32_t experts)
 // accumulator and weights behind the barrier: 2816 -> 2 x 704 gated, eight of 128 experts 6.07 -> 5.27, 704 -> 2816 level at 6.1;
 // 4096 -> 2 x 1408, six of 16, 10.6 -> 9.15, 1408 -> 4096 8.36 -> 7.76.)
 
-// What a wave sums over its passes first, first + stride, ... of a sub-tile; ONE: it has one.  between: what it does once its
-// loads are on their way.  An id that is no expert reads expert 0 and counts as zero (a branch would take the activations'
-// loads behind the id).
+// What a wave sums over its passes first, first + stride, ... of a sub-tile; ONE: it has one.  The loop over passes is the
+// pipelined one for f32 rows only: with f16 rows it takes all 128 registers of a sixteen-wave workgroup, where the plain one
+// takes 79 and two of them share a CU.  between: what it does once its loads are on their way.  An id that is no expert reads
+// expert 0 and counts as zero (a branch would take the activations' loads behind the id).
 template <bool AF32, bool ONE, class Between>
 __device__ __forceinline__ float bank_dot(const char *__restrict__ bank, size_t expert_bytes, uint32_t experts, const void *__restrict__ a_row,
                                           const float *__restrict__ id, uint32_t first, uint32_t stride, uint32_t tile, uint32_t col,
@@ -79,7 +80,7 @@ __device__ __forceinline__ float bank_dot(const char *__restrict__ bank, size_t 
         ok = eid < experts;
         const char *tbase = bank + (size_t)(ok ? eid : 0u) * expert_bytes + (size_t)tile * k_chunks * kColBlockBytes;
         const Gemv4Consts dq = make_gemv4_consts();
-        gemv4s_run_passes<SUB, false, 1, true>(
+        gemv4s_run_passes<SUB, false, 1, AF32>(
             first, stride, passes,
             [&](ChunkS<SUB> &r, uint32_t pass) {
                 uint32_t kc = pass * CPP + cg;
@@ -162,23 +163,23 @@ __global__ __launch_bounds__(1024) void k_bank_down_axpy(const float *__restrict
     const uint32_t lane = threadIdx.x & 63u, cl = lane % SUB;
     const uint32_t slot = (wave * (slots_wps >> 16)) >> 8, j = wave - slot * wps;
     const uint32_t on = st * SUB + cl;
-    float total = 0.f, w[kMaxBankSlots];
+    // (the weights one to a lane: sixteen registers of them, live across the pass loop, made the looped f16 form spill)
+    float total = 0.f, weight = 0.f;
     auto fetch = [&]() {
         if (wave != 0) return;
         if (on < n) total = accum[on];
-#pragma unroll
-        for (uint32_t s = 0; s < (uint32_t)kMaxBankSlots; s++) w[s] = weights[s < slots ? s : 0u];
+        weight = weights[lane < slots ? lane : 0u];
     };
     const void *a_row = (const char *)a_all + (size_t)slot * k * (AF32 ? 4 : 2);
     const float dot = bank_dot<AF32, ONE>(bank, expert_bytes, experts, a_row, ids + slot, j, wps, st / CPP, (st % CPP) * SUB + cl, k, (k + 127u) >> 7, fetch);
     if (lane < SUB) red[wave * SUB + cl] = dot;
     __syncthreads();
-    if (wave != 0 || lane >= SUB || on >= n) return;
+    if (wave != 0) return;
 #pragma unroll
     for (uint32_t s = 0; s < (uint32_t)kMaxBankSlots; s++) {
-        if (s < slots) total += w[s] * bank_sum(red + s * wps * SUB + cl, wps);
+        if (s < slots) total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), s)) * bank_sum(red + s * wps * SUB + cl, wps);
     }
-    accum[on] = total;
+    if (lane < SUB && on < n) accum[on] = total;
 }
 
 // ---- the same two launches on the reference's own slabs (no bank, nothing repacked) --------------------------
