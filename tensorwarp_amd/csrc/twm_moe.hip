@@ -14,6 +14,8 @@
 // q - 8, f32 sum per 32-wide group times f32(scale).  An id outside [0, experts) contributes zeros.
 #include "twm_gemv4_core.h"
 
+#include <type_traits>
+
 namespace twm {
 
 template <int ACT>
@@ -95,16 +97,30 @@ __device__ __forceinline__ float bank_dot(const char *__restrict__ bank, size_t 
     return ok ? dot : 0.f;
 }
 
-// The sum of count (<= 16) values at, at + 16, ... in their order: the reads are independent
+// The sum of count (<= R) values at, at + 16, ... in their order: the reads are independent
+template <int R>
 __device__ __forceinline__ float bank_sum(const float *at, uint32_t count)
 {
-    float x[16];
+    float x[R];
 #pragma unroll
-    for (uint32_t w = 0; w < 16; w++) x[w] = at[(w < count ? w : 0u) * 16u];
+    for (uint32_t w = 0; w < R; w++) x[w] = at[(w < count ? w : 0u) * 16u];
     float v = x[0];
 #pragma unroll
-    for (uint32_t w = 1; w < 16; w++) v += w < count ? x[w] : 0.f;
+    for (uint32_t w = 1; w < R; w++) v += w < count ? x[w] : 0.f;
     return v;
+}
+
+// then(R) with as many reads as count (<= 16) needs, rounded up to a power of two.  (Sixteen whatever the count, and that for each
+// of a down projection's slots, stood behind the last barrier: one pass per wave, f16 rows, 3 % of a per-slot launch and 8 % of a
+// down projection, in the mean of 500 random ones of 3 - 20 us.)
+template <class Then>
+__device__ __forceinline__ void bank_reads(uint32_t count, Then then)
+{
+    if (count == 1) then(std::integral_constant<int, 1>{});
+    else if (count == 2) then(std::integral_constant<int, 2>{});
+    else if (count <= 4) then(std::integral_constant<int, 4>{});
+    else if (count <= 8) then(std::integral_constant<int, 8>{});
+    else then(std::integral_constant<int, 16>{});
 }
 
 // Workgroup = `waves` waves on one sub-tile of one slot's expert; wave w takes passes w, w + waves, ...
@@ -134,7 +150,8 @@ __global__ __launch_bounds__(1024) void k_bank_gemv(const float *__restrict__ id
     if (lane < SUB) red[wave * SUB + cl] = dot;
     __syncthreads();
     if (wave != 0) return;
-    const float total = bank_sum(red + cl, waves);
+    float total = 0.f;
+    bank_reads(waves, [&](auto reads) { total = bank_sum<decltype(reads)::value>(red + cl, waves); });
     if (ACT == 0) {
         const uint32_t on = st * SUB + cl;
         if (lane < SUB && on < n) out[(size_t)slot * n + on] = total;
@@ -175,10 +192,13 @@ __global__ __launch_bounds__(1024) void k_bank_down_axpy(const float *__restrict
     if (lane < SUB) red[wave * SUB + cl] = dot;
     __syncthreads();
     if (wave != 0) return;
+    bank_reads(wps, [&](auto reads) {
+        constexpr int R = decltype(reads)::value;
 #pragma unroll
-    for (uint32_t s = 0; s < (uint32_t)kMaxBankSlots; s++) {
-        if (s < slots) total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), s)) * bank_sum(red + s * wps * SUB + cl, wps);
-    }
+        for (int s = 0; s < kMaxBankSlots / (R / 2 + 1); s++)   // (wps > R / 2, and slots * wps <= kMaxBankSlots)
+            if (s < (int)slots)
+                total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), s)) * bank_sum<R>(red + s * wps * SUB + cl, wps);
+    });
     if (lane < SUB && on < n) accum[on] = total;
 }
 
