@@ -204,9 +204,9 @@ void prefill_plan_of(uint32_t rows, uint32_t block_rows, uint32_t splits, uint32
 hipError_t launch_geglu_rows(hipStream_t s, const float *gu, float *out, uint32_t dim, uint32_t batch, bool paired);
 // act: 0 out[slot][n]; 1 gelu_tanh(gate) * up, 2 silu(gate) * up into out[slot][n/2] (paired bank)
 hipError_t launch_bank_gemv(hipStream_t s, const BankView &b, const void *a, bool a_f32, uint32_t a_slot_stride,
-                            const float *ids, uint32_t slots, int act, float *out, int force_waves = 0);
+                            const float *ids, uint32_t slots, int act, float *out, int force_sub = 0, int force_waves = 0);
 hipError_t launch_bank_down_axpy(hipStream_t s, const BankView &b, const void *a_all, bool a_f32, const float *ids,
-                                 const float *weights, uint32_t slots, float *accum, int force_waves = 0);
+                                 const float *weights, uint32_t slots, float *accum, int force_sub = 0, int force_waves = 0);
 
 // the same two launches on the reference's slabs, f32 activations (moe_batched_marlin.rs:153-214, quantize_indirect.rs:228-253)
 hipError_t launch_raw_gemv(hipStream_t s, const RawView &v, const float *a, uint32_t a_slot_stride, const float *ids,

@@ -10,7 +10,7 @@
 //   k_bank_down_axpy acc[n] += sum over slots, in slot order, of weight[slot] * (A[slot] x W[ids[slot]])
 //                    (batched_marlin_down_axpy, :78-134, whose float atomics add in no fixed order).
 //
-// Arithmetic per output as in the dense kernel: f16 activations (f32 ones are rounded on load), exact
+// Arithmetic per output as in the dense kernel: f16 activations (f32 ones as two f16 terms), exact
 // q - 8, f32 sum per 32-wide group times f32(scale).  An id outside [0, experts) contributes zeros.
 #include "twm_gemv4_core.h"
 
@@ -30,9 +30,9 @@ __device__ __forceinline__ uint32_t expert_of(float id, uint32_t experts)
     return (id >= 0.f && id < (float)experts) ? (uint32_t)id : experts;
 }
 
-// Both kernels work on sub-tiles of 16 columns (see twm_gemv4_core.h): a wave covers four consecutive chunks of them in one
-// pass, so that the short K of an expert matrix (a few chunks) still gives every wave of a workgroup one pass and the launch
-// many workgroups.
+// Both kernels work on sub-tiles of SUB = 16 or 32 columns (see twm_gemv4_core.h): a wave covers 64 / SUB consecutive chunks of
+// them in one pass, so that the short K of an expert matrix (a few chunks) still gives every wave of a workgroup one pass and
+// the launch many workgroups.
 // What bounds these launches is a chain of round trips, not the 9 or 18 MB of weights: the slot's expert id, then its weights,
 // then the store.  So nothing else waits: the arguments that the loads need arrive preloaded (thirteen words), the activations
 // are loaded ahead of the id, the accumulator and the slots' weights ahead of the weights, the wave's four chunks are summed by
@@ -46,12 +46,12 @@ __device__ __forceinline__ uint32_t expert_of(float id, uint32_t experts)
 // pipelined one for f32 rows only: with f16 rows it takes all 128 registers of a sixteen-wave workgroup, where the plain one
 // takes 79 and two of them share a CU.  between: what it does once its loads are on their way.  An id that is no expert reads
 // expert 0 and counts as zero (a branch would take the activations' loads behind the id).
-template <bool AF32, bool ONE, class Between>
+template <int SUB, bool AF32, bool ONE, class Between>
 __device__ __forceinline__ float bank_dot(const char *__restrict__ bank, size_t expert_bytes, uint32_t experts, const void *__restrict__ a_row,
                                           const float *__restrict__ id, uint32_t first, uint32_t stride, uint32_t tile, uint32_t col,
                                           uint32_t k, uint32_t k_chunks, Between between)
 {
-    constexpr int SUB = 16, CPP = 4;
+    constexpr int CPP = 64 / SUB;
     constexpr int TERMS = AF32 ? kTermsOneRowF32 : kTermsOneRow;   // one row: a lane loads one piece of its chunk
     const uint32_t lane = threadIdx.x & 63u, cl = lane % SUB, cg = lane / SUB;
     const uint32_t passes = (k_chunks + CPP - 1) / CPP;
@@ -97,13 +97,13 @@ __device__ __forceinline__ float bank_dot(const char *__restrict__ bank, size_t 
     return ok ? dot : 0.f;
 }
 
-// The sum of count (<= R) values at, at + 16, ... in their order: the reads are independent
-template <int R>
+// The sum of count (<= R) values at, at + SUB, ... in their order: the reads are independent
+template <int SUB, int R>
 __device__ __forceinline__ float bank_sum(const float *at, uint32_t count)
 {
     float x[R];
 #pragma unroll
-    for (uint32_t w = 0; w < R; w++) x[w] = at[(w < count ? w : 0u) * 16u];
+    for (uint32_t w = 0; w < R; w++) x[w] = at[(w < count ? w : 0u) * SUB];
     float v = x[0];
 #pragma unroll
     for (uint32_t w = 1; w < R; w++) v += w < count ? x[w] : 0.f;
@@ -125,16 +125,16 @@ __device__ __forceinline__ void bank_reads(uint32_t count, Then then)
 
 // Workgroup = `waves` waves on one sub-tile of one slot's expert; wave w takes passes w, w + waves, ...
 // grid = (sub-tiles, slots).  ACT 0: out[slot][n]; 1 / 2: paired bank (each 64-column tile is 32 gate columns,
-// then the up columns of the same features; the workgroup takes eight of each),
+// then the up columns of the same features; the workgroup takes SUB / 2 of each),
 // out[slot][n/2] = gelu_tanh / silu (gate) * up.
-template <bool AF32, int ACT, bool ONE>
+template <int SUB, bool AF32, int ACT, bool ONE>
 __global__ __launch_bounds__(1024) void k_bank_gemv(const float *__restrict__ ids, const void *__restrict__ a_any,
                                                      const char *__restrict__ bank, size_t expert_bytes, uint32_t experts,
                                                      uint32_t a_slot_stride, uint32_t k, uint32_t sub_tiles, uint32_t waves,
                                                      uint32_t n, float *__restrict__ out)
 {
-    constexpr int SUB = 16, CPP = 4;
-    __shared__ float red[16 * SUB];  // [waves][16]
+    constexpr int CPP = 64 / SUB;
+    __shared__ float red[16 * SUB];  // [waves][SUB]
     // (workgroups reach the eight XCDs in turn: a contiguous run of sub-tiles per XCD, so that the sub-tiles of a 64-column
     // tile, whose pieces interleave inside the copy's blocks, stream through one L2)
     const uint32_t st = (blockIdx.x & 7u) * ((sub_tiles + 7u) >> 3) + (blockIdx.x >> 3), slot = blockIdx.y;
@@ -144,14 +144,14 @@ __global__ __launch_bounds__(1024) void k_bank_gemv(const float *__restrict__ id
     const uint32_t tile = st / CPP, part = st % CPP;
     const uint32_t col = ACT ? (cl / (SUB / 2)) * 32u + part * (SUB / 2) + cl % (SUB / 2) : part * SUB + cl;
     const void *a_row = (const char *)a_any + (size_t)slot * a_slot_stride * (AF32 ? 4 : 2);
-    const float dot = bank_dot<AF32, ONE>(bank, expert_bytes, experts, a_row, ids + slot, wave, waves, tile, col, k, (k + 127u) >> 7, [&]() {
+    const float dot = bank_dot<SUB, AF32, ONE>(bank, expert_bytes, experts, a_row, ids + slot, wave, waves, tile, col, k, (k + 127u) >> 7, [&]() {
         asm volatile("" ::"s"(out), "s"(n));   // (the store's arguments, fetched meanwhile)
     });
     if (lane < SUB) red[wave * SUB + cl] = dot;
     __syncthreads();
     if (wave != 0) return;
     float total = 0.f;
-    bank_reads(waves, [&](auto reads) { total = bank_sum<decltype(reads)::value>(red + cl, waves); });
+    bank_reads(waves, [&](auto reads) { total = bank_sum<SUB, decltype(reads)::value>(red + cl, waves); });
     if (ACT == 0) {
         const uint32_t on = st * SUB + cl;
         if (lane < SUB && on < n) out[(size_t)slot * n + on] = total;
@@ -165,14 +165,14 @@ __global__ __launch_bounds__(1024) void k_bank_gemv(const float *__restrict__ id
 // Workgroup = slots * wps waves on one sub-tile: wave (slot, j) takes passes j, j + wps, ... of its slot's
 // expert with its slot's activation row; one thread per column then adds weight[slot] * dot to the accumulator
 // slot by slot.  slots_wps: slots | wps << 8 | ceil(256 / wps) << 16 (which makes wave / wps, up to 16, a product and a shift).
-template <bool AF32, bool ONE>
+template <int SUB, bool AF32, bool ONE>
 __global__ __launch_bounds__(1024) void k_bank_down_axpy(const float *__restrict__ ids, const void *__restrict__ a_all,
                                                           const char *__restrict__ bank, size_t expert_bytes, uint32_t experts,
                                                           uint32_t k, uint32_t sub_tiles, uint32_t slots_wps, uint32_t n,
                                                           const float *__restrict__ weights, float *__restrict__ accum)
 {
-    constexpr int SUB = 16, CPP = 4;
-    __shared__ float red[16 * SUB];  // [slots * wps][16]
+    constexpr int CPP = 64 / SUB;
+    __shared__ float red[16 * SUB];  // [slots * wps][SUB]
     const uint32_t slots = slots_wps & 255u, wps = (slots_wps >> 8) & 255u;
     const uint32_t st = (blockIdx.x & 7u) * ((sub_tiles + 7u) >> 3) + (blockIdx.x >> 3);  // (a contiguous run per XCD, as in k_bank_gemv)
     if (st >= sub_tiles) return;
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(1024) void k_bank_down_axpy(const float *__restrict
         weight = weights[lane < slots ? lane : 0u];
     };
     const void *a_row = (const char *)a_all + (size_t)slot * k * (AF32 ? 4 : 2);
-    const float dot = bank_dot<AF32, ONE>(bank, expert_bytes, experts, a_row, ids + slot, j, wps, st / CPP, (st % CPP) * SUB + cl, k, (k + 127u) >> 7, fetch);
+    const float dot = bank_dot<SUB, AF32, ONE>(bank, expert_bytes, experts, a_row, ids + slot, j, wps, st / CPP, (st % CPP) * SUB + cl, k, (k + 127u) >> 7, fetch);
     if (lane < SUB) red[wave * SUB + cl] = dot;
     __syncthreads();
     if (wave != 0) return;
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(1024) void k_bank_down_axpy(const float *__restrict
 #pragma unroll
         for (int s = 0; s < kMaxBankSlots / (R / 2 + 1); s++)   // (wps > R / 2, and slots * wps <= kMaxBankSlots)
             if (s < (int)slots)
-                total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), s)) * bank_sum<R>(red + s * wps * SUB + cl, wps);
+                total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), s)) * bank_sum<SUB, R>(red + s * wps * SUB + cl, wps);
     });
     if (lane < SUB && on < n) accum[on] = total;
 }
@@ -371,57 +371,80 @@ static uint32_t raw_sub(uint32_t n_pad, uint32_t slots, bool per_slot, int force
     return per_slot && (uint64_t)(n_pad / 32) * slots >= 256 ? 32 : 16;
 }
 
+// Sub-tile width of the bank kernels (force_sub = 16 or 32 overrides: a tuning knob of the context), from both widths timed on
+// 3800 random calls.  The down projection, whose workgroups hold every slot: 16 always (in the mean 32 is 4 - 25 % behind).  The
+// per-slot GEMV: 16, but 32
+// * where even sixteen waves make several passes (more than 64 chunks), once 32 columns give more than 128 workgroups (0.91, in
+//   the mean, of the time on 16: 8608 -> 2 x 10560 on six slots 111 / 134 us);
+// * up to eight chunks between 128 and 256 such workgroups (0.95), one to a CU, and from 1024 on (0.94);
+// * on many workgroups where a pass of four chunks would leave two or more of its lane groups without one, up to sixteen chunks
+//   from 768 workgroups on (0.95), up to 24 from 2048 on (2272 -> 2 x 10528 on six slots 27.4 / 30.1).
+static uint32_t bank_sub(const BankView &b, uint32_t slots, bool per_slot, int force_sub)
+{
+    if (force_sub == 16 || force_sub == 32) return (uint32_t)force_sub;
+    const uint64_t wgs = (uint64_t)(b.n_pad / 32) * slots;
+    const uint32_t chunks = b.k_chunks, idle = (4u - chunks % 4u) % 4u;
+    if (!per_slot) return 16;
+    if (chunks > 64) return wgs > 128 ? 32 : 16;
+    if (chunks <= 8 && ((wgs > 128 && wgs <= 256) || wgs >= 1024)) return 32;
+    return idle >= 2 && ((chunks <= 16 && wgs >= 768) || (chunks <= 24 && wgs >= 2048)) ? 32 : 16;
+}
+
+// go(width, f32 rows, one pass per wave) as compile-time values
+template <class Go>
+static void bank_form(uint32_t sub, bool a_f32, bool one, Go &&go)
+{
+    const std::true_type yes{};
+    const std::false_type no{};
+    auto rows = [&](auto subv) {
+        if (a_f32 && one) go(subv, yes, yes);
+        else if (a_f32) go(subv, yes, no);
+        else if (one) go(subv, no, yes);
+        else go(subv, no, no);
+    };
+    if (sub == 32) rows(std::integral_constant<int, 32>{});
+    else rows(std::integral_constant<int, 16>{});
+}
+
 hipError_t launch_bank_gemv(hipStream_t s, const BankView &b, const void *a, bool a_f32, uint32_t a_slot_stride,
-                            const float *ids, uint32_t slots, int act, float *out, int force_waves)
+                            const float *ids, uint32_t slots, int act, float *out, int force_sub, int force_waves)
 {
     if (slots == 0 || b.n == 0) return hipSuccess;
     if (!b.cq || act < 0 || act > 2 || slots > 65535u) return hipErrorInvalidValue;
     if (act != 0 && b.n % (2 * kPairWidth) != 0) return hipErrorInvalidValue;
-    const uint32_t sub_tiles = b.n_pad / 16, passes = (b.k_chunks + 3) / 4;
+    const uint32_t sub = bank_sub(b, slots, true, force_sub), sub_tiles = b.n_pad / sub, passes = (b.k_chunks + 64 / sub - 1) / (64 / sub);
     uint32_t waves = passes < 16 ? passes : 16;
     if (force_waves >= 1 && force_waves <= 16) waves = (uint32_t)force_waves;
-    const bool one = passes <= waves;
-    dim3 grid(((sub_tiles + 7) / 8) * 8, slots), block(waves * 64);  // (whole rounds of the eight XCDs: see k_bank_gemv)
-#define TWM_BANK_LAUNCH(F32, A, ONEV)                                                                                  \
-    hipLaunchKernelGGL((k_bank_gemv<F32, A, ONEV>), grid, block, 0, s, ids, a, (const char *)b.cq, b.expert_bytes,     \
-                       b.experts, a_slot_stride, b.k, sub_tiles, waves, b.n, out)
-#define TWM_BANK_ACT(F32, ONEV)                            \
-    do {                                                   \
-        if (act == 0) TWM_BANK_LAUNCH(F32, 0, ONEV);       \
-        else if (act == 1) TWM_BANK_LAUNCH(F32, 1, ONEV);  \
-        else TWM_BANK_LAUNCH(F32, 2, ONEV);                \
-    } while (0)
-    if (a_f32 && one) TWM_BANK_ACT(true, true);
-    else if (a_f32) TWM_BANK_ACT(true, false);
-    else if (one) TWM_BANK_ACT(false, true);
-    else TWM_BANK_ACT(false, false);
-#undef TWM_BANK_ACT
-#undef TWM_BANK_LAUNCH
+    const dim3 grid(((sub_tiles + 7) / 8) * 8, slots), block(waves * 64);  // (whole rounds of the eight XCDs: see k_bank_gemv)
+    auto go = [&](auto subv, auto f32, auto one) {
+        constexpr int SUB = decltype(subv)::value;
+        constexpr bool F32 = decltype(f32)::value, ONE = decltype(one)::value;
+        auto kernel = act == 0 ? k_bank_gemv<SUB, F32, 0, ONE> : act == 1 ? k_bank_gemv<SUB, F32, 1, ONE> : k_bank_gemv<SUB, F32, 2, ONE>;
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, ids, a, (const char *)b.cq, b.expert_bytes, b.experts, a_slot_stride, b.k, sub_tiles,
+                           waves, b.n, out);
+    };
+    bank_form(sub, a_f32, passes <= waves, go);
     return hipGetLastError();
 }
 
 hipError_t launch_bank_down_axpy(hipStream_t s, const BankView &b, const void *a_all, bool a_f32, const float *ids,
-                                 const float *weights, uint32_t slots, float *accum, int force_waves)
+                                 const float *weights, uint32_t slots, float *accum, int force_sub, int force_waves)
 {
     if (slots == 0 || b.n == 0) return hipSuccess;
     if (!b.cq || slots > (uint32_t)kMaxBankSlots) return hipErrorInvalidValue;
-    const uint32_t sub_tiles = b.n_pad / 16, passes = (b.k_chunks + 3) / 4;
+    const uint32_t sub = bank_sub(b, slots, false, force_sub), sub_tiles = b.n_pad / sub, passes = (b.k_chunks + 64 / sub - 1) / (64 / sub);
     uint32_t wps = 16 / slots;                // waves per slot: up to one per pass, sixteen waves in all
     if (wps > passes) wps = passes;
     if (force_waves >= 1 && (uint32_t)force_waves * slots <= 16) wps = (uint32_t)force_waves;
     if (wps == 0) wps = 1;
     const uint32_t slots_wps = slots | (wps << 8) | (((256u + wps - 1u) / wps) << 16);
-#define TWM_DOWN_LAUNCH(F32, ONEV)                                                                                     \
-    hipLaunchKernelGGL((k_bank_down_axpy<F32, ONEV>), dim3(((sub_tiles + 7) / 8) * 8), dim3(slots * wps * 64), 0, s, ids, a_all, \
-                       (const char *)b.cq, b.expert_bytes, b.experts, b.k, sub_tiles, slots_wps, b.n, weights, accum)
-    if (passes <= wps) {
-        if (a_f32) TWM_DOWN_LAUNCH(true, true);
-        else TWM_DOWN_LAUNCH(false, true);
-    } else {
-        if (a_f32) TWM_DOWN_LAUNCH(true, false);
-        else TWM_DOWN_LAUNCH(false, false);
-    }
-#undef TWM_DOWN_LAUNCH
+    auto go = [&](auto subv, auto f32, auto one) {
+        constexpr int SUB = decltype(subv)::value;
+        constexpr bool F32 = decltype(f32)::value, ONE = decltype(one)::value;
+        hipLaunchKernelGGL((k_bank_down_axpy<SUB, F32, ONE>), dim3(((sub_tiles + 7) / 8) * 8), dim3(slots * wps * 64), 0, s, ids, a_all,
+                           (const char *)b.cq, b.expert_bytes, b.experts, b.k, sub_tiles, slots_wps, b.n, weights, accum);
+    };
+    bank_form(sub, a_f32, passes <= wps, go);
     return hipGetLastError();
 }
 

@@ -592,6 +592,33 @@ def test_an_infinite_activation_of_a_bank_row_reaches_every_column_as_itself(dev
     bank.free()
 
 
+@pytest.mark.parametrize("k,slots", [(1184, 4), (9344, 1)])
+def test_bank_kernels_take_the_sub_tile_width_asked_for(dev, k, slots):
+    # the widths add a pass's chunks in another order, which shows in the last bits of some column
+    n, experts, ids_h = 192, 3, np.array([2, 0, 1, 1], np.float32)[:slots]
+    raw = [(O.synth_packed(k, n, 2051 + e), O.synth_scales(k, n, 2061 + e)) for e in range(experts)]
+    p, s = (T.GpuTensor.from_host(dev, np.concatenate([x[i].reshape(-1) for x in raw])) for i in (0, 1))
+    bank = T.ExpertBank.from_device(dev, p, s, raw[0][0].size, raw[0][1].size, k, n, experts)
+    ids, wts_h = T.GpuTensor.from_host(dev, ids_h), np.array([0.5, 0.25, 0.125, 1.0], np.float32)[:slots]
+    a16 = O.synth_act_f16(slots, k, 2071)
+    rows, a, wts = a16.view(np.float16).astype(np.float32).reshape(slots, k), T.GpuTensor.from_host(dev, a16, "f16"), T.GpuTensor.from_host(dev, wts_h)
+    truth = np.concatenate([O.gemm_f64(rows[i:i + 1], *raw[int(ids_h[i])], 1, k, n) for i in range(slots)])
+    got = {}
+    for width in (16, 32):
+        dev.set_option("sub", width)
+        try:
+            out, acc = T.GpuTensor.from_host(dev, np.full((slots, n), np.nan, np.float32)), T.GpuTensor.zeros(dev, (n,), "f32")
+            T.batched_marlin_gate_up(dev, a, bank, ids, out, slots, per_slot_rows=True)
+            T.batched_marlin_down_axpy(dev, a, bank, ids, wts, acc, slots)
+        finally:
+            dev.set_option("sub", 0)
+        got[width] = out.to_host(), acc.to_host()
+        close_rows(got[width][0], truth, F32_SUM)
+        close_rows(got[width][1].reshape(1, n), (wts_h.astype(np.float64)[:, None] * truth).sum(0, keepdims=True), F32_SUM)
+    assert not np.array_equal(got[16][0], got[32][0]) and not np.array_equal(got[16][1], got[32][1])
+    bank.free()
+
+
 # one chunk in part, the most chunks with one each per wave and one more, K one group past whole chunks, four chunks per wave of
 # sixteen waves; a column and a sub-tile more than whole tiles
 @pytest.mark.parametrize("k,n", [(32, 1), (96, 17), (1408, 81), (1440, 64), (2592, 130), (3616, 33), (8192, 65)])
