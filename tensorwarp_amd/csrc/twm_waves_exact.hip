@@ -530,7 +530,9 @@ hipError_t init_waves_exact()
 // Within those lines the form comes from a small cost model, fitted to the same sweeps (root mean square error 6.5 %; its forms
 // are 0.3 % above the best ones in the mean): a chunk costs a wave `fixed` + `tile` x nt us, more the longer the row of chunks;
 // a launch takes the larger of that and of its weights at 5.8 TB/s; a K-split adds the launch of the sum kernel and its
-// traffic.  Up to four tiles (3 excepted) a K-split is taken only up to 128 groups and from eight chunks on.
+// traffic.  Up to four tiles (3 excepted) a K-split is taken only up to 128 groups and from eight chunks on.  With the gated store
+// as without it: the kernel that adds the ranges applies the gate (17824 -> 2 x 128 at 24 f32 rows 45.0 us on 8 workgroups, 11.4 on
+// eight ranges of 16; 1180 random gated calls 0.91 with f16 rows and 0.72 with f32 rows of the time of the kernels of before).
 WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated)
 {
     const WavesPlan none = {0, 0, 0};
@@ -558,14 +560,15 @@ WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool
     WavesPlan best = none;
     double best_us = 1e30;
     for (uint32_t nt : {1u, 2u, 3u, 4u, 5u, 6u, 8u, 10u}) {
-        if ((gated && nt % 2) || (nt == 10 && a_f32 && !few_f32) || (nt > 4 && a_f32 && m > 16)) continue;
+        if ((nt == 10 && a_f32 && !few_f32) || (nt > 4 && a_f32 && m > 16)) continue;
         const uint32_t groups = (n_tiles + nt - 1) / nt;
         const bool whole = nt == 1 || nt == 2 || nt == 4;
         if (whole && groups > 256 && !(nt == 4 && a_f32 && m > 16)) continue;
         for (uint32_t sp = 1; sp <= 8 && sp <= k_chunks; sp++) {
             const uint32_t cps = (k_chunks + sp - 1) / sp;
             if ((k_chunks + cps - 1) / cps != sp) continue;   // same work as a smaller factor
-            if (sp > 1 && (gated || groups * sp > 256 || k_chunks / sp < 8 || (whole && groups > 128))) continue;
+            if (gated && sp == 1 && nt % 2) continue;         // (a gate tile and its up tile lie in one workgroup)
+            if (sp > 1 && (groups * sp > 256 || k_chunks / sp < 8 || (whole && groups > 128))) continue;
             const double e = 0.1 * ((cps + 7) / 8) + 0.9 * cps / 8.0;
             const double rounds = (double)((groups * sp + 255) / 256);
             const double work = rounds * e * (cost.fixed + cost.tile * nt) * (1.0 + cost.longer * e / nt);

@@ -264,6 +264,24 @@ def test_waves_gated_store_on_many_column_tiles(dev, m, dtype, ffn):
     w.free()
 
 
+# few features of a deep matrix: K in ranges whose sums the reduction gates
+@pytest.mark.parametrize("k,ffn,m,dtype", [(9344, 32, 9, "f16"), (9344, 96, 24, "f16"), (9376, 96, 25, "f32"), (12320, 160, 13, "f32"), (12288, 64, 8, "f32")])
+def test_waves_gated_store_with_a_planned_k_split(dev, k, ffn, m, dtype):
+    assert "k_splitk_reduce" in dev.plan(k, 2 * ffn, m, dtype=dtype, gated=True)
+    gate, up = [(O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (1521, 1523)]
+    pair = [tuple(T.GpuTensor.from_host(dev, x, t) for x, t in zip(w, ("u8", "f16"))) for w in (gate, up)]
+    w = T.MarlinWeight.gate_up(dev, *pair, k, ffn)
+    a16 = O.synth_act_f16(m, k, 1525)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+    if dtype == "f32":
+        a[1] *= np.float32(2.0 ** -21)
+    g, u = (O.gemm_f64(a, *x, m, k, ffn) for x in (gate, up))
+    out = T.GpuTensor.from_host(dev, np.full((m, ffn), np.nan, np.float32))
+    T.gemm_swiglu(dev, w, T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a), m, out)
+    close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
+    w.free()
+
+
 @pytest.mark.parametrize("m,dtype", [(5, "f32"), (8, "f32"), (9, "f16"), (13, "f32"), (32, "f16"), (40, "f16"), (64, "f32"), (96, "f16")])
 def test_waves_gated_store(dev, m, dtype):
     k, ffn = 1056, 96                                # 33 groups; three quads of gate and up tiles

@@ -203,6 +203,15 @@ def test_plans_of_the_few_row_kernels(lib):
     assert min(seen.values()) >= 400, seen
 
 
+@pytest.mark.parametrize("k,n,m,dtype", [(17824, 256, 24, "f32"), (16000, 256, 29, "f16"), (14976, 1344, 23, "f32"), (18176, 128, 9, "f16"),
+                                         (9344, 384, 25, "f32")])
+def test_few_gated_columns_of_a_deep_matrix_have_their_k_split(lib, k, n, m, dtype):
+    # (unsplit, the columns alone are a handful of workgroups that walk all of K)
+    dt = _lib.F32 if dtype == "f32" else _lib.F16
+    gated, plain = (parse(describe(lib, k, n, m, dt, g)) for g in (1, 0))
+    assert gated["splits"] > 1 and 2 * workgroups(gated, k, n, m) >= workgroups(plain, k, n, m), (gated["text"], plain["text"])
+
+
 def test_describe_rejects_what_twm_gemm_rejects(lib):
     buf = ctypes.create_string_buffer(64)
     assert lib.twm_plan_describe(None, 100, 64, 1, _lib.F16, 0, buf, 64) == _lib.SHAPE_ERROR       # K % 32
