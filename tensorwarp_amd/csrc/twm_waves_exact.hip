@@ -518,21 +518,32 @@ hipError_t init_waves_exact()
 //   (3584 -> 152064 at 8 f16 rows 66 / 54, at 32 92 / 78, at 8 f32 rows 73 / 82), as do wide matrices of up to eight chunks
 //   (896 -> 32000 at 16 rows 8.1 / 6.5);
 // * 17 .. 32 f32 rows end at the four tiles their registers allow (1856 -> 2 x 9312 at 32 rows 20.9 / 17.3; 1024 tiles and
-//   fewer are 5 - 50 % ahead) and at K of about 20000, 8192 above 512 tiles (28672 -> 8192 64 / 55, 13920 -> 11225 45.6 / 39.5);
+//   fewer are 5 - 50 % ahead) and at K of about 20000, 12800 above 340 tiles (17536 -> 5504 at 25 rows 36.5 / 31.6), 8192 above
+//   680 and 5120 on 513 .. 680, whose groups of three leave the CUs 70 - 85 % full (28672 -> 8192 64 / 55, 8064 -> 9792 at 23
+//   rows 30.5 / 25.6, 7296 -> 2 x 5280 at 27 30.7 / 27.0); nine rows and more on three chunks at 2048 tiles (128 -> 39553 at 16
+//   rows 8.1 / 7.3);
 // * f16, up to eight rows: the lane-per-column and streaming kernels keep 513 .. 1100 tiles (896 -> 2 x 4864 4.9 / 4.2, 2560 ->
 //   2 x 7168 8.5 / 7.5) and 1537 .. 2048 (3104 -> 28833 at 6 rows 14.1 / 12.8: eight tiles each leave the CUs 75 - 90 % full),
 //   K of 16 .. 32 chunks on 257 .. 512 tiles (3584 -> 4608 5.9 / 5.6), and up to six rows, seven up to K = 4096, every K from
-//   2200 on with up to 256 tiles (3584 -> 3584 at 5 rows 5.2 / 4.6);
-// * f16, deep K on 129 .. 256 tiles: from 72 chunks on up to sixteen rows (12192 -> 3584 at 8 rows 11.0 / 10.0), from 65 on above
-//   (17824 -> 3584 at 17 rows 16.8 / 15.6); f16 on a few chunks: four on 513 tiles and more (256 -> 14049 at 10 rows 4.0 / 3.75),
-//   nine to sixteen on 701 .. 1000 (1600 -> 2 x 6560 at 11 rows 6.75 / 6.5, 1600 -> 14798 at 30 9.6 / 8.9); 1801 .. 2048 tiles
-//   (2752 -> 2 x 15104 at 17 rows 16.0 / 15.0) and, up to sixteen rows, 961 .. 1024 (2752 -> 2 x 8192 at 12 rows 9.1 / 8.7).
+//   2200 on with up to 256 tiles (3584 -> 3584 at 5 rows 5.2 / 4.6), gated 2048 .. 4096 at eight rows too, where pairs of tiles
+//   are half as many workgroups (3072 -> 2 x 96 at 8 rows 4.75 / 4.24);
+// * f16, deep K on 129 .. 256 tiles: from 72 chunks on up to sixteen rows (12192 -> 3584 at 8 rows 11.0 / 10.0), up to 320 tiles
+//   from 67 on (9216 -> 4352 at 11 rows 10.9 / 9.8), from 65 on above (17824 -> 3584 at 17 rows 16.8 / 15.6); f16 on a few
+//   chunks: four on 513 tiles and more (256 -> 14049 at 10 rows 4.0 / 3.75), nine to sixteen on 701 .. 1000 (1600 -> 2 x 6560 at
+//   11 rows 6.75 / 6.5, 1600 -> 14798 at 30 9.6 / 8.9), up to eighteen above 1600, 1536 up to sixteen rows and 1300 up to eight
+//   (those up to ten): a wave has one to three chunks, unevenly, on seven to ten tiles (1152 -> 33728 at 19 rows 13.1 / 11.0, 1664
+//   -> 24966 at 9 10.4 / 8.9, 1152 -> 38272 at 9 10.6 / 9.4); 1801 .. 2048 tiles (2752 -> 2 x 15104 at 17 rows 16.0 / 15.0)
+//   and, up to sixteen rows, 961 .. 1024 (2752 -> 2 x 8192 at 12 rows 9.1 / 8.7).
 // Within those lines the form comes from a small cost model, fitted to the same sweeps (root mean square error 6.5 %; its forms
 // are 0.3 % above the best ones in the mean): a chunk costs a wave `fixed` + `tile` x nt us, more the longer the row of chunks;
 // a launch takes the larger of that and of its weights at 5.8 TB/s; a K-split adds the launch of the sum kernel and its
-// traffic.  Up to four tiles (3 excepted) a K-split is taken only up to 128 groups and from eight chunks on.  With the gated store
-// as without it: the kernel that adds the ranges applies the gate (17824 -> 2 x 128 at 24 f32 rows 45.0 us on 8 workgroups, 11.4 on
-// eight ranges of 16; 1180 random gated calls 0.91 with f16 rows and 0.72 with f32 rows of the time of the kernels of before).
+// traffic, 1.2 us more under a gate (5344 -> 2 x 2784 at 13 f32 rows 12.8 split, 11.3 not).  Up to four tiles (3 excepted) a
+// K-split is taken only up to 128 groups; from 32 chunks on, with f32 rows 28 up to sixteen rows and 16 above (3072 -> 128 at 25
+// f16 rows 5.5 split, 5.0 not; 2336 -> 2 x 608 at 5 f32 rows 6.2 / 5.1; but 3712 -> 448 at 11 f32 rows 6.2 / 7.5), and with eight
+// chunks and more to a range.  With the gated store as without it: the kernel that adds the ranges applies the gate (17824 -> 2 x
+// 128 at 24 f32 rows 45.0 us on 8 workgroups, 11.4 on eight ranges of 16).
+// 4000 random calls against the kernels of before, in the mean: f16 rows 0.95, gated 0.91, f32 rows 0.74, gated 0.71; 9 of them
+// more than 6 % slower.
 WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated)
 {
     const WavesPlan none = {0, 0, 0};
@@ -540,23 +551,27 @@ WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool
     const bool few_f32 = a_f32 && m <= 8;
     if (n_tiles > 4096 && !few_f32) return none;
     if (a_f32) {
-        if (m > 16 && (n_tiles > 1024 || k_chunks > (n_tiles > 512 ? 64u : 160u))) return none;
+        if (m > 16 && (n_tiles > 1024 || k_chunks > (n_tiles > 680 ? 64u : n_tiles > 512 ? 40u : n_tiles > 340 ? 100u : 160u))) return none;
+        if (m > 8 && n_tiles > 2048 && k_chunks <= 3) return none;
     } else {
         if (k_chunks <= 8 && n_tiles > (k_chunks <= 4 ? 512u : 1024u)) return none;
-        if (n_tiles > 128 && n_tiles <= 256 && k_chunks > (m <= 16 ? 71u : 64u)) return none;
+        if (n_tiles > 128 && n_tiles <= (m <= 16 ? 320u : 256u) && k_chunks > (m > 16 ? 64u : n_tiles > 256 ? 66u : 71u)) return none;
         if (n_tiles > 700 && n_tiles <= 1000 && k_chunks > 8 && k_chunks <= 16) return none;
         if (n_tiles > 1800 && n_tiles <= 2048) return none;
+        if (n_tiles > (m <= 8 && k_chunks <= 10 ? 1300u : m <= 16 ? 1536u : 1600u) && k_chunks <= 18) return none;
         if (m <= 16 && n_tiles > 960 && n_tiles <= 1024) return none;
         if (m <= 8) {
             if ((n_tiles > 512 && n_tiles <= 1100) || (n_tiles > 1536 && n_tiles <= 2048)) return none;
             if (n_tiles > 256 && n_tiles <= 512 && k_chunks >= 16 && k_chunks <= 32) return none;
             if (n_tiles <= 256 && k_chunks > 17 && (m <= 6 || (m == 7 && k_chunks <= 32))) return none;
+            if (n_tiles <= 256 && gated && k_chunks >= 16 && k_chunks <= 31) return none;
         }
     }
     static const struct { double fixed, tile, longer, split, split_mb; } kCost[] = {
         {0.12, 0.31, 0.045, 1.9, 1.0}, {0.37, 0.42, 0.026, 1.2, 1.0}, {0.20, 0.35, 0.026, 1.4, 1.0}, {0.54, 0.39, 0.05, 1.7, 0.5}, {1.5, 0.55, 0.02, 1.7, 0.5}};
     const auto &cost = kCost[!a_f32 ? (m <= 16 ? 0 : 1) : few_f32 ? 2 : m <= 16 ? 3 : 4];
     const double bytes_us = (double)n_tiles * k_chunks * 1152.0 / 5.8e6;
+    const uint32_t shallow = !a_f32 ? 32u : m <= 16 ? 28u : 16u;   // (K is not split below)
     WavesPlan best = none;
     double best_us = 1e30;
     for (uint32_t nt : {1u, 2u, 3u, 4u, 5u, 6u, 8u, 10u}) {
@@ -568,13 +583,13 @@ WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool
             const uint32_t cps = (k_chunks + sp - 1) / sp;
             if ((k_chunks + cps - 1) / cps != sp) continue;   // same work as a smaller factor
             if (gated && sp == 1 && nt % 2) continue;         // (a gate tile and its up tile lie in one workgroup)
-            if (sp > 1 && (groups * sp > 256 || k_chunks / sp < 8 || (whole && groups > 128))) continue;
+            if (sp > 1 && (groups * sp > 256 || k_chunks < shallow || k_chunks / sp < 8 || (whole && groups > 128))) continue;
             const double e = 0.1 * ((cps + 7) / 8) + 0.9 * cps / 8.0;
             const double rounds = (double)((groups * sp + 255) / 256);
             const double work = rounds * e * (cost.fixed + cost.tile * nt) * (1.0 + cost.longer * e / nt);
             const double t4 = work * work * work * work + bytes_us * bytes_us * bytes_us * bytes_us;
             double t = __builtin_sqrt(__builtin_sqrt(t4));
-            if (sp > 1) t += cost.split + cost.split_mb * sp * m * n_tiles * 128.0e-6;
+            if (sp > 1) t += cost.split + (gated ? 1.2 : 0.0) + cost.split_mb * sp * m * n_tiles * 128.0e-6;
             if (t < best_us) {
                 best_us = t;
                 best = WavesPlan{nt, 8, sp};

@@ -203,6 +203,23 @@ def test_plans_of_the_few_row_kernels(lib):
     assert min(seen.values()) >= 400, seen
 
 
+@pytest.mark.parametrize("k,n,m,dtype,gated", [(1152, 33728, 19, "f16", 0), (1664, 24966, 9, "f16", 0), (1152, 38272, 9, "f16", 0), (1792, 26560, 14, "f16", 0),
+                                               (128, 39553, 16, "f32", 0), (17536, 5504, 25, "f32", 0), (8064, 9792, 23, "f32", 0),
+                                               (7296, 10560, 27, "f32", 1), (3072, 192, 8, "f16", 1), (9216, 4352, 11, "f16", 0)])
+def test_shapes_on_which_the_other_kernels_stay_ahead(lib, k, n, m, dtype, gated):
+    # uneven chunks on many tiles, groups that leave CUs idle, gated pairs on few columns: measured 8 - 19 % slower on k_waves_exact
+    f = parse(describe(lib, k, n, m, _lib.F32 if dtype == "f32" else _lib.F16, gated))
+    assert f["kernel"] != "k_waves_exact", f["text"]
+
+
+@pytest.mark.parametrize("k,n,m,dtype,gated,split", [(3072, 128, 25, "f16", 0, False), (3584, 467, 24, "f16", 0, False), (2336, 1216, 5, "f32", 1, False),
+                                                     (3712, 448, 11, "f32", 0, True), (4096, 128, 25, "f16", 0, True)])
+def test_a_shallow_matrix_is_not_split(lib, k, n, m, dtype, gated, split):
+    # (the launch of the sum kernel costs more than a few chunks per wave)
+    f = parse(describe(lib, k, n, m, _lib.F32 if dtype == "f32" else _lib.F16, gated))
+    assert f["kernel"] == "k_waves_exact" and (f["splits"] > 1) == split, f["text"]
+
+
 @pytest.mark.parametrize("k,n,m,dtype", [(17824, 256, 24, "f32"), (16000, 256, 29, "f16"), (14976, 1344, 23, "f32"), (18176, 128, 9, "f16"),
                                          (9344, 384, 25, "f32")])
 def test_few_gated_columns_of_a_deep_matrix_have_their_k_split(lib, k, n, m, dtype):
