@@ -36,7 +36,7 @@ namespace twm {
 // three (two before: 4096 -> 2 x 11008 at 96 rows 32.8 -> 29.1 us on 96 x 128, at 64 rows 27.0 -> 25.3 on 64 x 256; a LLaMA-7B
 // layer at 512 rows 254.1 -> 249.7, at 2048 787.9 -> 783.4 on 128 x 256; 3584 -> 2 x 18944 at 96 rows, two workgroups on some
 // CUs, 43.1 -> 45.2).
-template <int MT, int NTW, bool HALF, int D>
+template <int MT, int NTW, bool HALF, int D, PrefillStore STORE>
 __device__ __forceinline__ void prefill_block(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc, const _Float16 *__restrict__ a_any,
                                               const OutSpec out, uint32_t m_rows, uint32_t k, uint32_t n, uint32_t n_tiles, uint32_t k_chunks,
                                               uint32_t chunks_per_split, float *__restrict__ partials, uint32_t row_store, uint32_t col_blocks,
@@ -326,7 +326,7 @@ __device__ __forceinline__ void prefill_block(const uint4v *__restrict__ qw, con
         // groups kb fall on different banks) so that a lane stores 16 bytes and sixteen lanes cover 256 consecutive bytes
         // of a row, instead of 64-byte pieces of four rows from 4-byte stores.
         const uint32_t col = nt0 * 16u + (lane & 15u) * 4u;
-        constexpr bool SEGS = NTW == 3;                        // (see launch_prefill_t)
+        constexpr bool SEGS = STORE == kStoreSegments;
         float *dst = partials ? partials + ((size_t)blockIdx.z * m_rows) * (n_tiles * 16u) : out.seg[0].ptr;
         uint32_t ld = partials ? n_tiles * 16u : n, at = col;
         bool mine = (lane & 15u) * 4u < 16u * NTW && col < ld;   // (ld is a multiple of 4)
@@ -407,7 +407,7 @@ __device__ __forceinline__ void prefill_block(const uint4v *__restrict__ qw, con
         }
         return;
     }
-    if (NTW == 3 && out.swiglu) {
+    if constexpr (STORE == kStoreGate) {
         // three quads of tiles on four waves of three: the gate and up tiles of a feature lie with different waves, so half of the
         // block's rows at a time go through LDS (rows of 196 floats: the four row groups kb fall on different banks) and every
         // thread gates and stores four features of a row, 24 lanes a row's 384 bytes
@@ -482,27 +482,27 @@ __device__ __forceinline__ void prefill_block(const uint4v *__restrict__ qw, con
     }
 }
 
-template <int MT, int NTW = 4, bool HALF = false, int D = HALF ? 2 : 3>
+template <int MT, int NTW = 4, bool HALF = false, int D = HALF ? 2 : 3, PrefillStore STORE = kStoreAny>
 __global__ __launch_bounds__(256) TWM_PF_OCC(HALF || NTW == 2) void k_prefill(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc,
                                                   const _Float16 *__restrict__ a_any, OutSpec out, uint32_t m_rows,
                                                   uint32_t k, uint32_t n, uint32_t n_tiles, uint32_t k_chunks,
                                                   uint32_t chunks_per_split, float *__restrict__ partials,
                                                   uint32_t row_store, uint32_t col_blocks, uint32_t row_blocks)
 {
-    prefill_block<MT, NTW, HALF, D>(qw, sc, a_any, out, m_rows, k, n, n_tiles, k_chunks, chunks_per_split, partials, row_store, col_blocks, row_blocks);
+    prefill_block<MT, NTW, HALF, D, STORE>(qw, sc, a_any, out, m_rows, k, n, n_tiles, k_chunks, chunks_per_split, partials, row_store, col_blocks, row_blocks);
 }
 
 // Blocks of 64 or 96 rows x 192 columns, for the shapes whose 128-column blocks put two on some CUs and whose 256-column blocks
 // leave many without (3584 -> 37888 at 64 rows 39.3 -> 28.3 us, at 96 39.6 -> 33.3; 4096 -> 22016 at 128 36.1 -> 31.2, at 192
 // 44.5 -> 38.7).
-template <int MT>
+template <int MT, PrefillStore STORE = kStoreAny>
 __global__ __launch_bounds__(256) TWM_PF_OCC(MT == 4) void k_prefill192(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc,
                                                   const _Float16 *__restrict__ a_any, OutSpec out, uint32_t m_rows,
                                                   uint32_t k, uint32_t n, uint32_t n_tiles, uint32_t k_chunks,
                                                   uint32_t chunks_per_split, float *__restrict__ partials,
                                                   uint32_t row_store, uint32_t col_blocks, uint32_t row_blocks)
 {
-    prefill_block<MT, 3, false, 3>(qw, sc, a_any, out, m_rows, k, n, n_tiles, k_chunks, chunks_per_split, partials, row_store, col_blocks, row_blocks);
+    prefill_block<MT, 3, false, 3, STORE>(qw, sc, a_any, out, m_rows, k, n, n_tiles, k_chunks, chunks_per_split, partials, row_store, col_blocks, row_blocks);
 }
 
 // The partial sums of one place, added in split order (deterministic): four loads in flight at a time.
@@ -785,9 +785,10 @@ static hipError_t launch_prefill_t(hipStream_t s, const WeightView &w, const _Fl
     const uint32_t col_blocks = (w.n_tiles + 4 * NTW - 1) / (4 * NTW), row_blocks = (m + 16 * MT - 1) / (16 * MT);
     dim3 grid(col_blocks * row_blocks, 1, splits);  // the kernel turns the linear id into an XCD-aware tile
     // 16-byte row stores: into the partial sums always (padded width, a multiple of 64); into the output when every four
-    // columns are whole 16-byte places of one segment.  Segments only from 192-column blocks: the others are no faster with
-    // the segment's search in them, not even where it is skipped (128 x 256 blocks, 3584 -> 4608 plain at 200 rows 22.4 us
-    // without it, 24.2 with it).
+    // columns are whole 16-byte places of one segment.  Segments only from 192-column blocks, in kernels of their own, as the gate
+    // there: compiled into one kernel they cost the plain store where they are skipped (128 x 192 blocks, 256 -> 33760 at 101 rows
+    // 8.1 us alone, 10.0 with both, 288 -> 16768 at 523 14.8 / 17.8; 128 x 256 blocks, 3584 -> 4608 at 200 rows 22.4 us without
+    // the segment's search, 24.2 with it).
     // (via_partials: the sums of a single split go through the partial-sum buffer too and k_splitk_reduce stores them:
     // it is the store that applies the rows' power-of-two factors of f32 activations ahead of a bias or a gate)
     via_partials = via_partials && partials != nullptr;
@@ -796,10 +797,16 @@ static hipError_t launch_prefill_t(hipStream_t s, const WeightView &w, const _Fl
         row_store = out.swiglu ? kRowsNone : row_store_of(out, w.n);
         if (NTW != 3 && row_store == kRowsSegments) row_store = kRowsNone;
     }
-    auto kernel = [] {
-        if constexpr (NTW == 3 && MT < 8) return k_prefill192<MT>;
-        else return k_prefill<MT, NTW, HALF, D>;
-    }();
+    auto kernel_of = [](auto store) {
+        constexpr PrefillStore STORE = decltype(store)::value;
+        if constexpr (NTW == 3 && MT < 8) return k_prefill192<MT, STORE>;
+        else return k_prefill<MT, NTW, HALF, D, STORE>;
+    };
+    auto kernel = kernel_of(std::integral_constant<PrefillStore, kStoreAny>{});
+    if constexpr (NTW == 3) {
+        if (splits == 1 && !via_partials && out.swiglu) kernel = kernel_of(std::integral_constant<PrefillStore, kStoreGate>{});
+        else if (row_store == kRowsSegments) kernel = kernel_of(std::integral_constant<PrefillStore, kStoreSegments>{});
+    }
     hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, (const uint4v *)w.qw, (const uint2v *)w.sc, a, out, m, w.k,
                        w.n, w.n_tiles, w.k_chunks, cps, splits > 1 || via_partials ? partials : nullptr, row_store, col_blocks, row_blocks);
     if (splits > 1 || via_partials) return launch_splitk_reduce(s, partials, out, m, w.n, w.n_tiles * 16, splits);
@@ -818,13 +825,19 @@ hipError_t init_prefill()
         return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, d * 16 * mt * kPfRowStride * (int)sizeof(_Float16));
     };
     hipError_t e = ask((const void *)k_prefill<8>, 8, 3);
-    if (e == hipSuccess) e = ask((const void *)k_prefill<8, 3>, 8, 3);
-    if (e == hipSuccess) e = ask((const void *)k_prefill<8, 3, true>, 8, 2);
+    auto ask192 = [&](auto store) {
+        constexpr PrefillStore STORE = decltype(store)::value;
+        if (e == hipSuccess) e = ask((const void *)k_prefill<8, 3, false, 3, STORE>, 8, 3);
+        if (e == hipSuccess) e = ask((const void *)k_prefill<8, 3, true, 2, STORE>, 8, 2);
+        if (e == hipSuccess) e = ask((const void *)k_prefill192<4, STORE>, 4, 3);
+        if (e == hipSuccess) e = ask((const void *)k_prefill192<6, STORE>, 6, 3);
+    };
+    ask192(std::integral_constant<PrefillStore, kStoreAny>{});
+    ask192(std::integral_constant<PrefillStore, kStoreSegments>{});
+    ask192(std::integral_constant<PrefillStore, kStoreGate>{});
     if (e == hipSuccess) e = ask((const void *)k_prefill<4, 2, false, 4>, 4, 4);
     if (e == hipSuccess) e = ask((const void *)k_prefill<6, 2>, 6, 3);
     if (e == hipSuccess) e = ask((const void *)k_prefill<8, 2>, 8, 3);
-    if (e == hipSuccess) e = ask((const void *)k_prefill192<4>, 4, 3);
-    if (e == hipSuccess) e = ask((const void *)k_prefill192<6>, 6, 3);
     return e;
 }
 

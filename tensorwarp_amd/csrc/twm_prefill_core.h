@@ -64,6 +64,9 @@ __device__ __forceinline__ void pf_store_out(const OutSpec &out, uint32_t m, uin
     }
 }
 
+// What a prefill kernel's store holds.  192-column blocks: rows of one matrix, rows of segments, and the gate in kernels of their
+// own; all other forms: kStoreAny, with a gate and without segments.
+enum PrefillStore { kStoreAny, kStoreSegments, kStoreGate };
 enum RowStore : uint32_t { kRowsNone, kRowsPlain, kRowsSegments };   // (see row_store_of)
 
 // Where columns col .. col + 3 of row 0 go (row r: r * ld further), and their bias; a segment's columns are multiples of four
