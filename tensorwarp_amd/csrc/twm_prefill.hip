@@ -667,6 +667,9 @@ hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutS
 // 8192, 86 blocks of 192 columns where 64 of 256 fill the CUs, stays with those).  Gated, the 192-column forms take 1.07 times
 // the plain ones (4096 -> 2 x 11008 at 512 rows 98.3 / 89.4, at 768 154 / 133, at 2048 356 / 346; 3584 -> 2 x 18944 at 2048 537 /
 // 507).
+// 128 x 192 gated not under a K-split, which it makes of many parts (13056 -> 2 x 32 at 929 rows 18.2 us on 17 parts of 64 x 256
+// blocks, 22.0 on 26 of these), and not on up to three chunks, 96 x 192 on two, where the gate's way through LDS is the launch
+// (128 -> 2 x 11616 at 833 rows 64 x 256 23.2, 128 x 192 24.8, 96 x 192 27.9).
 constexpr double kPf192 = 0.80, kPf192Gated = 1.07;
 constexpr uint32_t kNarrowMaxRows = 256, kNarrowMinTiles = 128, kMiddleMaxRows = 1024;
 static const struct { uint32_t form; double chunk[2]; } kMiddle[] = {{66, {0.94, 1.62}}, {98, {1.17, 2.10}}};
@@ -706,6 +709,7 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
             if (f.form == bm) chunk = f.chunk;
         for (uint32_t i = 0; i < n_cuts; i++) {
             const uint32_t sp = cuts[i].splits, cps = cuts[i].chunks;
+            if (gated && !force_rows && ((bm == 192 && (sp > 1 || k_chunks <= 3)) || (bm == 98 && k_chunks <= 2))) continue;
             if (!force_splits && sp > 1 && 5.5 + sp * partial_us >= best.us) break;  // (the sum kernel alone takes longer)
             const double total = wgs * sp;
             double t = 0.0;

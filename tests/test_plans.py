@@ -108,6 +108,14 @@ def test_plans_of_prefill(lib, k, n, m):
         assert f["block_rows"] == 128 and f["splits"] == 1 and wgs >= CUS, f["text"]        # enough tiles: the cheapest form per row
 
 
+@pytest.mark.parametrize("k,n,m", [(15360, 64, 525), (13056, 64, 929), (11136, 320, 579), (16640, 320, 446), (13344, 128, 992), (384, 18624, 205), (128, 23232, 833),
+                                   (160, 39552, 75)])
+def test_gated_prompts_where_192_column_blocks_are_behind(lib, k, n, m):
+    # under a K-split, which they make of many parts, and on a few chunks: 7 - 27 % behind the forms that run
+    f = parse(describe(lib, k, n, m, gated=1))
+    assert f["kernel"] == "k_prefill" and (f["block_cols"] != 192 or f["block_rows"] < (128 if k > 256 else 96)), f["text"]
+
+
 def test_plans_of_lm_head_and_small_shapes(lib):
     lm = parse(describe(lib, 3584, 152064, 1))
     assert lm["kernel"] in ("k_gemv4", "k_gemv4s") and lm["splits"] == 1 and workgroups(lm, 3584, 152064, 1) >= 8 * CUS, lm["text"]
