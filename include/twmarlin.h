@@ -108,7 +108,7 @@ int twm_stream_sync(twm_ctx *ctx, void *hip_stream);
 int twm_ctx_info(twm_ctx *ctx, char *buf, size_t buf_len);
 /* Tuning knobs for per-shape sweeps (the role AutoTuner::tune_gemm plays in
  * crates/kernels/src/autotune.rs:254-396); 0 = library's choice unless noted:
- *   "nt"            column tiles per workgroup of the decode kernels (1, 2, 4)
+ *   "nt"            column tiles per workgroup of the decode kernels (1 .. 4; 5, 6, 8, 10 with "kernel" 5 alone)
  *   "waves"         waves per workgroup of the decode kernels (1, 2, 4, 8, 16; streaming kernel 4 or 8)
  *   "sub"           M <= 4 and the expert kernels: 1 = whole 64-column tiles per workgroup, 16 or 32 = sub-tiles
  *                   of that many columns (with "waves" waves, default 8), 0 = the planner's choice per shape
@@ -116,8 +116,9 @@ int twm_ctx_info(twm_ctx *ctx, char *buf, size_t buf_len);
  *                   (M <= 4 only), 3 = batched-decode streaming kernel (32-row blocks), 4 = batched-decode kernel
  *                   with the activations shared through LDS (32-row blocks; "nt" 1 / 2 = tiles per wave, 4 / 3 =
  *                   two / three column quads per workgroup, "waves" 8 / 16 = two / four k-slices per workgroup),
- *                   5 = the kernels whose waves take k-chunks of their own ("nt" 1, 2, 4 = 16-column tiles per
- *                   workgroup; above 32 rows f16-rounded weights, as the prefill GEMM)
+ *                   5 = the kernels whose waves take k-chunks of their own ("nt" 1 .. 6, 8, 10 = 16-column tiles
+ *                   per workgroup, 9 .. 16 f32 rows up to 8, 17 .. 32 up to 4; above 32 rows 1, 2 and f16-rounded
+ *                   weights, as the prefill GEMM; a larger count takes the largest there is)
  *   "dequant_src"   which repacked copy twm_weight_dequant_f16 unpacks: 0 = 16-column tiles, 1 = column lanes
  *   "tune_on_upload" new weight handles (twm_weight_upload, twm_weight_from_device, twm_weight_fuse_n; not the paired
  *                   gate/up handles) get measured plans at once, as if twm_weight_tune had been called on them: 1 = for

@@ -200,7 +200,7 @@ int twm_ctx_info(twm_ctx *ctx, char *buf, size_t buf_len)
     return TWM_OK;
 }
 
-/* Tuning knobs for sweeps (0 = heuristic): "nt" = tiles per workgroup (1, 2, 4); "waves" = waves per
+/* Tuning knobs for sweeps (0 = heuristic): "nt" = tiles per workgroup; "waves" = waves per
  * workgroup; "kernel" = 2 the one-lane-per-column kernel (M <= 4), 3 the
  * streaming kernel, 4 the batched-decode kernel with LDS-shared activations, 5 the one whose waves take k-chunks of their own;
  * "dequant_src" = which weight copy twm_weight_dequant_f16 unpacks; "prefill_min_m" = smallest M that
@@ -209,7 +209,7 @@ int twm_ctx_set_option(twm_ctx *ctx, const char *key, int value)
 {
     if (!ctx || !key) return api_fail(TWM_INVALID_HANDLE, "twm_ctx_set_option: null argument");
     if (strcmp(key, "nt") == 0) {
-        if (value < 0 || value > 4) return api_fail(TWM_SHAPE_ERROR, "twm_ctx_set_option: nt must be 0 .. 4");
+        if (value < 0 || !nt_option(value)) return api_fail(TWM_SHAPE_ERROR, "twm_ctx_set_option: nt must be 0 .. 6, 8 or 10");
         ctx->force_nt = value;
         return TWM_OK;
     }

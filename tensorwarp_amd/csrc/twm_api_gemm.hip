@@ -258,10 +258,10 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
     const uint32_t n_ld = n_tiles * kTileN, tiles64 = n_ld / 64;
     f.splits = splits;
     WavesPlan wp = {0, 0, 0};
-    if (e.kernel == 5) {  // forced: "nt" 16-column tiles per workgroup (1, 2 or 4), "waves" waves (4 or 8)
-        wp = WavesPlan{e.nt == 1 || e.nt == 2 ? (uint32_t)e.nt : m > 32 ? 2u : 4u, e.waves == 4 ? 4u : 8u, 1};
-        if (wp.waves == 4 && (m <= 32 || wp.nt != 2)) wp.waves = 8;                       // (forms that do not exist: the nearest)
-        if (wp.nt == 4 && (m > 32 || (a_f32 && m > 16))) wp.nt = 2;
+    if (e.kernel == 5) {  // forced: "nt" 16-column tiles per workgroup, "waves" waves (4 or 8); forms that do not exist: the nearest
+        const uint32_t nt = e.nt ? (uint32_t)e.nt : a_f32 && m > 16 ? 2u : 4u;
+        wp = WavesPlan{m > 32 ? (nt < 2 ? nt : 2u) : waves_exact_tiles(nt, m, a_f32), e.waves == 4 ? 4u : 8u, 1};
+        if (wp.waves == 4 && (m <= 32 || wp.nt != 2)) wp.waves = 8;
     } else if (e.kernel == 0 && !e.nt && !e.waves && !e.sub && !splits && !e.prefill_bm && waves_arithmetic_asked_for(e, m)) {
         wp = m <= 32 ? plan_waves_exact(n_tiles, k_chunks, m, a_f32, gated) : plan_waves(n_tiles, k_chunks, m, gated);
         // A handle with the column-lane copy alone keeps the kernels that read that copy where there is one for this shape: a
@@ -622,6 +622,9 @@ static void tune_candidates(uint32_t m, uint32_t k_chunks, bool waves, std::vect
         for (int nt : {1, 2, 4})                                        // waves on k-ranges of their own
             for (int sp : {1, 2, 4})
                 if (nt != 4 || m <= 32) add(5, nt, 0, 0, 0, sp, 0);
+    if (waves && m > 4 && m <= 32)
+        for (int nt : {3, 5, 6, 8, 10})
+            for (int sp : {1, 2}) add(5, nt, 0, 0, 0, sp, 0);
     if (waves && m > 32 && m <= 64) add(5, 2, 4, 0, 0, 1, 0);           // (the four-wave form)
     if (m <= 4) {
     } else if (m <= 32) {

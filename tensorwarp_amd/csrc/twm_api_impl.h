@@ -67,6 +67,8 @@ struct TunedPlan {
     uint8_t valid, kernel, nt, waves, sub, sub_waves, splits, prefill_bm;
 };
 static_assert(sizeof(TunedPlan) == 8, "a tuned plan is eight bytes of the weight blob");
+// the values that option "nt" and a plan's nt take
+inline bool nt_option(int nt) { return nt <= 6 || nt == 8 || nt == 10; }
 constexpr int kTuneBuckets = 12;
 // row counts 1, 2, 3-4, 5-8, 9-16, 17-32, 33-64, 65-128, 129-256, 257-512, 513-1024, above
 inline int tune_bucket(uint32_t m)

@@ -385,7 +385,7 @@ twm_weight *twm_weight_import(twm_ctx *ctx, const void *blob_host, size_t blob_b
     w->paired = hd.paired != 0;
     memcpy(w->tuned, payload + hd.payload_bytes, kBlobTrailer);
     for (TunedPlan &p : w->tuned)   // (a plan is a set of option values: anything outside their ranges is dropped)
-        if (p.valid > 1 || p.kernel > 5 || p.kernel == 1 || p.nt > 4 || p.waves > 16 || p.sub_waves > 16 ||
+        if (p.valid > 1 || p.kernel > 5 || p.kernel == 1 || !nt_option(p.nt) || p.waves > 16 || p.sub_waves > 16 ||
             (p.sub != 0 && p.sub != 1 && p.sub != 16 && p.sub != 32) || (p.prefill_bm != 0 && !prefill_form_known(p.prefill_bm)))
             memset(&p, 0, sizeof p);
     return w;

@@ -175,6 +175,7 @@ struct WavesPlan {
     uint32_t nt, waves, splits;
 };
 WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated);
+uint32_t waves_exact_tiles(uint32_t nt, uint32_t m, bool a_f32);
 WavesPlan plan_waves(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool gated);
 uint32_t waves_block_rows(uint32_t m);  // rows per workgroup
 hipError_t launch_waves_exact(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out, uint32_t nt,

@@ -599,6 +599,14 @@ WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool
     return best;
 }
 
+// The largest count of column tiles up to nt that there is a form of at this row count and type.
+uint32_t waves_exact_tiles(uint32_t nt, uint32_t m, bool a_f32)
+{
+    const uint32_t most = !a_f32 || m <= 8 ? 10u : m <= 16 ? 8u : 4u;
+    if (nt > most) nt = most;
+    return nt == 7 || nt == 9 ? nt - 1u : nt < 1 ? 1u : nt;
+}
+
 // Up to 32 rows.  nt: 16-column tiles per workgroup (1 .. 6, 8, 10 as the form has them; a gated store without a K-split needs an
 // even number).  `scratch` holds the split-K sums; the split factor is cut to what fits.
 hipError_t launch_waves_exact(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out, uint32_t nt,

@@ -1,6 +1,7 @@
 """GPU tests of single kernels at the sizes where their tilings change: against the CPU oracle's f64 dequant-then-matmul or
 its byte-exact format functions, through the C ABI."""
 import ctypes as C
+import re
 import shutil
 from types import SimpleNamespace
 
@@ -223,7 +224,8 @@ def test_waves_on_their_own_k_ranges(dev, m, nt, waves, splits):
         w.free()
 
 
-# column groups of 3, 5, 6, 8 and 10 tiles whose last one is ragged, K one group past whole chunks and fewer chunks than two per
+# Matrices on which the planner takes column groups of several tiles, or a kernel that is ahead there (each form of k_waves_exact
+# by itself: the test behind these): a ragged last group, K one group past whole chunks and fewer chunks than two per
 # wave; one and two row blocks, f16 rows, f32 rows in one block and in two tiles with rows outside the f16 range
 @pytest.mark.parametrize("n", [12001, 17001, 22016, 30016, 40001])
 @pytest.mark.parametrize("m,dtype", [(9, "f16"), (16, "f32"), (20, "f16"), (7, "f32"), (32, "f32")])
@@ -245,7 +247,7 @@ def test_waves_on_many_column_tiles(dev, m, dtype, n):
     w.free()
 
 
-# the gated store of groups of four, six, eight and ten tiles, the last group ragged
+# the gated store of whichever form the planner takes there, the last group ragged
 @pytest.mark.parametrize("ffn", [6176, 10016, 14112, 18464])
 @pytest.mark.parametrize("m,dtype", [(9, "f16"), (13, "f32"), (8, "f32"), (32, "f16")])
 def test_waves_gated_store_on_many_column_tiles(dev, m, dtype, ffn):
@@ -262,6 +264,44 @@ def test_waves_gated_store_on_many_column_tiles(dev, m, dtype, ffn):
     T.gemm_swiglu(dev, w, T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a), m, out)
     close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
     w.free()
+
+
+# Every form of k_waves_exact: one and two row blocks, f16 rows, up to eight f32 rows in one block and more in two tiles; two column
+# groups of which the last has one whole tile and a ragged one, K one group past whole chunks on a wave or two more than once
+@pytest.mark.parametrize("m,dtype,most", [(9, "f16", 10), (17, "f16", 10), (32, "f16", 10), (6, "f32", 10), (13, "f32", 8), (29, "f32", 4)])
+@pytest.mark.parametrize("nt", [1, 2, 3, 4, 5, 6, 8, 10])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_every_form_of_waves_on_exact_weights(dev, m, dtype, most, nt, splits):
+    k, ffn = 1312, 96
+    n = 16 * nt + 21
+    packed, scales, w = weight(dev, k, n, 1601 + nt)
+    gate, up = [(O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (1611, 1613)]
+    pair = [tuple(T.GpuTensor.from_host(dev, x, t) for x, t in zip(p, ("u8", "f16"))) for p in (gate, up)]
+    wgu = T.MarlinWeight.gate_up(dev, *pair, k, ffn)
+    a16 = O.synth_act_f16(m, k, 1615 + m)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k).copy()
+    if dtype == "f32":
+        a[1] *= np.float32(2.0 ** -21)
+        a[2, 128:256] *= np.float32(2.0 ** -30)
+    rows = T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a)
+    c, out = (T.GpuTensor.from_host(dev, np.full((m, x), np.nan, np.float32)) for x in (n, ffn))
+    runs = min(nt, most)
+    dev.set_option("kernel", 5)
+    try:
+        dev.set_option("nt", nt)
+        plans = [dev.plan(k, x, m, dtype=dtype, gated=g) for x, g in ((n, False), (2 * ffn, True))]
+        T.gemm(dev, w, rows, m, c, splits)
+        T.gemm_swiglu(dev, wgu, rows, m, out, splits)
+    finally:
+        dev.set_option("nt", 0)
+        dev.set_option("kernel", 0)
+    assert re.match(r"k_waves_exact: \d+-row x %d-column" % (16 * runs), plans[0]), plans
+    assert re.match(r"k_waves_exact: \d+-row x %d-column" % (16 * (runs + runs % 2)), plans[1]), plans
+    close_rows(c.to_host(), O.gemm_f64(a, packed, scales, m, k, n), F32_SUM)
+    g, u = (O.gemm_f64(a, *x, m, k, ffn) for x in (gate, up))
+    close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
+    w.free()
+    wgu.free()
 
 
 # few features of a deep matrix: K in ranges whose sums the reduction gates
