@@ -517,6 +517,13 @@ hipError_t init_waves_exact()
 // * vocabularies (more than 4096 tiles) stay with the forms whose workgroups are short-lived, except up to eight f32 rows
 //   (3584 -> 152064 at 8 f16 rows 66 / 54, at 32 92 / 78, at 8 f32 rows 73 / 82), as do wide matrices of up to eight chunks
 //   (896 -> 32000 at 16 rows 8.1 / 6.5);
+// * so do f16 rows from where ten tiles each are more than one round of workgroups, 2560 tiles, at 9 .. 16 rows 2816 (2592 -> 51736
+//   at 28 rows 35.6 / 25.2, 3840 -> 52422 at 17 38.0 / 32.7, 2496 -> 64331 at 10 24.0 / 19.4, 2592 -> 2 x 28832 at 5 23.5 / 18.9), and
+//   f32 rows on a K that is shallow for it: up to eight rows four chunks, sixteen from 3840 tiles on (22 and 32 of them where the
+//   last round of ten-tile groups is the emptiest, eight between 8000 and 9000 tiles, where the other form's is: 12 chunks 0.78 of its
+//   time; 64 -> 84583 at 6 rows 19.2 / 10.2, 1184 -> 63459 at 8 18.6 / 17.0, 2080 -> 2 x 52384 at 6 39.1 / 36.1, 2400 -> 82295 at 5
+//   42.4 / 36.9), nine and more 5 .. 9 chunks, to 18 from 2700 tiles on, to 31 from 3328 (576 -> 2 x 24608 at 10 rows 13.5 / 12.4,
+//   1984 -> 59058 at 12 24.6 / 23.0);
 // * 17 .. 32 f32 rows end at the four tiles their registers allow (1856 -> 2 x 9312 at 32 rows 20.9 / 17.3; 1024 tiles and
 //   fewer are 5 - 50 % ahead) and at K of about 20000, 12800 above 340 tiles (17536 -> 5504 at 25 rows 36.5 / 31.6), 8192 above
 //   680 and 5120 on 513 .. 680, whose groups of three leave the CUs 70 - 85 % full (28672 -> 8192 64 / 55, 8064 -> 9792 at 23
@@ -527,8 +534,9 @@ hipError_t init_waves_exact()
 //   K of 16 .. 32 chunks on 257 .. 512 tiles (3584 -> 4608 5.9 / 5.6), and up to six rows, seven up to K = 4096, every K from
 //   2200 on with up to 256 tiles (3584 -> 3584 at 5 rows 5.2 / 4.6), gated 2048 .. 4096 at eight rows too, where pairs of tiles
 //   are half as many workgroups (3072 -> 2 x 96 at 8 rows 4.75 / 4.24);
-// * f16, deep K on 129 .. 256 tiles: from 72 chunks on up to sixteen rows (12192 -> 3584 at 8 rows 11.0 / 10.0), up to 320 tiles
-//   from 67 on (9216 -> 4352 at 11 rows 10.9 / 9.8), from 65 on above (17824 -> 3584 at 17 rows 16.8 / 15.6); f16 on a few
+// * f16, deep K on 129 .. 256 tiles: from 72 chunks on up to sixteen rows (12192 -> 3584 at 8 rows 11.0 / 10.0), up to 340 tiles
+//   from 67 on (9216 -> 4352 at 11 rows 10.9 / 9.8, 13600 -> 2 x 2720 at 7 14.4 / 12.9), from 65 on above (17824 -> 3584 at 17 rows
+//   16.8 / 15.6), gated from 61 on with 321 .. 400 tiles (10848 -> 2 x 2848 at 31 rows 20.0 / 17.9); f16 on a few
 //   chunks: four on 513 tiles and more (256 -> 14049 at 10 rows 4.0 / 3.75), nine to sixteen on 701 .. 1000 (1600 -> 2 x 6560 at
 //   11 rows 6.75 / 6.5, 1600 -> 14798 at 30 9.6 / 8.9), up to eighteen above 1600, 1536 up to sixteen rows and 1300 up to eight
 //   (those up to ten): a wave has one to three chunks, unevenly, on seven to ten tiles (1152 -> 33728 at 19 rows 13.1 / 11.0, 1664
@@ -550,12 +558,21 @@ WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool
     if (m < 5 || m > 32) return none;
     const bool few_f32 = a_f32 && m <= 8;
     if (n_tiles > 4096 && !few_f32) return none;
+    if (few_f32 && n_tiles > 3840) {
+        const uint32_t from = n_tiles > 8000 && n_tiles <= 9000 ? 8u : n_tiles > 5120 && n_tiles <= 5400 ? 32u : n_tiles > 6000 && n_tiles <= 7000 ? 22u : 16u;
+        if (k_chunks <= from) return none;
+    }
     if (a_f32) {
+        if (few_f32 && n_tiles > 2560 && k_chunks <= 4) return none;
+        if (!few_f32 && ((n_tiles > 2560 && k_chunks >= 5 && k_chunks <= 9) || (n_tiles > 2700 && k_chunks >= 10 && k_chunks <= 18) ||
+                         (n_tiles > 3328 && k_chunks >= 19 && k_chunks <= 31))) return none;
         if (m > 16 && (n_tiles > 1024 || k_chunks > (n_tiles > 680 ? 64u : n_tiles > 512 ? 40u : n_tiles > 340 ? 100u : 160u))) return none;
         if (m > 8 && n_tiles > 2048 && k_chunks <= 3) return none;
     } else {
+        if (n_tiles > (m <= 8 || m > 16 ? 2560u : 2816u)) return none;
         if (k_chunks <= 8 && n_tiles > (k_chunks <= 4 ? 512u : 1024u)) return none;
-        if (n_tiles > 128 && n_tiles <= (m <= 16 ? 320u : 256u) && k_chunks > (m > 16 ? 64u : n_tiles > 256 ? 66u : 71u)) return none;
+        if (n_tiles > 128 && n_tiles <= (m <= 16 ? 340u : 256u) && k_chunks > (m > 16 ? 64u : n_tiles > 256 ? 66u : 71u)) return none;
+        if (gated && m > 16 && n_tiles > 320 && n_tiles <= 400 && k_chunks > 60) return none;
         if (n_tiles > 700 && n_tiles <= 1000 && k_chunks > 8 && k_chunks <= 16) return none;
         if (n_tiles > 1800 && n_tiles <= 2048) return none;
         if (n_tiles > (m <= 8 && k_chunks <= 10 ? 1300u : m <= 16 ? 1536u : 1600u) && k_chunks <= 18) return none;

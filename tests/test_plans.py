@@ -213,11 +213,21 @@ def test_plans_of_the_few_row_kernels(lib):
 
 @pytest.mark.parametrize("k,n,m,dtype,gated", [(1152, 33728, 19, "f16", 0), (1664, 24966, 9, "f16", 0), (1152, 38272, 9, "f16", 0), (1792, 26560, 14, "f16", 0),
                                                (128, 39553, 16, "f32", 0), (17536, 5504, 25, "f32", 0), (8064, 9792, 23, "f32", 0),
-                                               (7296, 10560, 27, "f32", 1), (3072, 192, 8, "f16", 1), (9216, 4352, 11, "f16", 0)])
+                                               (7296, 10560, 27, "f32", 1), (3072, 192, 8, "f16", 1), (9216, 4352, 11, "f16", 0), (13600, 5440, 7, "f16", 1), (10848, 5696, 31, "f16", 1),
+                                               (2592, 51736, 28, "f16", 0), (3840, 52422, 17, "f16", 0), (2496, 64331, 10, "f16", 0), (2592, 57664, 5, "f16", 1),
+                                               (64, 84583, 6, "f32", 0), (2400, 82295, 5, "f32", 0), (2080, 104768, 6, "f32", 1), (896, 98304, 8, "f32", 0), (576, 49216, 10, "f32", 1), (1984, 59058, 12, "f32", 0)])
 def test_shapes_on_which_the_other_kernels_stay_ahead(lib, k, n, m, dtype, gated):
-    # uneven chunks on many tiles, groups that leave CUs idle, gated pairs on few columns: measured 8 - 19 % slower on k_waves_exact
+    # uneven chunks on many tiles, groups that leave CUs idle, gated pairs on few columns: measured 8 - 19 % slower on k_waves_exact;
+    # more tiles than one round of workgroups takes: 7 - 90 %
     f = parse(describe(lib, k, n, m, _lib.F32 if dtype == "f32" else _lib.F16, gated))
     assert f["kernel"] != "k_waves_exact", f["text"]
+
+
+@pytest.mark.parametrize("k,n,m,dtype,gated", [(2592, 37888, 28, "f16", 0), (3584, 37888, 8, "f16", 1), (4096, 22016, 13, "f32", 1), (3584, 152064, 8, "f32", 0)])
+def test_wide_shapes_that_one_round_of_workgroups_covers(lib, k, n, m, dtype, gated):
+    # (or, with up to eight f32 rows, a K deep enough that the other forms' conversion launch costs more)
+    f = parse(describe(lib, k, n, m, _lib.F32 if dtype == "f32" else _lib.F16, gated))
+    assert f["kernel"] == "k_waves_exact", f["text"]
 
 
 @pytest.mark.parametrize("k,n,m,dtype,gated,split", [(3072, 128, 25, "f16", 0, False), (3584, 467, 24, "f16", 0, False), (2336, 1216, 5, "f32", 1, False),
