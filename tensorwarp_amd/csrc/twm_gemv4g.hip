@@ -177,6 +177,11 @@ __global__ __launch_bounds__(1024) void k_gemv4g(const char *__restrict__ cw, co
 //   4.88; 3584 -> 2 x 18944 16.3 / 16.0; gated at four rows 2240 -> 2 x 7776 7.25 / 6.55).
 // * f32, one row: every lane splits a piece of its own for each group, four times what k_gemv4s's lanes do: K up to 1536 on 200
 //   column tiles (896 -> 151936 18.4 / 15.5, 2048 -> 2048 level), gated up to 3072 on 64 (2816 -> 2 x 704 3.54 / 3.88; 1472 -> 2 x 6048 4.97 / 4.79).
+//   On 150 column tiles and more the waves take two to four chunks; where those do not come out even many tiles stay with the other
+//   forms: two chunks gated (256 -> 2 x 7328 at three rows 3.68 / 3.34, 544 -> 2 x 14048 at one 5.24 / 4.59), five to seven (544 ->
+//   2 x 12544 at four rows 5.49 / 4.95, 576 -> 28479 at one 4.96 / 4.50), nine and thirteen to fifteen at one row (1088 -> 26584
+//   6.08 / 5.66, 1600 -> 30792 7.61 / 7.13); gated at two rows from nine chunks on (1088 -> 2 x 16352 7.69 / 6.86, 2048 -> 2 x 11136
+//   7.42 / 6.91).
 // One chunk per wave up to eleven of them on 150 column tiles, else up to four (4096 -> 4096 on 8 / 16 waves 3.58 / 3.62, 1536 ->
 // 12288 on 4 / 12 3.87 / 4.9; 3072 -> 5120 on 8 / 6 4.04 / 4.23), from 25 chunks on on an even number of waves; f32 one chunk up
 // to sixteen, then two.
@@ -190,6 +195,11 @@ uint32_t plan_gemv4g(uint32_t tiles64, uint32_t k_chunks, uint32_t m, bool a_f32
     const uint32_t deep = m == 1 ? 24u : m == 2 ? 21u : 20u, wide = m <= 2 ? 512u : 400u;
     if (gated && m >= 2 && k_chunks > (m == 2 ? 20u : 16u) && tiles64 > (m == 2 ? 256u : 200u)) return 0;
     if (!(k_chunks <= deep && tiles64 <= wide) && !(k_chunks <= 64 && tiles64 <= 64)) return 0;
+    if (k_chunks == 2 && tiles64 > (gated ? (m >= 3 ? 150u : m == 2 ? 400u : 330u) : m == 1 ? 440u : 512u)) return 0;
+    if (k_chunks == 5 && tiles64 > (gated ? (m >= 3 ? 150u : m == 2 ? 300u : 200u) : m == 1 ? 340u : 360u)) return 0;
+    if ((k_chunks == 6 || k_chunks == 7) && tiles64 > 340 && (gated || m == 1)) return 0;
+    if (gated && m == 2 && k_chunks >= 9 && tiles64 > 340) return 0;
+    if (m == 1 && ((k_chunks == 9 && tiles64 > (gated ? 260u : 320u)) || (k_chunks >= 13 && k_chunks <= 15 && tiles64 > (gated ? 320u : 430u)))) return 0;
     if (k_chunks <= 11 && tiles64 <= 150) return k_chunks;
     if (k_chunks > 24) return ((k_chunks + 3) / 4 + 1u) & ~1u;
     // three or four chunks per wave, whichever leaves fewer replayed; two where both leave several

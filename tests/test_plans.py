@@ -230,6 +230,15 @@ def test_wide_shapes_that_one_round_of_workgroups_covers(lib, k, n, m, dtype, ga
     assert f["kernel"] == "k_waves_exact", f["text"]
 
 
+@pytest.mark.parametrize("k,n,m,gated,group_lane", [(256, 14656, 3, 1, False), (544, 28096, 1, 1, False), (544, 25088, 4, 1, False), (576, 28479, 1, 0, False),
+                                                    (1088, 26584, 1, 0, False), (1152, 30080, 2, 1, False), (1600, 30792, 1, 0, False),
+                                                    (256, 14656, 3, 0, True), (384, 28096, 1, 1, True), (1024, 25088, 4, 1, True), (896, 1152, 1, 0, True)])
+def test_chunks_that_do_not_come_out_even_on_many_tiles(lib, k, n, m, gated, group_lane):
+    # where a wave of k_gemv4g has two to four chunks: 7 - 14 % behind the other kernels of up to four rows, or ahead of them
+    f = parse(describe(lib, k, n, m, gated=gated))
+    assert (f["kernel"] == "k_gemv4g") == group_lane, f["text"]
+
+
 @pytest.mark.parametrize("k,n,m,dtype,gated,split", [(3072, 128, 25, "f16", 0, False), (3584, 467, 24, "f16", 0, False), (2336, 1216, 5, "f32", 1, False),
                                                      (3712, 448, 11, "f32", 0, True), (4096, 128, 25, "f16", 0, True)])
 def test_a_shallow_matrix_is_not_split(lib, k, n, m, dtype, gated, split):
