@@ -436,7 +436,7 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
     switch (f.kind) {
     case kFormPrefill: {
         uint32_t bm = 0, sp = 0;
-        prefill_plan_of(m, 0, 0, n_tiles, k_chunks, e.ws_bytes, gated != 0, &bm, &sp);
+        prefill_plan_of(m, 0, 0, n_tiles, k_chunks, e.ws_bytes, gated != 0, n % 4 == 0, &bm, &sp);
         snprintf(text, bytes, "k_prefill: %u-row x %u-column blocks, %u K-split%s%s; 16-column tile copy", (bm & 1u) ? bm - 1u : bm == 66 || bm == 98 ? bm - 2u : bm == 64 ? 64u : 128u,
                  (bm & 1u) ? 128u : bm == 192 || bm == 66 || bm == 98 ? 192u : 256u, sp, sp == 1 ? "" : "s", sp > 1 ? " + k_splitk_reduce" : "");
         break;

@@ -670,6 +670,10 @@ hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutS
 // 128 x 192 gated not under a K-split, which it makes of many parts (13056 -> 2 x 32 at 929 rows 18.2 us on 17 parts of 64 x 256
 // blocks, 22.0 on 26 of these), and not on up to three chunks, 96 x 192 on two, where the gate's way through LDS is the launch
 // (128 -> 2 x 11616 at 833 rows 64 x 256 23.2, 128 x 192 24.8, 96 x 192 27.9).
+// 64 and 96 x 192 not in place of unsplit 48 x 128 where their store is the longer one: rows that are no whole 16-byte places
+// (832 -> 19155 at 107 rows 16.4 us, 48 x 128 14.3; 1056 -> 19537 at 110 18.7 / 17.2), and the 64-row gate up to twelve chunks (1248
+// -> 2 x 8672 at 120 rows 16.6 / 15.5); 96 x 192 not in K-splits of under six chunks, gated seven, whose fill and sum cost more than
+// the model has (2336 -> 2 x 5504 at 86 rows 20.5 on four splits, 48 x 128 unsplit 16.7; 5856 -> 2 x 2816 at 73 19.5 / 18.1).
 constexpr double kPf192 = 0.80, kPf192Gated = 1.07;
 constexpr uint32_t kNarrowMaxRows = 256, kNarrowMinTiles = 128, kMiddleMaxRows = 1024;
 static const struct { uint32_t form; double chunk[2]; } kMiddle[] = {{66, {0.94, 1.62}}, {98, {1.17, 2.10}}};
@@ -680,7 +684,7 @@ struct PrefillPlan {
     double us;
 };
 static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t force_splits, uint32_t n_tiles, uint32_t k_chunks,
-                                bool gated)
+                                bool gated, bool quads)
 {
     PrefillPlan best = {force_rows ? force_rows : 64u, force_splits ? force_splits : 1u, 1e30};
     const size_t n_ld = (size_t)n_tiles * 16;
@@ -710,6 +714,8 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
         for (uint32_t i = 0; i < n_cuts; i++) {
             const uint32_t sp = cuts[i].splits, cps = cuts[i].chunks;
             if (gated && !force_rows && ((bm == 192 && (sp > 1 || k_chunks <= 3)) || (bm == 98 && k_chunks <= 2))) continue;
+            if (middle && !force_rows && best.block_rows == 49 && best.splits == 1 && sp == 1 && (gated ? bm == 66 && k_chunks <= 12 : !quads)) continue;
+            if (bm == 98 && !force_rows && !force_splits && sp > 1 && cps < (gated ? 7u : 6u)) continue;
             if (!force_splits && sp > 1 && 5.5 + sp * partial_us >= best.us) break;  // (the sum kernel alone takes longer)
             const double total = wgs * sp;
             double t = 0.0;
@@ -749,10 +755,10 @@ static PrefillPlan plan_prefill(uint32_t rows, uint32_t force_rows, uint32_t for
 
 // The plan within what the scratch can hold of partial sums (ws_bytes = 0: no scratch, unsplit).
 static PrefillPlan plan_prefill_within(uint32_t rows, uint32_t block_rows, uint32_t splits, uint32_t n_tiles, uint32_t k_chunks,
-                                       size_t ws_bytes, bool gated)
+                                       size_t ws_bytes, bool gated, bool quads)
 {
     const size_t n_ld = (size_t)n_tiles * 16;
-    PrefillPlan plan = plan_prefill(rows, block_rows, splits, n_tiles, k_chunks, gated);
+    PrefillPlan plan = plan_prefill(rows, block_rows, splits, n_tiles, k_chunks, gated, quads);
     const size_t per_split = (size_t)rows * n_ld * 4;
     if (plan.splits > 1 && (ws_bytes == 0 || per_split == 0 || plan.splits > ws_bytes / per_split)) {
         // the scratch cannot hold that many partial sums: plan again within what it holds (at least unsplit)
@@ -762,7 +768,7 @@ static PrefillPlan plan_prefill_within(uint32_t rows, uint32_t block_rows, uint3
         else {
             PrefillPlan capped = {0, 0, 1e30};
             for (uint32_t sp = 1; sp <= cap; sp++) {
-                PrefillPlan c = plan_prefill(rows, block_rows, sp, n_tiles, k_chunks, gated);
+                PrefillPlan c = plan_prefill(rows, block_rows, sp, n_tiles, k_chunks, gated, quads);
                 if (c.us < capped.us) capped = c;
             }
             plan = capped;
@@ -772,9 +778,9 @@ static PrefillPlan plan_prefill_within(uint32_t rows, uint32_t block_rows, uint3
 }
 
 void prefill_plan_of(uint32_t rows, uint32_t block_rows, uint32_t splits, uint32_t n_tiles, uint32_t k_chunks, size_t ws_bytes,
-                     bool gated, uint32_t *block_rows_out, uint32_t *splits_out)
+                     bool gated, bool quads, uint32_t *block_rows_out, uint32_t *splits_out)
 {
-    const PrefillPlan plan = plan_prefill_within(rows, block_rows, splits, n_tiles, k_chunks, ws_bytes, gated);
+    const PrefillPlan plan = plan_prefill_within(rows, block_rows, splits, n_tiles, k_chunks, ws_bytes, gated, quads);
     *block_rows_out = plan.block_rows;
     *splits_out = plan.splits;
 }
@@ -857,7 +863,7 @@ hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, boo
     if (block_rows != 0 && !prefill_form_known(block_rows)) return hipErrorInvalidValue;
     uint32_t ran_splits = 1;  // of the last run
     auto run = [&](const _Float16 *a16, uint32_t rows, const OutSpec &o, void *ws, size_t ws_bytes, bool via = false) {
-        const PrefillPlan plan = plan_prefill_within(rows, block_rows, splits, w.n_tiles, w.k_chunks, ws ? ws_bytes : 0, o.swiglu != nullptr);
+        const PrefillPlan plan = plan_prefill_within(rows, block_rows, splits, w.n_tiles, w.k_chunks, ws ? ws_bytes : 0, o.swiglu != nullptr, row_store_of(o, w.n) != kRowsNone);
         const uint32_t cps = (w.k_chunks + plan.splits - 1) / plan.splits;
         ran_splits = (w.k_chunks + cps - 1) / cps;
         switch (plan.block_rows) {

@@ -239,6 +239,14 @@ def test_chunks_that_do_not_come_out_even_on_many_tiles(lib, k, n, m, gated, gro
     assert (f["kernel"] == "k_gemv4g") == group_lane, f["text"]
 
 
+@pytest.mark.parametrize("k,n,m,dtype,gated", [(832, 19155, 107, "f16", 0), (768, 12111, 210, "f32", 0), (1056, 19537, 110, "f16", 0), (1248, 17344, 120, "f16", 1),
+                                               (2336, 11008, 86, "f16", 1), (5856, 5632, 73, "f16", 1), (2528, 11456, 75, "f32", 1)])
+def test_prompts_that_stay_off_low_blocks_of_192_columns(lib, k, n, m, dtype, gated):
+    # rows that are no whole 16-byte places, the 64-row gate on up to twelve chunks, and K-splits of a few chunks: 5 - 23 % behind
+    f = parse(describe(lib, k, n, m, _lib.F32 if dtype == "f32" else _lib.F16, gated))
+    assert f["kernel"] == "k_prefill" and f["block_cols"] != 192, f["text"]
+
+
 @pytest.mark.parametrize("k,n,m,dtype,gated,split", [(3072, 128, 25, "f16", 0, False), (3584, 467, 24, "f16", 0, False), (2336, 1216, 5, "f32", 1, False),
                                                      (3712, 448, 11, "f32", 0, True), (4096, 128, 25, "f16", 0, True)])
 def test_a_shallow_matrix_is_not_split(lib, k, n, m, dtype, gated, split):
