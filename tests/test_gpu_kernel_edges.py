@@ -443,6 +443,25 @@ def test_saved_plans_of_every_kernel_come_back(dev):
     w.free()
 
 
+@pytest.mark.parametrize("nt,taken", [(5, True), (10, True), (7, False), (9, False), (11, False)])
+def test_column_tile_counts_of_saved_plans_and_of_the_option(dev, nt, taken):
+    w = weight(dev, 256, 128, 1711)[2]
+    blob = w.export_blob()
+    blob[-96 + 8 * 5:-96 + 8 * 6] = np.array([1, 5, nt, 0, 0, 0, 1, 0], np.uint8)
+    back = T.MarlinWeight.import_blob(dev, blob)
+    assert (back.tuned_plan(20) is not None) == taken
+    try:
+        if taken:
+            dev.set_option("nt", nt)
+        else:
+            with pytest.raises(T.DeviceError):
+                dev.set_option("nt", nt)
+    finally:
+        dev.set_option("nt", 0)
+    back.free()
+    w.free()
+
+
 # 48 .. 128-row blocks of 128 columns: a block's last row and the next one's first, K of one group, of two chunks and of an
 # odd number with a ragged end, N ragged below and above a block; K-split and plain stores, f16 rows and scaled f32 rows
 @pytest.mark.parametrize("form", [49, 65, 97, 129])
