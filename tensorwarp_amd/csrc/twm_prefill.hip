@@ -505,82 +505,6 @@ __global__ __launch_bounds__(256) TWM_PF_OCC(MT == 4) void k_prefill192(const ui
     prefill_block<MT, 3, false, 3, STORE>(qw, sc, a_any, out, m_rows, k, n, n_tiles, k_chunks, chunks_per_split, partials, row_store, col_blocks, row_blocks);
 }
 
-// The partial sums of one place, added in split order (deterministic): four loads in flight at a time.
-__device__ __forceinline__ float4v splitk_sum(const float4v *src, size_t stride4, uint32_t splits)
-{
-    float4v s = src[0];
-    uint32_t z = 1;
-    for (; z + 4u <= splits; z += 4u) {
-        float4v v[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = src[(z + j) * stride4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) s += v[j];
-    }
-    if (z + 2u <= splits) {
-        const float4v v = src[z * stride4], w = src[(z + 1u) * stride4];
-        s += v;
-        s += w;
-        z += 2u;
-    }
-    if (z < splits) s += src[z * stride4];
-    return s;
-}
-
-// out[row][col] = sum over splits of partials[split][row][col], one thread per four padded columns.  Bound: latency.  (A
-// loop of one load and one add per turn waited for memory once per split: nine splits of 96 x 3584 took 6.6 us in a kernel
-// trace, now 4.8, of which most is the launch; four splits of 32 x 3584 5.0 and 4.8.)
-template <RowStore ROWS>
-__global__ __launch_bounds__(256) void k_splitk_reduce(const float *__restrict__ partials, OutSpec out, uint32_t m_rows, uint32_t n,
-                                                         uint32_t n_ld, uint32_t splits)
-{
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t quads = n_ld / 4;
-    if (idx >= (size_t)m_rows * quads) return;
-    const uint32_t row = (uint32_t)(idx / quads), col = (uint32_t)(idx % quads) * 4u;
-    uint32_t ld = 0;
-    float4v bias = {0.f, 0.f, 0.f, 0.f};
-    float *dst = nullptr;
-    if (ROWS == kRowsSegments && col < n) dst = pf_quad_of(out, col, ld, bias);   // (the bias is on its way during the sum)
-    float4v s = splitk_sum((const float4v *)(partials + (size_t)row * n_ld + col), (size_t)m_rows * n_ld / 4, splits);
-    if (out.row_scale) s *= out.row_scale[row];  // (f32 rows scaled into the f16 range)
-    if constexpr (ROWS == kRowsPlain) {
-        if (col < n) *(float4v *)(out.seg[0].ptr + (size_t)row * n + col) = s;
-        return;
-    }
-    if constexpr (ROWS == kRowsSegments) {
-        if (out.seg[0].bias) s += bias;
-        if (dst) *(float4v *)(dst + (size_t)row * ld) = s;
-        return;
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < 4; j++)
-        if (col + j < n) pf_store_out(out, row, col + j, s[j]);
-}
-
-// The same sum for a paired gate/up weight: one thread per four features adds the gate and the up partials
-// (32 columns apart) in split order and stores silu(gate) * up.
-__global__ __launch_bounds__(256) void k_splitk_reduce_swiglu(const float *__restrict__ partials, float *__restrict__ gate_out,
-                                                                uint32_t m_rows, uint32_t ffn, uint32_t n_ld, uint32_t splits,
-                                                                uint32_t act, const float *__restrict__ row_scale)
-{
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t quads = ffn / 4;  // ffn is a multiple of 32
-    if (idx >= (size_t)m_rows * quads) return;
-    const uint32_t row = (uint32_t)(idx / quads), feat = (uint32_t)(idx % quads) * 4u;
-    const float4v *src = (const float4v *)(partials + (size_t)row * n_ld + paired_col(feat));
-    const size_t stride4 = (size_t)m_rows * n_ld / 4;
-    float4v g = splitk_sum(src, stride4, splits), u = splitk_sum(src + kPairWidth / 4, stride4, splits);
-    if (row_scale) {  // (f32 rows scaled into the f16 range)
-        g *= row_scale[row];
-        u *= row_scale[row];
-    }
-    float4v o;
-#pragma unroll
-    for (int j = 0; j < 4; j++) o[j] = gated_mul(act, g[j], u[j]);
-    *(float4v *)(gate_out + (size_t)row * ffn + feat) = o;
-}
-
 // out[row][:] *= row_scale[row] over every segment, for the rows whose factor is not 1.  Rows that need nothing are the
 // rule: a workgroup looks at the factors of kScaleRows rows with one load and usually ends there (2048 x 4096 without a factor,
 // in a kernel trace: 5.0 us in the median and 1.2 at least on 64 x 8 workgroups, 4.9 and 3.9 on one per row).
@@ -598,43 +522,6 @@ __global__ __launch_bounds__(256) void k_scale_rows(OutSpec out, const float *__
             for (uint32_t c = blockIdx.y * 256u + threadIdx.x; c < out.seg[sg].width; c += 256u * kScaleParts) p[c] *= rs;
         }
     }
-}
-
-// How rows are stored: kRowsPlain where the output is one [M, N] matrix without a bias, kRowsSegments where every four columns
-// are 16 aligned bytes of one segment and all segments have a bias or none (4096 -> 12288 split into three at 512 rows 57.5 ->
-// 50.9 us, at 2048 190.5 -> 179.5 against 4-byte stores; with K-splits 3584 -> 3584 + 2 * 512 with biases at 512 rows 34.4 ->
-// 31.4 us).
-static uint32_t row_store_of(const OutSpec &out, uint32_t n)
-{
-    for (uint32_t i = 0; i < out.count; i++)
-        if (out.seg[i].start % 4 != 0 || out.seg[i].width % 4 != 0 || ((uintptr_t)out.seg[i].ptr & 15) != 0 || !out.seg[i].bias != !out.seg[0].bias)
-            return kRowsNone;
-    if (out.count == 0) return kRowsNone;
-    return out.count == 1 && out.seg[0].start == 0 && out.seg[0].width == n && !out.seg[0].bias ? kRowsPlain : kRowsSegments;
-}
-
-hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutSpec &out, uint32_t m, uint32_t n,
-                                uint32_t n_ld, uint32_t splits)
-{
-    size_t quads = (size_t)m * n_ld / 4;
-    if (quads == 0) return hipSuccess;
-    // few places: one wave per workgroup, so that they spread over the CUs
-    auto block_of = [](size_t threads) { return threads < 256u * 256u ? 64u : 256u; };
-    if (out.swiglu) {
-        if (n % (2 * kPairWidth) != 0) return hipErrorInvalidValue;
-        const size_t fq = (size_t)m * (n / 2) / 4;
-        const unsigned block = block_of(fq);
-        hipLaunchKernelGGL(k_splitk_reduce_swiglu, dim3((unsigned)((fq + block - 1) / block)), dim3(block), 0, s, partials, out.swiglu, m,
-                           n / 2, n_ld, splits, out.gate_act, out.row_scale);
-        return hipGetLastError();
-    }
-    const uint32_t rows = row_store_of(out, n);
-    auto kernel = rows == kRowsPlain      ? k_splitk_reduce<kRowsPlain>
-                  : rows == kRowsSegments ? k_splitk_reduce<kRowsSegments>
-                                          : k_splitk_reduce<kRowsNone>;
-    const unsigned block = block_of(quads);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((quads + block - 1) / block)), dim3(block), 0, s, partials, out, m, n, n_ld, splits);
-    return hipGetLastError();
 }
 
 // Block form and split-K factor by a small cost model fitted to per-shape sweeps on MI355X (microseconds per

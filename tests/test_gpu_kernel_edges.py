@@ -186,6 +186,24 @@ def test_split_sums_of_every_count(dev, m, n, splits):
     w.free()
 
 
+@pytest.mark.parametrize("m,splits", [(24, 10), (24, 18), (40, 17), (65576, 2)])
+def test_split_sums_past_eight_in_flight_and_past_the_rows_of_a_grid(dev, m, splits):
+    # the sum kernel has eight loads in flight behind the first; more than 65535 rows are two launches
+    k, n = splits * 128, 72
+    packed, scales, w = weight(dev, k, n, 930 + splits)
+    a16 = O.synth_act_f16(m, k, 931 + splits)
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    dev.set_option("kernel", 4 if m <= 32 else 0)
+    try:
+        T.gemm(dev, w, T.GpuTensor.from_host(dev, a16, "f16"), m, c, splits)
+    finally:
+        dev.set_option("kernel", 0)
+    truth = gemm_truth(a16.view(np.float16).astype(np.float32).reshape(m, k), packed, scales, m, k, n)
+    err = np.abs(c.to_host() - truth) / np.maximum(np.abs(truth), 1e-3 * np.abs(truth).max(1, keepdims=True))
+    assert err.max() < (F32_SUM if m <= 32 else 1e-3)     # (NaN where a row was not stored)
+    w.free()
+
+
 def gemm_truth(a, packed, scales, m, k, n):
     """Exact weights up to 32 rows, the FP16 Q4 unpack above (the library's default arithmetic), f64 sums."""
     if m <= 32:
