@@ -7,7 +7,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libtwmarlin_hip.so")
-SOURCES = ["twm_kernels.hip", "twm_gemv4.hip", "twm_gemv4s.hip", "twm_gemv4g.hip", "twm_moe.hip", "twm_stream.hip", "twm_batch.hip", "twm_waves.hip", "twm_waves_exact.hip", "twm_splitk.hip", "twm_prefill.hip", "twm_debug_mix.hip", "twm_noalloc.hip", "twm_api.hip",
+SOURCES = ["twm_kernels.hip", "twm_gemv4.hip", "twm_gemv4s.hip", "twm_gemv4g.hip", "twm_moe.hip", "twm_stream.hip", "twm_batch.hip", "twm_waves.hip", "twm_waves_exact.hip", "twm_batch_range.hip", "twm_splitk.hip", "twm_prefill.hip", "twm_debug_mix.hip", "twm_noalloc.hip", "twm_api.hip",
            "twm_api_weights.hip", "twm_api_gemm.hip", "twm_api_moe.hip"]
 # The batched-decode kernels read every MFMA result with vector instructions right away (scale, add):
 # with the default choice the results land in AGPRs and each costs a v_accvgpr_read first.
@@ -16,6 +16,7 @@ PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 PER_FILE_FLAGS = {"twm_gemv4s.hip": PRELOAD, "twm_splitk.hip": PRELOAD, "twm_gemv4g.hip": PRELOAD, "twm_gemv4.hip": PRELOAD, "twm_moe.hip": PRELOAD, "twm_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] + PRELOAD,
                   "twm_batch.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] + PRELOAD,
                   "twm_waves_exact.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] + PRELOAD,
+                  "twm_batch_range.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] + PRELOAD,
                   "twm_waves.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] + PRELOAD}
 # -packed-fp32-ops off: v_pk_{add,mul,fma}_f32 are not to be generated on this hardware pool.
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",

@@ -86,7 +86,7 @@ twm_ctx *twm_ctx_create(int ordinal)
         return nullptr;
     }
     ok = ok && hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking) == hipSuccess;
-    ok = ok && init_prefill() == hipSuccess && init_waves() == hipSuccess && init_waves_exact() == hipSuccess;
+    ok = ok && init_prefill() == hipSuccess && init_waves() == hipSuccess && init_waves_exact() == hipSuccess && init_batch_range() == hipSuccess;
     ok = ok && noalloc_scratch_for_current_device("twm_ctx_create") != nullptr;
     c->stream = c->own_stream;
     c->ws_bytes = kWsBytes;

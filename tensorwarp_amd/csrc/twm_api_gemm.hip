@@ -218,7 +218,7 @@ static BatchPlan plan_batch(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, boo
 
 // ---- the launch form of a GEMM: chosen in one place, launched in another ---------------------------------
 // What twm_gemm will run for a weight's shape, a row count and the context's knobs.  Nothing here touches the device.
-enum FormKind { kFormPrefill = 0, kFormSubTile = 1, kFormWholeTile = 2, kFormBatch = 3, kFormStream = 4, kFormNone = 5, kFormWaves = 6, kFormGroupLane = 7 };
+enum FormKind { kFormPrefill = 0, kFormSubTile = 1, kFormWholeTile = 2, kFormBatch = 3, kFormStream = 4, kFormNone = 5, kFormWaves = 6, kFormGroupLane = 7, kFormBatchRange = 8 };
 struct LaunchForm {
     int kind;
     int copy;                 // the repacked order it reads (kCopyTile / kCopyCol)
@@ -268,6 +268,12 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
         // little slower (3584 -> 3584 at 16 rows 7.4 us, k_waves_exact 5.4), but the tile copy would be a second allocation of
         // the weight's size, and inside a graph capture a refusal.
         if (!(copies & kCopyTile) && !a_f32 && m <= 16 && (plan_gemv4_sub_rows(tiles64, k_chunks).sub || (m <= 8 && tiles64 > 128))) wp.nt = 0;
+        if (const uint32_t ranges = (copies & kCopyTile) ? plan_batch_range(n_tiles, k_chunks, m, a_f32, gated, e.ws_bytes) : 0u) {
+            f.kind = kFormBatchRange;
+            f.copy = kCopyTile;
+            f.splits = ranges;
+            return f;
+        }
     }
     if (wp.nt) {
         f.kind = kFormWaves;
@@ -411,6 +417,7 @@ uint32_t twm_pick_splits(uint32_t k, uint32_t n, uint32_t m)
     case kFormSubTile:
     case kFormGroupLane:
     case kFormWholeTile:
+    case kFormBatchRange:
     case kFormWaves: return f.splits;
     case kFormBatch: return plan_batch(n_tiles, k_chunks, m < 32 ? m : 32, false).splits;
     case kFormStream: return plan_stream(n_tiles, k_chunks, m < 32 ? m : 32);
@@ -466,6 +473,10 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
         snprintf(text, bytes, "%s: %u-row x %u-column blocks, %u waves on k-chunks of their own, %s weights, %u K-split%s%s; 16-column tile copy",
                  m <= 32 ? "k_waves_exact" : "k_waves", waves_block_rows(m), 16 * f.nt, f.waves, m <= 32 ? "exact" : "f16-rounded", f.splits,
                  f.splits == 1 ? "" : "s", f.splits > 1 ? " + k_splitk_reduce" : "");
+        break;
+    case kFormBatchRange:
+        snprintf(text, bytes, "k_batch: 1 quad per workgroup, %u tiles per wave, 2 k-slices, a range's rows staged at once (k_batch_range), %u K-splits + k_splitk_reduce; 16-column tile copy",
+                 m <= 16 ? 2u : 4u, f.splits);
         break;
     case kFormStream: {
         const uint32_t sp = plan_stream(n_tiles, k_chunks, mb);
@@ -531,6 +542,9 @@ static int gemm_dispatch(twm_ctx *ctx, const twm_weight *w, const void *a_dev, i
         HIP_TRY(m <= 32 ? launch_waves_exact(ctx->stream, v, a_dev, a_f32, m, gated, f.nt, f.splits, ctx->ws, ctx->ws_bytes)
                         : launch_waves(ctx->stream, v, a_dev, a_f32, m, gated, f.nt, f.waves, f.splits, ctx->ws, ctx->ws_bytes),
                 TWM_DEVICE_ERROR, "batched launch");
+        return TWM_OK;
+    case kFormBatchRange:
+        HIP_TRY(launch_batch_range(ctx->stream, v, (const float *)a_dev, m, gated, f.splits, ctx->ws, ctx->ws_bytes), TWM_DEVICE_ERROR, "batched launch");
         return TWM_OK;
     case kFormSubTile:
         HIP_TRY(launch_gemv4s(ctx->stream, v, a_dev, a_f32, m, gated, ctx->ws, ctx->counters, f.sub, f.waves, f.splits, ctx->trace), TWM_DEVICE_ERROR,

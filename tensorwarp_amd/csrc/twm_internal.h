@@ -169,6 +169,7 @@ bool prefill_form_known(uint32_t form);  // a prefill block form (see launch_pre
 hipError_t init_prefill();
 hipError_t init_waves();
 hipError_t init_waves_exact();
+hipError_t init_batch_range();
 // waves on k-chunks of their own: 5 .. 32 rows with exact weights (twm_waves_exact.hip), 33 .. 192 rows on narrow matrices with
 // f16-rounded ones (twm_waves.hip): 16-column tiles per workgroup (0: another form runs), waves, K-splits
 struct WavesPlan {
@@ -182,6 +183,11 @@ hipError_t launch_waves_exact(hipStream_t s, const WeightView &w, const void *a,
                               uint32_t splits, void *scratch, size_t scratch_bytes);
 hipError_t launch_waves(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out, uint32_t nt,
                         uint32_t waves, uint32_t splits, void *scratch, size_t scratch_bytes);
+// 5 .. 32 f32 rows on deep, narrow matrices, exact weights: K-ranges whose rows a workgroup stages at once (twm_batch_range.hip);
+// plan_batch_range: the number of ranges (0: another form runs)
+uint32_t plan_batch_range(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated, size_t scratch_bytes);
+hipError_t launch_batch_range(hipStream_t s, const WeightView &w, const float *a, uint32_t m, const OutSpec &out, uint32_t splits,
+                              void *scratch, size_t scratch_bytes);
 hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out,
                           uint32_t block_rows, uint32_t splits, void *scratch, size_t scratch_bytes);
 // out[row][col] = sum over splits (in order) of partials[split][row][col], partials rows n_ld floats wide

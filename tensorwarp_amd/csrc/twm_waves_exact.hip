@@ -27,48 +27,13 @@
 // 3584 -> 2 x 18944 at 32 24.4 -> 22.2, at 13 20.1 -> 17.8; 4096 -> 12288 at 32 14.3 -> 12.4.
 // Measured and not kept: activations two chunks ahead (896 -> 1152 at 8 rows 3.5 / 3.6, 4096 -> 4096 at 32 rows 8.0 / 8.5),
 // v_fma_mixlo_f16 for the two terms (it issues at half the rate of v_fma_mix_f32 and v_cvt_pk_f16_f32).
-#include "twm_device.h"
+#include "twm_waves_core.h"
 
 #include <type_traits>
 
 namespace twm {
 
 namespace {
-
-__device__ __forceinline__ const TWM_GLOBAL char *we_scalar_base(const void *p, size_t byte_offset)
-{
-    uint64_t v = (uint64_t)p + byte_offset;
-    asm("" : "+s"(v));  // a uniform base kept in scalar registers: loads take saddr + 32-bit lane offset
-    return (const TWM_GLOBAL char *)v;
-}
-
-struct WeConsts {
-    uint32_t mask_lo, mask_hi, magic_lo, magic_hi;
-};
-
-// eight nibbles of word w -> eight f16 values (q - 8), exact
-__device__ __forceinline__ half8 we_unpack(uint32_t w, const WeConsts &c)
-{
-    union { uint32_t u[4]; half2v h2[4]; half8 h; } r;
-    const half2v b_lo = {(_Float16)-1032.0f, (_Float16)-1032.0f};
-    const half2v b_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
-    const uint32_t w8 = w >> 8;
-    r.u[0] = (w & c.mask_lo) | c.magic_lo;
-    r.u[1] = (w & c.mask_hi) | c.magic_hi;
-    r.u[2] = (w8 & c.mask_lo) | c.magic_lo;
-    r.u[3] = (w8 & c.mask_hi) | c.magic_hi;
-    r.h2[0] += b_lo;
-    r.h2[1] += b_hi;
-    r.h2[2] += b_lo;
-    r.h2[3] += b_hi;
-    return r.h;
-}
-
-constexpr int kWeRow = 128;  // halves per LDS row (256 bytes)
-
-// What kind of rows: f16; up to eight f32 rows, whose second f16 terms are rows 8 .. 15 of the one block (which costs what
-// eight f16 rows cost); f32 rows as two tiles
-enum { kRowsF16 = 0, kRowsF32Few = 1, kRowsF32 = 2 };
 
 // The largest of m[j] over each sixteen lanes, in each of them, for NV values at once.  (A value read through DPP must have
 // been written two instructions before: the steps of several values are interleaved.)
@@ -219,49 +184,27 @@ __global__ __launch_bounds__(64 * W) void k_waves_exact(const uint4v *__restrict
             }
             float m[NV];
 #pragma unroll
-            for (int j = 0; j < NV; j++) {
-                float x[8];
-#pragma unroll
-                for (int l = 0; l < 2; l++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++) x[4 * l + q] = __uint_as_float(ar[j][l][q]);
-                float t;
-                asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(t) : "v"(x[0]), "v"(x[1]), "v"(x[2]));
-                asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(t) : "v"(t), "v"(x[3]), "v"(x[4]));
-                asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(t) : "v"(t), "v"(x[5]), "v"(x[6]));
-                asm("v_max_f32 %0, %1, |%2|" : "=v"(m[j]) : "v"(t), "v"(x[7]));
-            }
+            for (int j = 0; j < NV; j++) m[j] = we_max8(ar[j][0], ar[j][1]);
             rows16_max<NV>(m);
 #pragma unroll
             for (int j = 0; j < NV; j++) {
-                uint32_t e = __float_as_uint(m[j]) & 0x7F800000u;
-                e = e > (16u << 23) ? e : (16u << 23);
-                const float down = __uint_as_float((267u << 23) - e);   // 2^(13 - exponent); an infinity or a NaN stays one
+                const WeFactor factor = we_factor(m[j]);
                 const uint32_t row = 4u * j + (lane >> 4);
 #pragma unroll
                 for (int l = 0; l < 2; l++) {
-                    union { half2v h[2]; uint2v u; } hi, lo;
-#pragma unroll
-                    for (int q = 0; q < 2; q++) {
-                        const float f0 = __uint_as_float(ar[j][l][2 * q]), f1 = __uint_as_float(ar[j][l][2 * q + 1]);
-                        hi.h[q] = half2v{(_Float16)(f0 * down), (_Float16)(f1 * down)};
-                        asm("" : "+v"(hi.u[q]));        // (one conversion of the pair; its halves are read from the packed register)
-                        float r0 = __builtin_fmaf(f0, down, -(float)hi.h[q][0]), r1 = __builtin_fmaf(f1, down, -(float)hi.h[q][1]);
-                        asm("" : "+v"(r0), "+v"(r1));   // (v_fma_mixlo_f16, which would do both steps, issues at half the rate)
-                        lo.h[q] = half2v{(_Float16)r0, (_Float16)r1};
-                    }
+                    uint2v hi, lo;
+                    we_terms(ar[j][l], factor.down, hi, lo);
                     const uint32_t vec = (((uint32_t)l ^ odd) << 3) + (p >> 1);
-                    *(uint2v *)(region + row * kWeRow + ((vec ^ (row & 15u)) * 8u) + (p & 1u) * 4u) = hi.u;
+                    *(uint2v *)(region + row * kWeRow + ((vec ^ (row & 15u)) * 8u) + (p & 1u) * 4u) = hi;
                     if constexpr (MODE == kRowsF32Few)
-                        *(uint2v *)(region + (row + 8u) * kWeRow + ((vec ^ (row + 8u)) * 8u) + (p & 1u) * 4u) = lo.u;
+                        *(uint2v *)(region + (row + 8u) * kWeRow + ((vec ^ (row + 8u)) * 8u) + (p & 1u) * 4u) = lo;
                     else
-                        *(uint2v *)(region + kTile + row * kWeRow + ((vec ^ (row & 15u)) * 8u) + (p & 1u) * 4u) = lo.u;
+                        *(uint2v *)(region + kTile + row * kWeRow + ((vec ^ (row & 15u)) * 8u) + (p & 1u) * 4u) = lo;
                 }
                 if (p == 0) {
                     float *f = (float *)(region + TERMS * kTile);
-                    const float back = __uint_as_float(e - (13u << 23));
-                    f[row] = back;
-                    if (MODE == kRowsF32Few) f[row + 8u] = back;
+                    f[row] = factor.back;
+                    if (MODE == kRowsF32Few) f[row + 8u] = factor.back;
                 }
             }
         }

@@ -943,3 +943,45 @@ def test_prefill_gate_on_192_columns(dev, m, ffn, form):
         dev.set_option("prefill_bm", 0)
     close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, 2e-3)   # (a product of two sums at 1e-3 each)
     w.free()
+
+
+@pytest.mark.parametrize("m", [5, 8, 9, 16, 17, 31, 32])
+def test_ranges_staged_at_once(dev, m):
+    # k_batch_range: row blocks of 8, 16 and 32 rows and their remainders; ranges of an uneven number of chunks and a shorter last
+    # one; K that ends inside a chunk, N inside a workgroup's columns; rows beyond the f16 range on both sides, one infinite row;
+    # segments with biases
+    k, n = (20512, 1157) if m > 16 else (22624, 1725)
+    assert "k_batch_range" in dev.plan(k, n, m, dtype="f32")
+    packed, scales, w = weight(dev, k, n, 1700 + m)
+    a = O.synth_normal_f32(m * k, 1703 + m).reshape(m, k).copy()
+    a[0] *= np.float32(3e7)
+    a[1] *= np.float32(1e-9)
+    a[m - 1, k - 1] = np.float32(4e5)
+    a[2, ::3] *= np.float32(2.0 ** -20)
+    truth = O.gemm_f64(a, packed, scales, m, k, n)
+    a[3, k // 2] = np.inf
+    ns = [n - 500, 499, 1]
+    biases = [O.synth_normal_f32(x, 1709 + x) for x in ns]
+    outs = [T.GpuTensor.from_host(dev, np.full((m, x), np.nan, np.float32)) for x in ns]
+    T.gemm_split(dev, w, T.GpuTensor.from_host(dev, a), m, outs, ns, biases=[T.GpuTensor.from_host(dev, b) for b in biases])
+    got = np.concatenate([o.to_host() - b for o, b in zip(outs, biases)], 1).astype(np.float64)
+    keep = [r for r in range(m) if r not in (1, 3)]
+    assert not np.isfinite(got[3]).any()
+    close_rows(got[keep], truth[keep], F32_SUM)
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    T.gemm(dev, w, T.GpuTensor.from_host(dev, a), m, c)          # (without a bias the row of 1e-9 is seen to its last digits)
+    close_rows(c.to_host()[[1] + keep], truth[[1] + keep], F32_SUM)
+    w.free()
+
+
+def test_ranges_staged_at_once_under_a_gate(dev):
+    m, k, ffn = 23, 20256, 1344
+    assert "k_batch_range" in dev.plan(k, 2 * ffn, m, dtype="f32", gated=True)
+    gate, up = ((O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (1750, 1760))
+    w = T.MarlinWeight.gate_up(dev, *([T.GpuTensor.from_host(dev, p), T.GpuTensor.from_host(dev, s, "f16")] for p, s in (gate, up)), k, ffn)
+    a = 0.3 * O.synth_normal_f32(m * k, 1770).reshape(m, k)
+    g, u = (O.gemm_f64(a, *x, m, k, ffn) for x in (gate, up))
+    out = T.GpuTensor.from_host(dev, np.full((m, ffn), np.nan, np.float32))
+    T.gemm_swiglu(dev, w, T.GpuTensor.from_host(dev, a), m, out)
+    close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
+    w.free()
