@@ -514,7 +514,7 @@ int twm_argmax_f32(twm_ctx *ctx, const float *input_dev, uint32_t rows, uint32_t
     if (!ctx) return api_fail(TWM_INVALID_HANDLE, "twm_argmax_f32: null context");
     if (rows == 0) return TWM_OK;
     if (!out_dev || (cols != 0 && !input_dev)) return api_fail(TWM_INVALID_HANDLE, "twm_argmax_f32: null pointer");
-    HIP_TRY(launch_argmax(ctx->stream, input_dev, rows, cols, out_dev, ctx->ws, ctx->ws_bytes), TWM_DEVICE_ERROR, "argmax launch");
+    HIP_TRY(launch_argmax(ctx->stream, input_dev, rows, cols, out_dev, ctx->ws, ctx->ws_bytes, ctx->counters, ctx->n_counters), TWM_DEVICE_ERROR, "argmax launch");
     return TWM_OK;
 }
 

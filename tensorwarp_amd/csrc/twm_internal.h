@@ -135,7 +135,7 @@ hipError_t launch_pair_gate_up(hipStream_t s, const uint8_t *gate_packed, const 
                                const uint8_t *up_packed, const uint16_t *up_scales, uint32_t groups, uint32_t ffn,
                                uint8_t *packed_out, uint16_t *scales_out);
 hipError_t launch_argmax(hipStream_t s, const float *in, uint32_t rows, uint32_t cols, int *out, void *scratch,
-                         size_t scratch_bytes);
+                         size_t scratch_bytes, unsigned *counters, uint32_t n_counters);
 hipError_t launch_ref_gemv(hipStream_t s, const float *a, const uint8_t *packed, const uint16_t *scales, float *c,
                            uint32_t n, uint32_t k, uint32_t splits, uint32_t groups_per_split);
 hipError_t launch_repack(hipStream_t s, const uint8_t *packed, const uint16_t *scales, uint32_t k, uint32_t n,

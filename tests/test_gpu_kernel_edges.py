@@ -985,3 +985,19 @@ def test_ranges_staged_at_once_under_a_gate(dev):
     T.gemm_swiglu(dev, w, T.GpuTensor.from_host(dev, a), m, out)
     close_rows(out.to_host(), g / (1.0 + np.exp(-g)) * u, F32_SUM)
     w.free()
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 4095), (3, 4096), (3, 4097), (2, 8193), (1, 4096 * 65 + 1), (40, 4096 * 33), (1023, 8200), (1025, 4100), (2049, 70)])
+def test_argmax_at_the_edges_of_its_spans(dev, rows, cols):
+    # spans of 4096 columns, one or several to a workgroup; more spans than lanes merge them; ties across spans and between
+    # zeros of either sign, a largest value in the last column, rows without a candidate; a second call finds the counters clear
+    x = np.round(O.synth_normal_f32(rows * cols, 1800 + cols).reshape(rows, cols) * 2).astype(np.float32)
+    x[0, -1] = 1e9
+    x[rows // 2] = -np.abs(x[rows // 2])
+    x[rows // 2, cols // 3] = np.float32(-0.0)
+    if rows > 1:
+        x[rows - 1] = np.nan if cols % 2 else np.float32(-1e30)
+    xd, out = T.GpuTensor.from_host(dev, x), T.GpuTensor.from_host(dev, np.full(rows, -7, np.int32))
+    for _ in range(2):
+        T.argmax(dev, xd, out, rows, cols)
+        assert np.array_equal(out.to_host(), O.argmax(x, rows, cols))
