@@ -18,6 +18,10 @@
 //   tiles -- from memory in operand order they cost 3.5 times as much, 37 against 130 bytes per ns and CU;
 // * tile after tile, a tile's weight registers take the next chunk's loads as soon as its last group is unpacked: with up to
 //   four tiles two chunks are in flight, with more one, 92 KB per CU on ten tiles;
+// * the rows are loaded by quads, as many as there are (NV: 8, 12, 16, 24 or 32 rows): each costs the CU's load path, which
+//   delivers some 6.4 TB/s in all, weights and rows alike, once the weights come from HBM (16 and 32 rows whatever their number
+//   before: 3584 -> 3584 at 8 rows 5.45 -> 5.1, at 24 6.9 -> 6.4, 8192 -> 8192 at 8 11.5 -> 10.7, at 24 15.4 -> 14.7; with the
+//   conversion of f32 rows 4096 -> 12288 at 24 18.4 -> 16.5, 4096 -> 4096 at 20 12.2 -> 11.3);
 // * nothing in the store waits for a kernel argument: the output description is fetched behind the first loads (-0.3 us on
 //   896 -> 1152), and up to ten sums per lane four waves finish a tile, one register each (-0.5 us there).
 // f32 rows in one launch instead of a conversion launch and a GEMM on its two f16 arrays (us, before -> now): 4096 -> 2 x 11008
@@ -40,24 +44,28 @@ namespace {
 template <int NV>
 __device__ __forceinline__ void rows16_max(float (&m)[NV])
 {
-    static_assert(NV == 2 || NV % 4 == 0, "");
 #define TWM_MAX4(N)                                                             \
     "v_max_f32_dpp %0, %0, %0 row_ror:" #N " row_mask:0xf bank_mask:0xf\n"      \
     "v_max_f32_dpp %1, %1, %1 row_ror:" #N " row_mask:0xf bank_mask:0xf\n"      \
     "v_max_f32_dpp %2, %2, %2 row_ror:" #N " row_mask:0xf bank_mask:0xf\n"      \
     "v_max_f32_dpp %3, %3, %3 row_ror:" #N " row_mask:0xf bank_mask:0xf\n"
+#define TWM_MAX3(N)                                                             \
+    "v_max_f32_dpp %0, %0, %0 row_ror:" #N " row_mask:0xf bank_mask:0xf\n"      \
+    "v_max_f32_dpp %1, %1, %1 row_ror:" #N " row_mask:0xf bank_mask:0xf\n"      \
+    "v_max_f32_dpp %2, %2, %2 row_ror:" #N " row_mask:0xf bank_mask:0xf\n"
 #define TWM_MAX2(N)                                                             \
     "s_nop 1\n"                                                                 \
     "v_max_f32_dpp %0, %0, %0 row_ror:" #N " row_mask:0xf bank_mask:0xf\n"      \
     "v_max_f32_dpp %1, %1, %1 row_ror:" #N " row_mask:0xf bank_mask:0xf\n"
-    if constexpr (NV == 2) {
-        asm(TWM_MAX2(8) TWM_MAX2(4) TWM_MAX2(2) TWM_MAX2(1) : "+v"(m[0]), "+v"(m[1]));
-    } else {
 #pragma unroll
-        for (int j = 0; j < NV; j += 4)
-            asm("s_nop 1\n" TWM_MAX4(8) TWM_MAX4(4) TWM_MAX4(2) TWM_MAX4(1) : "+v"(m[j]), "+v"(m[j + 1]), "+v"(m[j + 2]), "+v"(m[j + 3]));
-    }
+    for (int j = 0; j + 4 <= NV; j += 4)
+        asm("s_nop 1\n" TWM_MAX4(8) TWM_MAX4(4) TWM_MAX4(2) TWM_MAX4(1) : "+v"(m[j]), "+v"(m[j + 1]), "+v"(m[j + 2]), "+v"(m[j + 3]));
+    constexpr int L = NV / 4 * 4;
+    if constexpr (NV % 4 == 3) asm("s_nop 1\n" TWM_MAX3(8) TWM_MAX3(4) TWM_MAX3(2) TWM_MAX3(1) : "+v"(m[L]), "+v"(m[L + 1]), "+v"(m[L + 2]));
+    if constexpr (NV % 4 == 2) asm(TWM_MAX2(8) TWM_MAX2(4) TWM_MAX2(2) TWM_MAX2(1) : "+v"(m[L]), "+v"(m[L + 1]));
+    static_assert(NV % 4 != 1, "");
 #undef TWM_MAX4
+#undef TWM_MAX3
 #undef TWM_MAX2
 }
 
@@ -65,7 +73,7 @@ __device__ __forceinline__ void rows16_max(float (&m)[NV])
 
 // grid: K-splits x column groups (the splits of a group are neighbours, so that with eight of them each XCD reads one stretch
 // of the activations).  The first arguments, which the loads need, arrive preloaded (thirteen words).
-template <int MT, int NT, int MODE, int W>
+template <int MT, int NT, int MODE, int W, int NV>
 __global__ __launch_bounds__(64 * W) void k_waves_exact(const uint4v *__restrict__ qw, const uint2v *__restrict__ sc,
                                                  const void *__restrict__ a_any, uint32_t m_rows, uint32_t k, uint32_t n_tiles,
                                                  uint32_t k_chunks, uint32_t chunks_per_split, uint32_t gated_u, uint32_t n,
@@ -76,7 +84,6 @@ __global__ __launch_bounds__(64 * W) void k_waves_exact(const uint4v *__restrict
     constexpr int SLOTS = NT <= 4 && !(MT == 2 && TERMS == 2) ? 2 : 1;
     constexpr int kTile = 16 * MT * kWeRow;                          // halves of one term's activation tile
     constexpr int kRegion = TERMS * kTile + (F32 ? 32 * MT : 0);     // halves of a wave's LDS region (behind the tiles: a factor per row)
-    constexpr int NV = MODE == kRowsF32Few ? 2 : 4 * MT;             // row quads that a wave loads per chunk
     constexpr int LD = F32 ? 2 : 1;                                  // 16-byte loads per lane and row quad
     extern __shared__ __attribute__((aligned(16))) _Float16 lds_all[];
 
@@ -398,7 +405,7 @@ __global__ __launch_bounds__(64 * W) void k_waves_exact(const uint4v *__restrict
 
 namespace {
 
-template <int MT, int NT, int MODE, int W> struct WavesExact {
+template <int MT, int NT, int MODE, int W, int NV> struct WavesExact {
     static constexpr size_t staging = (size_t)W * ((MODE == kRowsF32 ? 2 : 1) * 16 * MT * kWeRow + (MODE ? 32 * MT : 0)) * sizeof(_Float16);
     static constexpr size_t sums = (size_t)W * MT * NT * 1024;
     static constexpr size_t lds = staging > sums ? staging : sums;
@@ -406,7 +413,7 @@ template <int MT, int NT, int MODE, int W> struct WavesExact {
     static hipError_t init()
     {
         if (lds <= 64 * 1024) return hipSuccess;
-        return hipFuncSetAttribute((const void *)k_waves_exact<MT, NT, MODE, W>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        return hipFuncSetAttribute((const void *)k_waves_exact<MT, NT, MODE, W, NV>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     }
     static hipError_t launch(hipStream_t s, const WeightView &w, const void *a, uint32_t m, const OutSpec &out, uint32_t splits, float *partials)
     {
@@ -414,7 +421,7 @@ template <int MT, int NT, int MODE, int W> struct WavesExact {
         splits = (w.k_chunks + cps - 1) / cps;  // no empty split
         const bool gated = out.swiglu != nullptr;
         const uint32_t groups = (w.n_tiles + NT - 1) / NT;
-        hipLaunchKernelGGL((k_waves_exact<MT, NT, MODE, W>), dim3(splits, groups), dim3(64 * W), lds, s, (const uint4v *)w.qw, (const uint2v *)w.sc,
+        hipLaunchKernelGGL((k_waves_exact<MT, NT, MODE, W, NV>), dim3(splits, groups), dim3(64 * W), lds, s, (const uint4v *)w.qw, (const uint2v *)w.sc,
                            a, m, w.k, w.n_tiles, w.k_chunks, cps, gated && splits == 1 ? 1u : 0u, w.n, splits > 1 ? partials : nullptr, out);
         if (splits > 1) return launch_splitk_reduce(s, partials, out, m, w.n, w.n_tiles * 16, splits);
         return hipGetLastError();
@@ -423,15 +430,20 @@ template <int MT, int NT, int MODE, int W> struct WavesExact {
 
 // The forms that exist, eight waves each; the two-tile f32 rows' registers end at eight column tiles (four with 17 .. 32 rows).
 // fn gets the one of the runtime parameters (false: there is none), or every one in turn (mt = 0, until fn fails).
-template <typename F> bool waves_exact_form(uint32_t mt, uint32_t nt, uint32_t mode, hipError_t &e, F &&fn)
+template <typename F> bool waves_exact_form(uint32_t mt, uint32_t nt, uint32_t mode, uint32_t quads, hipError_t &e, F &&fn)
 {
     bool found = false;
     e = hipSuccess;
-#define TWM_WAVES(MT, NT, MODE)                                                       \
-    if (e == hipSuccess && (mt == 0 || (mt == MT && nt == NT && mode == MODE))) {     \
-        found = true;                                                                 \
-        e = fn(WavesExact<MT, NT, MODE, 8>{});                                        \
+#define TWM_WAVES_ROWS(MT, NT, MODE, NV)                                                              \
+    if (e == hipSuccess && (mt == 0 || (mt == MT && nt == NT && mode == MODE && quads == NV))) {      \
+        found = true;                                                                                 \
+        e = fn(WavesExact<MT, NT, MODE, 8, NV>{});                                                    \
     }
+#define TWM_WAVES(MT, NT, MODE)                                                       \
+    if constexpr (MT == 2) { TWM_WAVES_ROWS(MT, NT, MODE, 6) TWM_WAVES_ROWS(MT, NT, MODE, 8) }              \
+    else if constexpr (MODE == kRowsF32Few) { TWM_WAVES_ROWS(MT, NT, MODE, 2) }                             \
+    else if constexpr (MODE == kRowsF32) { TWM_WAVES_ROWS(MT, NT, MODE, 3) TWM_WAVES_ROWS(MT, NT, MODE, 4) } \
+    else { TWM_WAVES_ROWS(MT, NT, MODE, 2) TWM_WAVES_ROWS(MT, NT, MODE, 3) TWM_WAVES_ROWS(MT, NT, MODE, 4) }
 #define TWM_WAVES_4(MT, MODE) TWM_WAVES(MT, 1, MODE) TWM_WAVES(MT, 2, MODE) TWM_WAVES(MT, 3, MODE) TWM_WAVES(MT, 4, MODE)
 #define TWM_WAVES_8(MT, MODE) TWM_WAVES_4(MT, MODE) TWM_WAVES(MT, 5, MODE) TWM_WAVES(MT, 6, MODE) TWM_WAVES(MT, 8, MODE)
     TWM_WAVES_8(1, kRowsF16) TWM_WAVES(1, 10, kRowsF16)
@@ -442,6 +454,7 @@ template <typename F> bool waves_exact_form(uint32_t mt, uint32_t nt, uint32_t m
 #undef TWM_WAVES_8
 #undef TWM_WAVES_4
 #undef TWM_WAVES
+#undef TWM_WAVES_ROWS
     return found;
 }
 
@@ -451,7 +464,7 @@ template <typename F> bool waves_exact_form(uint32_t mt, uint32_t nt, uint32_t m
 hipError_t init_waves_exact()
 {
     hipError_t e;
-    waves_exact_form(0, 0, 0, e, [](auto form) { return decltype(form)::init(); });
+    waves_exact_form(0, 0, 0, 0, e, [](auto form) { return decltype(form)::init(); });
     return e;
 }
 
@@ -472,11 +485,17 @@ hipError_t init_waves_exact()
 //   680 and 5120 on 513 .. 680, whose groups of three leave the CUs 70 - 85 % full (28672 -> 8192 64 / 55, 8064 -> 9792 at 23
 //   rows 30.5 / 25.6, 7296 -> 2 x 5280 at 27 30.7 / 27.0); nine rows and more on three chunks at 2048 tiles (128 -> 39553 at 16
 //   rows 8.1 / 7.3);
-// * f16, up to eight rows: the lane-per-column and streaming kernels keep 513 .. 1100 tiles (896 -> 2 x 4864 4.9 / 4.2, 2560 ->
-//   2 x 7168 8.5 / 7.5) and 1537 .. 2048 (3104 -> 28833 at 6 rows 14.1 / 12.8: eight tiles each leave the CUs 75 - 90 % full),
-//   K of 16 .. 32 chunks on 257 .. 512 tiles (3584 -> 4608 5.9 / 5.6), and up to six rows, seven up to K = 4096, every K from
-//   2200 on with up to 256 tiles (3584 -> 3584 at 5 rows 5.2 / 4.6), gated 2048 .. 4096 at eight rows too, where pairs of tiles
-//   are half as many workgroups (3072 -> 2 x 96 at 8 rows 4.75 / 4.24);
+// * f16, up to eight rows: the lane-per-column and streaming kernels keep 513 .. 1100 tiles (896 -> 2 x 4864 4.9 / 4.2; 820 .. 1024
+//   tiles 2 - 17 % ahead) but for a deeper K on up to 820 of them (700 tiles, nine chunks and more: 0.97 of their time, 33 and more
+//   0.79 .. 0.87, gated 0.97; 33 and more on 820 0.85 .. 0.9) and 17 chunks and more above 1024, where their second round of
+//   workgroups is nearly empty (0.67 .. 0.89); 1537 .. 2048 tiles (3104 -> 28833 at 6 rows 14.1 / 12.8: eight tiles each leave the
+//   CUs 75 - 90 % full); K of 16 .. 32 chunks on 341 .. 512 tiles (gated up to 18 chunks 0.93, else level to 10 % behind; on 257 ..
+//   340 0.93 .. 0.97); and up to six rows, seven up to K = 4096, every K from 2200 on with up to 256 tiles (3584 -> 3584 at 5 rows
+//   5.2 / 4.6) but for more than 64 chunks on up to 128 (0.75 .. 0.87 of k_stream's time), gated 2048 .. 4096 at eight rows too,
+//   where pairs of tiles are half as many workgroups (3072 -> 2 x 96 at 8 rows 4.75 / 4.24);
+// * f16, 9 .. 12 and 17 .. 24 rows, whose row blocks are not loaded whole: a few more of the shapes below (two to four chunks on
+//   513 .. 820 tiles 0.92 .. 0.95 of k_batch's time, nine to sixteen on 701 .. 820 0.91 .. 0.96, 33 and more on 1801 .. 2048 0.93 ..
+//   0.96);
 // * f16, deep K on 129 .. 256 tiles: from 72 chunks on up to sixteen rows (12192 -> 3584 at 8 rows 11.0 / 10.0), up to 340 tiles
 //   from 67 on (9216 -> 4352 at 11 rows 10.9 / 9.8, 13600 -> 2 x 2720 at 7 14.4 / 12.9), from 65 on above (17824 -> 3584 at 17 rows
 //   16.8 / 15.6), gated from 61 on with 321 .. 400 tiles (10848 -> 2 x 2848 at 31 rows 20.0 / 17.9); f16 on a few
@@ -513,17 +532,19 @@ WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool
         if (m > 8 && n_tiles > 2048 && k_chunks <= 3) return none;
     } else {
         if (n_tiles > (m <= 8 || m > 16 ? 2560u : 2816u)) return none;
-        if (k_chunks <= 8 && n_tiles > (k_chunks <= 4 ? 512u : 1024u)) return none;
+        const bool part = (m >= 9 && m <= 12) || (m >= 17 && m <= 24);   // (a row block that is not loaded whole)
+        if (k_chunks <= 8 && n_tiles > (k_chunks > 4 ? 1024u : part && k_chunks > 1 ? 820u : 512u)) return none;
         if (n_tiles > 128 && n_tiles <= (m <= 16 ? 340u : 256u) && k_chunks > (m > 16 ? 64u : n_tiles > 256 ? 66u : 71u)) return none;
         if (gated && m > 16 && n_tiles > 320 && n_tiles <= 400 && k_chunks > 60) return none;
-        if (n_tiles > 700 && n_tiles <= 1000 && k_chunks > 8 && k_chunks <= 16) return none;
-        if (n_tiles > 1800 && n_tiles <= 2048) return none;
+        if (n_tiles > (part ? 820u : 700u) && n_tiles <= 1000 && k_chunks > 8 && k_chunks <= 16) return none;
+        if (n_tiles > 1800 && n_tiles <= 2048 && !(part && k_chunks > 32)) return none;
         if (n_tiles > (m <= 8 && k_chunks <= 10 ? 1300u : m <= 16 ? 1536u : 1600u) && k_chunks <= 18) return none;
         if (m <= 16 && n_tiles > 960 && n_tiles <= 1024) return none;
         if (m <= 8) {
-            if ((n_tiles > 512 && n_tiles <= 1100) || (n_tiles > 1536 && n_tiles <= 2048)) return none;
-            if (n_tiles > 256 && n_tiles <= 512 && k_chunks >= 16 && k_chunks <= 32) return none;
-            if (n_tiles <= 256 && k_chunks > 17 && (m <= 6 || (m == 7 && k_chunks <= 32))) return none;
+            const bool deep = n_tiles > 1024 ? k_chunks > 16 : n_tiles <= 700 ? k_chunks > (gated ? 32u : 8u) : n_tiles <= 820 && k_chunks > 32 && !gated;
+            if ((n_tiles > 512 && n_tiles <= 1100 && !deep) || (n_tiles > 1536 && n_tiles <= 2048)) return none;
+            if (n_tiles > 340 && n_tiles <= 512 && k_chunks >= 16 && k_chunks <= 32 && !(gated && k_chunks <= 18)) return none;
+            if (n_tiles <= 256 && k_chunks > 17 && (m <= 6 || (m == 7 && k_chunks <= 32)) && !(n_tiles <= 128 && k_chunks > 64)) return none;
             if (n_tiles <= 256 && gated && k_chunks >= 16 && k_chunks <= 31) return none;
         }
     }
@@ -582,7 +603,8 @@ hipError_t launch_waves_exact(hipStream_t s, const WeightView &w, const void *a,
     if (splits < 1) splits = 1;
     if (out.swiglu && splits == 1 && nt % 2) nt++;
     hipError_t e;
-    const bool found = waves_exact_form(m <= 16 ? 1u : 2u, nt, mode, e, [&](auto form) {
+    const uint32_t quads = m <= 8 ? 2u : m <= 12 ? 3u : m <= 16 ? 4u : m <= 24 ? 6u : 8u;
+    const bool found = waves_exact_form(m <= 16 ? 1u : 2u, nt, mode, quads, e, [&](auto form) {
         return decltype(form)::launch(s, w, a, m, out, splits, (float *)scratch);
     });
     return found ? e : hipErrorInvalidValue;

@@ -987,6 +987,31 @@ def test_ranges_staged_at_once_under_a_gate(dev):
     w.free()
 
 
+@pytest.mark.parametrize("m,dtype", [(1, "f16"), (4, "f16"), (5, "f16"), (8, "f16"), (9, "f16"), (12, "f16"), (13, "f16"), (16, "f16"), (17, "f16"), (24, "f16"),
+                                     (25, "f16"), (9, "f32"), (12, "f32"), (13, "f32"), (17, "f32"), (24, "f32"), (25, "f32")])
+@pytest.mark.parametrize("nt", [1, 3, 8])
+def test_row_quads_of_waves_on_exact_weights(dev, m, dtype, nt):
+    # k_waves_exact loads the rows by quads: the rows of a block behind them are whatever the LDS holds, here NaNs that a launch on
+    # rows of them has left, and touch no other row
+    k, n = 1312, 16 * nt + 21
+    packed, scales, w = weight(dev, k, n, 1651 + nt)
+    a16 = O.synth_act_f16(m, k, 1655 + m)
+    a = a16.view(np.float16).astype(np.float32).reshape(m, k)
+    rows = T.GpuTensor.from_host(dev, a16, "f16") if dtype == "f16" else T.GpuTensor.from_host(dev, a)
+    nans = T.GpuTensor.from_host(dev, np.full((32, k), np.nan, np.float32))
+    c, junk = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32)), T.GpuTensor.zeros(dev, (32, n), "f32")
+    dev.set_option("kernel", 5)
+    try:
+        dev.set_option("nt", nt)
+        T.gemm(dev, w, nans, 32, junk)
+        T.gemm(dev, w, rows, m, c)
+    finally:
+        dev.set_option("nt", 0)
+        dev.set_option("kernel", 0)
+    close_rows(c.to_host(), O.gemm_f64(a, packed, scales, m, k, n), F32_SUM)
+    w.free()
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (3, 4095), (3, 4096), (3, 4097), (2, 8193), (1, 4096 * 65 + 1), (40, 4096 * 33), (1023, 8200), (1025, 4100), (2049, 70)])
 def test_argmax_at_the_edges_of_its_spans(dev, rows, cols):
     # spans of 4096 columns, one or several to a workgroup; more spans than lanes merge them; ties across spans and between
