@@ -5,50 +5,66 @@ namespace twm {
 
 namespace {
 
-// The partial sums of one place, added in split order (deterministic): up to eight loads in flight.  (Byte offsets: the partial
-// sums of a launch fit the context's scratch, 256 MB.)
+// N more partial sums of one place, all loads in flight, added in split order
+template <int N> __device__ __forceinline__ void splitk_add(float4v &s, const TWM_GLOBAL char *base, uint32_t &offset, uint32_t stride)
+{
+    float4v v[N];
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        offset += stride;
+        v[j] = *(const TWM_GLOBAL float4v *)(base + offset);
+    }
+#pragma unroll
+    for (int j = 0; j < N; j++) s += v[j];
+}
+
+// The partial sums of one place, added in split order (deterministic).  (Byte offsets: the partial sums of a launch fit the
+// context's scratch, 256 MB.)
 __device__ __forceinline__ float4v splitk_sum(const float *partials, uint32_t offset, uint32_t stride, uint32_t splits)
 {
     const TWM_GLOBAL char *base = (const TWM_GLOBAL char *)partials;
     float4v s = *(const TWM_GLOBAL float4v *)(base + offset);
-    for (uint32_t z = 1; z < splits; z += 8u) {
-        float4v v[8];
-#pragma unroll
-        for (uint32_t j = 0; j < 8u; j++) {
-            if (z + j < splits) {
-                offset += stride;
-                v[j] = *(const TWM_GLOBAL float4v *)(base + offset);
-            }
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < 8u; j++)
-            if (z + j < splits) s += v[j];
+    uint32_t left = splits - 1u;
+    for (; left >= 8u; left -= 8u) splitk_add<8>(s, base, offset, stride);
+    switch (left) {
+    case 1: splitk_add<1>(s, base, offset, stride); break;
+    case 2: splitk_add<2>(s, base, offset, stride); break;
+    case 3: splitk_add<3>(s, base, offset, stride); break;
+    case 4: splitk_add<4>(s, base, offset, stride); break;
+    case 5: splitk_add<5>(s, base, offset, stride); break;
+    case 6: splitk_add<6>(s, base, offset, stride); break;
+    case 7: splitk_add<7>(s, base, offset, stride); break;
     }
     return s;
 }
 
 }  // namespace
 
-// One thread per four padded columns, one grid row per output row; stride: bytes from one split's sums to the next.  Bound:
-// latency: a launch takes about 1.8 us with a single load and store, this one 2.4 for four splits of 8 x 3584 and 3.1 for seven
-// of 96 x 4608 in a graph.  A grid row per output row instead of a division by the quads of a row, the arguments of the loads
-// preloaded, and eight loads in flight instead of four: 0.2 - 0.4 us a launch (3584 -> 4608 at 96 rows on seven splits 16.56 ->
-// 16.25, 18944 -> 3584 at 8 f32 rows on four 16.1 -> 15.9; a decode layer with one such launch 64.3 -> 63.7 at 32 rows, 45.3 ->
-// 44.8 at 8).  Sixteen in flight were no faster.
+// One thread per four padded columns; stride: bytes from one split's sums to the next.  Bound: latency, and on many rows the
+// traffic: a launch takes about 1.8 us with a single load and store, this one 2.4 for four splits of 8 x 3584 and 3.1 for seven of
+// 96 x 4608 in a graph.  A 32-bit division by the quads of a row in place of a 64-bit one, the arguments of the loads preloaded, and
+// all loads of up to nine splits in flight instead of one, four or two in turn: 0.2 - 0.6 us a launch (3584 -> 4608 at 96 rows on
+// seven splits 16.6 -> 16.0, 18944 -> 3584 at 8 f32 rows on four 16.1 -> 15.9, the four launches of a layer of 1152 values at 394
+// f32 rows 87.0 -> 85.6 with three of these; a decode layer with one 64.3 -> 63.7 at 32 rows, 45.3 -> 44.8 at 8).  Sixteen loads
+// in flight were no faster; eight under conditions instead of a form per remainder 1.5 % behind on few splits of many rows; a grid
+// row per output row instead of the division left most lanes of a row's last workgroup idle.
 template <RowStore ROWS, uint32_t BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_splitk_reduce(const float *__restrict__ partials, uint32_t n_ld, uint32_t splits, uint32_t stride,
-                                                         uint32_t n, const float *__restrict__ row_scale, uint32_t row0, OutSpec out)
+                                                         uint32_t n, const float *__restrict__ row_scale, uint32_t m_rows, OutSpec out)
 {
-    const uint32_t col = (blockIdx.x * BLOCK + threadIdx.x) * 4u, row = row0 + blockIdx.y;
-    if (col >= n_ld) return;
+    const uint32_t idx = blockIdx.x * BLOCK + threadIdx.x, quads = n_ld / 4u, row = idx / quads, col = (idx - row * quads) * 4u;
+    if (row >= m_rows) return;
+    uint32_t ld = 0;
+    float4v bias = {0.f, 0.f, 0.f, 0.f};
+    float *dst = nullptr, scale = 1.f;
+    // (the factor and the bias are on their way during the sum)
+    if (row_scale) scale = row_scale[row];
+    if (ROWS == kRowsSegments && col < n) dst = pf_quad_of(out, col, ld, bias);
     float4v s = splitk_sum(partials, (row * n_ld + col) * 4u, stride, splits);
-    if (row_scale) s *= row_scale[row];  // (f32 rows scaled into the f16 range)
+    if (row_scale) s *= scale;  // (f32 rows scaled into the f16 range)
     if constexpr (ROWS == kRowsPlain) {
         if (col < n) *(float4v *)(out.seg[0].ptr + (size_t)row * n + col) = s;
     } else if constexpr (ROWS == kRowsSegments) {
-        uint32_t ld = 0;
-        float4v bias = {0.f, 0.f, 0.f, 0.f};
-        float *dst = col < n ? pf_quad_of(out, col, ld, bias) : nullptr;
         if (out.seg[0].bias) s += bias;
         if (dst) *(float4v *)(dst + (size_t)row * ld) = s;
     } else {
@@ -62,15 +78,15 @@ __global__ __launch_bounds__(BLOCK) void k_splitk_reduce(const float *__restrict
 // (32 columns apart) in split order and stores silu(gate) * up.
 template <uint32_t BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_splitk_reduce_swiglu(const float *__restrict__ partials, uint32_t n_ld, uint32_t splits, uint32_t stride,
-                                                                uint32_t ffn, const float *__restrict__ row_scale, uint32_t row0,
+                                                                uint32_t ffn, const float *__restrict__ row_scale, uint32_t m_rows,
                                                                 uint32_t act, float *__restrict__ gate_out)
 {
-    const uint32_t feat = (blockIdx.x * BLOCK + threadIdx.x) * 4u, row = row0 + blockIdx.y;
-    if (feat >= ffn) return;   // (ffn is a multiple of 32)
+    const uint32_t idx = blockIdx.x * BLOCK + threadIdx.x, quads = ffn / 4u, row = idx / quads, feat = (idx - row * quads) * 4u;   // (ffn is a multiple of 32)
+    if (row >= m_rows) return;
     const uint32_t at = (row * n_ld + paired_col(feat)) * 4u;
+    const float scale = row_scale ? row_scale[row] : 1.f;
     float4v g = splitk_sum(partials, at, stride, splits), u = splitk_sum(partials, at + kPairWidth * 4u, stride, splits);
     if (row_scale) {
-        const float scale = row_scale[row];
         g *= scale;
         u *= scale;
     }
@@ -94,11 +110,9 @@ hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutS
     auto plain = rows == kRowsPlain      ? (few ? k_splitk_reduce<kRowsPlain, 64> : k_splitk_reduce<kRowsPlain, 256>)
                  : rows == kRowsSegments ? (few ? k_splitk_reduce<kRowsSegments, 64> : k_splitk_reduce<kRowsSegments, 256>)
                                          : (few ? k_splitk_reduce<kRowsNone, 64> : k_splitk_reduce<kRowsNone, 256>);
-    for (uint32_t row0 = 0; row0 < m; row0 += 65535u) {   // (the most rows of a grid)
-        const dim3 grid((quads + block - 1) / block, m - row0 < 65535u ? m - row0 : 65535u);
-        if (out.swiglu) hipLaunchKernelGGL(gated, grid, dim3(block), 0, s, partials, n_ld, splits, stride, n / 2, out.row_scale, row0, out.gate_act, out.swiglu);
-        else hipLaunchKernelGGL(plain, grid, dim3(block), 0, s, partials, n_ld, splits, stride, n, out.row_scale, row0, out);
-    }
+    const dim3 grid((unsigned)(((uint64_t)m * quads + block - 1) / block));
+    if (out.swiglu) hipLaunchKernelGGL(gated, grid, dim3(block), 0, s, partials, n_ld, splits, stride, n / 2, out.row_scale, m, out.gate_act, out.swiglu);
+    else hipLaunchKernelGGL(plain, grid, dim3(block), 0, s, partials, n_ld, splits, stride, n, out.row_scale, m, out);
     return hipGetLastError();
 }
 

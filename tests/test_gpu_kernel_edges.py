@@ -187,8 +187,8 @@ def test_split_sums_of_every_count(dev, m, n, splits):
 
 
 @pytest.mark.parametrize("m,splits", [(24, 10), (24, 18), (40, 17), (65576, 2)])
-def test_split_sums_past_eight_in_flight_and_past_the_rows_of_a_grid(dev, m, splits):
-    # the sum kernel has eight loads in flight behind the first; more than 65535 rows are two launches
+def test_split_sums_past_eight_in_flight_and_of_many_rows(dev, m, splits):
+    # the sum kernel has eight loads in flight behind the first, then what is left; one-wave and four-wave workgroups, rows of 32 quads
     k, n = splits * 128, 72
     packed, scales, w = weight(dev, k, n, 930 + splits)
     a16 = O.synth_act_f16(m, k, 931 + splits)
