@@ -15,7 +15,10 @@
 // * two k-slices of four waves beside each other; per group the wave reads the rows' operands once for its two or four tiles;
 //   a unit's scaling and the next one's unpack stand between its matrix instructions (a v_mfma_f32_16x16x32 leaves the vector unit
 //   two of its four issue slots: four in a row with the seventeen vector instructions behind them take 114 cycles, spread 104).
-// What is left: the partial sums (17 x 32 x 3584 floats in the example), written and read back by k_splitk_reduce, 4.7 of 22.3 us.
+// The rounding error of the sums is that of the kernels before or less (a chunk's four groups are summed first, the ranges by
+// pairs: 18944 -> 3584 at 32 rows 1.14e-7 of the result against 64 bits, k_waves_exact 1.14e-7; at 8 rows 1.06e-7 and 1.23e-7; with one
+// chain each 1.33e-7 and 1.36e-7).
+// What is left: the partial sums (17 x 32 x 3584 floats in the example), written and read back by k_splitk_reduce, 4.7 of 22.7 us.
 #include "twm_waves_core.h"
 
 #include <type_traits>
@@ -199,14 +202,18 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
     };
     // A unit is a group of a tile.  Its MFMAs are followed by the scaling of the unit before and the unpack of the next one,
     // so that no vector instruction waits for the matrix pipe.
-    float4v d[2][MT];
+    // (a chunk's four groups are summed first: one long chain of additions would double the rounding error of the sum)
+    float4v d[2][MT], sum[MT][NT];
     float scale = 0.f;
     half8 bf;
     auto scaled = [&](int u, int t) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) acc[mt][t][r] += d[u & 1][mt][r] * scale;
+            for (int r = 0; r < 4; r++) {
+                sum[mt][t][r] = u < NT ? d[u & 1][mt][r] * scale : __builtin_fmaf(d[u & 1][mt][r], scale, sum[mt][t][r]);
+                if (u >= 3 * NT) acc[mt][t][r] += sum[mt][t][r];
+            }
     };
     auto step = [&](int slot, uint32_t i) {
         bf = we_unpack(wq[slot][0][0], dq);
@@ -331,10 +338,10 @@ hipError_t init_batch_range()
 // How many K-ranges a GEMM is cut into (0: another form runs): one round of workgroups, each with as many chunks as its staging
 // takes, or fewer where the round fills the CUs with them.  Lines from random calls, 5 .. 32 f32 rows on 60 .. 600 column tiles,
 // K of 3000 .. 24000 (us, k_waves_exact or above 160 chunks k_batch / this kernel):
-// * 17 .. 32 rows: from a work of 21500 tiles times chunks on, gated 26500 (18944 -> 3584 at 32 rows 26.6 / 22.3, 8192 -> 8192 at
+// * 17 .. 32 rows: from a work of 21500 tiles times chunks on, gated 26500 (18944 -> 3584 at 32 rows 26.6 / 22.7, 8192 -> 8192 at
 //   17 21.6 / 19.1, 12672 -> 5824 at 17 25.6 / 20.5; below, 7296 -> 4608 at 28 rows gains 1 %, 4608 -> 5120 at 32 is 13.6 / 15.8),
 //   and above 160 chunks, where k_waves_exact ends, from 72 tiles on (22656 -> 1344 at 32 rows 23.3 / 17.2);
-// * up to sixteen rows: 108 .. 360 tiles and a work of 19000 (18944 -> 3584 at 8 rows 15.9 / 13.7, 11008 -> 4096 at 13 15.0 / 12.9,
+// * up to sixteen rows: 108 .. 360 tiles and a work of 19000 (18944 -> 3584 at 8 rows 15.9 / 13.9, 11008 -> 4096 at 13 15.0 / 12.9,
 //   14336 -> 4096 at 16 16.3 / 15.1; 84 tiles at a work of 13000 - 15000 8 % behind, 440 .. 520 tiles, where k_waves_exact does not
 //   cut K, 0 - 25 %; 13824 -> 5120 at 16 rows, 320 tiles, level), and not gated: the kernel that adds the ranges reads twice the
 //   sums per value (0.92 .. 1.13 of the time).
