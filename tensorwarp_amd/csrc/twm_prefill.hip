@@ -357,7 +357,7 @@ __device__ __forceinline__ void prefill_block(const uint4v *__restrict__ qw, con
         return;
     }
     if (partials) {
-        // split-K: plain [split][row][padded column] partial sums, added up in split order by k_splitk_reduce
+        // split-K: plain [split][row][padded column] partial sums, added up by k_splitk_reduce
         const uint32_t n_ld = n_tiles * 16u;
         float *dst = partials + ((size_t)blockIdx.z * m_rows) * n_ld;
 #pragma unroll

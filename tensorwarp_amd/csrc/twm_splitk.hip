@@ -80,7 +80,7 @@ __global__ __launch_bounds__(BLOCK) void k_splitk_reduce(const float *__restrict
 }
 
 // The same sum for a paired gate/up weight: one thread per four features adds the gate and the up partials
-// (32 columns apart) in split order and stores silu(gate) * up.
+// (32 columns apart) and stores silu(gate) * up.
 template <uint32_t BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_splitk_reduce_swiglu(const float *__restrict__ partials, uint32_t n_ld, uint32_t splits, uint32_t stride,
                                                                 uint32_t ffn, const float *__restrict__ row_scale, uint32_t m_rows,
