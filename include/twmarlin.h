@@ -347,8 +347,8 @@ int twm_weight_dequant_f16(twm_ctx *ctx, const twm_weight *w, uint16_t *out_kn_d
  * Up to M = 32 f32 activations enter as two f16 terms, a first term and the residual, about 21 bits.  Any finite f32
  * row is taken, as by the reference's kernels, which multiply in f32 (quantize.rs:1188, 186-246): values beyond the f16
  * range, and rows too small for it, are scaled by a power of two first and the sums back, both exact -- per stretch of
- * a row inside the kernels up to M = 32, except that from M = 5 on some forms (wide or shallow matrices, very deep ones at
- * M = 17 .. 32) have it done per row by a conversion kernel ahead of the GEMM.
+ * a row (128 values from M = 5 on) inside the kernels up to M = 32, except that from M = 5 on some forms (wide or shallow
+ * matrices, some very deep ones at M = 17 .. 32) have it done per row by a conversion kernel ahead of the GEMM.
  * M  > 32: prefill GEMM on the FP16 Q4 unpack (the arithmetic of the reference's FP16 route, DequantizedF16Weights +
  *          HGEMM, quantize.rs:620-670).  f32 activations are scaled per row in the same way and then rounded to ONE f16
  *          term: a deviation from gemm_q4_0 (quantize.rs:1825-1858), which multiplies f32 A by f32 weights -- about

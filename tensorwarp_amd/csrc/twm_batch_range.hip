@@ -2,8 +2,10 @@
 //
 // Semantics: those of k_waves_exact (twm_waves_exact.hip; crates/kernels/src/quantize.rs:1219-1238): per 32-deep group the
 // products a * (q - 8) are summed in f32 by MFMA, the group sum is scaled once by f32(scale) and added to the running f32 sum; f32
-// rows enter as two f16 terms, with a power of two per row and k-slice (up to nine chunks) that brings the row's largest
-// magnitude there to [2^13, 2^14), exactly undone on the slice's sums.
+// rows enter as two f16 terms, with a power of two per row and 128-deep chunk that brings the row's largest magnitude there to
+// [2^13, 2^14), exactly undone on the chunk's sums.  (One per row and k-slice, up to nine chunks, was no faster -- 18944 -> 3584 at 8
+// rows 13.8, now 13.9 us, at 32 23.2 and 23.0 -- and a value far above its neighbours took the bits of 1151 of them instead of 127: with
+// one of 1e6 in each of 8 rows the columns where its weight is 0 were 2.87e-7 off the 64-bit product, now 1.38e-7, k_waves_exact 1.53e-7.)
 //
 // What bounds these launches: each workgroup of k_waves_exact converts every row of its K-range itself, for one to four column
 // tiles, and fetches 4 bytes per value for them (18944 -> 3584 at 32 rows: 56 column groups, 136 MB from L2 for 38 MB of weights,
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
         for (int t = 0; t < NT; t++) load_b(s, t, (uint32_t)s);
     __builtin_amdgcn_sched_barrier(0);
 
-    float *factors = (float *)(lds_all + chunks_per_split * kChunk);   // [k-slice][16 MT]
+    float *factors = (float *)(lds_all + chunks_per_split * kChunk);   // [chunk][16 MT]
 #pragma unroll
     for (uint32_t i = 0; i < UNITS; i++) {
         uint32_t quad, of, at, n;
@@ -153,14 +155,10 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
                 }
             }
         }
-        float largest = 0.f;
-#pragma unroll
-        for (uint32_t j = 0; j < kSlice; j++)
-            if (j < n) largest = fmaxf(largest, we_max8(ar[i][j][0], ar[i][j][1]));
-        const WeFactor factor = we_factor(row16_max(largest));
 #pragma unroll
         for (uint32_t j = 0; j < kSlice; j++) {
             if (j < n) {
+                const WeFactor factor = we_factor(row16_max(we_max8(ar[i][j][0], ar[i][j][1])));
                 _Float16 *dst = lds_all + (at + j) * kChunk;
 #pragma unroll
                 for (int l = 0; l < 2; l++) {
@@ -173,12 +171,12 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
                     else
                         *(uint2v *)(dst + kTile + row * kWeRow + ((vec ^ (row & 15u)) * 8u) + (p & 1u) * 4u) = lo;
                 }
+                if (p == 0) {
+                    float *f = factors + (at + j) * 16u * MT;
+                    f[row] = factor.back;
+                    if (MODE == kRowsF32Few) f[row + 8u] = factor.back;
+                }
             }
-        }
-        if (p == 0 && n != 0) {
-            float *f = factors + of * 16u * MT;
-            f[row] = factor.back;
-            if (MODE == kRowsF32Few) f[row + 8u] = factor.back;
         }
     }
     __syncthreads();
@@ -202,8 +200,9 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
     };
     // A unit is a group of a tile.  Its MFMAs are followed by the scaling of the unit before and the unpack of the next one,
     // so that no vector instruction waits for the matrix pipe.
-    // (a chunk's four groups are summed first: one long chain of additions would double the rounding error of the sum)
-    float4v d[2][MT], sum[MT][NT];
+    // (a chunk's four groups are summed first, its factors taken back on their sum: one long chain of additions would double the
+    // rounding error)
+    float4v d[2][MT], sum[MT][NT], back[MT];
     float scale = 0.f;
     half8 bf;
     auto scaled = [&](int u, int t) {
@@ -212,7 +211,7 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 sum[mt][t][r] = u < NT ? d[u & 1][mt][r] * scale : __builtin_fmaf(d[u & 1][mt][r], scale, sum[mt][t][r]);
-                if (u >= 3 * NT) acc[mt][t][r] += sum[mt][t][r];
+                if (u >= 3 * NT) acc[mt][t][r] = __builtin_fmaf(sum[mt][t][r], back[mt][r], acc[mt][t][r]);
             }
     };
     auto step = [&](int slot, uint32_t i) {
@@ -221,6 +220,10 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
         for (int u = 0; u < 4 * NT; u++) {
             const int g = u / NT, t = u % NT;
             if (t == 0) load_a((g + 1) & 1, g == 3 ? i + 1u : i, (g + 1) & 3);
+            if (u == 2 * NT) {
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) back[mt] = *(const float4v *)(factors + (base + i) * 16u * MT + 16 * mt + 4u * kb);
+            }
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) d[u & 1][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[g & 1][0][mt], bf, float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
             if constexpr (TERMS == 2) {
@@ -253,12 +256,6 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
 #pragma unroll
             for (int s = 0; s < SLOTS; s++)
                 if (i + s < count) step(s, i + s);
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const float4v back = *(const float4v *)(factors + slice * 16u * MT + 16 * mt + 4u * kb);
-#pragma unroll
-            for (int t = 0; t < NT; t++) acc[mt][t] *= back;
         }
     }
     __syncthreads();
@@ -293,16 +290,11 @@ namespace {
 
 template <int MT, int MODE, int NT> struct BatchRange {
     static constexpr uint32_t tiles = COLS * NT;   // 16-column tiles of a workgroup
-    static constexpr size_t chunk = (MODE == kRowsF32 ? 2 : 1) * 16 * MT * kWeRow * sizeof(_Float16);
-    static constexpr size_t factors = KS * 16 * MT * sizeof(float);
+    static constexpr size_t chunk = (MODE == kRowsF32 ? 2 : 1) * 16 * MT * kWeRow * sizeof(_Float16) + 16 * MT * sizeof(float);   // staged values and factors
     static constexpr size_t sums = (size_t)KS * 16 * MT * (tiles * 16 + 4) * sizeof(float);
     static constexpr size_t most = 160 * 1024;
-    static constexpr uint32_t max_chunks = (most - factors) / chunk < KS * range_slice(NT) ? (uint32_t)((most - factors) / chunk) : KS * range_slice(NT);
-    static size_t lds(uint32_t cps)
-    {
-        const size_t staging = cps * chunk + factors;
-        return staging > sums ? staging : sums;
-    }
+    static constexpr uint32_t max_chunks = most / chunk < KS * range_slice(NT) ? (uint32_t)(most / chunk) : KS * range_slice(NT);
+    static size_t lds(uint32_t cps) { return cps * chunk > sums ? cps * chunk : sums; }
     static hipError_t init()
     {
         return hipFuncSetAttribute((const void *)k_batch_range<MT, MODE, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds(max_chunks));

@@ -974,6 +974,26 @@ def test_ranges_staged_at_once(dev, m):
     w.free()
 
 
+@pytest.mark.parametrize("m", [5, 8, 16, 17, 32])
+def test_large_values_of_other_chunks_take_no_bits_in_ranges_staged_at_once(dev, m):
+    # f32 rows of k_batch_range: every fourth chunk holds a 2^40 alone, on weights of 0 in the first half of the columns; there the
+    # results are the other chunks' sums, whose values keep their bits
+    k, n = (20512, 1157) if m > 16 else (22624, 1725)
+    assert "k_batch_range" in dev.plan(k, n, m, dtype="f32")
+    half, packed, scales = n // 2, O.synth_packed(k, n, 1721).reshape(k // 32, n, 16), O.synth_scales(k, n, 1722)
+    a = O.synth_normal_f32(m * k, 1723 + m).reshape(m, k).copy()
+    for c in range(1, k // 128, 4):
+        a[:, 128 * c: 128 * (c + 1)] = 0
+        a[:, 128 * c + 32 + c % 32] = np.float32(2.0 ** 40)
+        packed[4 * c + 1, :half] = 0x88                           # (the group that holds it)
+    truth = O.gemm_f64(a, packed, scales, m, k, n)
+    w = T.MarlinWeight.upload(dev, packed, scales, k, n)
+    c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+    T.gemm(dev, w, T.GpuTensor.from_host(dev, a), m, c)
+    close_rows(c.to_host()[:, :half], truth[:, :half], F32_SUM)
+    w.free()
+
+
 def test_ranges_staged_at_once_under_a_gate(dev):
     m, k, ffn = 23, 20256, 1344
     assert "k_batch_range" in dev.plan(k, 2 * ffn, m, dtype="f32", gated=True)
