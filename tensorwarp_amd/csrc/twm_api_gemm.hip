@@ -268,7 +268,8 @@ static LaunchForm choose_form(const FormEnv &e, uint32_t n_tiles, uint32_t k_chu
         // little slower (3584 -> 3584 at 16 rows 7.4 us, k_waves_exact 5.4), but the tile copy would be a second allocation of
         // the weight's size, and inside a graph capture a refusal.
         if (!(copies & kCopyTile) && !a_f32 && m <= 16 && (plan_gemv4_sub_rows(tiles64, k_chunks).sub || (m <= 8 && tiles64 > 128))) wp.nt = 0;
-        if (const uint32_t ranges = (copies & kCopyTile) ? plan_batch_range(n_tiles, k_chunks, m, a_f32, gated, e.ws_bytes) : 0u) {
+        // (whichever copies the handle holds: all forms for five and more f32 rows read the tile copy)
+        if (const uint32_t ranges = plan_batch_range(n_tiles, k_chunks, m, a_f32, gated, e.ws_bytes)) {
             f.kind = kFormBatchRange;
             f.copy = kCopyTile;
             f.splits = ranges;

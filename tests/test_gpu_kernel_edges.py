@@ -994,6 +994,27 @@ def test_large_values_of_other_chunks_take_no_bits_in_ranges_staged_at_once(dev,
     w.free()
 
 
+@pytest.mark.parametrize("k,n,m", [(22624, 1725, 8), (22624, 1725, 16), (20512, 1157, 20)])
+def test_f32_rows_run_alike_whichever_copy_a_handle_holds(dev, k, n, m):
+    # k_batch_range on a handle of the column-lane copy alone: the first call, which builds the tile copy, is the launch of every
+    # later one
+    assert "k_batch_range" in dev.plan(k, n, m, dtype="f32")
+    packed, scales, both = weight(dev, k, n, 1790)
+    dev.set_option("weight_copies", T.MarlinWeight.COPY_COLUMN_LANE)
+    one = T.MarlinWeight.upload(dev, packed, scales, k, n)
+    dev.set_option("weight_copies", 0)
+    a = T.GpuTensor.from_host(dev, O.synth_normal_f32(m * k, 1791).reshape(m, k))
+    got = []
+    for w in (both, one, one):
+        c = T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+        T.gemm(dev, w, a, m, c)
+        got.append(c.to_host().view(np.uint32))
+    assert one.copies == 3
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    both.free()
+    one.free()
+
+
 def test_ranges_staged_at_once_under_a_gate(dev):
     m, k, ffn = 23, 20256, 1344
     assert "k_batch_range" in dev.plan(k, 2 * ffn, m, dtype="f32", gated=True)
