@@ -476,8 +476,8 @@ int twm_plan_describe(const twm_ctx *ctx, uint32_t k, uint32_t n, uint32_t m, in
                  f.splits == 1 ? "" : "s", f.splits > 1 ? " + k_splitk_reduce" : "");
         break;
     case kFormBatchRange:
-        snprintf(text, bytes, "k_batch: 1 quad per workgroup, %u tiles per wave, 2 k-slices, a range's rows staged at once (k_batch_range), %u K-splits + k_splitk_reduce; 16-column tile copy",
-                 m <= 16 ? 2u : 4u, f.splits);
+        snprintf(text, bytes, "k_batch_range: %u-row x %u-column blocks, ranges of up to %u chunks staged at once, %u K-splits + k_splitk_reduce; 16-column tile copy",
+                 m <= 8 ? 8u : m <= 16 ? 16u : 32u, batch_range_columns(m), (k_chunks + f.splits - 1) / f.splits, f.splits);
         break;
     case kFormStream: {
         const uint32_t sp = plan_stream(n_tiles, k_chunks, mb);

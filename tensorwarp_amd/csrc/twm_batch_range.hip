@@ -354,7 +354,12 @@ uint32_t plan_batch_range(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool 
     return splits;
 }
 
-// 1 .. 32 rows; splits >= 1 K-ranges of at most slab_max_chunks() chunks, their sums in `scratch`.
+uint32_t batch_range_columns(uint32_t m)
+{
+    return 16 * range_form(m, [](auto form) { return decltype(form)::tiles; });
+}
+
+// 1 .. 32 rows; splits >= 1 K-ranges of at most BatchRange::max_chunks chunks, their sums in `scratch`.
 hipError_t launch_batch_range(hipStream_t s, const WeightView &w, const float *a, uint32_t m, const OutSpec &out, uint32_t splits,
                               void *scratch, size_t scratch_bytes)
 {

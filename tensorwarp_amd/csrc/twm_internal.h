@@ -184,8 +184,9 @@ hipError_t launch_waves_exact(hipStream_t s, const WeightView &w, const void *a,
 hipError_t launch_waves(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out, uint32_t nt,
                         uint32_t waves, uint32_t splits, void *scratch, size_t scratch_bytes);
 // 5 .. 32 f32 rows on deep, narrow matrices, exact weights: K-ranges whose rows a workgroup stages at once (twm_batch_range.hip);
-// plan_batch_range: the number of ranges (0: another form runs)
+// plan_batch_range: the number of ranges (0: another form runs); batch_range_columns: columns per workgroup
 uint32_t plan_batch_range(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool a_f32, bool gated, size_t scratch_bytes);
+uint32_t batch_range_columns(uint32_t m);
 hipError_t launch_batch_range(hipStream_t s, const WeightView &w, const float *a, uint32_t m, const OutSpec &out, uint32_t splits,
                               void *scratch, size_t scratch_bytes);
 hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out,

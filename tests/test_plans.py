@@ -51,7 +51,7 @@ def workgroups(f, k, n, m):
         return -(-(n_pad // 64) // (f["quads"] * f["tiles_per_wave"])) * f["splits"]
     if f["kernel"] == "k_stream":
         return n_pad // 64 * f["splits"]
-    if f["kernel"] in ("k_prefill", "k_waves", "k_waves_exact"):
+    if f["kernel"] in ("k_prefill", "k_waves", "k_waves_exact", "k_batch_range"):
         return -(-m // f["block_rows"]) * -(-n_pad // f["block_cols"]) * f["splits"]
     raise AssertionError(f["text"])
 
@@ -209,6 +209,30 @@ def test_plans_of_the_few_row_kernels(lib):
             continue
         seen[f["kernel"]] += 1
     assert min(seen.values()) >= 400, seen
+
+
+def test_plans_of_ranges_staged_at_once(lib):
+    # k_batch_range: 5 .. 32 f32 rows, one round of workgroups that keeps at least 70 % of the CUs busy, no more chunks than a
+    # workgroup's LDS holds, the partial sums within the default scratch; gated only from 17 rows on
+    rng = np.random.default_rng(17)
+    seen = {8: 0, 16: 0, 32: 0}
+    for _ in range(6000):
+        k, n = 32 * int(rng.integers(100, 900)), int(rng.integers(900, 10000))
+        m, gated = int(rng.integers(4, 35)), int(rng.integers(0, 2))
+        n = n // 64 * 64 + 64 if gated else n
+        assert not describe(lib, k, n, m, _lib.F16, gated).startswith("k_batch_range"), (k, n, m)
+        f = parse(describe(lib, k, n, m, _lib.F32, gated))
+        if f["kernel"] != "k_batch_range":
+            continue
+        rows, k_chunks, wgs = f["block_rows"], (k // 32 + 3) // 4, workgroups(f, k, n, m)
+        assert 5 <= m <= 32 and rows == (8 if m <= 8 else 16 if m <= 16 else 32) and not (gated and m <= 16), f["text"]
+        assert f["copy"] == "16-column tile copy" and "+ k_splitk_reduce" in f["text"], f["text"]
+        assert f["block_cols"] == (128 if m <= 16 else 256) and f["chunks"] <= (18 if m <= 16 else 9), f["text"]
+        assert f["splits"] >= 2 and (f["splits"] - 1) * f["chunks"] < k_chunks <= f["splits"] * f["chunks"], f["text"]
+        assert wgs <= CUS and 10 * k_chunks * ((n + 63) // 64 * 64) >= 7 * CUS * f["chunks"] * f["block_cols"], f["text"]
+        assert f["splits"] * m * ((n + 63) // 64 * 64) * 4 <= 256 << 20, f["text"]
+        seen[rows] += 1
+    assert min(seen.values()) >= 25, seen
 
 
 @pytest.mark.parametrize("k,n,m,dtype,gated", [(1152, 33728, 19, "f16", 0), (1664, 24966, 9, "f16", 0), (1152, 38272, 9, "f16", 0), (1792, 26560, 14, "f16", 0),
