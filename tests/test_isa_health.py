@@ -1,7 +1,7 @@
 """What the compiler made of the kernels whose speed hangs on its instruction scheduling and register allocation, checked
 on the CPU from the gfx950 assembly: no register spills, and no prefetch moved down to its first use.
 
-k_batch and k_prefill keep several chunks of loads in flight; their source pins every prefetch in place, but the
+k_batch, k_batch_range and k_prefill keep several chunks of loads in flight; their source pins every prefetch in place, but the
 compiler's choices move with unrelated code (a multiply added to k_batch's store loops once moved the main loop's weight
 loads of one instantiation down to their use, each followed by a wait for everything in flight: 19.2 -> 22.3 us on
 3584 -> 37888 at 16 rows; the same multiply in k_prefill's store made its 128 x 256 form spill and run six times
@@ -18,7 +18,8 @@ import pytest
 from tensorwarp_amd import build
 
 CSRC = build.CSRC
-FILES = ["twm_batch.hip", "twm_prefill.hip", "twm_gemv4s.hip", "twm_gemv4g.hip", "twm_moe.hip", "twm_waves.hip", "twm_waves_exact.hip"]
+FILES = ["twm_batch.hip", "twm_prefill.hip", "twm_gemv4s.hip", "twm_gemv4g.hip", "twm_moe.hip", "twm_waves.hip", "twm_waves_exact.hip", "twm_batch_range.hip",
+         "twm_splitk.hip"]
 # The sub-tile kernel's looping forms with many rows (and with four f32 rows on 16 columns) run out of registers with
 # two register sets live.  No planner chooses them (five rows and up run only where one pass per wave covers K; f32
 # rows on a deep K take 32 columns or whole tiles); only the option knobs reach them, and the parity tests do.
@@ -52,6 +53,10 @@ def kernels():
 
 def test_no_kernel_spills(kernels):
     assert len(kernels) > 80
+    # every file's kernels are among them: one that moves to another file takes its check along
+    for kernel, forms in (("k_batch", 10), ("k_prefill", 10), ("k_prefill192", 4), ("k_gemv4s", 20), ("k_gemv4g", 4), ("k_bank_gemv", 20), ("k_bank_down_axpy", 2),
+                          ("k_waves", 4), ("k_waves_exact", 60), ("k_batch_range", 3), ("k_splitk_reduce", 6), ("k_splitk_reduce_swiglu", 2)):
+        assert sum("%d%sI" % (len(kernel), kernel) in name for name in kernels) >= forms, kernel
     spilled = {name: scratch for name, (body, scratch) in kernels.items() if scratch and not any(f in name for f in FORCED_ONLY_SPILLS)}
     assert not spilled, spilled
 
@@ -61,7 +66,7 @@ def test_no_prefetch_was_moved_down_to_its_use(kernels):
     pattern = re.compile(r"(?:global_load_dwordx[24]|global_load_lds_dwordx4) [^\n]*\n\s*s_waitcnt vmcnt\(0\)")
     checked = 0
     for name, (body, _) in kernels.items():
-        if "7k_batchI" in name or "9k_prefillILi8ELi4ELb0E" in name or "9k_prefillILi4E" in name or "12k_prefill192I" in name:
+        if "7k_batchI" in name or "9k_prefillILi8ELi4ELb0E" in name or "9k_prefillILi4E" in name or "12k_prefill192I" in name or "13k_batch_rangeI" in name:
             checked += 1
             assert not pattern.search(body), name
     assert checked >= 40
