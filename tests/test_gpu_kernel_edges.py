@@ -994,6 +994,45 @@ def test_large_values_of_other_chunks_take_no_bits_in_ranges_staged_at_once(dev,
     w.free()
 
 
+@pytest.mark.parametrize("m,k,n,gated,chunks,splits", [(8, 39712, 1707, False, 18, 18), (5, 32800, 1835, False, 16, 17), (16, 39712, 1707, False, 18, 18),
+                                                       (13, 32800, 1835, False, 16, 17), (32, 43936, 1323, False, 9, 39), (20, 43808, 1323, False, 9, 39),
+                                                       (17, 43680, 1323, False, 9, 38), (27, 43808, 1344, True, 9, 39)])
+def test_ranges_of_as_many_chunks_as_a_workgroup_stages(dev, m, k, n, gated, chunks, splits):
+    # k_batch_range: the longest ranges, 147 KB of staged rows, and last ranges of all chunks, two and one (whose second k-slice is
+    # empty) with a K that ends inside them; f32 values with a second term.  The sums of a range's chunks are a chain of up to nine
+    # additions, those of the ranges a tree: 1.0 - 1.3e-7 of a row's norm (a lost second term would be 1e-4)
+    assert dev.plan(k, n, m, dtype="f32", gated=gated).startswith("k_batch_range: ")
+    assert "ranges of up to %d chunks staged at once, %d K-splits" % (chunks, splits) in dev.plan(k, n, m, dtype="f32", gated=gated)
+    a = O.synth_normal_f32(m * k, 1803 + m).reshape(m, k) * np.float32(0.3)
+    rows = T.GpuTensor.from_host(dev, a)
+    if gated:
+        ffn = n // 2
+        parts = [(O.synth_packed(k, ffn, s), O.synth_scales(k, ffn, s + 1)) for s in (1811, 1821)]
+        w = T.MarlinWeight.gate_up(dev, *([T.GpuTensor.from_host(dev, p), T.GpuTensor.from_host(dev, s, "f16")] for p, s in parts), k, ffn)
+        g, u = (O.gemm_f64(a, *x, m, k, ffn) for x in parts)
+        truth, c = g / (1.0 + np.exp(-g)) * u, T.GpuTensor.from_host(dev, np.full((m, ffn), np.nan, np.float32))
+        T.gemm_swiglu(dev, w, rows, m, c)
+    else:
+        packed, scales, w = weight(dev, k, n, 1801)
+        truth, c = O.gemm_f64(a, packed, scales, m, k, n), T.GpuTensor.from_host(dev, np.full((m, n), np.nan, np.float32))
+        T.gemm(dev, w, rows, m, c)
+    err = np.linalg.norm(c.to_host() - truth, axis=1) / np.linalg.norm(truth, axis=1)
+    assert err.max() < (2e-6 if gated else 1e-6), err
+    w.free()
+
+
+def test_options_that_ask_for_other_forms_get_them(dev):
+    # k_batch_range runs only where nothing is asked for
+    k, n, m = 22624, 1725, 8
+    for option, value in (("kernel", 4), ("kernel", 5), ("nt", 2), ("waves", 8), ("prefill_bm", 64)):
+        assert dev.plan(k, n, m, dtype="f32").startswith("k_batch_range: ")
+        dev.set_option(option, value)
+        try:
+            assert "k_batch_range" not in dev.plan(k, n, m, dtype="f32"), option
+        finally:
+            dev.set_option(option, 0)
+
+
 @pytest.mark.parametrize("k,n,m", [(22624, 1725, 8), (22624, 1725, 16), (20512, 1157, 20)])
 def test_f32_rows_run_alike_whichever_copy_a_handle_holds(dev, k, n, m):
     # k_batch_range on a handle of the column-lane copy alone: the first call, which builds the tile copy, is the launch of every
