@@ -492,13 +492,14 @@ __global__ __launch_bounds__(256) void k_pair_gate_up(const uint4v *__restrict__
 // first index whose value is greater than every earlier candidate, starting from -1e30 at index 0 (so
 // values <= -1e30 and NaNs are never chosen, and an empty or all-small row yields 0).
 //
-// A workgroup takes a span of 4096 columns, sixteen loads per thread in flight; of a row's several spans each leaves its
+// A workgroup takes a span of sixteen columns a thread, all loads in flight; of a row's several spans each leaves its
 // candidate in the scratch, and the workgroup that arrives last picks among them and clears the row's counter.  Bound: latency.
+// Workgroups of 512 and 1024 threads hold rows of up to 8192 and 16384 columns whole, since a hand-over costs a microsecond.
 // A value and its index are one 64-bit key, larger for a larger value and, among equal values, for the smaller index; the
 // largest of a wave's keys is found half by half, values and then indices, by DPP steps and four scalar reads.
 // (152064 columns: two launches, of 8192 columns a workgroup each merging through an LDS tree of ten steps and of one workgroup a
 // row for the candidates, 5.7 us in a graph, now 3.9; 16 rows 6.8, now 4.3; 512 rows of 32000 16.7, now 12.7.)
-constexpr uint32_t kArgmaxThreads = 256, kArgmaxEach = 16, kArgmaxSpan = kArgmaxThreads * kArgmaxEach;
+constexpr uint32_t kArgmaxEach = 16;
 constexpr uint32_t kArgmaxCounterStep = 32;   // a row's counter has a cache line of its own (16 rows in one line: 10.5 us, now 4.3)
 
 // a number that orders as the float does (-0 as 0)
@@ -527,31 +528,32 @@ __device__ __forceinline__ uint64_t wave_max_key(uint64_t key)
     return (uint64_t)hi << 32 | wave_max_u32((uint32_t)(key >> 32) == hi ? (uint32_t)key : 0u);
 }
 
-__global__ __launch_bounds__(kArgmaxThreads) void k_argmax(const float *__restrict__ in, uint32_t cols, uint32_t spans, uint64_t *__restrict__ candidates,
-                                                           unsigned *__restrict__ counters, int *__restrict__ out)
+template <uint32_t THREADS>
+__global__ __launch_bounds__(THREADS) void k_argmax(const float *__restrict__ in, uint32_t cols, uint32_t spans, uint64_t *__restrict__ candidates,
+                                                    unsigned *__restrict__ counters, int *__restrict__ out)
 {
-    constexpr uint32_t kWaves = kArgmaxThreads / 64;
+    constexpr uint32_t kWaves = THREADS / 64, kSpan = THREADS * kArgmaxEach;
     __shared__ uint64_t found[kWaves];
     __shared__ uint32_t last;
     const uint32_t row = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const float *src = in + (size_t)row * cols;
     float best = -1e30f;
     uint32_t idx = 0xFFFFFFFFu;  // "none yet"
-    for (uint64_t c0 = (uint64_t)blockIdx.y * kArgmaxSpan; c0 < cols; c0 += (uint64_t)spans * kArgmaxSpan) {
+    for (uint64_t c0 = (uint64_t)blockIdx.y * kSpan; c0 < cols; c0 += (uint64_t)spans * kSpan) {
         // past the end the last column again, under a larger index than its own
         const float *from = src + c0;
         const uint32_t most = cols - (uint32_t)c0 - 1u;
         float v[kArgmaxEach];
 #pragma unroll
         for (uint32_t j = 0; j < kArgmaxEach; j++) {
-            const uint32_t c = threadIdx.x + kArgmaxThreads * j;
+            const uint32_t c = threadIdx.x + THREADS * j;
             v[j] = from[c < most ? c : most];
         }
 #pragma unroll
         for (uint32_t j = 0; j < kArgmaxEach; j++) {  // (in increasing index order)
             if (v[j] > best) {
                 best = v[j];
-                idx = (uint32_t)c0 + threadIdx.x + kArgmaxThreads * j;
+                idx = (uint32_t)c0 + threadIdx.x + THREADS * j;
             }
         }
     }
@@ -592,12 +594,17 @@ hipError_t launch_argmax(hipStream_t s, const float *in, uint32_t rows, uint32_t
                          size_t scratch_bytes, unsigned *counters, uint32_t n_counters)
 {
     if (rows == 0) return hipSuccess;
-    uint32_t spans = (uint32_t)(((uint64_t)cols + kArgmaxSpan - 1) / kArgmaxSpan);
+    // Whole rows in one workgroup up to 16384 columns of up to 512 rows (1 x 5000 3.4 us in two spans, 2.35 whole, 1 x 16384 3.4 and
+    // 2.9, 512 x 9000 5.1 and 4.4; beyond that many rows the larger workgroups wait for room on the CUs: 600 x 9000 4.2 and 5.2)
+    const uint32_t threads = rows > 512u || cols <= 256u * kArgmaxEach || cols > 1024u * kArgmaxEach ? 256u : cols <= 512u * kArgmaxEach ? 512u : 1024u;
+    const uint32_t span = threads * kArgmaxEach;
+    uint32_t spans = (uint32_t)(((uint64_t)cols + span - 1) / span);
     // about a thousand workgroups at most: with many rows a workgroup takes several spans
     const uint32_t most = rows < 1024u ? 1024u / rows : 1u;
     if (spans > most) spans = most;
     if (spans == 0 || !scratch || !counters || (uint64_t)rows * kArgmaxCounterStep > n_counters || (size_t)rows * spans * 8 > scratch_bytes) spans = 1;
-    hipLaunchKernelGGL(k_argmax, dim3(rows, spans), dim3(kArgmaxThreads), 0, s, in, cols, spans, (uint64_t *)scratch, counters, out);
+    auto kernel = threads == 256u ? k_argmax<256> : threads == 512u ? k_argmax<512> : k_argmax<1024>;
+    hipLaunchKernelGGL(kernel, dim3(rows, spans), dim3(threads), 0, s, in, cols, spans, (uint64_t *)scratch, counters, out);
     return hipGetLastError();
 }
 

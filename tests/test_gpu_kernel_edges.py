@@ -1092,9 +1092,10 @@ def test_row_quads_of_waves_on_exact_weights(dev, m, dtype, nt):
     w.free()
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 4095), (3, 4096), (3, 4097), (2, 8193), (1, 4096 * 65 + 1), (40, 4096 * 33), (1023, 8200), (1025, 4100), (2049, 70)])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 4095), (3, 4096), (3, 4097), (2, 8193), (1, 4096 * 65 + 1), (40, 4096 * 33), (1023, 8200), (1025, 4100), (2049, 70),
+                                       (2, 8192), (512, 5000), (513, 5000), (3, 16383), (3, 16384), (2, 16385), (512, 8200), (513, 12300)])
 def test_argmax_at_the_edges_of_its_spans(dev, rows, cols):
-    # spans of 4096 columns, one or several to a workgroup; more spans than lanes merge them; ties across spans and between
+    # spans of 4096, 8192 and 16384 columns, one or several to a workgroup; more spans than lanes merge them; ties across spans and between
     # zeros of either sign, a largest value in the last column, rows without a candidate; a second call finds the counters clear
     x = np.round(O.synth_normal_f32(rows * cols, 1800 + cols).reshape(rows, cols) * 2).astype(np.float32)
     x[0, -1] = 1e9
