@@ -486,16 +486,21 @@ hipError_t init_waves_exact()
 //   rows 30.5 / 25.6, 7296 -> 2 x 5280 at 27 30.7 / 27.0); nine rows and more on three chunks at 2048 tiles (128 -> 39553 at 16
 //   rows 8.1 / 7.3);
 // * f16, up to eight rows: the lane-per-column and streaming kernels keep 513 .. 1100 tiles (896 -> 2 x 4864 4.9 / 4.2; 820 .. 1024
-//   tiles 2 - 17 % ahead) but for a deeper K on up to 820 of them (700 tiles, nine chunks and more: 0.97 of their time, 33 and more
-//   0.79 .. 0.87, gated 0.97; 33 and more on 820 0.85 .. 0.9) and 17 chunks and more above 1024, where their second round of
-//   workgroups is nearly empty (0.67 .. 0.89); 1537 .. 2048 tiles (3104 -> 28833 at 6 rows 14.1 / 12.8: eight tiles each leave the
-//   CUs 75 - 90 % full); K of 16 .. 32 chunks on 341 .. 512 tiles (gated up to 18 chunks 0.93, else level to 10 % behind; on 257 ..
-//   340 0.93 .. 0.97); and up to six rows, seven up to K = 4096, every K from 2200 on with up to 256 tiles (3584 -> 3584 at 5 rows
+//   tiles 2 - 17 % ahead) but for a deeper K on up to 820 of them (up to 700 tiles nine chunks and more: 3072 -> 8922 at 8 rows 7.2
+//   / 8.1, 8448 -> 10775 at 8 13.3 / 16.8, gated from 33 on 0.97; up to 768, three tiles each, 33 and more: 5760 -> 11678 at 6 10.7 /
+//   12.5; up to 820, four each, 49 and more: 9856 -> 12562 at 5 17.6 / 18.6, but 4640 -> 12716 at 5 11.1 / 10.6) and 17 chunks and
+//   more above 1024, where their second round of workgroups is nearly empty (0.67 .. 0.89); 1537 .. 2048 tiles (3104 -> 28833 at 6
+//   rows 14.1 / 12.8: eight tiles each leave the CUs 75 - 90 % full); K of 16 .. 32 chunks on 257 .. 512 tiles (2784 -> 4611 at 5 rows
+//   5.45 / 5.0; but gated up to 340 tiles 0.89 .. 1.01 of k_gemv4s's time, 3200 -> 2 x 2336 at 8 rows 5.8 / 6.5, and up to 18 chunks
+//   0.93); and up to six rows, seven up to K = 4096, every K from 2200 on with up to 256 tiles (3584 -> 3584 at 5 rows
 //   5.2 / 4.6) but for more than 64 chunks on up to 128 (0.75 .. 0.87 of k_stream's time), gated 2048 .. 4096 at eight rows too,
 //   where pairs of tiles are half as many workgroups (3072 -> 2 x 96 at 8 rows 4.75 / 4.24);
-// * f16, 9 .. 12 and 17 .. 24 rows, whose row blocks are not loaded whole: a few more of the shapes below (two to four chunks on
-//   513 .. 820 tiles 0.92 .. 0.95 of k_batch's time, nine to sixteen on 701 .. 820 0.91 .. 0.96, 33 and more on 1801 .. 2048 0.93 ..
-//   0.96);
+// * f16, 9 .. 12 and 17 .. 24 rows, whose row blocks are not loaded whole: a few more of the shapes below, against k_batch: three and
+//   four chunks on up to 768 tiles (512 -> 12208 at 10 rows 4.2 / 4.5, 448 -> 11338 at 21 5.1 / 5.6; three chunks 0.91 .. 1.02), two
+//   under a gate from 19 rows on (160 -> 2 x 4672 at 21 4.4 / 4.7; without one 160 -> 12385 at 24 5.2 / 4.6, and at 17 rows 160 -> 2 x
+//   6080 4.5 / 4.3), nine to sixteen on 701 .. 768 tiles (2048 -> 11391 at 9 6.5 / 7.4, 1408 -> 12134 at 21 7.1 / 8.3), up to 820
+//   under a gate and from 21 rows on (2016 -> 2 x 6464 at 21 8.9 / 10.2; but 1600 -> 12768 at 9 7.0 / 6.7), 33 and more on 1801 .. 2048
+//   (5312 -> 29504 at 12 20.3 / 22.2, 8416 -> 2 x 15328 at 24 35.9 / 41.4);
 // * f16, deep K on 129 .. 256 tiles: from 72 chunks on up to sixteen rows (12192 -> 3584 at 8 rows 11.0 / 10.0), up to 340 tiles
 //   from 67 on (9216 -> 4352 at 11 rows 10.9 / 9.8, 13600 -> 2 x 2720 at 7 14.4 / 12.9), from 65 on above (17824 -> 3584 at 17 rows
 //   16.8 / 15.6), gated from 61 on with 321 .. 400 tiles (10848 -> 2 x 2848 at 31 rows 20.0 / 17.9); f16 on a few
@@ -533,17 +538,17 @@ WavesPlan plan_waves_exact(uint32_t n_tiles, uint32_t k_chunks, uint32_t m, bool
     } else {
         if (n_tiles > (m <= 8 || m > 16 ? 2560u : 2816u)) return none;
         const bool part = (m >= 9 && m <= 12) || (m >= 17 && m <= 24);   // (a row block that is not loaded whole)
-        if (k_chunks <= 8 && n_tiles > (k_chunks > 4 ? 1024u : part && k_chunks > 1 ? 820u : 512u)) return none;
+        if (k_chunks <= 8 && n_tiles > (k_chunks > 4 ? 1024u : part && k_chunks > (gated && m > 18 ? 1u : 2u) ? 768u : 512u)) return none;
         if (n_tiles > 128 && n_tiles <= (m <= 16 ? 340u : 256u) && k_chunks > (m > 16 ? 64u : n_tiles > 256 ? 66u : 71u)) return none;
         if (gated && m > 16 && n_tiles > 320 && n_tiles <= 400 && k_chunks > 60) return none;
-        if (n_tiles > (part ? 820u : 700u) && n_tiles <= 1000 && k_chunks > 8 && k_chunks <= 16) return none;
+        if (n_tiles > (!part ? 700u : gated || m > 20 ? 820u : 768u) && n_tiles <= 1000 && k_chunks > 8 && k_chunks <= 16) return none;
         if (n_tiles > 1800 && n_tiles <= 2048 && !(part && k_chunks > 32)) return none;
         if (n_tiles > (m <= 8 && k_chunks <= 10 ? 1300u : m <= 16 ? 1536u : 1600u) && k_chunks <= 18) return none;
         if (m <= 16 && n_tiles > 960 && n_tiles <= 1024) return none;
         if (m <= 8) {
-            const bool deep = n_tiles > 1024 ? k_chunks > 16 : n_tiles <= 700 ? k_chunks > (gated ? 32u : 8u) : n_tiles <= 820 && k_chunks > 32 && !gated;
+            const bool deep = n_tiles > 1024 ? k_chunks > 16 : n_tiles <= 700 ? k_chunks > (gated ? 32u : 8u) : n_tiles <= 820 && k_chunks > (n_tiles <= 768 ? 32u : 48u) && !gated;
             if ((n_tiles > 512 && n_tiles <= 1100 && !deep) || (n_tiles > 1536 && n_tiles <= 2048)) return none;
-            if (n_tiles > 340 && n_tiles <= 512 && k_chunks >= 16 && k_chunks <= 32 && !(gated && k_chunks <= 18)) return none;
+            if (n_tiles > 256 && n_tiles <= 512 && k_chunks >= 16 && k_chunks <= 32 && !(gated && (n_tiles <= 340 || k_chunks <= 18))) return none;
             if (n_tiles <= 256 && k_chunks > 17 && (m <= 6 || (m == 7 && k_chunks <= 32)) && !(n_tiles <= 128 && k_chunks > 64)) return none;
             if (n_tiles <= 256 && gated && k_chunks >= 16 && k_chunks <= 31) return none;
         }
