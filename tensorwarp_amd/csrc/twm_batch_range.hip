@@ -121,7 +121,7 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
     __builtin_amdgcn_s_barrier();   // (no wave's weights ahead of another's activations)
     __builtin_amdgcn_sched_barrier(0);
 
-    // ---- this wave's weights: two chunks of its four tiles in flight.  Past the end every lane reads the first bytes of the wave's
+    // ---- this wave's weights: 8 / NT chunks of its NT tiles in flight.  Past the end every lane reads the first bytes of the wave's
     // first chunk instead (one line per load, never used).
     uint4v wq[SLOTS][NT];
     uint2v ws[SLOTS][NT];
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(64 * kRangeWaves) void k_batch_range(const uint4v *
     }
     __syncthreads();
 
-    // ---- the products: group after group of a chunk on the four tiles, one read of the activations for all of them
+    // ---- the products: group after group of a chunk on the NT tiles, one read of the activations for all of them
     float4v acc[MT][NT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)

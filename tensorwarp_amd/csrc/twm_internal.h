@@ -191,7 +191,8 @@ hipError_t launch_batch_range(hipStream_t s, const WeightView &w, const float *a
                               void *scratch, size_t scratch_bytes);
 hipError_t launch_prefill(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out,
                           uint32_t block_rows, uint32_t splits, void *scratch, size_t scratch_bytes);
-// out[row][col] = sum over splits (in order) of partials[split][row][col], partials rows n_ld floats wide
+// out[row][col] = sum over splits of partials[split][row][col], added by pairs in an order that their number alone decides;
+// partials rows n_ld floats wide
 hipError_t launch_splitk_reduce(hipStream_t s, const float *partials, const OutSpec &out, uint32_t m, uint32_t n,
                                 uint32_t n_ld, uint32_t splits);
 hipError_t launch_stream(hipStream_t s, const WeightView &w, const void *a, bool a_f32, uint32_t m, const OutSpec &out,
