@@ -5,30 +5,35 @@ namespace twm {
 
 namespace {
 
-// N more partial sums of one place, all loads in flight, added by pairs (a chain of additions in split order had a tenth more
-// rounding error in the whole result on seventeen splits)
-template <int N> __device__ __forceinline__ void splitk_add(float4v &s, const TWM_GLOBAL char *base, uint32_t &offset, uint32_t stride)
+// N more partial sums of P places kPairWidth columns apart, all loads in flight, added by pairs (a chain of additions in split order
+// had a tenth more rounding error in the whole result on seventeen splits)
+template <int N, int P> __device__ __forceinline__ void splitk_add(float4v (&s)[P], const TWM_GLOBAL char *base, uint32_t &offset, uint32_t stride)
 {
-    float4v v[N + 1];
-    v[0] = s;
+    float4v v[N + 1][P];
 #pragma unroll
     for (int j = 1; j <= N; j++) {
         offset += stride;
-        v[j] = *(const TWM_GLOBAL float4v *)(base + offset);
+#pragma unroll
+        for (int p = 0; p < P; p++) v[j][p] = *(const TWM_GLOBAL float4v *)(base + offset + p * kPairWidth * 4u);
     }
 #pragma unroll
-    for (int step = 1; step <= N; step *= 2)
+    for (int p = 0; p < P; p++) {
+        v[0][p] = s[p];
 #pragma unroll
-        for (int j = 0; j + step <= N; j += 2 * step) v[j] += v[j + step];
-    s = v[0];
+        for (int step = 1; step <= N; step *= 2)
+#pragma unroll
+            for (int j = 0; j + step <= N; j += 2 * step) v[j][p] += v[j + step][p];
+        s[p] = v[0][p];
+    }
 }
 
-// The partial sums of one place, added in an order that their number alone decides.  (Byte offsets: the partial sums of a launch fit the
+// The partial sums of P places, added in an order that their number alone decides.  (Byte offsets: the partial sums of a launch fit the
 // context's scratch, 256 MB.)
-__device__ __forceinline__ float4v splitk_sum(const float *partials, uint32_t offset, uint32_t stride, uint32_t splits)
+template <int P> __device__ __forceinline__ void splitk_sum(float4v (&s)[P], const float *partials, uint32_t offset, uint32_t stride, uint32_t splits)
 {
     const TWM_GLOBAL char *base = (const TWM_GLOBAL char *)partials;
-    float4v s = *(const TWM_GLOBAL float4v *)(base + offset);
+#pragma unroll
+    for (int p = 0; p < P; p++) s[p] = *(const TWM_GLOBAL float4v *)(base + offset + p * kPairWidth * 4u);
     uint32_t left = splits - 1u;
     for (; left >= 8u; left -= 8u) splitk_add<8>(s, base, offset, stride);
     switch (left) {
@@ -40,7 +45,6 @@ __device__ __forceinline__ float4v splitk_sum(const float *partials, uint32_t of
     case 6: splitk_add<6>(s, base, offset, stride); break;
     case 7: splitk_add<7>(s, base, offset, stride); break;
     }
-    return s;
 }
 
 }  // namespace
@@ -65,7 +69,9 @@ __global__ __launch_bounds__(BLOCK) void k_splitk_reduce(const float *__restrict
     // (the factor and the bias are on their way during the sum)
     if (row_scale) scale = row_scale[row];
     if (ROWS == kRowsSegments && col < n) dst = pf_quad_of(out, col, ld, bias);
-    float4v s = splitk_sum(partials, (row * n_ld + col) * 4u, stride, splits);
+    float4v sum[1];
+    splitk_sum(sum, partials, (row * n_ld + col) * 4u, stride, splits);
+    float4v s = sum[0];
     if (row_scale) s *= scale;  // (f32 rows scaled into the f16 range)
     if constexpr (ROWS == kRowsPlain) {
         if (col < n) *(float4v *)(out.seg[0].ptr + (size_t)row * n + col) = s;
@@ -80,7 +86,8 @@ __global__ __launch_bounds__(BLOCK) void k_splitk_reduce(const float *__restrict
 }
 
 // The same sum for a paired gate/up weight: one thread per four features adds the gate and the up partials
-// (32 columns apart) and stores silu(gate) * up.
+// (32 columns apart) and stores silu(gate) * up.  The loads of both places are in flight together, also the only ones of one split, which
+// f32 prompt rows under a gate come as (one place after the other cost a second latency: 160 -> 2 x 64 at 204 f32 rows 11.5, now 11.0 us).
 template <uint32_t BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_splitk_reduce_swiglu(const float *__restrict__ partials, uint32_t n_ld, uint32_t splits, uint32_t stride,
                                                                 uint32_t ffn, const float *__restrict__ row_scale, uint32_t m_rows,
@@ -90,7 +97,9 @@ __global__ __launch_bounds__(BLOCK) void k_splitk_reduce_swiglu(const float *__r
     if (row >= m_rows) return;
     const uint32_t at = (row * n_ld + paired_col(feat)) * 4u;
     const float scale = row_scale ? row_scale[row] : 1.f;
-    float4v g = splitk_sum(partials, at, stride, splits), u = splitk_sum(partials, at + kPairWidth * 4u, stride, splits);
+    float4v sum[2];
+    splitk_sum(sum, partials, at, stride, splits);
+    float4v g = sum[0], u = sum[1];
     if (row_scale) {
         g *= scale;
         u *= scale;

@@ -115,3 +115,12 @@ def test_plain_stores_of_192_column_blocks_carry_no_other_store(kernels):
         plain, segments, gate = (by_store[i] for i in range(3))
         assert "v_exp_f32" in gate and "v_exp_f32" not in plain + segments, which
         assert len(plain) < len(segments), which
+
+
+def test_the_gated_sum_has_both_places_in_flight(kernels):
+    # the gate's and the up projection's first partial sums are loaded before either is waited for
+    forms = [(name, body) for name, (body, _) in kernels.items() if "k_splitk_reduce_swiglu" in name]
+    assert len(forms) == 2
+    for name, body in forms:
+        second = [m.start() for m in re.finditer(r"global_load_dwordx4", body)][1]
+        assert "vmcnt" not in body[:second], name
