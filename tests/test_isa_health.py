@@ -118,9 +118,9 @@ def test_plain_stores_of_192_column_blocks_carry_no_other_store(kernels):
 
 
 def test_the_gated_sum_has_both_places_in_flight(kernels):
-    # the gate's and the up projection's first partial sums are loaded before either is waited for
+    # the gate's and the up projection's first partial sums are loaded before either is waited for, whatever the splits
     forms = [(name, body) for name, (body, _) in kernels.items() if "k_splitk_reduce_swiglu" in name]
     assert len(forms) == 2
     for name, body in forms:
-        second = [m.start() for m in re.finditer(r"global_load_dwordx4", body)][1]
-        assert "vmcnt" not in body[:second], name
+        first, second = [m.start() for m in re.finditer(r"global_load_dwordx4", body)][:2]
+        assert not re.search(r"vmcnt|branch|\n\.LBB", body[first:second]), name
